@@ -5,10 +5,11 @@ Artefacts (all under vq_gemm_amd/lib/):
   libvqgemm_ref.so    hipBLASLt fp16 baseline
   mfma_ceiling        stand-alone program: what a register-only MFMA loop sustains on the device
   launch_floor        stand-alone program: what an empty kernel costs per launch in a replayed graph
+  vq_gemm_torch_ops.so the torch operators (torch.ops.vq_gemm_amd.*) and the layers' direct calls
   vq_gemm_cuda_<k>.so one torch extension module per variant, named as the reference's
                       harness imports them (reference compile_kernels.py:55-68, bench.py:6-11)
 
-The torch modules are built from one host-only C++ file (csrc/bind.cpp) with the host
+The torch modules are built from host-only C++ files (csrc/bind.cpp, csrc/torch_ops.cpp) with the host
 compiler and linked against libvqgemm.so; no source passes through hipify.
 """
 from __future__ import annotations
@@ -174,8 +175,11 @@ def build_launch_floor(force: bool = True) -> str:
     return out
 
 
+TORCH_OPS = "vq_gemm_torch_ops"
+
+
 def build_ext(keys=None, force: bool = True, jobs: int = 6):
-    """Torch extension modules, one per variant key (host C++ only)."""
+    """Torch extension modules (host C++ only): the operators, and one module per variant key."""
     import torch  # noqa: F401  (needed for its include/lib paths)
     from torch.utils import cpp_extension as ce
 
@@ -184,32 +188,34 @@ def build_ext(keys=None, force: bool = True, jobs: int = 6):
         if k not in VARIANTS:
             raise KeyError(f"unknown kernel variant {k!r}; known: {', '.join(VARIANTS)}")
     os.makedirs(LIB_DIR, exist_ok=True)
-    src = os.path.join(CSRC, "bind.cpp")
     cxx = os.environ.get("CXX", "g++")
     torch_lib = ce.library_paths()[0]
     incs = [f"-I{p}" for p in ce.include_paths()] + [f"-I{sysconfig.get_paths()['include']}", f"-I{ROCM}/include"]
     abi = int(getattr(__import__("torch")._C, "_GLIBCXX_USE_CXX11_ABI", True))
     hdrs = _headers()
 
-    def one(k):
-        variant, is_ref = VARIANTS[k]
-        name = module_name(k)
+    def one(name, source, lib, defines):
+        src = os.path.join(CSRC, source)
         out = os.path.join(LIB_DIR, name + ".so")
         if not force and _newer(out, [src] + hdrs):
             return out
         cmd = [cxx, "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", "-Wno-unused-function",
                "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
-               f"-DTORCH_EXTENSION_NAME={name}", "-DTORCH_API_INCLUDE_EXTENSION_H", f"-DVQ_VARIANT={variant}"]
-        if is_ref:
-            cmd.append("-DVQ_REF_MODULE=1")
-        cmd += incs + [src, "-o", out, f"-L{LIB_DIR}"] + (["-lvqgemm_ref"] if is_ref else ["-lvqgemm"]) + [
+               f"-DTORCH_EXTENSION_NAME={name}", "-DTORCH_API_INCLUDE_EXTENSION_H"] + defines
+        cmd += incs + [src, "-o", out, f"-L{LIB_DIR}", f"-l{lib}",
                        f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python",
                        "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}"]
         _run(cmd)
         return out
 
+    def variant(k):
+        v, is_ref = VARIANTS[k]
+        return one(module_name(k), "bind.cpp", "vqgemm_ref" if is_ref else "vqgemm",
+                   [f"-DVQ_VARIANT={v}"] + (["-DVQ_REF_MODULE=1"] if is_ref else []))
+
     with ThreadPoolExecutor(max_workers=jobs) as ex:
-        return list(ex.map(one, keys))
+        ops = ex.submit(one, TORCH_OPS, "torch_ops.cpp", "vqgemm", [])
+        return list(ex.map(variant, keys)) + [ops.result()]
 
 
 def build_all(keys=None, force: bool = True):

@@ -10,6 +10,7 @@
 //   -DTORCH_EXTENSION_NAME=vq_gemm_cuda_<k>  -DVQ_VARIANT=<VQGEMM_VARIANT_*>  [-DVQ_REF_MODULE]
 // mirroring the reference's one-extension-per-strategy scheme (compile_kernels.py:55-68).
 #include <torch/extension.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/core/DeviceGuard.h>
 
@@ -46,6 +47,12 @@ torch::Tensor canon(const torch::Tensor &t)
     torch::Tensor c = t.contiguous();
     if ((reinterpret_cast<uintptr_t>(c.data_ptr()) & 15) != 0) c = c.clone();
     return c;
+}
+
+// fp16 [m, n] on t's device, without a dispatch
+torch::Tensor new_result(int64_t m, int64_t n, const torch::Tensor &t)
+{
+    return at::detail::empty_cuda({m, n}, at::kHalf, t.device(), c10::nullopt);
 }
 
 void *cur_stream(const torch::Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
@@ -142,7 +149,7 @@ torch::Tensor e2e_gemm(torch::Tensor input, torch::Tensor w, torch::Tensor codeb
         TORCH_CHECK(out.is_contiguous() && (reinterpret_cast<uintptr_t>(out.data_ptr()) & 15) == 0,
                     "out must be contiguous and 16-byte aligned");
     } else {
-        out = torch::empty({g.M, g.N}, input.options());
+        out = new_result(g.M, g.N, input);
     }
     check_code_range(c, g.code_bits, g.entries, cur_stream(input));
     torch::Tensor ws;
@@ -183,7 +190,7 @@ torch::Tensor gemm(torch::Tensor input, torch::Tensor w)
     TORCH_CHECK(w.device() == input.device(), "input and w must be on the same device");
     c10::DeviceGuard guard(input.device());
     torch::Tensor x = canon(input), ww = canon(w);
-    torch::Tensor out = torch::empty({input.size(0), w.size(1)}, input.options());
+    torch::Tensor out = new_result(input.size(0), w.size(1), input);
     check_rc(vqgemm_gemm_f16(x.data_ptr(), ww.data_ptr(), out.data_ptr(), input.size(0), input.size(1), w.size(1),
                              cur_stream(input)),
              "gemm");
@@ -233,7 +240,7 @@ torch::Tensor gemm(torch::Tensor input, torch::Tensor w)
     TORCH_CHECK(w.device() == input.device(), "input and w must be on the same device");
     c10::DeviceGuard guard(input.device());
     torch::Tensor x = canon(input), ww = canon(w);
-    torch::Tensor out = torch::empty({input.size(0), w.size(1)}, input.options());
+    torch::Tensor out = new_result(input.size(0), w.size(1), input);
     check_rc(vqref_gemm_f16(x.data_ptr(), ww.data_ptr(), out.data_ptr(), input.size(0), input.size(1), w.size(1),
                             /*w_is_nk=*/0, cur_stream(input)),
              "gemm (hipBLASLt)");

@@ -1,0 +1,256 @@
+// The torch operators of the package (torch.ops.vq_gemm_amd.*) and the direct calls behind its layers.  Host-only C++:
+// tensors are checked, the result is allocated with torch's allocator, raw pointers and the current stream go to the
+// C ABI of libvqgemm.so.
+//
+// A decode-size product is a kernel of three to twelve microseconds, so what surrounds the launch is what a layer call
+// costs: as a Python custom operator over ctypes it took 26 us per call on 4096 x 4096 with one row of X (the kernel:
+// 3.7).  The operators are therefore registered here, and the layers (vq_gemm_amd/nn.py) call `linear` and `gated` below
+// without going through the dispatcher at all; those two step aside (return None) whenever something else is to see
+// the call - a fake or wrapped tensor, a dispatch mode, a tracer - and the layer then calls the registered operator.
+#include <torch/extension.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/record_function.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/hip/HIPStream.h>
+
+#include "../../include/vq_gemm.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = c10::optional<Tensor>;
+
+void check_rc(int rc, const char *what)
+{
+    TORCH_CHECK(rc == 0, what, " failed with code ", rc, ": ", vqgemm_error_string(rc));
+}
+
+bool aligned16(const Tensor &t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+
+// An activation as the kernels want it: contiguous and 16-byte aligned (a view into a larger buffer may start anywhere,
+// and a copy costs far less than the scalar kernel that takes unaligned operands).
+Tensor dense(const Tensor &t)
+{
+    Tensor c = t.is_contiguous() ? t : t.contiguous();
+    return aligned16(c) ? c : c.clone();
+}
+
+// Sizes of a product, after every check that raw pointers need: types, devices, element counts.
+struct Dims {
+    int64_t M, K, N;
+    int vec, entries, books, bits;
+};
+
+Dims check_linear(const char *name, const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias,
+                  int64_t k_repeat)
+{
+    TORCH_CHECK_VALUE(codes.dim() == 2 && (codebook.dim() == 2 || codebook.dim() == 3) && x.dim() >= 1, name,
+                      ": x [..., K], codes [N, K/vec], codebook [E, vec] or [G, E, vec]");
+    const bool u8 = codes.scalar_type() == at::kByte;
+    TORCH_CHECK_VALUE(u8 || codes.scalar_type() == at::kUInt16, name, ": codes must be uint8 or uint16, got ", codes.scalar_type());
+    TORCH_CHECK_VALUE(x.scalar_type() == at::kHalf && codebook.scalar_type() == at::kHalf, name, ": x and codebook must be float16");
+    Dims d;
+    d.vec = (int)codebook.size(-1);
+    d.entries = (int)codebook.size(-2);
+    d.books = codebook.dim() == 3 ? (int)codebook.size(0) : 1;
+    d.bits = u8 ? 8 : 16;
+    d.N = codes.size(0);
+    d.K = codes.size(1) * d.vec;
+    TORCH_CHECK_VALUE(x.size(-1) * k_repeat == d.K, name, ": x has ", x.size(-1), " features, codes x vec give ", d.K, " / ", k_repeat);
+    TORCH_CHECK_VALUE(d.books > 0 && d.N % d.books == 0, name, ": rows of codes must be a multiple of the number of codebooks");
+    d.M = 1;
+    for (int64_t i = 0; i + 1 < x.dim(); i++) d.M *= x.size(i);
+    const c10::Device dev = x.device();
+    TORCH_CHECK_VALUE(dev.is_cuda() && codes.device() == dev && codebook.device() == dev, name,
+                      ": all tensors must be on one device, in GPU memory");
+    if (bias.has_value() && bias->defined())
+        TORCH_CHECK_VALUE(bias->scalar_type() == at::kHalf && bias->dim() == 1 && bias->size(0) == d.N && bias->device() == dev, name,
+                          ": bias must be a float16 tensor on x's device with one entry per output column");
+    return d;
+}
+
+Tensor new_result(const Tensor &x, int64_t columns)
+{
+    c10::SmallVector<int64_t, 6> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = columns;
+    return at::detail::empty_cuda(shape, at::kHalf, x.device(), c10::nullopt);
+}
+
+void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+// x @ W.T (+ bias), W in k_repeat stages side by side along K that all multiply the same x
+Tensor linear_impl(const Tensor &x_in, const Tensor &codes_in, const Tensor &codebook_in, const OptTensor &bias_in, int64_t k_repeat,
+                   int variant = VQGEMM_VARIANT_AUTO)
+{
+    const Dims d = check_linear("vq_linear", x_in, codes_in, codebook_in, bias_in, k_repeat);
+    const c10::OptionalDeviceGuard guard(x_in.device());
+    Tensor x = dense(x_in), codes = codes_in.contiguous(), codebook = codebook_in.contiguous(), bias;
+    if (bias_in.has_value() && bias_in->defined()) bias = bias_in->contiguous();
+    if (k_repeat > 1) {
+        c10::SmallVector<int64_t, 6> times(x.dim(), 1);
+        times.back() = k_repeat;
+        x = x.repeat(times);
+    }
+    Tensor y = new_result(x_in, d.N);
+    void *bias_p = bias.defined() ? bias.data_ptr() : nullptr;
+    void *s = stream_of(x);
+    // scratch for the shapes where the automatic choice may split K; the caching allocator hands out stream-ordered blocks
+    const int64_t need = variant == VQGEMM_VARIANT_AUTO && d.M > 16
+                             ? vqgemm_workspace_bytes_b(d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, variant) : 0;
+    int rc;
+    if (need > 0) {
+        Tensor ws = at::detail::empty_cuda({need}, at::kByte, x.device(), c10::nullopt);
+        rc = vqgemm_e2e_gemm_b_ws(x.data_ptr(), codes.data_ptr(), codebook.data_ptr(), bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec,
+                                  d.entries, d.books, d.bits, variant, ws.data_ptr(), need, s);
+    } else {
+        rc = vqgemm_e2e_gemm_b_bias(x.data_ptr(), codes.data_ptr(), codebook.data_ptr(), bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec,
+                                    d.entries, d.books, d.bits, variant, nullptr, s);
+    }
+    check_rc(rc, "vq_linear");
+    return y;
+}
+
+Tensor gated_impl(const Tensor &x_in, const Tensor &codes_in, const Tensor &codebook_in, const OptTensor &bias_in)
+{
+    const Dims d = check_linear("vq_gated_linear", x_in, codes_in, codebook_in, bias_in, 1);
+    TORCH_CHECK_VALUE(d.N % 32 == 0, "vq_gated_linear: the interleaved gate/up rows come in whole groups of 32");
+    const c10::OptionalDeviceGuard guard(x_in.device());
+    const Tensor x = dense(x_in), codes = codes_in.contiguous(), codebook = codebook_in.contiguous();
+    Tensor bias;
+    if (bias_in.has_value() && bias_in->defined()) bias = bias_in->contiguous();
+    Tensor y = new_result(x_in, d.N / 2);
+    check_rc(vqgemm_e2e_gemm_b_gated(x.data_ptr(), codes.data_ptr(), codebook.data_ptr(), bias.defined() ? bias.data_ptr() : nullptr,
+                                     y.data_ptr(), d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, VQGEMM_VARIANT_AUTO, nullptr,
+                                     stream_of(x)),
+             "vq_gated_linear");
+    return y;
+}
+
+Tensor silu_mul_impl(const Tensor &gate_up)
+{
+    TORCH_CHECK_VALUE(gate_up.scalar_type() == at::kHalf && gate_up.dim() >= 1 && gate_up.size(-1) % 2 == 0,
+                      "silu_mul: expected a float16 tensor with an even last dimension");
+    const c10::OptionalDeviceGuard guard(gate_up.device());
+    const Tensor a = gate_up.contiguous();
+    const int64_t n2 = a.size(-1), m = n2 > 0 ? a.numel() / n2 : 0;
+    Tensor y = new_result(a, n2 / 2);
+    check_rc(vqgemm_silu_mul(a.data_ptr(), y.data_ptr(), m, n2 / 2, stream_of(a)), "silu_mul");
+    return y;
+}
+
+// ---- the registered operators ---------------------------------------------------------------------------------
+
+Tensor vq_linear(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
+{
+    return linear_impl(x, codes, codebook, bias, 1);
+}
+
+Tensor vq_linear_packed(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
+{
+    return linear_impl(x, codes, codebook, bias, 1, VQGEMM_VARIANT_DECODE_PACKED);
+}
+
+// No gradient flows: an input that wants one gets a result whose backward raises.
+struct NoGradient : torch::autograd::Function<NoGradient> {
+    static Tensor forward(torch::autograd::AutogradContext *, const Tensor &y_of, const Tensor &y)
+    {
+        (void)y_of;
+        return y.view_as(y);
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *, torch::autograd::variable_list)
+    {
+        TORCH_CHECK(false, "the vector-quantised products are for inference: no backward formula is registered");
+    }
+};
+
+Tensor no_gradient(Tensor y, std::initializer_list<const Tensor *> inputs)
+{
+    if (at::GradMode::is_enabled())
+        for (const Tensor *t : inputs)
+            if (t->defined() && t->requires_grad()) return NoGradient::apply(*t, y);
+    return y;
+}
+
+// The autograd kernels call the device implementation directly: one dispatch per call instead of two.
+template <Tensor (*Impl)(const Tensor &, const Tensor &, const Tensor &, const OptTensor &)>
+Tensor with_autograd(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
+{
+    Tensor y;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        y = Impl(x, codes, codebook, bias);
+    }
+    const Tensor b = bias.has_value() ? *bias : Tensor();
+    return no_gradient(y, {&x, &codebook, &b});
+}
+
+Tensor silu_mul_autograd(const Tensor &gate_up)
+{
+    Tensor y;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        y = silu_mul_impl(gate_up);
+    }
+    return no_gradient(y, {&gate_up});
+}
+
+// ---- the layers' direct calls ---------------------------------------------------------------------------------
+
+// Whether nothing but this library is to see a call on `x`: an ordinary tensor in GPU memory, no dispatch mode, no
+// functional transform, no tracer.
+bool plain_call(const Tensor &x)
+{
+    if (!x.defined() || !x.is_cuda()) return false;
+    constexpr c10::DispatchKeySet wrappers({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::Functionalize,
+                                            c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                            c10::DispatchKey::BatchedNestedTensor, c10::DispatchKey::NestedTensor});
+    if (x.key_set().has_any(wrappers)) return false;
+    return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
+}
+
+py::object linear(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias, int64_t k_repeat)
+{
+    if (!plain_call(x)) return py::none();
+    RECORD_FUNCTION("vq_gemm_amd::vq_linear", c10::ArrayRef<const c10::IValue>());
+    return py::cast(linear_impl(x, codes, codebook, bias, k_repeat));
+}
+
+py::object gated(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
+{
+    if (!plain_call(x)) return py::none();
+    RECORD_FUNCTION("vq_gemm_amd::vq_gated_linear", c10::ArrayRef<const c10::IValue>());
+    return py::cast(gated_impl(x, codes, codebook, bias));
+}
+
+}  // namespace
+
+TORCH_LIBRARY(vq_gemm_amd, m)
+{
+    m.def("vq_linear(Tensor x, Tensor codes, Tensor codebook, Tensor? bias=None) -> Tensor");
+    m.def("vq_linear_packed(Tensor x, Tensor codes_packed, Tensor codebook, Tensor? bias=None) -> Tensor");
+    m.def("vq_gated_linear(Tensor x, Tensor codes, Tensor codebook, Tensor? bias=None) -> Tensor");
+    m.def("silu_mul(Tensor gate_up) -> Tensor");
+}
+
+TORCH_LIBRARY_IMPL(vq_gemm_amd, CUDA, m)
+{
+    m.impl("vq_linear", &vq_linear);
+    m.impl("vq_linear_packed", &vq_linear_packed);
+    m.impl("vq_gated_linear", &gated_impl);
+    m.impl("silu_mul", &silu_mul_impl);
+}
+
+TORCH_LIBRARY_IMPL(vq_gemm_amd, AutogradCUDA, m)
+{
+    m.impl("vq_linear", &with_autograd<vq_linear>);
+    m.impl("vq_linear_packed", &with_autograd<vq_linear_packed>);
+    m.impl("vq_gated_linear", &with_autograd<gated_impl>);
+    m.impl("silu_mul", &silu_mul_autograd);
+}
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
+{
+    m.def("linear", &linear, "x @ W.T (+ bias) on plain GPU tensors; None where the registered operator is to be called instead");
+    m.def("gated", &gated, "silu(gate) * up likewise");
+}

@@ -12,7 +12,7 @@ import torch
 
 from . import cabi
 from .quantize import kmeans_quantize, residual_quantize
-from .torch_ops import silu_mul, vq_gated_linear, vq_linear, vq_linear_packed
+from .torch_ops import native, silu_mul, vq_gated_linear, vq_linear, vq_linear_packed
 
 
 class VQLinear(torch.nn.Module):
@@ -90,8 +90,20 @@ class VQLinear(torch.nn.Module):
             return w
         return w.view(self.out_features, self.k_repeat, self.in_features).float().sum(dim=1).half()
 
-    @torch.no_grad()
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # Called eagerly on an ordinary GPU tensor, the layer is one native call (no dispatch, no autograd bookkeeping:
+        # what surrounds a kernel of a few microseconds is most of a decode call's time); under a tracer, a dispatch
+        # mode or torch.compile it is the registered operator.
+        if not torch.compiler.is_compiling():
+            b = self._buffers
+            if b["codes_packed"] is None:
+                y = native.linear(x, b["codes"], b["codebook"], b["bias"], self.k_repeat)
+                if y is not None:
+                    return y
+        return self._forward_op(x)
+
+    @torch.no_grad()
+    def _forward_op(self, x: torch.Tensor) -> torch.Tensor:
         if x.dtype != torch.float16 or x.shape[-1] != self.in_features:
             raise ValueError(f"expected an fp16 input with {self.in_features} features")
         if self.k_repeat > 1:
@@ -138,8 +150,16 @@ class VQGatedMLP(torch.nn.Module):
                                  None, iters, seed)
         return cls(gu, VQLinear.from_float(down, vec, entries, n_codebooks, None, iters, seed + 1), interleaved=True)
 
-    @torch.no_grad()
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if self.interleaved and not torch.compiler.is_compiling():
+            b = self.gate_up._buffers
+            h = native.gated(x, b["codes"], b["codebook"], b["bias"])
+            if h is not None:
+                return self.down(h)
+        return self._forward_op(x)
+
+    @torch.no_grad()
+    def _forward_op(self, x: torch.Tensor) -> torch.Tensor:
         if self.interleaved:
             gu = self.gate_up
             if x.dtype != torch.float16 or x.shape[-1] != gu.in_features:

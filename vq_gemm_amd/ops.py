@@ -23,23 +23,28 @@ def load_module(key: str = DEFAULT_VARIANT):
     if key not in VARIANT_KEYS:
         raise KeyError(f"unknown kernel variant {key!r}; known: {', '.join(VARIANT_KEYS)}")
     if key not in _modules:
-        name = f"vq_gemm_cuda_{key}"
-        path = os.path.join(_LIB_DIR, name + ".so")
-        if not os.path.exists(path):
-            raise ImportError(
-                f"{path} is missing: build the HIP extension first "
-                f"(python compile_kernels.py build_ext --inplace). There is no CPU fallback.")
-        spec = importlib.util.spec_from_file_location(name, path)
-        mod = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(mod)
-        _modules[key] = mod
+        _modules[key] = load_extension(f"vq_gemm_cuda_{key}")
     return _modules[key]
+
+
+def load_extension(name: str):
+    """Import the compiled extension module `name` from vq_gemm_amd/lib.  Raises if it has not been built."""
+    path = os.path.join(_LIB_DIR, name + ".so")
+    if not os.path.exists(path):
+        raise ImportError(
+            f"{path} is missing: build the HIP extension first "
+            f"(python compile_kernels.py build_ext --inplace). There is no CPU fallback.")
+    spec = importlib.util.spec_from_file_location(name, path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
 
 
 def e2e_gemm(input, w, codebook, variant: str = DEFAULT_VARIANT, out=None):
     """Fused VQ GEMM; same positional arguments as the reference's e2e_gemm.  `out` (fp16 [M,N],
     contiguous, on input's device) receives the result instead of a new tensor."""
-    return load_module(variant).e2e_gemm(input, w, codebook, out=out)
+    mod = _modules.get(variant) or load_module(variant)
+    return mod.e2e_gemm(input, w, codebook, out)
 
 
 def gemm(input, w, variant: str = DEFAULT_VARIANT):
