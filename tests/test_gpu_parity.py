@@ -1824,3 +1824,50 @@ def test_sized_workspace_entry_point_passes_the_other_variants_through():
         cabi.e2e_gemm_b_ws(x[:, :128].contiguous(), codes[:, :16].contiguous(), cb, variant=cabi.VARIANT_PREFILL_SPLITK,
                            workspace=torch.empty(1 << 20, dtype=torch.uint8, device=DEV))
     assert err.value.code == -4
+
+
+RAGGED_B = [
+    # name, M, K, N, vec, E, bits: K that ends inside a code tile or a K slice, N that ends inside a tile
+    ("shortest", 16, 192, 16, 8, 256, 8),
+    ("one_lane_load_over", 3, 320, 33, 8, 256, 8),
+    ("three_lane_loads_over", 16, 2240, 47, 8, 200, 8),
+    ("two_chunks_of_k", 5, 4160, 130, 8, 256, 8),
+    ("slabs", 70, 1088, 1000, 8, 256, 8),
+    ("many_tiles", 17, 576, 9001, 8, 256, 8),
+    ("split_k", 130, 2880, 264, 8, 256, 8),
+    ("prefill", 300, 1984, 520, 8, 256, 8),
+    ("v8_u16", 9, 448, 50, 8, 700, 16),
+    ("v4_u8", 12, 832, 61, 4, 256, 8),
+    ("v4_u16", 16, 4288, 77, 4, 4096, 16),
+]
+
+
+@pytest.mark.parametrize("row", RAGGED_B, ids=[r[0] for r in RAGGED_B])
+def test_widths_that_are_no_multiple_of_a_tile_or_a_slice(row):
+    name, M, K, N, v, E, bits = row
+    spec = ProblemSpec(name, GEOM_B, M, K, N, v, E, 1, bits, codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=81, device=DEV)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(3)).half().to(DEV)
+    want = _np(x).astype(np.float64) @ vo.dequant_b(_np(codes), _np(cb)).astype(np.float64).T
+    ran = []
+    for variant in (cabi.VARIANT_AUTO, cabi.VARIANT_DECODE, cabi.VARIANT_PREFILL, cabi.VARIANT_PREFILL_NARROW, cabi.VARIANT_PREFILL_SMALL,
+                    cabi.VARIANT_PREFILL_SPLITK):
+        for b in (None, bias):
+            _say(name, M, K, N, "variant", cabi.VARIANT_NAMES[variant], "bias", b is not None)
+            try:
+                y = cabi.e2e_gemm_b_ws(x, codes, cb, variant=variant, bias=b)
+            except cabi.VqGemmError as e:
+                assert e.code == -4
+                continue
+            torch.cuda.synchronize()
+            e1, _ = vo.rel_err(_np(y), want if b is None else want + _np(b).astype(np.float64))
+            assert e1 <= TOL, (name, variant, e1)
+            ran.append(variant)
+    assert {cabi.VARIANT_AUTO, cabi.VARIANT_DECODE, cabi.VARIANT_PREFILL} <= set(ran)
+    assert cabi.VARIANT_PREFILL_SPLITK in ran or name != "split_k"
+    if N >= 32:  # the gated epilogue on the same widths
+        n = N // 32 * 32
+        y = cabi.e2e_gemm_b_gated(x, codes[:n].contiguous(), cb)
+        torch.cuda.synchronize()
+        e1, e2 = vo.rel_err(_np(y), vo.gated_gemm_b(_np(x), _np(codes)[:n], _np(cb)).astype(np.float64))
+        assert e2 <= TOL and e1 <= 2 * TOL, (name, "gated", e1, e2)

@@ -30,10 +30,12 @@ bool aligned16(const Tensor &t) { return (reinterpret_cast<uintptr_t>(t.data_ptr
 
 // An activation as the kernels want it: contiguous and 16-byte aligned (a view into a larger buffer may start anywhere,
 // and a copy costs far less than the scalar kernel that takes unaligned operands).
-Tensor dense(const Tensor &t)
+void *dense_of(const Tensor &t, Tensor &hold)
 {
-    Tensor c = t.is_contiguous() ? t : t.contiguous();
-    return aligned16(c) ? c : c.clone();
+    if (t.is_contiguous() && aligned16(t)) return t.data_ptr();
+    hold = t.is_contiguous() ? t.clone() : t.contiguous();
+    if (!aligned16(hold)) hold = hold.clone();
+    return hold.data_ptr();
 }
 
 // Sizes of a product, after every check that raw pointers need: types, devices, element counts.
@@ -79,50 +81,61 @@ Tensor new_result(const Tensor &x, int64_t columns)
 
 void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
+// A tensor's own data where the kernels can read it as it lies, else the data of a copy kept in `hold`.
+void *data_of(const Tensor &t, Tensor &hold)
+{
+    if (t.is_contiguous()) return t.data_ptr();
+    hold = t.contiguous();
+    return hold.data_ptr();
+}
+
 // x @ W.T (+ bias), W in k_repeat stages side by side along K that all multiply the same x
-Tensor linear_impl(const Tensor &x_in, const Tensor &codes_in, const Tensor &codebook_in, const OptTensor &bias_in, int64_t k_repeat,
+Tensor linear_impl(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias, int64_t k_repeat,
                    int variant = VQGEMM_VARIANT_AUTO)
 {
-    const Dims d = check_linear("vq_linear", x_in, codes_in, codebook_in, bias_in, k_repeat);
-    const c10::OptionalDeviceGuard guard(x_in.device());
-    Tensor x = dense(x_in), codes = codes_in.contiguous(), codebook = codebook_in.contiguous(), bias;
-    if (bias_in.has_value() && bias_in->defined()) bias = bias_in->contiguous();
+    const Dims d = check_linear("vq_linear", x, codes, codebook, bias, k_repeat);
+    const c10::OptionalDeviceGuard guard(x.device());
+    Tensor hold_x, hold_codes, hold_cb, hold_bias;
+    const void *xp, *codes_p = data_of(codes, hold_codes), *cb_p = data_of(codebook, hold_cb);
     if (k_repeat > 1) {
         c10::SmallVector<int64_t, 6> times(x.dim(), 1);
         times.back() = k_repeat;
-        x = x.repeat(times);
+        hold_x = x.repeat(times);
+        xp = hold_x.data_ptr();
+    } else {
+        xp = dense_of(x, hold_x);
     }
-    Tensor y = new_result(x_in, d.N);
-    void *bias_p = bias.defined() ? bias.data_ptr() : nullptr;
+    const void *bias_p = bias.has_value() && bias->defined() ? data_of(*bias, hold_bias) : nullptr;
+    Tensor y = new_result(x, d.N);
     void *s = stream_of(x);
-    // scratch for the shapes where the automatic choice may split K; the caching allocator hands out stream-ordered blocks
+    // scratch for the shapes where the automatic choice may split K (never with a slab of 16 rows or fewer); the
+    // caching allocator hands out stream-ordered blocks
     const int64_t need = variant == VQGEMM_VARIANT_AUTO && d.M > 16
                              ? vqgemm_workspace_bytes_b(d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, variant) : 0;
     int rc;
     if (need > 0) {
         Tensor ws = at::detail::empty_cuda({need}, at::kByte, x.device(), c10::nullopt);
-        rc = vqgemm_e2e_gemm_b_ws(x.data_ptr(), codes.data_ptr(), codebook.data_ptr(), bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec,
-                                  d.entries, d.books, d.bits, variant, ws.data_ptr(), need, s);
+        rc = vqgemm_e2e_gemm_b_ws(xp, codes_p, cb_p, bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, variant,
+                                  ws.data_ptr(), need, s);
     } else {
-        rc = vqgemm_e2e_gemm_b_bias(x.data_ptr(), codes.data_ptr(), codebook.data_ptr(), bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec,
-                                    d.entries, d.books, d.bits, variant, nullptr, s);
+        rc = vqgemm_e2e_gemm_b_bias(xp, codes_p, cb_p, bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, variant,
+                                    nullptr, s);
     }
     check_rc(rc, "vq_linear");
     return y;
 }
 
-Tensor gated_impl(const Tensor &x_in, const Tensor &codes_in, const Tensor &codebook_in, const OptTensor &bias_in)
+Tensor gated_impl(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
 {
-    const Dims d = check_linear("vq_gated_linear", x_in, codes_in, codebook_in, bias_in, 1);
+    const Dims d = check_linear("vq_gated_linear", x, codes, codebook, bias, 1);
     TORCH_CHECK_VALUE(d.N % 32 == 0, "vq_gated_linear: the interleaved gate/up rows come in whole groups of 32");
-    const c10::OptionalDeviceGuard guard(x_in.device());
-    const Tensor x = dense(x_in), codes = codes_in.contiguous(), codebook = codebook_in.contiguous();
-    Tensor bias;
-    if (bias_in.has_value() && bias_in->defined()) bias = bias_in->contiguous();
-    Tensor y = new_result(x_in, d.N / 2);
-    check_rc(vqgemm_e2e_gemm_b_gated(x.data_ptr(), codes.data_ptr(), codebook.data_ptr(), bias.defined() ? bias.data_ptr() : nullptr,
-                                     y.data_ptr(), d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, VQGEMM_VARIANT_AUTO, nullptr,
-                                     stream_of(x)),
+    const c10::OptionalDeviceGuard guard(x.device());
+    Tensor hold_x, hold_codes, hold_cb, hold_bias;
+    const void *xp = dense_of(x, hold_x), *codes_p = data_of(codes, hold_codes), *cb_p = data_of(codebook, hold_cb);
+    const void *bias_p = bias.has_value() && bias->defined() ? data_of(*bias, hold_bias) : nullptr;
+    Tensor y = new_result(x, d.N / 2);
+    check_rc(vqgemm_e2e_gemm_b_gated(xp, codes_p, cb_p, bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits,
+                                     VQGEMM_VARIANT_AUTO, nullptr, stream_of(x)),
              "vq_gated_linear");
     return y;
 }
@@ -172,31 +185,6 @@ Tensor no_gradient(Tensor y, std::initializer_list<const Tensor *> inputs)
     return y;
 }
 
-// The autograd kernels call the device implementation directly: one dispatch per call instead of two.
-template <Tensor (*Impl)(const Tensor &, const Tensor &, const Tensor &, const OptTensor &)>
-Tensor with_autograd(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
-{
-    Tensor y;
-    {
-        at::AutoDispatchBelowADInplaceOrView below;
-        y = Impl(x, codes, codebook, bias);
-    }
-    const Tensor b = bias.has_value() ? *bias : Tensor();
-    return no_gradient(y, {&x, &codebook, &b});
-}
-
-Tensor silu_mul_autograd(const Tensor &gate_up)
-{
-    Tensor y;
-    {
-        at::AutoDispatchBelowADInplaceOrView below;
-        y = silu_mul_impl(gate_up);
-    }
-    return no_gradient(y, {&gate_up});
-}
-
-// ---- the layers' direct calls ---------------------------------------------------------------------------------
-
 // Whether nothing but this library is to see a call on `x`: an ordinary tensor in GPU memory, no dispatch mode, no
 // functional transform, no tracer.
 bool plain_call(const Tensor &x)
@@ -208,6 +196,48 @@ bool plain_call(const Tensor &x)
     if (x.key_set().has_any(wrappers)) return false;
     return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
 }
+
+// The autograd kernels call the device implementation directly (one dispatch per call instead of two), unless the tensors
+// only stand for data: then the call goes on to whoever wrapped them.
+typedef Tensor (*LinearFn)(const Tensor &, const Tensor &, const Tensor &, const OptTensor &);
+
+template <LinearFn Impl, const char *Name>
+Tensor with_autograd(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
+{
+    const bool plain = plain_call(x);
+    Tensor y;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        if (plain) {
+            y = Impl(x, codes, codebook, bias);
+        } else {
+            static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow(Name, "").typed<Tensor(const Tensor &, const Tensor &, const Tensor &, const OptTensor &)>();
+            y = op.call(x, codes, codebook, bias);
+        }
+    }
+    const Tensor b = bias.has_value() ? *bias : Tensor();
+    return no_gradient(y, {&x, &codebook, &b});
+}
+
+Tensor silu_mul_autograd(const Tensor &gate_up)
+{
+    const bool plain = plain_call(gate_up);
+    Tensor y;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        if (plain) {
+            y = silu_mul_impl(gate_up);
+        } else {
+            static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("vq_gemm_amd::silu_mul", "").typed<Tensor(const Tensor &)>();
+            y = op.call(gate_up);
+        }
+    }
+    return no_gradient(y, {&gate_up});
+}
+
+constexpr char kLinear[] = "vq_gemm_amd::vq_linear", kLinearPacked[] = "vq_gemm_amd::vq_linear_packed", kGated[] = "vq_gemm_amd::vq_gated_linear";
+
+// ---- the layers' direct calls ---------------------------------------------------------------------------------
 
 py::object linear(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias, int64_t k_repeat)
 {
@@ -243,9 +273,9 @@ TORCH_LIBRARY_IMPL(vq_gemm_amd, CUDA, m)
 
 TORCH_LIBRARY_IMPL(vq_gemm_amd, AutogradCUDA, m)
 {
-    m.impl("vq_linear", &with_autograd<vq_linear>);
-    m.impl("vq_linear_packed", &with_autograd<vq_linear_packed>);
-    m.impl("vq_gated_linear", &with_autograd<gated_impl>);
+    m.impl("vq_linear", &with_autograd<vq_linear, kLinear>);
+    m.impl("vq_linear_packed", &with_autograd<vq_linear_packed, kLinearPacked>);
+    m.impl("vq_gated_linear", &with_autograd<gated_impl, kGated>);
     m.impl("silu_mul", &silu_mul_autograd);
 }
 

@@ -1,7 +1,7 @@
 // Decode path (at most 64 rows of X, 16 per launch): Y[M,N] = X[M,K] . W^T with W given as
-// codes + codebook.  This file holds the batched kernel, which takes the common shapes (one
-// codebook, K a multiple of 256 up to 4096, N a multiple of 16), and the dispatch; every other
-// shape goes to the general kernel of vq_decode_general.hip.
+// codes + codebook.  This file holds the batched kernel, which takes the common shapes (K a multiple
+// of 64, any N from 16 on, the rows of a codebook a multiple of 16 where there are several), and the
+// dispatch; every other shape goes to the general kernel of vq_decode_general.hip.
 //
 // The path is bound by the HBM stream of the code matrix (N*K/vec code bytes), so the design
 // goal is one pass over the codes with every other operand resident on the CU:
@@ -230,8 +230,7 @@ __device__ __forceinline__ void wait_vmcnt_upto(int n)
 }
 
 // ---- batched kernel -----------------------------------------------------------------------
-// The common case (one codebook, K a multiple of 256 and at most 4096, N a multiple of 16) gets
-// a loop that is lean in instructions: a CU issues one vector and one scalar instruction per
+// The common case gets a loop that is lean in instructions: a CU issues one vector and one scalar instruction per
 // cycle in total, whatever the number of waves, and a loop that spends a hundred instructions
 // per wave and tile on control flow, addresses and the reduction is bound by exactly that.
 //   * A wave works through TB consecutive tiles (its K slice of each) before the waves meet, so
@@ -293,7 +292,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // K goes in n_chunks chunks of (at most) n_waves slices of 256 k: wave w owns slice w of the
     // current chunk; the last chunk may leave the upper waves without one.
     const int n_waves = blockDim.x >> 6;
-    const int total_slices = K / kSliceK;
+    const int total_slices = (K + kSliceK - 1) / kSliceK;  // (the last one may end short: K is a multiple of a lane load's k)
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int r16 = lane & 15;  // W row within the tile (A operand) / X row m (B operand)
@@ -327,21 +326,42 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // lie 4*LB bytes apart in each of 16 rows.  Packed layout (pack_codes_kernel below): the 64 lane
     // loads of a wave load are contiguous, [tile][slice][load][lane], so that a wave instruction
     // reads 64*LB consecutive bytes instead of 16 pieces of 4*LB.
-    constexpr int kLoadPitch = PACKED ? 64 * C::LB : 4 * C::LB;  // bytes between the loads of a slice
-    const uint32_t voff = PACKED ? (uint32_t)((w * C::LPT * 64 + lane) * C::LB)
-                                 : (uint32_t)((r16 * J + (w * kSliceK + kq * C::K_LANE) / VEC) * (int)sizeof(CodeT));
-    const int64_t tile_bytes = (int64_t)kTileN * J * (int)sizeof(CodeT);
+    constexpr int kLoadPitch = 64 * C::LB;  // packed: bytes between the loads of a slice
+    // A lane load past the end of K (in a short last slice) reads the chunk's first codes instead, against zeros of X.
+    uint32_t voff[PACKED ? 1 : C::LPT];
+    auto set_voff = [&]() {
+        if constexpr (PACKED) {
+            voff[0] = (uint32_t)((w * C::LPT * 64 + lane) * C::LB);
+        } else {
+#pragma unroll
+            for (int t = 0; t < C::LPT; t++) {
+                const int k = w * kSliceK + t * C::K_WAVE + kq * C::K_LANE;  // inside the chunk
+                voff[t] = (uint32_t)((r16 * J + k / VEC) * (int)sizeof(CodeT));
+                if (K % kSliceK != 0 && chunk * n_waves * kSliceK + k >= K) voff[t] = (uint32_t)(r16 * J * (int)sizeof(CodeT));
+            }
+        }
+    };
+    set_voff();
+    const int row_bytes = J * (int)sizeof(CodeT);
+    // first row of W of a tile: a last tile that N cuts short is moved up to end with N (its first rows are computed twice,
+    // with the same result)
+    auto tile_row = [&](int tile) { return min(tile * kTileN, N - kTileN); };
     const int chunk_bytes = n_waves * kSliceK / VEC * (int)sizeof(CodeT) * (PACKED ? kTileN : 1);
     auto load_unit = [&](int q, Codes (&cw)[TB]) {
 #pragma unroll
         for (int j = 0; j < TB; j++) {
             const int tile = tile_begin + q * TB + j;
             if (tile >= tile_end) break;
-            const uint8_t *sbase = reinterpret_cast<const uint8_t *>(codes) + tile * tile_bytes + chunk * chunk_bytes;
-            if constexpr (C::LPT >= 1) cw[j].template load_async_s<0>(0, voff, sbase);
-            if constexpr (C::LPT >= 2) cw[j].template load_async_s<kLoadPitch>(1, voff, sbase);
-            if constexpr (C::LPT >= 3) cw[j].template load_async_s<2 * kLoadPitch>(2, voff, sbase);
-            if constexpr (C::LPT >= 4) cw[j].template load_async_s<3 * kLoadPitch>(3, voff, sbase);
+            const uint8_t *sbase = reinterpret_cast<const uint8_t *>(codes) + (int64_t)tile_row(tile) * row_bytes + chunk * chunk_bytes;
+            if constexpr (PACKED) {
+                cw[j].template load_async_s<0>(0, voff[0], sbase);
+                if constexpr (C::LPT >= 2) cw[j].template load_async_s<kLoadPitch>(1, voff[0], sbase);
+                if constexpr (C::LPT >= 3) cw[j].template load_async_s<2 * kLoadPitch>(2, voff[0], sbase);
+                if constexpr (C::LPT >= 4) cw[j].template load_async_s<3 * kLoadPitch>(3, voff[0], sbase);
+            } else {
+#pragma unroll
+                for (int t = 0; t < C::LPT; t++) cw[j].template load_async_s<0>(t, voff[t], sbase);
+            }
             static_assert(C::LPT <= 4, "at most four lane loads per slice");
         }
     };
@@ -427,6 +447,13 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
             uint4_t v = {0u, 0u, 0u, 0u};
             if (active && row < M) v = *reinterpret_cast<const uint4_t *>(smem + win + k * 2);
             xr[s] = as_half8(v);
+        }
+        // a slice that K cuts short: zeros behind its end (a branch of its own, so that whole slices test nothing)
+        const int k_left = K - chunk * n_waves * kSliceK - k0;
+        if (k_left < kSliceK) {
+#pragma unroll
+            for (int s = 0; s < kSteps; s++)
+                if ((s / C::SPL) * C::K_WAVE + kg * C::K_LANE + (s % C::SPL) * 8 >= k_left) xr[s] = half8_t{};
         }
     };
     stage_x();
@@ -527,7 +554,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
             // with several chunks the sums are carried from chunk to chunk in the LDS, one entry per slot of the range
             t.carry = (uint32_t)acc_off + (uint32_t)(q * n_slots + slot) * 16u;
             // D[i][j] of the tile: the slot holds rows i = 4*kq .. 4*kq+3 of column j = m.
-            t.n = tile * kTileN + 4 * (jq & 3);
+            t.n = tile_row(tile) + 4 * (jq & 3);
             t.dst = GATED ? y + (int64_t)m * ldy + (tile >> 1) * kTileN + 4 * (jq & 3) : y + (int64_t)m * N + t.n;
             t.live = pass < n_passes && out < n_out_slots && tile < tile_end;
             return t;
@@ -554,7 +581,8 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
             if (!last) {
                 *carry = sum;
             } else if constexpr (kHasBias) {
-                const half4_t b = *reinterpret_cast<const half4_t *>(bias + n_bias);
+                half4_t b;  // (eight bytes at any even address: N may be any number)
+                __builtin_memcpy(&b, bias + n_bias, 8);
                 sum += float4_t{(float)b[0], (float)b[1], (float)b[2], (float)b[3]};
             }
             return sum;
@@ -570,8 +598,8 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
                 for (int e = 0; e < 4; e++) sum[e] = silu_f32(sum[e]) * up[e];
             }
             if (last) {
-                half4_t h = {(half_t)sum[0], (half_t)sum[1], (half_t)sum[2], (half_t)sum[3]};
-                *reinterpret_cast<half4_t *>(t.dst) = h;
+                const half4_t h = {(half_t)sum[0], (half_t)sum[1], (half_t)sum[2], (half_t)sum[3]};
+                __builtin_memcpy(t.dst, &h, 8);
             }
         };
         // The waves take the passes in turn; a wave's first pass is located before the barrier,
@@ -603,6 +631,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
         }
         n_act = min(n_waves, total_slices - chunk * n_waves);
         active = w < n_act;
+        if (n_chunks > 1 && K % kSliceK != 0) set_voff();
         // The first codes are requested before the table or X are replaced, to overlap the latencies.
         load_first_units();
         __syncthreads();  // every gather from the old table has been consumed, every slot read
@@ -646,23 +675,27 @@ struct BatchedPlan {
     size_t smem;
 };
 
-// K a multiple of 256, N and the rows per codebook multiples of 16; the LDS must hold the table,
+// K a multiple of 64 (of 256 on packed codes), N at least 16, with several codebooks the rows of each a multiple of 16; the
+// LDS must hold the table,
 // the slots, the staged X and, when K goes in chunks, the carried sums of the workgroup's tiles.
 template <int VEC, typename CodeT>
 BatchedPlan plan_batched(const ProblemB &p)
 {
     typedef DecodeCfg<VEC, CodeT> C;
     BatchedPlan g = {};
-    if (p.K % kSliceK != 0 || p.N % kTileN != 0 || p.rows_per_cb % kTileN != 0) return g;
+    if (p.K % 64 != 0 || p.N < kTileN || (p.n_codebooks > 1 && p.rows_per_cb % kTileN != 0)) return g;
+    if (p.packed && (p.K % kSliceK != 0 || p.N % kTileN != 0)) return g;
+    static_assert(64 % C::K_LANE == 0, "a lane load is whole or past the end of K");
+    if (p.entries > (p.code_bits == 8 ? 256 : 65536) || ((size_t)p.entries * VEC * 2) % 16 != 0) return g;
     // gated: whole pairs of a gate and an up tile per codebook, dealt to the workgroups as pairs, in batches of an even
     // number of tiles; the packed code layout is not read
     const int deal = p.gated ? 2 : 1;
     if (p.gated && (p.rows_per_cb % (2 * kTileN) != 0 || C::TB % 2 != 0 || p.packed)) return g;
-    const int slices = p.K / kSliceK;
+    const int slices = (p.K + kSliceK - 1) / kSliceK;
     g.n_chunks = (slices + kMaxWaves - 1) / kMaxWaves;
     g.n_waves = (slices + g.n_chunks - 1) / g.n_chunks;
     const int m_slab = p.M < kTileN ? p.M : kTileN;  // rows of X one workgroup multiplies
-    g.tiles_per_cb = p.rows_per_cb / kTileN;
+    g.tiles_per_cb = (p.rows_per_cb + kTileN - 1) / kTileN;
     g.per_cu = kMaxWaves / g.n_waves;
     g.n_slabs = (p.M + kTileN - 1) / kTileN;
     // As many workgroups as the device holds at once, shared among the slabs.  Within a slab a
@@ -827,7 +860,9 @@ bool batched_supports(const ProblemB &p) { return plan_batched(p).ok; }
 
 bool decode_packed_supports(const ProblemB &p)
 {
-    return p.M >= 1 && p.M <= kBatchedMaxM && decode_general_supports(p) && batched_supports(p);
+    ProblemB q = p;
+    q.packed = true;
+    return p.M >= 1 && p.M <= kBatchedMaxM && decode_general_supports(p) && batched_supports(q);
 }
 
 bool pack_codes_supports(int64_t N, int64_t K, int vec, int code_bits)
@@ -852,8 +887,8 @@ bool decode_gated_supports(const ProblemB &p) { return p.gated && decode_support
 
 bool decode_supports(const ProblemB &p)
 {
-    if (p.M < 1 || !decode_general_supports(p)) return false;
-    return p.M <= kGeneralMaxM || (p.M <= kBatchedMaxM && batched_supports(p));
+    if (p.M < 1 || (p.vec != 2 && p.vec != 4 && p.vec != 8)) return false;
+    return (p.M <= kGeneralMaxM && decode_general_supports(p)) || (p.M <= kBatchedMaxM && batched_supports(p));
 }
 
 // Rough times (us) of the two tiled kernels on a shape both can take; the automatic choice takes

@@ -31,8 +31,10 @@
 //
 // K is walked in order: stage i is k in [64 i, 64 i + 64), MFMA step s of it the 32 k from
 // 32 s on, and lane group g (lanes 16g..16g+15) holds the 8 k from 8 g on.  K must be a
-// multiple of the k that 16 bytes of codes cover; a last stage of 32 k runs in the TAIL
-// instantiation, which points the W operands of the missing step at zeros.
+// multiple of the k that 16 bytes of codes cover, or for 8-vectors with 8-bit codes (128 k) of 64.
+// What does not end with a whole code tile runs in the TAIL instantiation: a last stage of 32 k
+// points the W operands of the missing step at zeros; a last code tile of one stage is left after
+// that stage, its 8 bytes of codes per row being read as the upper half of the 16 that end the row.
 #include "vq_prefill_common.h"
 
 #include <type_traits>
@@ -58,6 +60,8 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
     // The launch covers the W rows (columns of Y) [n_begin, N) of a problem with ldn rows in all:
     // ldn is the row stride of Y and counts the codebooks, N bounds the rows that are touched.
     typedef PrefillCfg<VEC, CodeT> C;
+    // TAIL: a last stage of 32 k, or (HALF: a code tile covers two stages) a last code tile of one stage
+    constexpr bool TAIL32 = TAIL && C::STAGES == 1, HALF = TAIL && C::STAGES == 2;
     static_assert(NS >= 2 && NS <= 4, "two to four X stages");
     constexpr int D = NS - 1;                 // loads run D stages ahead of the MFMAs
     constexpr int NC = C::code_bufs(NS);
@@ -106,7 +110,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
     // buffer; the lane looks up which (row, chunk) lives in its slot under the swizzle and reads
     // that.  Chunk cc of a row is the 8 k from 8 cc on.
     uint32_t x_voff[kChunksPerThread];
-    uint32_t x_voff_tail[TAIL ? kChunksPerThread : 1];  // last stage of 32 k: chunks 4..7 re-read chunks 0..3
+    uint32_t x_voff_tail[TAIL32 ? kChunksPerThread : 1];  // last stage of 32 k: chunks 4..7 re-read chunks 0..3
 #pragma unroll
     for (int i = 0; i < kChunksPerThread; i++) {
         const int slot = (4 * i + wave) * 64 + lane;
@@ -115,7 +119,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
         const int row = 2 * bank_row + (v >> 3), cc = v & 7;
         const int gm = min(m0 + row, M - 1) - m0;
         x_voff[i] = (uint32_t)(((int64_t)gm * K + cc * 8) * 2);
-        if (TAIL) x_voff_tail[i] = x_voff[i] - (cc >= 4 ? 64u : 0u);
+        if (TAIL32) x_voff_tail[i] = x_voff[i] - (cc >= 4 ? 64u : 0u);
     }
     const half_t *x_tile = x + (int64_t)m0 * K;
     // X load i (0..7) of stage `stage` into buffer `buf`: one 16-byte chunk per lane, 1 KB per
@@ -124,7 +128,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
         const bool is_last = stage >= n_stage - 1;
         const half_t *sbase = x_tile + min(stage, n_stage - 1) * kStageK;
         uint32_t voff = x_voff[i];
-        if (TAIL) voff = is_last ? x_voff_tail[i] : voff;
+        if (TAIL32) voff = is_last ? x_voff_tail[i] : voff;
         load_to_lds_16(buf * kStageBytes + (4 * i + wave) * 1024, voff, sbase);
     };
     // Code tile of a super stage: chunk c of tile row w*64 + lane goes to [c][row]; 1 KB per wave.
@@ -133,9 +137,10 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
     auto issue_codes = [&](int c, int cbuf, int super) {
         const bool is_last = super >= n_super - 1;
         super = min(super, n_super - 1);
-        // a last stage of 32 k has only chunk 0; read it twice
-        const int chunk = (TAIL && is_last) ? 0 : c;
-        const uint8_t *sbase = reinterpret_cast<const uint8_t *>(code_tile) + (int64_t)super * (C::K_SUPER / VEC * C::CSZ) + chunk * 16;
+        // a last stage of 32 k has only chunk 0; read it twice.  A last code tile of one stage has 8 bytes: the 16 that end
+        // with them are read (rows are 8-byte aligned then, and nothing past the end of the matrix is touched)
+        const int chunk = (TAIL32 && is_last) ? 0 : c;
+        const uint8_t *sbase = reinterpret_cast<const uint8_t *>(code_tile) + (int64_t)super * (C::K_SUPER / VEC * C::CSZ) + chunk * 16 - (HALF && is_last ? 8 : 0);
         load_to_lds_16(kCodeBase + cbuf * C::kTileBytes + c * (BN * 16) + wave * 1024, code_voff, sbase);
     };
 
@@ -164,9 +169,9 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
         xp[i] = *reinterpret_cast<const half8_t *>(smem + buf * kStageBytes + x_rd[i & 1][s] + (i >> 1) * 4096);
     };
     // the codes of W piece j for MFMA step s of stage t (of its super stage) out of code buffer `cbuf`
-    auto load_c1 = [&](int set, int j, int cbuf, int t, int s) {
+    auto load_c1 = [&](int set, int j, int cbuf, int shift, int t, int s) {
         const int pos = (t % C::STAGES) * 2 * C::HALF + s * C::HALF;   // + kg*RB stays inside the 16-byte chunk
-        cr[set][j & 3] = read_codes<C::RB>(smem + code_rd + cbuf * C::kTileBytes + (pos / 16) * (BN * 16) + j * 256 + pos % 16);
+        cr[set][j & 3] = read_codes<C::RB>(smem + code_rd + cbuf * C::kTileBytes + shift + (pos / 16) * (BN * 16) + j * 256 + pos % 16);
     };
     // the two halves of W piece j from the codes read before
     // 8-vectors out of the plain table: one 16-byte gather per operand.  (This kernel is bound by the energy it spends,
@@ -176,16 +181,16 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
     auto load_w1 = [&](int set, int j, bool zero) {
         if constexpr (kWholeGather) {
             uint32_t a = book[j] + cr[set][j & 3] * 16u;
-            if (TAIL) a = zero ? zero_off : a;
+            if (TAIL32) a = zero ? zero_off : a;
             const half8_t v = *reinterpret_cast<const half8_t *>(smem + a);
             wlo[j] = __builtin_shufflevector(v, v, 0, 1, 2, 3);
             whi[j] = __builtin_shufflevector(v, v, 4, 5, 6, 7);
         } else {
-            wlo[j] = gather4<VEC, CodeT, TAIL, SPLIT>(smem, book[j], cr[set][j & 3], 0, zero, zero_off);
+            wlo[j] = gather4<VEC, CodeT, TAIL32, SPLIT>(smem, book[j], cr[set][j & 3], 0, zero, zero_off);
         }
     };
     auto load_w2 = [&](int set, int j, bool zero) {
-        if constexpr (!kWholeGather) whi[j] = gather4<VEC, CodeT, TAIL, SPLIT>(smem, book[j], cr[set][j & 3], 1, zero, zero_off);
+        if constexpr (!kWholeGather) whi[j] = gather4<VEC, CodeT, TAIL32, SPLIT>(smem, book[j], cr[set][j & 3], 1, zero, zero_off);
     };
     // MFMA f of group p of the 4x4 quadrant (jh, ih): a group is W piece p against the four X
     // pieces, or (x_outer) X piece p against the four W pieces
@@ -246,8 +251,8 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
     int cbuf = 0;  // code buffer of the current super stage; super+j lives in (cbuf + j) % NC
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-        load_c1(0, p, cbuf, 0, 0);
-        load_c1(1, 4 + p, cbuf, 0, 0);
+        load_c1(0, p, cbuf, 0, 0, 0);
+        load_c1(1, 4 + p, cbuf, 0, 0, 0);
     }
 #pragma unroll
     for (int p = 0; p < 4; p++) {
@@ -273,8 +278,8 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
         mfma_one(jh, ih, p_, 1, x_outer); VQ_FENCE;                                 \
         LOADP##2(p_); CODEP(p_); VQ_FENCE;                                          \
         mfma_one(jh, ih, p_, 2, x_outer); VQ_FENCE;                                 \
-        if (p_ == 0) { issue_x(xi, TGT##_buf, TGT##_stage); VQ_FENCE; }             \
-        if (p_ == 2 && TGT##_codes && xi < C::CH) { issue_codes(xi, TGT##_cbuf, TGT##_super); VQ_FENCE; } \
+        if (!kLast && p_ == 0) { issue_x(xi, TGT##_buf, TGT##_stage); VQ_FENCE; }             \
+        if (!kLast && p_ == 2 && TGT##_codes && xi < C::CH) { issue_codes(xi, TGT##_cbuf, TGT##_super); VQ_FENCE; } \
         mfma_one(jh, ih, p_, 3, x_outer); VQ_FENCE;                                 \
     }
 
@@ -311,8 +316,11 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
     constexpr bool same_super = t + 1 < C::STAGES;                                  \
     const int cbuf_n = same_super ? cbuf : (cbuf + 1 == NC ? 0 : cbuf + 1);         \
     constexpr int t_n = same_super ? t + 1 : 0;                                     \
+    /* the codes of a last code tile of one stage lie in the upper half of its chunks */ \
+    const int cshift = HALF && super == n_super - 1 ? 8 : 0;                        \
+    const int cshift_n = HALF && super + (same_super ? 0 : 1) >= n_super - 1 ? 8 : 0; \
     /* a last stage of 32 k has no step 1 */                                       \
-    const bool no_b = TAIL && stage == n_stage - 1;                                 \
+    const bool no_b = TAIL32 && stage == n_stage - 1;                                 \
     /* publish stage+1: in flight may be what stages +2..+D bring along */         \
     constexpr int in_flight = [&]() constexpr {                                     \
         int n = 0;                                                                  \
@@ -324,39 +332,39 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
 #define L_XHI_A(p) load_x1(4 + (p), buf, 0)
 #define L_XLO_B(p) load_x1((p), buf, 1)
 #define L_XHI_B(p) load_x1(4 + (p), buf, 1)
-#define L_XLO_N(p) load_x1((p), buf_next, 0)
+#define L_XLO_N(p) if (!kLast) load_x1((p), buf_next, 0)
 #define L_XHI_A2(p) do {} while (0)
 #define L_XLO_B2(p) do {} while (0)
 #define L_XHI_B2(p) do {} while (0)
 #define L_XLO_N2(p) do {} while (0)
     if (!mirrored) {
-        for (int super = 0; super < n_super; super++) {
-            // stage t (a compile-time 0 or 1) of the super stage
-            auto stage_body = [&](auto t_const) {
-                VQ_STAGE_SETUP;
-                // W low/X low are in registers, the codes of W high in cr[1]
+        // stage t (a compile-time 0 or 1) of the super stage
+        auto stage_body = [&](int super, auto t_const, auto last_const) {
+            constexpr bool kLast = decltype(last_const)::value;  // nothing is loaded for a stage behind this one
+            VQ_STAGE_SETUP;
+            // W low/X low are in registers, the codes of W high in cr[1]
 #define L_WHI_A(p) load_w1(1, 4 + (p), false)
 #define L_WHI_A2(p) load_w2(1, 4 + (p), false)
 #define L_WHI_B(p) load_w1(0, 4 + (p), no_b)
 #define L_WHI_B2(p) load_w2(0, 4 + (p), no_b)
 #define L_WLO_B(p) load_w1(1, (p), no_b)
 #define L_WLO_B2(p) load_w2(1, (p), no_b)
-#define L_WLO_N(p) load_w1(0, (p), false)
-#define L_WLO_N2(p) load_w2(0, (p), false)
-#define C_WHI_B(p) load_c1(0, 4 + (p), cbuf, t, 1)
-#define C_WLO_B(p) load_c1(1, (p), cbuf, t, 1)
-#define C_WLO_N(p) load_c1(0, (p), cbuf_n, t_n, 0)
-#define C_WHI_N(p) load_c1(1, 4 + (p), cbuf_n, t_n, 0)
-                VQ_QUADRANT(L_WHI_A, VQ_NONE, 0, 0, false, 2, tgt_a);   // W low (just loaded) x X low
-                VQ_QUADRANT(L_XHI_A, VQ_NONE, 1, 0, false, 3, tgt_a);   // W high (just loaded) x X low
-                VQ_QUADRANT(L_XLO_B, C_WHI_B, 1, 1, true, 4, tgt_a);    // W high x X high (just loaded)
-                VQ_QUADRANT(L_WHI_B, C_WLO_B, 0, 1, false, 5, tgt_a);   // W low x X high
-                VQ_QUADRANT(L_WLO_B, VQ_NONE, 1, 0, false, 6, tgt_a);   // W high' (just loaded) x X low'
-                VQ_QUADRANT(L_XHI_B, VQ_NONE, 0, 0, false, 7, tgt_a);   // W low' (just loaded) x X low'
-                wait_vmcnt<in_flight>();
-                __syncthreads();
-                VQ_QUADRANT(L_XLO_N, C_WLO_N, 0, 1, true, 0, tgt_b);    // W low' x X high' (just loaded)
-                VQ_QUADRANT(L_WLO_N, C_WHI_N, 1, 1, false, 1, tgt_b);   // W high' x X high'
+#define L_WLO_N(p) if (!kLast) load_w1(0, (p), false)
+#define L_WLO_N2(p) if (!kLast) load_w2(0, (p), false)
+#define C_WHI_B(p) load_c1(0, 4 + (p), cbuf, cshift, t, 1)
+#define C_WLO_B(p) load_c1(1, (p), cbuf, cshift, t, 1)
+#define C_WLO_N(p) if (!kLast) load_c1(0, (p), cbuf_n, cshift_n, t_n, 0)
+#define C_WHI_N(p) if (!kLast) load_c1(1, 4 + (p), cbuf_n, cshift_n, t_n, 0)
+            VQ_QUADRANT(L_WHI_A, VQ_NONE, 0, 0, false, 2, tgt_a);   // W low (just loaded) x X low
+            VQ_QUADRANT(L_XHI_A, VQ_NONE, 1, 0, false, 3, tgt_a);   // W high (just loaded) x X low
+            VQ_QUADRANT(L_XLO_B, C_WHI_B, 1, 1, true, 4, tgt_a);    // W high x X high (just loaded)
+            VQ_QUADRANT(L_WHI_B, C_WLO_B, 0, 1, false, 5, tgt_a);   // W low x X high
+            VQ_QUADRANT(L_WLO_B, VQ_NONE, 1, 0, false, 6, tgt_a);   // W high' (just loaded) x X low'
+            VQ_QUADRANT(L_XHI_B, VQ_NONE, 0, 0, false, 7, tgt_a);   // W low' (just loaded) x X low'
+            wait_vmcnt<in_flight>();
+            __syncthreads();
+            VQ_QUADRANT(L_XLO_N, C_WLO_N, 0, 1, true, 0, tgt_b);    // W low' x X high' (just loaded)
+            VQ_QUADRANT(L_WLO_N, C_WHI_N, 1, 1, false, 1, tgt_b);   // W high' x X high'
 #undef L_WHI_A
 #undef L_WHI_A2
 #undef L_WHI_B
@@ -369,39 +377,42 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
 #undef C_WLO_B
 #undef C_WLO_N
 #undef C_WHI_N
-                buf = buf_next;
+            buf = buf_next;
             };
-            stage_body(std::integral_constant<int, 0>{});
-            if constexpr (C::STAGES == 2) stage_body(std::integral_constant<int, 1>{});
+        int super = 0;
+        do {
+            stage_body(super, std::integral_constant<int, 0>{}, std::false_type{});
+            if constexpr (C::STAGES == 2) stage_body(super, std::integral_constant<int, 1>{}, std::false_type{});
             cbuf = cbuf + 1 == NC ? 0 : cbuf + 1;
-        }
+        } while (++super < n_super - (HALF ? 1 : 0));
+        if constexpr (HALF) stage_body(n_super - 1, std::integral_constant<int, 0>{}, std::true_type{});  // (behind the loop: an exit from its middle costs spills)
     } else {
-        for (int super = 0; super < n_super; super++) {
-            auto stage_body = [&](auto t_const) {
-                VQ_STAGE_SETUP;
-                // W low/X low are in registers
-#define C_WHI_A(p) load_c1(0, 4 + (p), cbuf, t, 0)
+        auto stage_body = [&](int super, auto t_const, auto last_const) {
+            constexpr bool kLast = decltype(last_const)::value;  // nothing is loaded for a stage behind this one
+            VQ_STAGE_SETUP;
+            // W low/X low are in registers
+#define C_WHI_A(p) load_c1(0, 4 + (p), cbuf, cshift, t, 0)
 #define L_WHI_A(p) load_w1(0, 4 + (p), false)
 #define L_WHI_A2(p) load_w2(0, 4 + (p), false)
-#define C_WLO_B(p) load_c1(1, (p), cbuf, t, 1)
+#define C_WLO_B(p) load_c1(1, (p), cbuf, cshift, t, 1)
 #define L_WLO_B(p) load_w1(1, (p), no_b)
 #define L_WLO_B2(p) load_w2(1, (p), no_b)
-#define C_WHI_B(p) load_c1(0, 4 + (p), cbuf, t, 1)
+#define C_WHI_B(p) load_c1(0, 4 + (p), cbuf, cshift, t, 1)
 #define L_WHI_B(p) load_w1(0, 4 + (p), no_b)
 #define L_WHI_B2(p) load_w2(0, 4 + (p), no_b)
-#define C_WLO_N(p) load_c1(1, (p), cbuf_n, t_n, 0)
-#define L_WLO_N(p) load_w1(1, (p), false)
-#define L_WLO_N2(p) load_w2(1, (p), false)
-                VQ_QUADRANT(L_XHI_A, C_WHI_A, 0, 0, true, 3, tgt_a);    // W low x X low (just loaded)
-                VQ_QUADRANT(L_WHI_A, C_WLO_B, 0, 1, true, 4, tgt_a);    // W low x X high (just loaded)
-                VQ_QUADRANT(L_WLO_B, VQ_NONE, 1, 1, false, 5, tgt_a);   // W high (just loaded) x X high
-                VQ_QUADRANT(L_XHI_B, VQ_NONE, 1, 0, false, 6, tgt_a);   // W high x X low
-                VQ_QUADRANT(L_XLO_B, C_WHI_B, 0, 1, true, 7, tgt_a);    // W low' x X high' (just loaded)
-                wait_vmcnt<in_flight>();
-                __syncthreads();
-                VQ_QUADRANT(L_WHI_B, C_WLO_N, 0, 0, true, 0, tgt_b);    // W low' x X low' (just loaded)
-                VQ_QUADRANT(L_WLO_N, VQ_NONE, 1, 0, false, 1, tgt_b);   // W high' (just loaded) x X low'
-                VQ_QUADRANT(L_XLO_N, VQ_NONE, 1, 1, false, 2, tgt_b);   // W high' x X high'
+#define C_WLO_N(p) if (!kLast) load_c1(1, (p), cbuf_n, cshift_n, t_n, 0)
+#define L_WLO_N(p) if (!kLast) load_w1(1, (p), false)
+#define L_WLO_N2(p) if (!kLast) load_w2(1, (p), false)
+            VQ_QUADRANT(L_XHI_A, C_WHI_A, 0, 0, true, 3, tgt_a);    // W low x X low (just loaded)
+            VQ_QUADRANT(L_WHI_A, C_WLO_B, 0, 1, true, 4, tgt_a);    // W low x X high (just loaded)
+            VQ_QUADRANT(L_WLO_B, VQ_NONE, 1, 1, false, 5, tgt_a);   // W high (just loaded) x X high
+            VQ_QUADRANT(L_XHI_B, VQ_NONE, 1, 0, false, 6, tgt_a);   // W high x X low
+            VQ_QUADRANT(L_XLO_B, C_WHI_B, 0, 1, true, 7, tgt_a);    // W low' x X high' (just loaded)
+            wait_vmcnt<in_flight>();
+            __syncthreads();
+            VQ_QUADRANT(L_WHI_B, C_WLO_N, 0, 0, true, 0, tgt_b);    // W low' x X low' (just loaded)
+            VQ_QUADRANT(L_WLO_N, VQ_NONE, 1, 0, false, 1, tgt_b);   // W high' (just loaded) x X low'
+            VQ_QUADRANT(L_XLO_N, VQ_NONE, 1, 1, false, 2, tgt_b);   // W high' x X high'
 #undef C_WHI_A
 #undef L_WHI_A
 #undef L_WHI_A2
@@ -414,12 +425,15 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
 #undef C_WLO_N
 #undef L_WLO_N
 #undef L_WLO_N2
-                buf = buf_next;
+            buf = buf_next;
             };
-            stage_body(std::integral_constant<int, 0>{});
-            if constexpr (C::STAGES == 2) stage_body(std::integral_constant<int, 1>{});
+        int super = 0;
+        do {
+            stage_body(super, std::integral_constant<int, 0>{}, std::false_type{});
+            if constexpr (C::STAGES == 2) stage_body(super, std::integral_constant<int, 1>{}, std::false_type{});
             cbuf = cbuf + 1 == NC ? 0 : cbuf + 1;
-        }
+        } while (++super < n_super - (HALF ? 1 : 0));
+        if constexpr (HALF) stage_body(n_super - 1, std::integral_constant<int, 0>{}, std::true_type{});  // (behind the loop: an exit from its middle costs spills)
     }
 #undef L_XHI_A
 #undef L_XHI_A2
@@ -437,6 +451,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
     __syncthreads();
     // the last MFMAs must have left the pipe before the accumulators are read
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    if constexpr (HALF) hold_accumulators(acc);
     // ---- epilogue: lane holds Y[m = i*16 + r16][n = j*16 + 4*kg + 0..3] of its wave tile ------
     auto epilogue = [&](auto has_bias_const) {
         constexpr bool HB = decltype(has_bias_const)::value;
@@ -527,6 +542,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
                                                                      int cb_lds_count, int gated)
 {
     typedef PrefillCfg<VEC, CodeT> C;
+    constexpr bool TAIL32 = TAIL && C::STAGES == 1, HALF = TAIL && C::STAGES == 2;  // as in prefill_kernel
     constexpr int NS = 4, D = NS - 1;
     constexpr int NC = C::code_bufs(NS);
     constexpr int kTile = C::CH * BNN * 16;   // code tile: [chunk][128 rows][16 bytes]
@@ -564,7 +580,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
     }
 
     uint32_t x_voff[kChunksPerThread];
-    uint32_t x_voff_tail[TAIL ? kChunksPerThread : 1];
+    uint32_t x_voff_tail[TAIL32 ? kChunksPerThread : 1];
 #pragma unroll
     for (int i = 0; i < kChunksPerThread; i++) {
         const int slot = (4 * i + wave) * 64 + lane;
@@ -573,14 +589,14 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
         const int row = 2 * bank_row + (v >> 3), cc = v & 7;
         const int gm = min(m0 + row, M - 1) - m0;
         x_voff[i] = (uint32_t)(((int64_t)gm * K + cc * 8) * 2);
-        if (TAIL) x_voff_tail[i] = x_voff[i] - (cc >= 4 ? 64u : 0u);
+        if (TAIL32) x_voff_tail[i] = x_voff[i] - (cc >= 4 ? 64u : 0u);
     }
     const half_t *x_tile = x + (int64_t)m0 * K;
     auto issue_x = [&](int i, int buf, int stage) {
         const bool is_last = stage >= n_stage - 1;
         const half_t *sbase = x_tile + min(stage, n_stage - 1) * kStageK;
         uint32_t voff = x_voff[i];
-        if (TAIL) voff = is_last ? x_voff_tail[i] : voff;
+        if (TAIL32) voff = is_last ? x_voff_tail[i] : voff;
         load_to_lds_16(buf * kStageBytes + (4 * i + wave) * 1024, voff, sbase);
     };
     // The code tile has 128 rows, two waves' worth: the waves of the lower half of the tile load
@@ -590,8 +606,8 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
     auto issue_codes = [&](int c, int cbuf, int super) {
         const bool is_last = super >= n_super - 1;
         super = min(super, n_super - 1);
-        const int chunk = (TAIL && is_last) ? 0 : c;
-        const uint8_t *sbase = reinterpret_cast<const uint8_t *>(code_tile) + (int64_t)super * (C::K_SUPER / VEC * C::CSZ) + chunk * 16;
+        const int chunk = (TAIL32 && is_last) ? 0 : c;
+        const uint8_t *sbase = reinterpret_cast<const uint8_t *>(code_tile) + (int64_t)super * (C::K_SUPER / VEC * C::CSZ) + chunk * 16 - (HALF && is_last ? 8 : 0);
         load_to_lds_16(kCodeBase + cbuf * kTile + c * (BNN * 16) + wn * 1024, code_voff, sbase);
     };
 
@@ -615,12 +631,12 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
     auto load_x1 = [&](int set, int i, int buf, int s) {
         xp[set][i] = *reinterpret_cast<const half8_t *>(smem + buf * kStageBytes + x_rd[i & 1][s] + (i >> 1) * 4096);
     };
-    auto load_c1 = [&](int cset, int j, int cbuf, int t, int s) {
+    auto load_c1 = [&](int cset, int j, int cbuf, int shift, int t, int s) {
         const int pos = (t % C::STAGES) * 2 * C::HALF + s * C::HALF;
-        cr[cset][j & 1] = read_codes<C::RB>(smem + code_rd + cbuf * kTile + (pos / 16) * (BNN * 16) + j * 256 + pos % 16);
+        cr[cset][j & 1] = read_codes<C::RB>(smem + code_rd + cbuf * kTile + shift + (pos / 16) * (BNN * 16) + j * 256 + pos % 16);
     };
     auto load_w_half = [&](int set, int cset, int j, int h, bool zero) {
-        const half4_t v = gather4<VEC, CodeT, TAIL, SPLIT>(smem, book[j], cr[cset][j & 1], h, zero, zero_off);
+        const half4_t v = gather4<VEC, CodeT, TAIL32, SPLIT>(smem, book[j], cr[cset][j & 1], h, zero, zero_off);
         if (h == 0) wlo[set][j] = v;
         else whi[set][j] = v;
     };
@@ -664,8 +680,8 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
     // step 0 of stage 0: all of its operands; and the codes of the first W pair of step 1
 #pragma unroll
     for (int j = 0; j < NPN; j += 2) {
-        load_c1(0, j, cbuf, 0, 0);
-        load_c1(0, j + 1, cbuf, 0, 0);
+        load_c1(0, j, cbuf, 0, 0, 0);
+        load_c1(0, j + 1, cbuf, 0, 0, 0);
         load_w_half(0, 0, j, 0, false);
         load_w_half(0, 0, j, 1, false);
         load_w_half(0, 0, j + 1, 0, false);
@@ -673,8 +689,8 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
     }
 #pragma unroll
     for (int i = 0; i < MP; i++) load_x1(0, i, buf, 0);
-    load_c1(0, 0, cbuf, 0, 1);
-    load_c1(0, 1, cbuf, 0, 1);
+    load_c1(0, 0, cbuf, 0, 0, 1);
+    load_c1(0, 1, cbuf, 0, 0, 1);
 
 #define VQ_FENCE __builtin_amdgcn_sched_barrier(0)
     // One quadrant: W pieces 0..3 of operand set `set` against X pieces ih*4.. of the same set.
@@ -695,46 +711,47 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
         }                                                                           \
     }
 
-    for (int super = 0; super < n_super; super++) {
-        auto stage_body = [&](auto t_const) {
-            constexpr int t = decltype(t_const)::value;
-            const int stage = super * C::STAGES + t;
-            const int buf_next = buf + 1 == NS ? 0 : buf + 1;
-            // first quadrant: X loads 6, 7 of stage+2; the others: X loads 0..5 of stage+3 and its code tile
-            const int tgt_a_buf = (buf + 2) % NS, tgt_a_stage = stage + 2;
-            constexpr bool tgt_a_codes = false;
-            const int tgt_a_cbuf = 0, tgt_a_super = 0;
-            const int tgt_b_buf = buf == 0 ? NS - 1 : buf - 1, tgt_b_stage = stage + D;
-            constexpr bool tgt_b_codes = (t + D) % C::STAGES == 0;
-            constexpr int d_super = (t + D) / C::STAGES;
-            const int tgt_b_super = super + d_super;
-            const int tgt_b_cbuf = (cbuf + d_super) % NC;
-            constexpr bool same_super = t + 1 < C::STAGES;
-            const int cbuf_n = same_super ? cbuf : (cbuf + 1 == NC ? 0 : cbuf + 1);
-            constexpr int t_n = same_super ? t + 1 : 0;
-            const bool no_b = TAIL && stage == n_stage - 1;
-            VQ_FENCE;
-            // step 0 multiplies (set 0); step 1's operands are loaded into set 1
+    auto stage_body = [&](int super, auto t_const) {
+        constexpr int t = decltype(t_const)::value;
+        const int stage = super * C::STAGES + t;
+        const int buf_next = buf + 1 == NS ? 0 : buf + 1;
+        // first quadrant: X loads 6, 7 of stage+2; the others: X loads 0..5 of stage+3 and its code tile
+        const int tgt_a_buf = (buf + 2) % NS, tgt_a_stage = stage + 2;
+        constexpr bool tgt_a_codes = false;
+        const int tgt_a_cbuf = 0, tgt_a_super = 0;
+        const int tgt_b_buf = buf == 0 ? NS - 1 : buf - 1, tgt_b_stage = stage + D;
+        constexpr bool tgt_b_codes = (t + D) % C::STAGES == 0;
+        constexpr int d_super = (t + D) / C::STAGES;
+        const int tgt_b_super = super + d_super;
+        const int tgt_b_cbuf = (cbuf + d_super) % NC;
+        constexpr bool same_super = t + 1 < C::STAGES;
+        const int cbuf_n = same_super ? cbuf : (cbuf + 1 == NC ? 0 : cbuf + 1);
+        constexpr int t_n = same_super ? t + 1 : 0;
+        const int cshift = HALF && super == n_super - 1 ? 8 : 0;
+        const int cshift_n = HALF && super + (same_super ? 0 : 1) >= n_super - 1 ? 8 : 0;
+        const bool no_b = TAIL32 && stage == n_stage - 1;
+        VQ_FENCE;
+        // step 0 multiplies (set 0); step 1's operands are loaded into set 1
 #define LX_B_LO(p) load_x1(1, (p), buf, 1)
 #define LX_B_HI(p) load_x1(1, 4 + (p), buf, 1)
 #define LW_B_01(p) load_w_half(1, 0, (p) >> 1, (p) & 1, no_b)
 #define LW_B_23(p) load_w_half(1, 1, 2 + ((p) >> 1), (p) & 1, no_b)
-#define LC_B_23(q) load_c1(1, 2 + (q), cbuf, t, 1)
-#define LC_N_01(q) load_c1(0, (q), cbuf_n, t_n, 0)
-            VQ_NQUADRANT(0, 0, LX_B_LO, LW_B_01, LC_B_23, 6, tgt_a);
-            // Publish stage+1: only what stage+2 brings along may still be in flight.
-            wait_vmcnt<loads_of(t + 2)>();
-            __syncthreads();
-            VQ_NQUADRANT(0, 1, LX_B_HI, LW_B_23, LC_N_01, 0, tgt_b);
-            // step 1 multiplies (set 1); the next stage's step 0 operands are loaded into set 0
+#define LC_B_23(q) load_c1(1, 2 + (q), cbuf, cshift, t, 1)
+#define LC_N_01(q) load_c1(0, (q), cbuf_n, cshift_n, t_n, 0)
+        VQ_NQUADRANT(0, 0, LX_B_LO, LW_B_01, LC_B_23, 6, tgt_a);
+        // Publish stage+1: only what stage+2 brings along may still be in flight.
+        wait_vmcnt<loads_of(t + 2)>();
+        __syncthreads();
+        VQ_NQUADRANT(0, 1, LX_B_HI, LW_B_23, LC_N_01, 0, tgt_b);
+        // step 1 multiplies (set 1); the next stage's step 0 operands are loaded into set 0
 #define LX_N_LO(p) load_x1(0, (p), buf_next, 0)
 #define LX_N_HI(p) load_x1(0, 4 + (p), buf_next, 0)
 #define LW_N_01(p) load_w_half(0, 0, (p) >> 1, (p) & 1, false)
 #define LW_N_23(p) load_w_half(0, 1, 2 + ((p) >> 1), (p) & 1, false)
-#define LC_N_23(q) load_c1(1, 2 + (q), cbuf_n, t_n, 0)
-#define LC_NB_01(q) load_c1(0, (q), cbuf_n, t_n, 1)
-            VQ_NQUADRANT(1, 0, LX_N_LO, LW_N_01, LC_N_23, 2, tgt_b);
-            VQ_NQUADRANT(1, 1, LX_N_HI, LW_N_23, LC_NB_01, 4, tgt_b);
+#define LC_N_23(q) load_c1(1, 2 + (q), cbuf_n, cshift_n, t_n, 0)
+#define LC_NB_01(q) load_c1(0, (q), cbuf_n, cshift_n, t_n, 1)
+        VQ_NQUADRANT(1, 0, LX_N_LO, LW_N_01, LC_N_23, 2, tgt_b);
+        VQ_NQUADRANT(1, 1, LX_N_HI, LW_N_23, LC_NB_01, 4, tgt_b);
 #undef LX_B_LO
 #undef LX_B_HI
 #undef LW_B_01
@@ -747,17 +764,21 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
 #undef LW_N_23
 #undef LC_N_23
 #undef LC_NB_01
-            buf = buf_next;
+        buf = buf_next;
         };
-        stage_body(std::integral_constant<int, 0>{});
-        if constexpr (C::STAGES == 2) stage_body(std::integral_constant<int, 1>{});
+    int super = 0;
+    do {
+        stage_body(super, std::integral_constant<int, 0>{});
+        if constexpr (C::STAGES == 2) stage_body(super, std::integral_constant<int, 1>{});
         cbuf = cbuf + 1 == NC ? 0 : cbuf + 1;
-    }
+    } while (++super < n_super - (HALF ? 1 : 0));
+    if constexpr (HALF) stage_body(n_super - 1, std::integral_constant<int, 0>{});  // (behind the loop: an exit from its middle costs spills)
 #undef VQ_NQUADRANT
 #undef VQ_FENCE
     wait_vmcnt<0>();
     __syncthreads();
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    if constexpr (HALF) hold_accumulators(acc);
 
     // ---- epilogue: lane holds Y[m = i*16 + r16][n = j*16 + 4*kg + 0..3] of its 128x64 wave tile --
     auto epilogue = [&](auto has_bias_const) {
@@ -881,7 +902,7 @@ TilePlan plan_tiles(const ProblemB &p)
 template <int VEC, typename CodeT>
 hipError_t launch_prefill_typed(const ProblemB &p, hipStream_t s, int tile, int n_end = 0)
 {
-    const bool tail = (p.K % kStageK) != 0;
+    const bool tail = (p.K % PrefillCfg<VEC, CodeT>::K_SUPER) != 0;
     const int tiles_m = (p.M + BM - 1) / BM;
     if (n_end <= 0 || n_end > p.N) n_end = p.N;
     int n_split = n_end;
@@ -933,8 +954,8 @@ hipError_t launch_prefill_typed(const ProblemB &p, hipStream_t s, int tile, int 
 template <int VEC, typename CodeT>
 bool prefill_cfg_supports(const ProblemB &p)
 {
-    // whole 16-byte code chunks per row, a tile's code offsets within 32 bits
-    return p.K % PrefillCfg<VEC, CodeT>::KC == 0 && lds_bytes<VEC, CodeT>(p, 2) <= kLdsLimit &&
+    // whole 16-byte code chunks per row (or a half one at its end), a tile's code offsets within 32 bits
+    return prefill_k_ok<VEC, CodeT>(p.K) && lds_bytes<VEC, CodeT>(p, 2) <= kLdsLimit &&
            (int64_t)BN * (p.K / VEC) * (int64_t)sizeof(CodeT) < ((int64_t)1 << 31) &&
            (int64_t)BM * p.K * 2 < ((int64_t)1 << 32);
 }

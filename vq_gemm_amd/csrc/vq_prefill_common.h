@@ -33,6 +33,15 @@ struct PrefillCfg {
     static constexpr int code_bufs(int ns) { return STAGES == 1 ? ns : 3; }
 };
 
+// K the kernels walk: whole 16-byte chunks of codes per row, or - where a chunk spans two stages - a last chunk of one
+// stage (8 bytes) behind at least one whole one.
+template <int VEC, typename CodeT>
+inline bool prefill_k_ok(int K)
+{
+    typedef PrefillCfg<VEC, CodeT> C;
+    return K % C::KC == 0 || (C::STAGES == 2 && K % kStageK == 0 && K > C::KC);
+}
+
 // Byte offset inside a stage buffer of logical 16-byte chunk cc (0..7) of X-tile row `row`.
 __device__ __forceinline__ int x_offset(int row, int cc)
 {

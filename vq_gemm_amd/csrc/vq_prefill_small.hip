@@ -16,10 +16,11 @@
 // One barrier per stage publishes stage+1 (X and, when it opens a code tile, the tile) and frees
 // the buffer of stage-1, into which the loads of stage+3 go.
 //
-// K must be a multiple of the k one code tile covers (64, or 128 for 8-vectors with 8-bit codes).
+// K must be a multiple of 64.  (A code tile covers 64 k, or 128 for 8-vectors with 8-bit codes; the HALF instantiation
+// ends with one of 64.)
 //
 // Split K.  Where even these tiles are fewer than the compute units, `splits` workgroups share a tile, each
-// multiplying k_len = K / splits of K.  Nothing waits for anything: a workgroup writes its fp32 sums to a partial
+// multiplying its share of K (whole code tiles).  Nothing waits for anything: a workgroup writes its fp32 sums to a partial
 // buffer with device-scope stores, waits for them, and counts itself in on the tile's counter; the one that
 // finds itself last adds the partial sums up in the order of the slices and runs the epilogue.  The sum is the same whoever comes last, so
 // results do not depend on the order in which the workgroups finish.
@@ -45,7 +46,8 @@ constexpr int small_code_bufs(int ns)
 }
 
 // SPLIT: the codebooks lie in the LDS in the split layout (vq_prefill_common.h).
-template <int VEC, typename CodeT, int NS, bool SPLIT>
+// HALF: K ends with a code tile of one stage (8-vectors with 8-bit codes, K % 128 == 64; as in prefill_kernel).
+template <int VEC, typename CodeT, int NS, bool SPLIT, bool HALF>
 __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t *__restrict__ x,
                                                                     const CodeT *__restrict__ codes,
                                                                     const half_t *__restrict__ cb,
@@ -53,7 +55,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
                                                                     const half_t *__restrict__ bias, int M, int K,
                                                                     int N, int n_begin, int ldn, int entries,
                                                                     int rows_per_cb, int tiles_m,
-                                                                    int tiles_n, int cb_lds_count, int gated, int k_len,
+                                                                    int tiles_n, int cb_lds_count, int gated,
                                                                     int splits, float4_t *__restrict__ partials,
                                                                     unsigned int *__restrict__ counters, int fenced)
 {
@@ -82,8 +84,12 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
     const int tm = wg / tiles_n, tn = wg % tiles_n;
     // The launch covers the W rows (columns of Y) [n_begin, N) of a problem with ldn rows in all.
     const int m0 = tm * SBM, n0 = n_begin + tn * SBN;
-    const int n_stage = k_len / kStageK;
-    const int n_super = n_stage / C::STAGES;
+    // K in whole code tiles, dealt to the slices as evenly as they go
+    const int k_supers = (K + C::K_SUPER - 1) / C::K_SUPER;
+    const int super0 = (int)((uint32_t)(split * k_supers) / (uint32_t)splits);
+    const int n_super = (int)((uint32_t)((split + 1) * k_supers) / (uint32_t)splits) - super0;
+    const bool half = HALF && split == splits - 1;  // this slice ends with a code tile of one stage
+    const int n_stage = n_super * C::STAGES - (half ? 1 : 0);
 
     // ---- per-lane codebook bases ------------------------------------------------------------
     const int g_first = n0 / rows_per_cb;
@@ -110,18 +116,22 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
         const int row = 2 * bank_row + (v >> 3), cc = v & 7;
         x_voff[i] = (uint32_t)(((int64_t)(min(m0 + row, M - 1) - m0) * K + cc * 8) * 2);
     }
-    const half_t *x_tile = x + (int64_t)m0 * K + (int64_t)split * k_len;
+    const half_t *x_tile = x + (int64_t)m0 * K + (int64_t)super0 * C::K_SUPER;
     // X load i (0..3) of a stage that starts at `xb` into buffer `buf`.
     auto issue_x = [&](int i, int buf, const half_t *xb) {
         load_to_lds_16(buf * kSmallStage + (4 * i + wave) * 1024, x_voff[i], xb);
     };
     // The code tile has 128 rows, two waves' worth: the waves of the lower half of the tile load
     // the same chunks to the same place again, which keeps every wave's load count the same.
-    const uint8_t *code_tile = reinterpret_cast<const uint8_t *>(codes + (int64_t)n0 * J + (int64_t)split * (k_len / VEC));
+    const uint8_t *code_tile = reinterpret_cast<const uint8_t *>(codes + (int64_t)n0 * J + (int64_t)super0 * (C::K_SUPER / VEC));
     uint32_t code_voff[C::CH];
 #pragma unroll
     for (int c = 0; c < C::CH; c++) code_voff[c] = (uint32_t)(min(wn * 64 + lane, N - 1 - n0) * J * C::CSZ) + c * 16;
     constexpr int kSuperBytes = C::K_SUPER / VEC * C::CSZ;  // bytes of one row's codes per code tile
+    // where code tile i (clamped to the last) starts; a last one of one stage is read as the 16 bytes that end the row
+    auto code_at = [&](int i) {
+        return code_tile + (int64_t)min(i, n_super - 1) * kSuperBytes - (half && i >= n_super - 1 ? 8 : 0);
+    };
     auto issue_codes = [&](int c, int cbuf, const uint8_t *cbase) {
         load_to_lds_16(kCodeBase + cbuf * kTile + c * (SBN * 16) + wn * 1024, code_voff[c], cbase);
     };
@@ -129,7 +139,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
     // Past the end the last stage (tile) is read again (harmless) instead of branching, so that
     // every stage brings the same number of loads; the pointers move on once per stage.
     const half_t *x_ahead = x_tile + min(D, n_stage - 1) * kStageK;
-    const uint8_t *c_ahead = code_tile + (int64_t)min(D / C::STAGES, n_super - 1) * kSuperBytes;
+    const uint8_t *c_ahead = code_at(D / C::STAGES);
 
     float4_t acc[SNP][SMP];
 #pragma unroll
@@ -152,9 +162,9 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
         xp[set][i] = *reinterpret_cast<const half8_t *>(smem + buf * kSmallStage + x_rd[i & 1][s] + (i >> 1) * 4096);
     };
     // the codes of W piece j for MFMA step s of stage t (of its code tile) out of code buffer `cbuf`
-    auto load_c1 = [&](int j, int cbuf, int t, int s) {
+    auto load_c1 = [&](int j, int cbuf, int shift, int t, int s) {
         const int pos = (t % C::STAGES) * 2 * C::HALF + s * C::HALF;
-        cr[j] = read_codes<C::RB>(smem + code_rd + cbuf * kTile + (pos / 16) * (SBN * 16) + j * 256 + pos % 16);
+        cr[j] = read_codes<C::RB>(smem + code_rd + cbuf * kTile + shift + (pos / 16) * (SBN * 16) + j * 256 + pos % 16);
     };
     auto load_w_half = [&](int set, int j, int h) {
         const half4_t v = gather4<VEC, CodeT, false, SPLIT>(smem, book[j], cr[j], h, false, 0);
@@ -183,7 +193,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
         if (d % C::STAGES == 0) {
 #pragma unroll
             for (int c = 0; c < C::CH; c++)
-                issue_codes(c, (d / C::STAGES) % NC, code_tile + (int64_t)min(d / C::STAGES, n_super - 1) * kSuperBytes);
+                issue_codes(c, (d / C::STAGES) % NC, code_at(d / C::STAGES));
         }
 #pragma unroll
         for (int i = 0; i < kSmallXLoads; i++) issue_x(i, d, x_tile + min(d, n_stage - 1) * kStageK);
@@ -206,7 +216,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
     int buf = 0, cbuf = 0;
     // step 0 of stage 0: all of its operands; then the codes of step 1
 #pragma unroll
-    for (int j = 0; j < SNP; j++) load_c1(j, cbuf, 0, 0);
+    for (int j = 0; j < SNP; j++) load_c1(j, cbuf, 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < SNP; j++) {
         load_w_half(0, j, 0);
@@ -215,75 +225,87 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
 #pragma unroll
     for (int i = 0; i < SMP; i++) load_x1(0, i, buf, 0);
 #pragma unroll
-    for (int j = 0; j < SNP; j++) load_c1(j, cbuf, 0, 1);
+    for (int j = 0; j < SNP; j++) load_c1(j, cbuf, 0, 0, 1);
 
 #define VQ_FENCE __builtin_amdgcn_sched_barrier(0)
-    for (int super = 0; super < n_super; super++) {
-        auto stage_body = [&](auto t_const) {
-            constexpr int t = decltype(t_const)::value;
-            const int stage = super * C::STAGES + t;
-            const int buf_next = buf + 1 == NS ? 0 : buf + 1;
-            // the loads of stage+D go into the buffer stage-1 was read from
-            const int tgt_buf = buf == 0 ? NS - 1 : buf - 1;
-            constexpr bool tgt_codes = (t + D) % C::STAGES == 0;
-            constexpr int d_super = (t + D) / C::STAGES;
-            const int tgt_cbuf = (cbuf + d_super) % NC;
-            // the stage after this one: same code tile or the next
-            constexpr bool same_super = t + 1 < C::STAGES;
-            const int cbuf_n = same_super ? cbuf : (cbuf + 1 == NC ? 0 : cbuf + 1);
-            constexpr int t_n = same_super ? t + 1 : 0;
-            // Publish stage+1: only what the stages behind it bring along may still be in flight.
-            constexpr int in_flight = [&]() constexpr {
-                int n = 0;
-                for (int d = 2; d < D; d++) n += loads_of(t + d);
-                return n;
-            }();
-            wait_vmcnt<in_flight>();
-            __syncthreads();
-            VQ_FENCE;
-            // A step: 16 MFMAs of set `set`; between them the gathers (in halves) and X reads of the
-            // next step into the other set, the codes of the step after that, and this step's share
-            // of the global loads.  A wave issues one instruction every four cycles and an MFMA holds
-            // the pipe for sixteen: a few instructions fit between two MFMAs.
+    auto stage_body = [&](int super, auto t_const) {
+        constexpr int t = decltype(t_const)::value;
+        const int stage = super * C::STAGES + t;
+        const int buf_next = buf + 1 == NS ? 0 : buf + 1;
+        // the loads of stage+D go into the buffer stage-1 was read from
+        const int tgt_buf = buf == 0 ? NS - 1 : buf - 1;
+        constexpr bool tgt_codes = (t + D) % C::STAGES == 0;
+        constexpr int d_super = (t + D) / C::STAGES;
+        const int tgt_cbuf = (cbuf + d_super) % NC;
+        // the stage after this one: same code tile or the next
+        constexpr bool same_super = t + 1 < C::STAGES;
+        const int cbuf_n = same_super ? cbuf : (cbuf + 1 == NC ? 0 : cbuf + 1);
+        constexpr int t_n = same_super ? t + 1 : 0;
+        const int cshift_n = HALF && half && super + (same_super ? 0 : 1) >= n_super - 1 ? 8 : 0;
+        // Publish stage+1: only what the stages behind it bring along may still be in flight.
+        constexpr int in_flight = [&]() constexpr {
+            int n = 0;
+            for (int d = 2; d < D; d++) n += loads_of(t + d);
+            return n;
+        }();
+        wait_vmcnt<in_flight>();
+        __syncthreads();
+        VQ_FENCE;
+        // A step: 16 MFMAs of set `set`; between them the gathers (in halves) and X reads of the
+        // next step into the other set, the codes of the step after that, and this step's share
+        // of the global loads.  A wave issues one instruction every four cycles and an MFMA holds
+        // the pipe for sixteen: a few instructions fit between two MFMAs.
 #pragma unroll
-            for (int step = 0; step < 2; step++) {
+        for (int step = 0; step < 2; step++) {
 #pragma unroll
-                for (int m = 0; m < SNP * SMP; m++) {
-                    mfma_one(step, m >> 2, m & 3);
+            for (int m = 0; m < SNP * SMP; m++) {
+                mfma_one(step, m >> 2, m & 3);
+                VQ_FENCE;
+                if (m < 2 * SNP) {
+                    load_w_half(step ^ 1, m >> 1, m & 1);
                     VQ_FENCE;
-                    if (m < 2 * SNP) {
-                        load_w_half(step ^ 1, m >> 1, m & 1);
+                    if (m & 1) {
+                        if (step == 0) load_x1(1, m >> 1, buf, 1);
+                        else load_x1(0, m >> 1, buf_next, 0);
                         VQ_FENCE;
-                        if (m & 1) {
-                            if (step == 0) load_x1(1, m >> 1, buf, 1);
-                            else load_x1(0, m >> 1, buf_next, 0);
-                            VQ_FENCE;
-                        }
-                    } else if (m < 3 * SNP) {
-                        // the gathers above have taken their addresses from cr[]: read the next codes
-                        if (step == 0) load_c1(m - 2 * SNP, cbuf_n, t_n, 0);
-                        else load_c1(m - 2 * SNP, cbuf_n, t_n, 1);
+                    }
+                } else if (m < 3 * SNP) {
+                    // the gathers above have taken their addresses from cr[]: read the next codes
+                    if (step == 0) load_c1(m - 2 * SNP, cbuf_n, cshift_n, t_n, 0);
+                    else load_c1(m - 2 * SNP, cbuf_n, cshift_n, t_n, 1);
+                    VQ_FENCE;
+                } else {
+                    const int q = m - 3 * SNP;  // 0..3
+                    if ((q & 1) == 0) {
+                        issue_x(2 * step + (q >> 1), tgt_buf, x_ahead);
                         VQ_FENCE;
-                    } else {
-                        const int q = m - 3 * SNP;  // 0..3
-                        if ((q & 1) == 0) {
-                            issue_x(2 * step + (q >> 1), tgt_buf, x_ahead);
-                            VQ_FENCE;
-                        } else if (tgt_codes && 2 * step + (q >> 1) < C::CH) {
-                            issue_codes(2 * step + (q >> 1), tgt_cbuf, c_ahead);
-                            VQ_FENCE;
-                        }
+                    } else if (tgt_codes && 2 * step + (q >> 1) < C::CH) {
+                        issue_codes(2 * step + (q >> 1), tgt_cbuf, c_ahead);
+                        VQ_FENCE;
                     }
                 }
             }
-            // the next stage loads stage+D+1, and with it the code tile that stage may open
-            x_ahead += stage + D + 1 < n_stage ? kStageK : 0;
-            if ((t + D + 1) % C::STAGES == 0) c_ahead += (stage + D + 1) / C::STAGES < n_super ? kSuperBytes : 0;
-            buf = buf_next;
-        };
-        stage_body(std::integral_constant<int, 0>{});
-        if constexpr (C::STAGES == 2) stage_body(std::integral_constant<int, 1>{});
+        }
+        // the next stage loads stage+D+1, and with it the code tile that stage may open
+        x_ahead += stage + D + 1 < n_stage ? kStageK : 0;
+        if ((t + D + 1) % C::STAGES == 0) {
+            const int next = (stage + D + 1) / C::STAGES;
+            c_ahead += next < n_super ? (HALF && half && next == n_super - 1 ? kSuperBytes - 8 : kSuperBytes) : 0;
+        }
+        buf = buf_next;
+    };
+    const int n_whole = n_super - (half ? 1 : 0);  // (at least one)
+    int super = 0;
+    do {
+        stage_body(super, std::integral_constant<int, 0>{});
+        if constexpr (C::STAGES == 2) stage_body(super, std::integral_constant<int, 1>{});
         cbuf = cbuf + 1 == NC ? 0 : cbuf + 1;
+    } while (++super < n_whole);
+    if constexpr (HALF) {
+        // (the MFMAs are opaque to the compiler: let them leave the pipe ahead of a branch, where it may copy accumulators)
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        VQ_FENCE;
+        if (half) stage_body(n_super - 1, std::integral_constant<int, 0>{});
     }
 #undef VQ_FENCE
     // Drain the clamped loads still in flight before the stage buffers are reused.
@@ -291,6 +313,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
     __syncthreads();
     // the last MFMAs must have left the pipe before the accumulators are read
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    if constexpr (HALF) hold_accumulators(acc);
 
     // ---- split K: partial sums out, and the workgroup that comes last adds them up -------------------
     // The partial sums are written and read with device-scope memory instructions (sc1: through the L2 of the
@@ -424,7 +447,7 @@ template <int VEC, typename CodeT>
 bool small_cfg_supports(const ProblemB &p)
 {
     typedef PrefillCfg<VEC, CodeT> C;
-    return p.K >= C::K_SUPER && p.K % C::K_SUPER == 0 && lds_bytes_small<VEC, CodeT>(p, 4) <= kLdsLimit &&
+    return p.K >= C::K_SUPER && (p.K % C::K_SUPER == 0 || (C::STAGES == 2 && prefill_k_ok<VEC, CodeT>(p.K))) && lds_bytes_small<VEC, CodeT>(p, 4) <= kLdsLimit &&
            (int64_t)SBN * (p.K / VEC) * (int64_t)sizeof(CodeT) < ((int64_t)1 << 31) &&
            (int64_t)SBM * p.K * 2 < ((int64_t)1 << 32);
 }
@@ -438,7 +461,7 @@ hipError_t launch_small_typed(const ProblemB &p, hipStream_t s, int splits, void
 {
     typedef PrefillCfg<VEC, CodeT> C;
     if (!small_cfg_supports<VEC, CodeT>(p)) return hipErrorInvalidValue;
-    if (splits < 1 || p.K % splits != 0 || (p.K / splits) % C::K_SUPER != 0 || (splits > 1 && !workspace)) return hipErrorInvalidValue;
+    if (splits < 1 || (splits > 1 && (!workspace || p.K / C::K_SUPER < 2 * splits))) return hipErrorInvalidValue;
     if (n_begin < 0 || n_begin >= p.N || n_begin % SBN != 0) return hipErrorInvalidValue;
     const int tiles_m = (p.M + SBM - 1) / SBM, tiles_n = (p.N - n_begin + SBN - 1) / SBN;
     // workspace: the tiles' counters (cleared here, by a kernel: the launch may be captured), then the partial sums
@@ -454,12 +477,15 @@ hipError_t launch_small_typed(const ProblemB &p, hipStream_t s, int splits, void
     // the split codebook layout is built out of a copy in the last X buffer
     constexpr bool can_split = VEC == 8 && sizeof(CodeT) == 1;
     const bool split = can_split && split_layout_applies(p, codebooks_per_tile(p, SBN), kSmallStage);
-    auto kern = split ? prefill_small_kernel<VEC, CodeT, 4, can_split> : prefill_small_kernel<VEC, CodeT, 4, false>;
+    constexpr bool can_half = C::STAGES == 2;
+    const bool half = p.K % C::K_SUPER != 0;
+    auto kern = half ? (split ? prefill_small_kernel<VEC, CodeT, 4, can_split, can_half> : prefill_small_kernel<VEC, CodeT, 4, false, can_half>)
+                     : (split ? prefill_small_kernel<VEC, CodeT, 4, can_split, false> : prefill_small_kernel<VEC, CodeT, 4, false, false>);
     const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), smem);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(kThreads), smem, s, p.x,
                        static_cast<const CodeT *>(p.codes), p.cb, p.y, p.bias, p.M, p.K, p.N, n_begin, p.N, p.entries,
-                       p.rows_per_cb, tiles_m, tiles_n, codebooks_per_tile(p, SBN), p.gated ? 1 : 0, p.K / splits, splits, partials, counters,
+                       p.rows_per_cb, tiles_m, tiles_n, codebooks_per_tile(p, SBN), p.gated ? 1 : 0, splits, partials, counters,
                        tuning().splitk_validate_fences >= 1.0 ? 1 : 0);
     return hipGetLastError();
 }
@@ -524,10 +550,10 @@ size_t prefill_splitk_workspace_bytes(const ProblemB &p, int splits)
     return prefill_splitk_counter_bytes(tiles) + (size_t)tiles * splits * kPartialBytes;
 }
 
+// (a slice is at least two code tiles: the loads run that far ahead)
 bool prefill_splitk_supports(const ProblemB &p, int splits)
 {
-    return splits >= 2 && splits <= 8 && prefill_small_supports(p) && p.K % splits == 0 && (p.K / splits) % small_k_super(p) == 0 &&
-           p.K / splits >= 2 * small_k_super(p);
+    return splits >= 2 && splits <= 8 && prefill_small_supports(p) && p.K / small_k_super(p) >= 2 * splits;
 }
 
 // The number of slices of K (1: none) that the cost model expects to be fastest with 128x128 tiles, and its time.

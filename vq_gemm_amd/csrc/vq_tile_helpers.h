@@ -33,6 +33,18 @@ __device__ __forceinline__ void st_global_16_streaming(void *p, uint4_t v)
     __builtin_nontemporal_store(v, reinterpret_cast<uint4_t *>(p));
 }
 
+// Holds the accumulators where they are (the AGPRs) up to here.  Called behind the wait for the last MFMAs: the compiler
+// does not see what an inline-assembly MFMA is still writing, and where a loop's last pass is peeled off it would copy
+// each accumulator out right behind its last MFMA.
+template <int A, int B>
+__device__ __forceinline__ void hold_accumulators(float4_t (&acc)[A][B])
+{
+#pragma unroll
+    for (int a = 0; a < A; a++)
+#pragma unroll
+        for (int b = 0; b < B; b++) asm volatile("" : "+a"(acc[a][b]));
+}
+
 }  // namespace
 
 }  // namespace vq
