@@ -212,6 +212,24 @@ int vqgemm_encode_b(const void *w, const void *codebook, void *codes_out,
                     int32_t n_codebooks, int32_t code_bits, void *stream);
 
 /*
+ * Lloyd iterations (k-means) of the quantiser as one call, geometry B: `iters` times assignment (vqgemm_encode_b's rule) and
+ * centroid update, then a last assignment.  Entry e of codebook g starts as vector pick[g*entries + e] (int32) of the
+ * codebook's block, rows [g*N/n_codebooks, (g+1)*N/n_codebooks) of w read as a flat array of vectors; an entry nothing was
+ * assigned to keeps its value.  codes_out [N, K/vec] and codebook_out [n_codebooks, entries, vec] fp16 belong together
+ * (the codes are the nearest entries of the codebook returned); errors_out[0 .. iters] is the sum of squared differences
+ * after each assignment, in double.  workspace: vqgemm_kmeans_workspace_bytes_b() bytes of device memory, 256-byte
+ * aligned; w must be 8-byte aligned.  VQGEMM_E_VARIANT (also the size function's answer) where the per-entry sums do not fit
+ * the LDS (more than about 1400 entries of 8-vectors).
+ * No counterpart in the reference.
+ */
+int64_t vqgemm_kmeans_workspace_bytes_b(int64_t N, int64_t K, int32_t vec, int32_t entries,
+                                        int32_t n_codebooks, int32_t code_bits);
+int vqgemm_kmeans_b(const void *w, const int32_t *pick, void *codes_out, void *codebook_out,
+                    double *errors_out, int64_t N, int64_t K, int32_t vec, int32_t entries,
+                    int32_t n_codebooks, int32_t code_bits, int32_t iters, void *workspace,
+                    int64_t workspace_bytes, void *stream);
+
+/*
  * Element-wise pass behind a gate/up projection pair (the MLP shapes among the measured
  * configurations): out[m, n] = silu(gate_up[m, n]) * gate_up[m, N + n], gate_up [M, 2N] fp16 being
  * one fused VQ GEMM over the gate rows of W stacked on its up rows; silu(g) = g / (1 + exp(-g)),

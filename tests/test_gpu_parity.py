@@ -1871,3 +1871,49 @@ def test_widths_that_are_no_multiple_of_a_tile_or_a_slice(row):
         torch.cuda.synchronize()
         e1, e2 = vo.rel_err(_np(y), vo.gated_gemm_b(_np(x), _np(codes)[:n], _np(cb)).astype(np.float64))
         assert e2 <= TOL and e1 <= 2 * TOL, (name, "gated", e1, e2)
+
+
+LLOYD_B = [
+    # N, K, vec, entries, G: codebooks in several workgroups, entries nothing is assigned to, a last tile of entries cut short
+    (512, 1024, 8, 256, 2),
+    (48, 264, 8, 33, 1),
+    (96, 128, 4, 700, 3),
+    (10, 64, 2, 5, 5),
+    (8, 32, 8, 64, 1),      # fewer vectors than entries
+]
+
+
+@pytest.mark.parametrize("row", LLOYD_B, ids=["x".join(map(str, r)) for r in LLOYD_B])
+def test_lloyd_iterations_on_the_device_against_the_definition(row):
+    from vq_gemm_amd.quantize import _initial_vectors
+    from vq_gemm_amd.torch_ops import native
+    N, K, v, E, G = row
+    _say("lloyd", row)
+    g = torch.Generator(device="cpu").manual_seed(7)
+    w = (torch.randn(N, K, generator=g) * 0.05).half().to(DEV)
+    bits = 8 if E <= 256 else 16
+    per_cb = N // G * (K // v)
+    pick = _initial_vectors(per_cb, E, G, 3)
+    vectors = _np(w).reshape(G, per_cb, v)
+    book = np.stack([vectors[i][pick[i].numpy()] for i in range(G)])
+    for iters in (0, 1, 2):
+        codes, cb, errors = native.kmeans(w, pick, v, E, G, bits, iters)
+        torch.cuda.synchronize()
+        # the codes are the encoder's for the codebook returned, the last error is theirs
+        assert torch.equal(codes, cabi.encode_b(w, cb, bits))
+        c = _np(codes).astype(np.int64).reshape(G, per_cb)
+        got = _np(cb)
+        sq = sum(((got[i][c[i]].astype(np.float64) - vectors[i].astype(np.float64)) ** 2).sum() for i in range(G))
+        assert errors.shape == (iters + 1,) and float(errors[-1]) == pytest.approx(sq, rel=1e-5, abs=1e-12)
+        if iters == 0:
+            assert np.array_equal(got, book)
+        elif iters == 1:
+            # the update of the first assignment: means in float64, an fp16 last place for the order of the fp32 sums
+            c0 = c_oracle.encode_b(_np(w), book, bits).astype(np.int64).reshape(G, per_cb)
+            for i in range(G):
+                for e in range(E):
+                    mine = vectors[i][c0[i] == e].astype(np.float64)
+                    if len(mine) == 0:
+                        assert np.array_equal(got[i, e], book[i, e])
+                    else:
+                        assert np.allclose(got[i, e].astype(np.float64), mine.mean(axis=0), rtol=1.1e-3, atol=1e-6)

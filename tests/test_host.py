@@ -183,3 +183,13 @@ def test_vqlinear_codes_key_works_on_inference_tensors():
     k2 = layer2._codes_key()
     layer2.codes.add_(1)
     assert layer2._codes_key() != k2
+
+
+@pytest.mark.parametrize("n,count,books,seed", [(1, 1, 3, 0), (2, 2, 2, 5), (256, 256, 4, 1), (700, 256, 3, 4294967295), (5000, 1, 2, 7), (262144, 256, 3, 0)])
+def test_start_of_a_seeded_permutation_is_torch_randperm_s(n, count, books, seed):
+    from vq_gemm_amd.quantize import _initial_vectors
+    from vq_gemm_amd.torch_ops import native
+    gen = torch.Generator().manual_seed(seed)
+    want = torch.stack([torch.randperm(n, generator=gen)[:count] for _ in range(books)]).to(torch.int32)
+    assert torch.equal(native.first_of_permutations(n, count, books, seed), want)
+    assert torch.equal(_initial_vectors(n, count, books, seed), want)

@@ -15,6 +15,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include "../../include/vq_gemm.h"
+#include "seeded_pick.h"
 
 namespace {
 
@@ -253,6 +254,41 @@ py::object gated(const Tensor &x, const Tensor &codes, const Tensor &codebook, c
     return py::cast(gated_impl(x, codes, codebook, bias));
 }
 
+// ---- the quantiser --------------------------------------------------------------------------------------------
+
+// int32 [books, count] on the host: row g is the start of the g-th permutation of 0 .. n-1 that a generator seeded with `seed` makes
+Tensor first_of_permutations(int64_t n, int64_t count, int64_t books, int64_t seed)
+{
+    TORCH_CHECK_VALUE(count >= 0 && count <= n && n <= (int64_t(1) << 24) && books >= 1, "first_of_permutations: 0 <= count <= n <= 2^24");
+    Tensor pick = at::empty({books, count}, at::kInt);
+    vq::Mt19937 gen((uint32_t)((uint64_t)seed & 0xffffffffu));
+    for (int64_t g = 0; g < books; g++) {
+        vq::first_of_permutation(gen, n, count, g + 1 < books, pick.data_ptr<int32_t>() + g * count);
+    }
+    return pick;
+}
+
+// (codes, codebook, squared errors [iters + 1] on the device) of Lloyd iterations from the vectors `pick`, or None where the library
+// has no kernel for the codebook's size.  The caller has checked w: fp16 [N, K] on the GPU, contiguous.
+py::object kmeans(const Tensor &w, const Tensor &pick, int64_t vec, int64_t entries, int64_t books, int64_t code_bits, int64_t iters)
+{
+    const int64_t N = w.size(0), K = w.size(1);
+    TORCH_CHECK_VALUE(w.is_cuda() && w.scalar_type() == at::kHalf && w.is_contiguous() && pick.scalar_type() == at::kInt &&
+                          pick.numel() == books * entries && pick.is_contiguous() && vec > 0 && K % vec == 0 && books > 0 && N % books == 0,
+                      "kmeans: w fp16 [N, K] on the GPU, pick int32 [books, entries]");
+    const int64_t need = vqgemm_kmeans_workspace_bytes_b(N, K, (int)vec, (int)entries, (int)books, (int)code_bits);
+    if (need < 0 || (reinterpret_cast<uintptr_t>(w.data_ptr()) & 7) != 0) return py::none();
+    const c10::OptionalDeviceGuard guard(w.device());
+    const Tensor pick_d = pick.to(w.device());
+    auto on_device = [&](at::IntArrayRef shape, at::ScalarType t) { return at::detail::empty_cuda(shape, t, w.device(), c10::nullopt); };
+    Tensor codes = on_device({N, K / vec}, code_bits == 8 ? at::kByte : at::kUInt16);
+    Tensor codebook = on_device({books, entries, vec}, at::kHalf), errors = on_device({iters + 1}, at::kDouble), ws = on_device({need}, at::kByte);
+    check_rc(vqgemm_kmeans_b(w.data_ptr(), pick_d.data_ptr<int32_t>(), codes.data_ptr(), codebook.data_ptr(), errors.data_ptr<double>(), N, K,
+                             (int)vec, (int)entries, (int)books, (int)code_bits, (int)iters, ws.data_ptr(), need, stream_of(w)),
+             "kmeans");
+    return py::make_tuple(codes, codebook, errors);
+}
+
 }  // namespace
 
 TORCH_LIBRARY(vq_gemm_amd, m)
@@ -282,5 +318,7 @@ TORCH_LIBRARY_IMPL(vq_gemm_amd, AutogradCUDA, m)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.def("linear", &linear, "x @ W.T (+ bias) on plain GPU tensors; None where the registered operator is to be called instead");
+    m.def("first_of_permutations", &first_of_permutations, "the first elements of seeded random permutations");
+    m.def("kmeans", &kmeans, "Lloyd iterations on the device; None where the codebook is too large for them");
     m.def("gated", &gated, "silu(gate) * up likewise");
 }

@@ -644,6 +644,33 @@ int vqgemm_encode_b(const void *w, const void *codebook, void *codes_out, int64_
     return static_cast<int>(launch_encode_b(static_cast<const half_t *>(w), p, codes_out, static_cast<hipStream_t>(stream)));
 }
 
+int64_t vqgemm_kmeans_workspace_bytes_b(int64_t N, int64_t K, int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits)
+{
+    const int rc = check_b(0, K, N, vec, entries, n_codebooks, code_bits);
+    if (rc != VQGEMM_OK) return rc;
+    if (N == 0 || K == 0) return VQGEMM_E_VARIANT;
+    const ProblemB p = make_b(nullptr, nullptr, nullptr, nullptr, 0, K, N, vec, entries, n_codebooks, code_bits);
+    if (!lloyd_supports(p) || (int64_t)p.rows_per_cb * (K / vec) > INT_MAX) return VQGEMM_E_VARIANT;
+    return (int64_t)lloyd_workspace_bytes(p);
+}
+
+int vqgemm_kmeans_b(const void *w, const int32_t *pick, void *codes_out, void *codebook_out, double *errors_out, int64_t N, int64_t K,
+                    int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits, int32_t iters, void *workspace,
+                    int64_t workspace_bytes, void *stream)
+{
+    const int64_t need = vqgemm_kmeans_workspace_bytes_b(N, K, vec, entries, n_codebooks, code_bits);
+    if (need < 0) return (int)need;
+    if (iters < 0) return VQGEMM_E_SHAPE;
+    if (!w || !pick || !codes_out || !codebook_out || !errors_out || !workspace) return VQGEMM_E_NULL;
+    if (!aligned(w, 8) || !aligned(pick, 4) || !aligned(codebook_out, 4) || !aligned(codes_out, code_bits / 8) || !aligned(errors_out, 8) ||
+        !aligned(workspace, 256))
+        return VQGEMM_E_ALIGN;
+    if (workspace_bytes < need) return VQGEMM_E_SCRATCH;
+    const ProblemB p = make_b(nullptr, nullptr, nullptr, nullptr, 0, K, N, vec, entries, n_codebooks, code_bits);
+    return static_cast<int>(launch_lloyd(static_cast<const half_t *>(w), p, pick, iters, codes_out, static_cast<half_t *>(codebook_out),
+                                         errors_out, workspace, static_cast<hipStream_t>(stream)));
+}
+
 int vqgemm_silu_mul(const void *gate_up, void *out, int64_t M, int64_t N, void *stream)
 {
     if (M < 0 || N < 0 || M > INT_MAX / 2 || N > INT_MAX / 4) return VQGEMM_E_SHAPE;

@@ -79,6 +79,13 @@ hipError_t launch_dequant_a(const ProblemA &p, half_t *w_out, hipStream_t s);
 bool encode_supports(const ProblemB &p);
 hipError_t launch_encode_b(const half_t *w, const ProblemB &p, void *codes_out, hipStream_t s);
 
+// Lloyd iterations from the entries `pick` (int32 [G, E], vectors of each codebook's block): codes and codebook of the last
+// assignment, and errors[0 .. iters] = the sum of squared differences after each assignment (vq_lloyd.hip)
+bool lloyd_supports(const ProblemB &p);
+size_t lloyd_workspace_bytes(const ProblemB &p);
+hipError_t launch_lloyd(const half_t *w, const ProblemB &p, const int32_t *pick, int iters, void *codes_out, half_t *cb_out,
+                        double *errors, void *workspace, hipStream_t s);
+
 hipError_t launch_generic_b(const ProblemB &p, hipStream_t s);
 hipError_t launch_generic_a(const ProblemA &p, hipStream_t s);
 

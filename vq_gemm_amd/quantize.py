@@ -2,9 +2,10 @@
 
 The reference only ever multiplies random codes (its harness draws them, bench.py:84); this is
 the step before the path for real weights.  Plain Lloyd iterations per codebook block: the
-assignment step (by far the heaviest: every vector against every entry) runs in the library's HIP
-encoder (vqgemm_encode_b), the centroid update is a handful of torch reductions on the device.
-Nothing here runs on the CPU and nothing falls back to it.
+assignment step (every vector against every entry) and the centroid update run in the library
+(vqgemm_kmeans_b), nothing coming back to the host in between; codebooks too large for its kernels take the
+encoder (vqgemm_encode_b) and a handful of torch reductions on the device.  Only the initial entries are drawn on the
+host; nothing falls back to the CPU.
 
 `residual_quantize` is the additive ("residual") mode the reference names in an unused macro
 (`RESIDUAL`, strategy_1/src.cu:18-19) and never implements: W ~ sum over stages s of
@@ -37,16 +38,18 @@ def kmeans_quantize(w, vec: int, entries: int, n_codebooks: int = 1, iters: int 
     w = w.contiguous()
     G, J = n_codebooks, K // vec
     per_cb = (N // G) * J                                     # vectors per codebook block
-    vectors = w.view(G, per_cb, vec)
-    gen = torch.Generator(device="cpu").manual_seed(seed)
-    # initial entries: distinct random vectors of the block (with repetition when the block is small)
-    if per_cb >= entries:
-        pick = torch.stack([torch.randperm(per_cb, generator=gen)[:entries] for _ in range(G)])
-    else:
-        pick = torch.randint(0, per_cb, (G, entries), generator=gen)
-    pick = pick.to(w.device)
-    codebook = torch.gather(vectors, 1, pick[:, :, None].expand(G, entries, vec)).contiguous()
     code_bits = 8 if entries <= 256 else 16
+    pick = _initial_vectors(per_cb, entries, G, seed)
+    if vec in (2, 4, 8) and 0 < per_cb < 2 ** 31 and iters >= 0:
+        # the iterations as one call on the device (None: more entries than its kernels keep sums for)
+        from .torch_ops import native
+        done = native.kmeans(w, pick, vec, entries, G, code_bits, iters)
+        if done is not None:
+            codes, codebook, errors = done
+            return codes, codebook, (errors / w.numel()).tolist()
+    vectors = w.view(G, per_cb, vec)
+    pick = pick.to(w.device).to(torch.int64)
+    codebook = torch.gather(vectors, 1, pick[:, :, None].expand(G, entries, vec)).contiguous()
     vf = vectors.float()
     history = []
     codes = None
@@ -65,6 +68,28 @@ def kmeans_quantize(w, vec: int, entries: int, n_codebooks: int = 1, iters: int 
         # an entry nothing was assigned to keeps its value
         codebook = torch.where(counts[:, :, None] > 0, mean, codebook.float()).half().contiguous()
     return codes, codebook, history
+
+
+_permutation_start_known = None  # whether `native.first_of_permutations` is what torch.randperm makes on this build
+
+
+def _initial_vectors(per_cb: int, entries: int, n_codebooks: int, seed: int):
+    """int32 [G, entries] on the host: which vectors of each codebook's block the entries start as - distinct random ones (the
+    start of a random permutation), with repetition where the block is smaller than the codebook."""
+    import torch
+
+    global _permutation_start_known
+    gen = torch.Generator(device="cpu").manual_seed(seed)
+    if per_cb < entries:
+        return torch.randint(0, per_cb, (n_codebooks, entries), generator=gen).to(torch.int32)
+    from .torch_ops import native
+    if _permutation_start_known is None:
+        probe = torch.Generator(device="cpu").manual_seed(2024)
+        want = torch.stack([torch.randperm(1500, generator=probe, dtype=torch.int32)[:700] for _ in range(2)])
+        _permutation_start_known = torch.equal(native.first_of_permutations(1500, 700, 2, 2024), want)
+    if _permutation_start_known and 0 <= seed < 2 ** 32 and per_cb <= 2 ** 24:
+        return native.first_of_permutations(per_cb, entries, n_codebooks, seed)
+    return torch.stack([torch.randperm(per_cb, generator=gen)[:entries] for _ in range(n_codebooks)]).to(torch.int32)
 
 
 def residual_quantize(w, vec: int, entries: int, stages: int = 2, n_codebooks: int = 1, iters: int = 10, seed: int = 0):
