@@ -15,12 +15,41 @@
 
 namespace vq {
 
+namespace {
+
+// the current device while a DeviceScope is alive on this thread, and how many are
+thread_local int t_device = -1, t_scopes = 0;
+
+int current_device()
+{
+    if (t_scopes > 0) return t_device;
+    int dev = -1;
+    return hipGetDevice(&dev) == hipSuccess ? dev : -1;
+}
+
+struct ResolvedKernel {
+    const void *kernel = nullptr;
+    int device = -1;
+    hipFunction_t function = nullptr;
+    size_t granted = 48 * 1024;  // dynamic LDS a launch may ask for; this much needs no leave
+};
+
+}  // namespace
+
+DeviceScope::DeviceScope()
+{
+    if (t_scopes == 0) t_device = current_device();
+    t_scopes++;
+}
+
+DeviceScope::~DeviceScope() { t_scopes--; }
+
 int device_cu_count()
 {
     constexpr int kMaxDev = 64;
     static std::atomic<int> cache[kMaxDev];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return 256;
+    const int dev = current_device();
+    if (dev < 0 || dev >= kMaxDev) return 256;
     int v = cache[dev].load(std::memory_order_relaxed);
     if (v > 0) return v;
     int cus = 0;
@@ -29,20 +58,37 @@ int device_cu_count()
     return cus;
 }
 
-hipError_t ensure_dynamic_lds(const void *kernel, size_t bytes)
+hipError_t resolve_kernel(const void *kernel, size_t lds_bytes, hipFunction_t *function)
 {
-    if (bytes <= 48 * 1024) return hipSuccess;  // within the default limit
+    // a small table per thread in front of the shared one: a serving thread launches few kernels, again and again
+    constexpr int kSlots = 64;
+    thread_local ResolvedKernel recent[kSlots];
     static std::mutex mu;
-    static std::map<std::pair<int, const void *>, size_t> granted;
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(mu);
-    size_t &g = granted[{dev, kernel}];
-    if (bytes <= g) return hipSuccess;
-    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e == hipSuccess) g = bytes;
-    return e;
+    static std::map<std::pair<int, const void *>, ResolvedKernel> known;
+    const int dev = current_device();
+    if (dev < 0) return hipErrorInvalidDevice;
+    ResolvedKernel &slot = recent[((reinterpret_cast<uintptr_t>(kernel) >> 4) * 0x9e3779b97f4a7c15ull) >> 58];
+    if (slot.kernel != kernel || slot.device != dev || lds_bytes > slot.granted) {
+        std::lock_guard<std::mutex> lock(mu);
+        ResolvedKernel &k = known[{dev, kernel}];
+        if (!k.function) {
+            const hipError_t e = hipGetFuncBySymbol(&k.function, kernel);
+            if (e != hipSuccess) {
+                k.function = nullptr;
+                return e;
+            }
+            k.kernel = kernel;
+            k.device = dev;
+        }
+        if (lds_bytes > k.granted) {
+            const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+            if (e != hipSuccess) return e;
+            k.granted = lds_bytes;
+        }
+        slot = k;
+    }
+    *function = slot.function;
+    return hipSuccess;
 }
 
 namespace {
@@ -271,6 +317,7 @@ const char *vqgemm_error_string(int code)
 int vqgemm_select_variant_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks,
                             int32_t code_bits)
 {
+    const DeviceScope device;
     const int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
     if (rc != VQGEMM_OK) return rc;
     const ProblemB p = make_b(nullptr, nullptr, nullptr, nullptr, M, K, N, vec, entries, n_codebooks, code_bits);
@@ -281,6 +328,7 @@ int vqgemm_e2e_gemm_b_bias(const void *x, const void *codes, const void *codeboo
                            int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks,
                            int32_t code_bits, int32_t variant, void *workspace, void *stream)
 {
+    const DeviceScope device;
     int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
     if (rc != VQGEMM_OK) return rc;
     if (variant < VQGEMM_VARIANT_AUTO || variant > VQGEMM_VARIANT_DECODE_GEMV) return VQGEMM_E_VARIANT;
@@ -400,6 +448,7 @@ WorkspaceChoice workspace_auto(const ProblemB &p, bool all_aligned16)
 int64_t vqgemm_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks,
                                  int32_t code_bits, int32_t variant)
 {
+    const DeviceScope device;
     const int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
     if (rc != VQGEMM_OK) return rc;
     if (M == 0 || N == 0 || K == 0) return 0;
@@ -415,6 +464,7 @@ int vqgemm_e2e_gemm_b_ws(const void *x, const void *codes, const void *codebook,
                          int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits,
                          int32_t variant, void *workspace, int64_t workspace_bytes, void *stream)
 {
+    const DeviceScope device;
     if (workspace_bytes < 0 || (workspace_bytes > 0 && !workspace)) return VQGEMM_E_NULL;
     if (variant == VQGEMM_VARIANT_TWOPASS) {
         if (workspace_bytes < N * K * 2) return VQGEMM_E_SCRATCH;
@@ -453,6 +503,7 @@ int vqgemm_e2e_gemm_b_gated(const void *x, const void *codes, const void *codebo
                             int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits,
                             int32_t variant, void *workspace, void *stream)
 {
+    const DeviceScope device;
     int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
     if (rc != VQGEMM_OK) return rc;
     if (N % 32 != 0) return VQGEMM_E_SHAPE;  // whole pairs of 16 gate rows and 16 up rows
@@ -543,6 +594,7 @@ int vqgemm_e2e_gemm_b(const void *x, const void *codes, const void *codebook, vo
 int vqgemm_e2e_gemm_a(const void *x, const void *w, const void *codebook, void *out, int64_t M, int64_t K,
                       int64_t Nc, int32_t variant, void *workspace, void *stream)
 {
+    const DeviceScope device;
     if (M < 0 || K < 0 || Nc < 0 || M > INT_MAX / 2 || K > INT_MAX / 2 || Nc > INT_MAX / 4) return VQGEMM_E_SHAPE;
     if (Nc % 4 != 0) return VQGEMM_E_SHAPE;
     if (variant < VQGEMM_VARIANT_AUTO || variant > VQGEMM_VARIANT_TWOPASS) return VQGEMM_E_VARIANT;
@@ -586,6 +638,7 @@ int vqgemm_e2e_gemm_a(const void *x, const void *w, const void *codebook, void *
 
 int vqgemm_select_variant_a(int64_t M, int64_t K, int64_t Nc, int32_t has_workspace)
 {
+    const DeviceScope device;
     if (M < 0 || K < 0 || Nc < 0 || M > INT_MAX / 2 || K > INT_MAX / 2 || Nc > INT_MAX / 4 || Nc % 4 != 0) return VQGEMM_E_SHAPE;
     ProblemA p = {};
     p.M = (int)M; p.K = (int)K; p.Nc = (int)Nc;
@@ -596,6 +649,7 @@ int vqgemm_select_variant_a(int64_t M, int64_t K, int64_t Nc, int32_t has_worksp
 int vqgemm_dequant_b(const void *codes, const void *codebook, void *w_out, int64_t N, int64_t K, int32_t vec,
                      int32_t entries, int32_t n_codebooks, int32_t code_bits, void *stream)
 {
+    const DeviceScope device;
     const int rc = check_b(0, K, N, vec, entries, n_codebooks, code_bits);
     if (rc != VQGEMM_OK) return rc;
     if (N == 0 || K == 0) return VQGEMM_OK;
@@ -608,6 +662,7 @@ int vqgemm_dequant_b(const void *codes, const void *codebook, void *w_out, int64
 int vqgemm_pack_codes_b(const void *codes, void *codes_out, int64_t N, int64_t K, int32_t vec, int32_t code_bits,
                         int32_t inverse, void *stream)
 {
+    const DeviceScope device;
     if (N < 0 || K < 0 || N > INT_MAX / 2 || K > INT_MAX / 2) return VQGEMM_E_SHAPE;
     if (code_bits != 8 && code_bits != 16) return VQGEMM_E_CODEBITS;
     if (vec < 1 || K % vec != 0) return VQGEMM_E_SHAPE;
@@ -623,6 +678,7 @@ int vqgemm_pack_codes_b(const void *codes, void *codes_out, int64_t N, int64_t K
 int vqgemm_decode_packed_supports(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks,
                                   int32_t code_bits)
 {
+    const DeviceScope device;
     const int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
     if (rc != VQGEMM_OK) return rc;
     if (M == 0 || N == 0 || K == 0) return 0;
@@ -634,6 +690,7 @@ int vqgemm_decode_packed_supports(int64_t M, int64_t K, int64_t N, int32_t vec, 
 int vqgemm_encode_b(const void *w, const void *codebook, void *codes_out, int64_t N, int64_t K, int32_t vec,
                     int32_t entries, int32_t n_codebooks, int32_t code_bits, void *stream)
 {
+    const DeviceScope device;
     const int rc = check_b(0, K, N, vec, entries, n_codebooks, code_bits);
     if (rc != VQGEMM_OK) return rc;
     if (N == 0 || K == 0) return VQGEMM_OK;
@@ -646,6 +703,7 @@ int vqgemm_encode_b(const void *w, const void *codebook, void *codes_out, int64_
 
 int64_t vqgemm_kmeans_workspace_bytes_b(int64_t N, int64_t K, int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits)
 {
+    const DeviceScope device;
     const int rc = check_b(0, K, N, vec, entries, n_codebooks, code_bits);
     if (rc != VQGEMM_OK) return rc;
     if (N == 0 || K == 0) return VQGEMM_E_VARIANT;
@@ -658,6 +716,7 @@ int vqgemm_kmeans_b(const void *w, const int32_t *pick, void *codes_out, void *c
                     int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits, int32_t iters, void *workspace,
                     int64_t workspace_bytes, void *stream)
 {
+    const DeviceScope device;
     const int64_t need = vqgemm_kmeans_workspace_bytes_b(N, K, vec, entries, n_codebooks, code_bits);
     if (need < 0) return (int)need;
     if (iters < 0) return VQGEMM_E_SHAPE;
@@ -673,6 +732,7 @@ int vqgemm_kmeans_b(const void *w, const int32_t *pick, void *codes_out, void *c
 
 int vqgemm_silu_mul(const void *gate_up, void *out, int64_t M, int64_t N, void *stream)
 {
+    const DeviceScope device;
     if (M < 0 || N < 0 || M > INT_MAX / 2 || N > INT_MAX / 4) return VQGEMM_E_SHAPE;
     if (M == 0 || N == 0) return VQGEMM_OK;
     if (!gate_up || !out) return VQGEMM_E_NULL;
@@ -683,6 +743,7 @@ int vqgemm_silu_mul(const void *gate_up, void *out, int64_t M, int64_t N, void *
 
 int vqgemm_max_code(const void *codes, int64_t count, int32_t code_bits, void *max_out, void *stream)
 {
+    const DeviceScope device;
     if (count < 0) return VQGEMM_E_SHAPE;
     if (code_bits != 8 && code_bits != 16) return VQGEMM_E_CODEBITS;
     if (!max_out || (count > 0 && !codes)) return VQGEMM_E_NULL;
@@ -693,6 +754,7 @@ int vqgemm_max_code(const void *codes, int64_t count, int32_t code_bits, void *m
 
 int vqgemm_dequant_a(const void *w, const void *codebook, void *w_out, int64_t K, int64_t Nc, void *stream)
 {
+    const DeviceScope device;
     if (K < 0 || Nc < 0 || K > INT_MAX / 2 || Nc > INT_MAX / 4 || Nc % 4 != 0) return VQGEMM_E_SHAPE;
     if (K == 0 || Nc == 0) return VQGEMM_OK;
     if (!w || !codebook || !w_out) return VQGEMM_E_NULL;
@@ -708,6 +770,7 @@ int vqgemm_dequant_a(const void *w, const void *codebook, void *w_out, int64_t K
 
 int vqgemm_gemm_f16(const void *x, const void *w, void *y, int64_t M, int64_t K, int64_t N, void *stream)
 {
+    const DeviceScope device;
     if (M < 0 || K < 0 || N < 0 || M > INT_MAX / 2 || K > INT_MAX / 2 || N > INT_MAX / 2) return VQGEMM_E_SHAPE;
     if (M == 0 || N == 0) return VQGEMM_OK;
     if (!y || (K > 0 && (!x || !w))) return VQGEMM_E_NULL;

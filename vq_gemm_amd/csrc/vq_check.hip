@@ -54,24 +54,21 @@ hipError_t launch_clear_words(uint32_t *words, int64_t n, hipStream_t s)
     if (n <= 0) return hipSuccess;
     int64_t blocks = (n + 255) / 256;
     if (blocks > 64) blocks = 64;
-    hipLaunchKernelGGL(clear_words_kernel, dim3((unsigned)blocks), dim3(256), 0, s, words, n);
-    return hipGetLastError();
+    return launch_kernel(clear_words_kernel, dim3((unsigned)blocks), dim3(256), 0, s, words, n);
 }
 
 hipError_t launch_max_code(const void *codes, int64_t count, int code_bits, uint32_t *out, hipStream_t s)
 {
-    hipLaunchKernelGGL(clear_word_kernel, dim3(1), dim3(64), 0, s, out);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_kernel(clear_word_kernel, dim3(1), dim3(64), 0, s, out);
     if (e != hipSuccess || count == 0) return e;
     int64_t blocks = (count / (code_bits == 8 ? 16 : 8) + 255) / 256;
     const int64_t cap = (int64_t)device_cu_count() * 8;
     if (blocks > cap) blocks = cap;
     if (blocks < 1) blocks = 1;
     if (code_bits == 8)
-        hipLaunchKernelGGL(max_code_kernel<uint8_t>, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<const uint8_t *>(codes), count, out);
+        return launch_kernel(max_code_kernel<uint8_t>, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<const uint8_t *>(codes), count, out);
     else
-        hipLaunchKernelGGL(max_code_kernel<uint16_t>, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<const uint16_t *>(codes), count, out);
-    return hipGetLastError();
+        return launch_kernel(max_code_kernel<uint16_t>, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<const uint16_t *>(codes), count, out);
 }
 
 }  // namespace vq

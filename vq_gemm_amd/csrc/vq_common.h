@@ -4,6 +4,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <tuple>
+#include <type_traits>
+
 namespace vq {
 
 typedef _Float16 half_t;
@@ -182,7 +185,16 @@ hipError_t launch_max_code(const void *codes, int64_t count, int code_bits, uint
 // words[0 .. n) = 0, by a kernel (a launch that may be captured into a graph records no memset)
 hipError_t launch_clear_words(uint32_t *words, int64_t n, hipStream_t s);
 
+// compute units of the current device
 int device_cu_count();
+
+// Held by an entry point of the library: the current device is asked for once and not for every question about it.
+struct DeviceScope {
+    DeviceScope();
+    ~DeviceScope();
+    DeviceScope(const DeviceScope &) = delete;
+    DeviceScope &operator=(const DeviceScope &) = delete;
+};
 
 // The constants of the cost models behind the automatic kernel choice.  The compiled-in values were fitted to
 // measurements on one 256-CU MI355X; vqgemm_tuning_set / a file named by VQGEMM_TUNING_FILE (written by
@@ -250,8 +262,27 @@ struct Tuning {
 };
 const Tuning &tuning();
 
-// Raises a kernel's dynamic-LDS limit when `bytes` needs it; remembers what was granted per
-// (device, kernel) so that steady-state launches make no attribute call.
-hipError_t ensure_dynamic_lds(const void *kernel, size_t bytes);
+// The function handle of `kernel` on the current device, its dynamic-LDS limit raised to `lds_bytes` where that needs it.  Both
+// are looked up once per (device, kernel) and remembered per thread.
+hipError_t resolve_kernel(const void *kernel, size_t lds_bytes, hipFunction_t *function);
+
+// Enqueues kernel(args...).  What a launch statement does, less what it does again on every call: the search for the kernel
+// behind the host pointer, the push and pop of the launch configuration, the query of the last error (a decode launch
+// through the C ABI: 3.5 -> 2.9 us on the host, of which the runtime's own launch is 2.5).
+template <typename... P, typename... A>
+inline hipError_t launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream, A... args)
+{
+    static_assert(sizeof...(P) == sizeof...(A), "one argument per kernel parameter");
+    hipFunction_t f;
+    const hipError_t e = resolve_kernel(reinterpret_cast<const void *>(kernel), lds_bytes, &f);
+    if (e != hipSuccess) return e;
+    std::tuple<std::remove_cv_t<P>...> values(static_cast<P>(args)...);
+    return std::apply(
+        [&](auto &...v) {
+            void *pointers[] = {const_cast<void *>(static_cast<const void *>(&v))...};
+            return hipModuleLaunchKernel(f, grid.x, grid.y, grid.z, block.x, block.y, block.z, (unsigned)lds_bytes, stream, pointers, nullptr);
+        },
+        values);
+}
 
 }  // namespace vq

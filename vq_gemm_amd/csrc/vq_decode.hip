@@ -782,14 +782,11 @@ hipError_t launch_decode_batched(const ProblemB &p, hipStream_t s)
     const int dealt = p.gated ? g.tiles_per_cb / 2 : g.tiles_per_cb;  // what the workgroups of a codebook share: tiles, or pairs
     // the same launch for the instantiation with a bias argument and the one without
     auto launch = [&](auto kern, auto... bias) {
-        hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), g.smem);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, dim3(g.per_slab, g.n_slabs), dim3(g.n_waves * 64), g.smem, s, p.x,
+        return launch_kernel(kern, dim3(g.per_slab, g.n_slabs), dim3(g.n_waves * 64), g.smem, s, p.x,
                            static_cast<const CodeT *>(p.codes), p.cb, p.y, p.M, p.K, p.N, p.entries, p.n_codebooks,
                            g.wgs_per_cb, g.books_per_wg, g.tiles_per_cb, dealt / g.wgs_per_cb,
                            dealt % g.wgs_per_cb, g.n_chunks, g.red_off, g.stage_off, g.stage_over, g.acc_off,
                            (65536 + tail_rows - 1) / tail_rows, bias...);
-        return hipGetLastError();
     };
     // a full batch of one tile is the only case with a replicated table and TB = 1
     const int tb = g.full ? C::TB : 1;
@@ -849,9 +846,8 @@ hipError_t launch_pack(const void *src, void *dst, int64_t N, int64_t K, bool in
     const int64_t n_pieces = N * row_bytes / C::LB;
     if (n_pieces == 0) return hipSuccess;
     const unsigned blocks = (unsigned)((n_pieces + 255) / 256);
-    hipLaunchKernelGGL(pack_codes_kernel<C::LB>, dim3(blocks), dim3(256), 0, s, static_cast<const uint8_t *>(src),
+    return launch_kernel(pack_codes_kernel<C::LB>, dim3(blocks), dim3(256), 0, s, static_cast<const uint8_t *>(src),
                        static_cast<uint8_t *>(dst), n_pieces, row_bytes, inverse);
-    return hipGetLastError();
 }
 
 bool batched_supports(const ProblemB &p) { return plan_batched(p).ok; }

@@ -770,10 +770,9 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
     // single row per wave is over before a turn would come
     const int rotate_priority = tuning().gemv_wide_rotate_priority >= 1.0 && (n_dealt + waves - 1) / waves >= 2 ? 1 : 0;
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, block, 0, s, p.x, codes, p.cb, p.entries, n_dealt / waves, n_dealt % waves, n_dealt,
+        return launch_kernel(kern, grid, block, 0, s, p.x, codes, p.cb, p.entries, n_dealt / waves, n_dealt % waves, n_dealt,
                            (int)((p.gated ? 0x80000000u : 0u) | (uint32_t)(p.K / 8)), p.rows_per_cb,
                            1.0f / (float)p.rows_per_cb, p.n_codebooks, p.bias, p.y, rotate_priority);
-        return hipGetLastError();
     };
     using std::integral_constant;
     const int g = wide_rows_per_group(p);
@@ -905,31 +904,29 @@ hipError_t launch_gemv_format(const ProblemB &p, hipStream_t s)
     const dim3 grid(p.N / kGemvTile), block(kGemvWaves * 64);
     const CodeT *codes = static_cast<const CodeT *>(p.codes);
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, block, 0, s, p.x, codes, p.cb, p.y, p.bias, p.K, p.N, p.entries, p.rows_per_cb);
+        return launch_kernel(kern, grid, block, 0, s, p.x, codes, p.cb, p.y, p.bias, p.K, p.N, p.entries, p.rows_per_cb);
     };
     switch ((p.K / kRunK) * 10 + p.M) {
-    case 11: launch(decode_gemv_kernel<VEC, CodeT, 1, 1, GATED>); break;
-    case 12: launch(decode_gemv_kernel<VEC, CodeT, 1, 2, GATED>); break;
-    case 21: launch(decode_gemv_kernel<VEC, CodeT, 2, 1, GATED>); break;
-    case 22: launch(decode_gemv_kernel<VEC, CodeT, 2, 2, GATED>); break;
-    case 31: launch(decode_gemv_kernel<VEC, CodeT, 3, 1, GATED>); break;
-    case 32: launch(decode_gemv_kernel<VEC, CodeT, 3, 2, GATED>); break;
-    case 41: launch(decode_gemv_kernel<VEC, CodeT, 4, 1, GATED>); break;
-    case 42: launch(decode_gemv_kernel<VEC, CodeT, 4, 2, GATED>); break;
+    case 11: return launch(decode_gemv_kernel<VEC, CodeT, 1, 1, GATED>);
+    case 12: return launch(decode_gemv_kernel<VEC, CodeT, 1, 2, GATED>);
+    case 21: return launch(decode_gemv_kernel<VEC, CodeT, 2, 1, GATED>);
+    case 22: return launch(decode_gemv_kernel<VEC, CodeT, 2, 2, GATED>);
+    case 31: return launch(decode_gemv_kernel<VEC, CodeT, 3, 1, GATED>);
+    case 32: return launch(decode_gemv_kernel<VEC, CodeT, 3, 2, GATED>);
+    case 41: return launch(decode_gemv_kernel<VEC, CodeT, 4, 1, GATED>);
+    case 42: return launch(decode_gemv_kernel<VEC, CodeT, 4, 2, GATED>);
     default:
         if constexpr (VEC == 8 && sizeof(CodeT) == 1) {
             switch ((p.K / kRunK) * 10 + p.M) {
-            case 13: launch(decode_gemv_kernel<8, uint8_t, 1, 3, GATED>); break;
-            case 14: launch(decode_gemv_kernel<8, uint8_t, 1, 4, GATED>); break;
-            case 23: launch(decode_gemv_kernel<8, uint8_t, 2, 3, GATED>); break;
-            case 24: launch(decode_gemv_kernel<8, uint8_t, 2, 4, GATED>); break;
-            default: return hipErrorInvalidValue;
+            case 13: return launch(decode_gemv_kernel<8, uint8_t, 1, 3, GATED>);
+            case 14: return launch(decode_gemv_kernel<8, uint8_t, 1, 4, GATED>);
+            case 23: return launch(decode_gemv_kernel<8, uint8_t, 2, 3, GATED>);
+            case 24: return launch(decode_gemv_kernel<8, uint8_t, 2, 4, GATED>);
+            default: break;
             }
-            break;
         }
         return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 template <bool GATED>

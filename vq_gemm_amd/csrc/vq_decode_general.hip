@@ -399,12 +399,9 @@ hipError_t launch_decode_steps(const ProblemB &p, hipStream_t s)
         grid = n_dealt < cus * per_cu ? n_dealt : cus * per_cu;
     }
     auto kern = repl ? decode_general_kernel<VEC, CodeT, STEPS, true> : decode_general_kernel<VEC, CodeT, STEPS, false>;
-    hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), smem);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(n_waves * 64), smem, s, p.x, static_cast<const CodeT *>(p.codes), p.cb,
+    return launch_kernel(kern, dim3(grid), dim3(n_waves * 64), smem, s, p.x, static_cast<const CodeT *>(p.codes), p.cb,
                        p.y, p.bias, p.M, p.K, p.N, p.entries, p.rows_per_cb, n_dealt / grid, n_dealt % grid, n_chunks, stage_off, aliased,
                        p.gated ? 1 : 0);
-    return hipGetLastError();
 }
 
 template <int VEC, typename CodeT>

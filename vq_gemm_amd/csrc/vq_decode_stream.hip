@@ -316,9 +316,8 @@ hipError_t launch_decode_stream(const ProblemB &p, hipStream_t s)
     const int pieces = stream_pieces_per_wave(p);
     const bool repl = (double)(pieces * t * kPieceSteps) >= tuning().decode_stream_replicated_min_gathers;
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, block, 0, s, p.x, static_cast<const uint8_t *>(p.codes), p.cb, p.y, p.bias, p.M, p.K, p.N,
+        return launch_kernel(kern, grid, block, 0, s, p.x, static_cast<const uint8_t *>(p.codes), p.cb, p.y, p.bias, p.M, p.K, p.N,
                            p.entries, p.rows_per_cb, n_groups / wgs, n_groups % wgs, n_tiles);
-        return hipGetLastError();
     };
     using std::integral_constant;
     auto pick = [&](auto t_c, auto np_c) {

@@ -59,12 +59,11 @@ static hipError_t dequant_b_typed(const ProblemB &p, half_t *w_out, hipStream_t 
     // Vector copies need codeword-aligned source and destination; otherwise copy scalars.
     const bool aligned = (((uintptr_t)w_out | (uintptr_t)p.cb) % (uintptr_t)(p.vec * 2)) == 0;
     switch (aligned ? p.vec : 0) {
-    case 2: hipLaunchKernelGGL((dequant_b_kernel<2, CodeT>), grid, block, 0, s, codes, p.cb, w_out, p.N, J, p.entries, p.rows_per_cb); break;
-    case 4: hipLaunchKernelGGL((dequant_b_kernel<4, CodeT>), grid, block, 0, s, codes, p.cb, w_out, p.N, J, p.entries, p.rows_per_cb); break;
-    case 8: hipLaunchKernelGGL((dequant_b_kernel<8, CodeT>), grid, block, 0, s, codes, p.cb, w_out, p.N, J, p.entries, p.rows_per_cb); break;
-    default: hipLaunchKernelGGL((dequant_b_anyvec_kernel<CodeT>), grid, block, 0, s, codes, p.cb, w_out, p.N, J, p.vec, p.entries, p.rows_per_cb); break;
+    case 2: return launch_kernel((dequant_b_kernel<2, CodeT>), grid, block, 0, s, codes, p.cb, w_out, p.N, J, p.entries, p.rows_per_cb);
+    case 4: return launch_kernel((dequant_b_kernel<4, CodeT>), grid, block, 0, s, codes, p.cb, w_out, p.N, J, p.entries, p.rows_per_cb);
+    case 8: return launch_kernel((dequant_b_kernel<8, CodeT>), grid, block, 0, s, codes, p.cb, w_out, p.N, J, p.entries, p.rows_per_cb);
+    default: return launch_kernel((dequant_b_anyvec_kernel<CodeT>), grid, block, 0, s, codes, p.cb, w_out, p.N, J, p.vec, p.entries, p.rows_per_cb);
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_dequant_b(const ProblemB &p, half_t *w_out, hipStream_t s)
@@ -96,8 +95,7 @@ hipError_t launch_dequant_a(const ProblemA &p, half_t *w_out, hipStream_t s)
     int64_t blocks = (total + 255) / 256;
     const int64_t cap = (int64_t)device_cu_count() * 32;
     if (blocks > cap) blocks = cap;
-    hipLaunchKernelGGL(dequant_a_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p.w, p.cb, w_out, p.K, p.Nc);
-    return hipGetLastError();
+    return launch_kernel(dequant_a_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p.w, p.cb, w_out, p.K, p.Nc);
 }
 
 }  // namespace vq

@@ -419,11 +419,8 @@ hipError_t launch_scan(const half_t *w, const ProblemB &p, void *codes_out, floa
     const int wgs_per_cb = scan_workgroups(p, ACCUMULATE);
     const size_t smem = scan_lds_bytes(p, ACCUMULATE);
     auto kern = p.entries < kScanWideGroupEntries ? encode_scan_kernel<VEC, CodeT, 8, ACCUMULATE> : encode_scan_kernel<VEC, CodeT, 16, ACCUMULATE>;
-    const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), smem);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem, s, w, p.cb,
+    return launch_kernel(kern, dim3((unsigned)(wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem, s, w, p.cb,
                        static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, wgs_per_cb, partials);
-    return hipGetLastError();
 }
 
 template <int VEC, typename CodeT>
@@ -436,9 +433,8 @@ hipError_t encode_b_typed(const half_t *w, const ProblemB &p, void *codes_out, h
     const int64_t want = ((int64_t)device_cu_count() * 8 + p.n_codebooks - 1) / p.n_codebooks;
     const int64_t have = (vectors_per_cb + kEncThreads * kEncPerThread - 1) / (kEncThreads * kEncPerThread);
     const int wgs_per_cb = (int)(want < have ? want : have);
-    hipLaunchKernelGGL((encode_b_kernel<VEC, CodeT>), dim3((unsigned)(wgs_per_cb * p.n_codebooks)), dim3(kEncThreads), 0, s, w,
+    return launch_kernel((encode_b_kernel<VEC, CodeT>), dim3((unsigned)(wgs_per_cb * p.n_codebooks)), dim3(kEncThreads), 0, s, w,
                        p.cb, static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, wgs_per_cb);
-    return hipGetLastError();
 }
 
 }  // namespace

@@ -57,13 +57,12 @@ hipError_t launch_silu_mul(const half_t *a, half_t *out, int64_t M, int64_t N, h
     if (blocks > cap) blocks = cap;
     const dim3 grid((unsigned)blocks), block(256);
     if (interleaved) {
-        if (vec8) hipLaunchKernelGGL((silu_mul_kernel<true, true>), grid, block, 0, s, a, out, M, N);
-        else hipLaunchKernelGGL((silu_mul_kernel<false, true>), grid, block, 0, s, a, out, M, N);
+        if (vec8) return launch_kernel((silu_mul_kernel<true, true>), grid, block, 0, s, a, out, M, N);
+        else return launch_kernel((silu_mul_kernel<false, true>), grid, block, 0, s, a, out, M, N);
     } else {
-        if (vec8) hipLaunchKernelGGL((silu_mul_kernel<true, false>), grid, block, 0, s, a, out, M, N);
-        else hipLaunchKernelGGL((silu_mul_kernel<false, false>), grid, block, 0, s, a, out, M, N);
+        if (vec8) return launch_kernel((silu_mul_kernel<true, false>), grid, block, 0, s, a, out, M, N);
+        else return launch_kernel((silu_mul_kernel<false, false>), grid, block, 0, s, a, out, M, N);
     }
-    return hipGetLastError();
 }
 
 }  // namespace vq

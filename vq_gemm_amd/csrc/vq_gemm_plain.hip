@@ -135,8 +135,7 @@ hipError_t launch_plain(const half_t *x, const half_t *w, half_t *y, int M, int 
     const int w_cols = W_IS_KN ? N : K;
     const bool w_vec = (w_cols % 8 == 0) && (((uintptr_t)w & 15) == 0);
     dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
-    hipLaunchKernelGGL((gemm_plain_kernel<W_IS_KN>), grid, dim3(256), 0, s, x, w, y, M, K, N, x_vec, w_vec);
-    return hipGetLastError();
+    return launch_kernel((gemm_plain_kernel<W_IS_KN>), grid, dim3(256), 0, s, x, w, y, M, K, N, x_vec, w_vec);
 }
 
 }  // namespace

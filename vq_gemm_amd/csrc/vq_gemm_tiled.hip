@@ -621,11 +621,8 @@ hipError_t launch_tiled(const half_t *x, const half_t *w, half_t *y, int M, int 
     typedef TileCfg<NP, MPW> C;
     const int tiles_m = (M + C::BM - 1) / C::BM, tiles_n = (N + C::BN - 1) / C::BN;
     auto kern = gemm_tiled_kernel<W_IS_KN, NP, MPW>;
-    const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), C::kLdsBytes);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads), C::kLdsBytes, s, x, w, y, M, K, N,
+    return launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads), C::kLdsBytes, s, x, w, y, M, K, N,
                        tiles_m, tiles_n);
-    return hipGetLastError();
 }
 
 }  // namespace
@@ -685,11 +682,8 @@ hipError_t launch_fused_a(const ProblemA &p, hipStream_t s)
     const bool tall = (double)((n_tall + cus - 1) / cus) <= 0.8 * (double)((n_short + cus - 1) / cus);
     auto launch = [&](auto kern, int bm, size_t lds) {
         const int tiles_m = (p.M + bm - 1) / bm;
-        const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads), lds, s, p.x, p.w, p.cb, p.y, p.M, p.K,
+        return launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads), lds, s, p.x, p.w, p.cb, p.y, p.M, p.K,
                            p.Nc, tiles_m, tiles_n);
-        return hipGetLastError();
     };
     return tall ? launch(gemm_a_fused_kernel<8>, 256, FusedACfg<8>::kLdsBytes) : launch(gemm_a_fused_kernel<4>, 128, FusedACfg<4>::kLdsBytes);
 }

@@ -77,22 +77,20 @@ hipError_t launch_generic_b(const ProblemB &p, hipStream_t s)
         dim3 block(64, 4);
         dim3 grid((p.N / 2 + 63) / 64, (unsigned)(((p.M + 3) / 4) < 32768 ? (p.M + 3) / 4 : 32768));
         if (p.code_bits == 8)
-            hipLaunchKernelGGL((generic_b_gated_kernel<uint8_t>), grid, block, 0, s, p.x, static_cast<const uint8_t *>(p.codes),
+            return launch_kernel((generic_b_gated_kernel<uint8_t>), grid, block, 0, s, p.x, static_cast<const uint8_t *>(p.codes),
                                p.cb, p.y, p.bias, p.M, p.K, p.N, p.vec, p.entries, p.rows_per_cb);
         else
-            hipLaunchKernelGGL((generic_b_gated_kernel<uint16_t>), grid, block, 0, s, p.x, static_cast<const uint16_t *>(p.codes),
+            return launch_kernel((generic_b_gated_kernel<uint16_t>), grid, block, 0, s, p.x, static_cast<const uint16_t *>(p.codes),
                                p.cb, p.y, p.bias, p.M, p.K, p.N, p.vec, p.entries, p.rows_per_cb);
-        return hipGetLastError();
     }
     dim3 block(64, 4);
     dim3 grid((p.N + 63) / 64, (unsigned)(((p.M + 3) / 4) < 32768 ? (p.M + 3) / 4 : 32768));
     if (p.code_bits == 8)
-        hipLaunchKernelGGL((generic_b_kernel<uint8_t>), grid, block, 0, s, p.x, static_cast<const uint8_t *>(p.codes),
+        return launch_kernel((generic_b_kernel<uint8_t>), grid, block, 0, s, p.x, static_cast<const uint8_t *>(p.codes),
                            p.cb, p.y, p.bias, p.M, p.K, p.N, p.vec, p.entries, p.rows_per_cb);
     else
-        hipLaunchKernelGGL((generic_b_kernel<uint16_t>), grid, block, 0, s, p.x, static_cast<const uint16_t *>(p.codes),
+        return launch_kernel((generic_b_kernel<uint16_t>), grid, block, 0, s, p.x, static_cast<const uint16_t *>(p.codes),
                            p.cb, p.y, p.bias, p.M, p.K, p.N, p.vec, p.entries, p.rows_per_cb);
-    return hipGetLastError();
 }
 
 // Geometry A: out[m, 2n + r] = sum_k x[m,k] * cb[n/4][w[k,n]][r].  One thread per code
@@ -124,8 +122,7 @@ hipError_t launch_generic_a(const ProblemA &p, hipStream_t s)
     if (p.M == 0 || p.Nc == 0) return hipSuccess;
     dim3 block(64, 4);
     dim3 grid((p.Nc + 63) / 64, (unsigned)(((p.M + 3) / 4) < 32768 ? (p.M + 3) / 4 : 32768));
-    hipLaunchKernelGGL(generic_a_kernel, grid, block, 0, s, p.x, p.w, p.cb, p.y, p.M, p.K, p.Nc);
-    return hipGetLastError();
+    return launch_kernel(generic_a_kernel, grid, block, 0, s, p.x, p.w, p.cb, p.y, p.M, p.K, p.Nc);
 }
 
 }  // namespace vq

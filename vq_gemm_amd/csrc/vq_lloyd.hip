@@ -108,18 +108,16 @@ hipError_t lloyd_typed(const half_t *w, const ProblemB &p, const int32_t *pick, 
     const int picks = p.n_codebooks * p.entries;
     ProblemB q = p;
     half_t *book = iters == 0 ? cb_out : books[0];
-    hipLaunchKernelGGL(lloyd_pick_kernel<VEC>, dim3((picks + 255) / 256), dim3(256), 0, s, w, pick, book,
+    hipError_t e = launch_kernel(lloyd_pick_kernel<VEC>, dim3((picks + 255) / 256), dim3(256), 0, s, w, pick, book,
                        (int64_t)p.rows_per_cb * (p.K / VEC), p.entries, picks);
-    hipError_t e = hipGetLastError();
     for (int it = 0; it <= iters && e == hipSuccess; it++) {
         q.cb = book;
         e = launch_lloyd_assign(w, q, codes_out, partials, s);
         if (e != hipSuccess) return e;
         half_t *next = it == iters ? nullptr : it + 1 == iters ? cb_out : books[(it + 1) & 1];
         const int wgs = next ? p.n_codebooks * ((p.entries + kUpdateEntries - 1) / kUpdateEntries) : 1;
-        hipLaunchKernelGGL(lloyd_update_kernel<VEC>, dim3(wgs), dim3(kUpdateThreads), 0, s, partials, rows, book, next, p.entries,
+        e = launch_kernel(lloyd_update_kernel<VEC>, dim3(wgs), dim3(kUpdateThreads), 0, s, partials, rows, book, next, p.entries,
                            p.n_codebooks, errors + it);
-        e = hipGetLastError();
         book = next;
     }
     return e;

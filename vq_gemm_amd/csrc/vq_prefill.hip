@@ -925,12 +925,9 @@ hipError_t launch_prefill_typed(const ProblemB &p, hipStream_t s, int tile, int 
         auto kern = ns == 4   ? (tail ? pick(std::true_type{}, integral_constant<int, 4>{}) : pick(std::false_type{}, integral_constant<int, 4>{}))
                     : ns == 3 ? (tail ? pick(std::true_type{}, integral_constant<int, 3>{}) : pick(std::false_type{}, integral_constant<int, 3>{}))
                               : (tail ? pick(std::true_type{}, integral_constant<int, 2>{}) : pick(std::false_type{}, integral_constant<int, 2>{}));
-        hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), smem);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(kThreads), smem, s, p.x,
+        const hipError_t e = launch_kernel(kern, dim3(tiles_m * tiles_n), dim3(kThreads), smem, s, p.x,
                            static_cast<const CodeT *>(p.codes), p.cb, p.y, p.bias, p.M, p.K, n_split, 0, p.N, p.entries,
                            p.rows_per_cb, tiles_m, tiles_n, n_cb, p.gated ? 1 : 0);
-        e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     if (n_split < n_end) {
@@ -941,12 +938,9 @@ hipError_t launch_prefill_typed(const ProblemB &p, hipStream_t s, int tile, int 
         const bool split = can_split && split_layout_applies(p, codebooks_per_tile(p, BNN), kStageBytes);
         auto kern = split ? (tail ? prefill_narrow_kernel<VEC, CodeT, true, can_split> : prefill_narrow_kernel<VEC, CodeT, false, can_split>)
                           : (tail ? prefill_narrow_kernel<VEC, CodeT, true, false> : prefill_narrow_kernel<VEC, CodeT, false, false>);
-        hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), smem);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(kThreads), smem, s, p.x,
+        return launch_kernel(kern, dim3(tiles_m * tiles_n), dim3(kThreads), smem, s, p.x,
                            static_cast<const CodeT *>(p.codes), p.cb, p.y, p.bias, p.M, p.K, n_end, n_split, p.N, p.entries,
                            p.rows_per_cb, tiles_m, tiles_n, codebooks_per_tile(p, BNN), p.gated ? 1 : 0);
-        return hipGetLastError();
     }
     return hipSuccess;
 }

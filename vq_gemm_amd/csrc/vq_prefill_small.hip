@@ -481,13 +481,10 @@ hipError_t launch_small_typed(const ProblemB &p, hipStream_t s, int splits, void
     const bool half = p.K % C::K_SUPER != 0;
     auto kern = half ? (split ? prefill_small_kernel<VEC, CodeT, 4, can_split, can_half> : prefill_small_kernel<VEC, CodeT, 4, false, can_half>)
                      : (split ? prefill_small_kernel<VEC, CodeT, 4, can_split, false> : prefill_small_kernel<VEC, CodeT, 4, false, false>);
-    const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), smem);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(kThreads), smem, s, p.x,
+    return launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(kThreads), smem, s, p.x,
                        static_cast<const CodeT *>(p.codes), p.cb, p.y, p.bias, p.M, p.K, p.N, n_begin, p.N, p.entries,
                        p.rows_per_cb, tiles_m, tiles_n, codebooks_per_tile(p, SBN), p.gated ? 1 : 0, splits, partials, counters,
                        tuning().splitk_validate_fences >= 1.0 ? 1 : 0);
-    return hipGetLastError();
 }
 
 }  // namespace
