@@ -126,6 +126,22 @@ int64_t vqgemm_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t vec, i
                                  int32_t n_codebooks, int32_t code_bits, int32_t variant);
 
 /*
+ * The product over additive ("residual") stages: codes [N, K/vec] hold `stages` blocks of K/stages columns of W side by side, all of
+ * which multiply the same x [M, K/stages]: y = sum over the stages of x . W_s^T, in one fp32 sum.  The kernel is the automatic
+ * choice's for K; the decode kernel reads x as it is, the others from a copy repeated along K in the workspace
+ * (vqgemm_stages_workspace_bytes_b bytes, 256-byte aligned; what is beyond the copy serves split K as in
+ * vqgemm_e2e_gemm_b_ws).  VQGEMM_E_SCRATCH when the workspace does not hold a copy that is needed.  No counterpart in the reference.
+ */
+int64_t vqgemm_stages_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t vec,
+                                        int32_t entries, int32_t n_codebooks, int32_t code_bits,
+                                        int32_t stages);
+int vqgemm_e2e_gemm_b_stages(const void *x, const void *codes, const void *codebook,
+                             const void *bias, void *y, int64_t M, int64_t K, int64_t N,
+                             int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits,
+                             int32_t stages, void *workspace, int64_t workspace_bytes, void *stream);
+
+
+/*
  * The fused VQ GEMM with a gated epilogue, for a gate/up projection pair (the MLP shapes among the measured
  * configurations): the rows of W (as codes) are the gate rows and the up rows of the pair interleaved in groups of
  * 16 - rows 32g .. 32g+15 are gate rows 16g .. 16g+15, rows 32g+16 .. 32g+31 the up rows of the same columns -

@@ -1917,3 +1917,18 @@ def test_lloyd_iterations_on_the_device_against_the_definition(row):
                         assert np.array_equal(got[i, e], book[i, e])
                     else:
                         assert np.allclose(got[i, e].astype(np.float64), mine.mean(axis=0), rtol=1.1e-3, atol=1e-6)
+
+
+@pytest.mark.parametrize("M,K,N,v,entries,stages,bits", [(5, 4096, 80, 8, 256, 2, 16), (16, 320, 50, 8, 100, 3, 16), (3, 4160, 33, 8, 128, 2, 8),
+                                                         (20, 2048, 64, 4, 256, 4, 16), (1, 2048, 64, 8, 128, 2, 8), (130, 512, 72, 8, 128, 2, 8)])
+def test_stages_multiply_the_same_x_without_a_copy_of_it(M, K, N, v, entries, stages, bits):
+    from vq_gemm_amd.nn import VQLinear
+    _say("stages", M, K, N, v, entries, stages)
+    spec = ProblemSpec("stages", GEOM_B, M, stages * K, N, v, stages * entries, 1, bits, codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=17, device=DEV)
+    x = x[:, :K].contiguous()
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(1)).half().to(DEV)
+    for b in (None, bias):
+        y = VQLinear(codes, cb, b, k_repeat=stages)(x)
+        torch.cuda.synchronize()
+        assert torch.equal(y, cabi.e2e_gemm_b_ws(x.repeat(1, stages), codes, cb, bias=b))

@@ -90,7 +90,7 @@ def _newer(target: str, deps) -> bool:
 # zero VGPR spills and zero bytes of private segment.  (A scalar register that the compiler parks in a lane
 # of a vector register - an "SGPR spill" that never touches memory - is tolerated in small numbers: it costs
 # one lane write and read outside the hand-scheduled loops.)
-MAX_SGPR_SPILLS = 4
+MAX_SGPR_SPILLS = 8
 
 
 def _check_no_spills(asm_path: str) -> None:

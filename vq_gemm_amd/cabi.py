@@ -26,6 +26,8 @@ _SIGNATURES = {
     "vqgemm_e2e_gemm_b_bias": (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _P, _P]),
     "vqgemm_e2e_gemm_b_gated": (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _P, _P]),
     "vqgemm_e2e_gemm_b_ws": (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _P, _I64, _P]),
+    "vqgemm_stages_workspace_bytes_b": (_I64, [_I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32]),
+    "vqgemm_e2e_gemm_b_stages": (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _P, _I64, _P]),
     "vqgemm_workspace_bytes_b": (_I64, [_I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32]),
     "vqgemm_e2e_gemm_a": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, _I64, _I32, _P, _P]),
     "vqgemm_e2e_gemm_a_noalloc": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, _I64, _I32, _P]),

@@ -97,31 +97,30 @@ Tensor linear_impl(const Tensor &x, const Tensor &codes, const Tensor &codebook,
     const Dims d = check_linear("vq_linear", x, codes, codebook, bias, k_repeat);
     const c10::OptionalDeviceGuard guard(x.device());
     Tensor hold_x, hold_codes, hold_cb, hold_bias;
-    const void *xp, *codes_p = data_of(codes, hold_codes), *cb_p = data_of(codebook, hold_cb);
-    if (k_repeat > 1) {
-        c10::SmallVector<int64_t, 6> times(x.dim(), 1);
-        times.back() = k_repeat;
-        hold_x = x.repeat(times);
-        xp = hold_x.data_ptr();
-    } else {
-        xp = dense_of(x, hold_x);
-    }
+    const void *xp = dense_of(x, hold_x), *codes_p = data_of(codes, hold_codes), *cb_p = data_of(codebook, hold_cb);
     const void *bias_p = bias.has_value() && bias->defined() ? data_of(*bias, hold_bias) : nullptr;
     Tensor y = new_result(x, d.N);
     void *s = stream_of(x);
-    // scratch for the shapes where the automatic choice may split K (never with a slab of 16 rows or fewer); the
-    // caching allocator hands out stream-ordered blocks
-    const int64_t need = variant == VQGEMM_VARIANT_AUTO && d.M > 16
-                             ? vqgemm_workspace_bytes_b(d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, variant) : 0;
+    // scratch for the shapes where the automatic choice may split K (never with a slab of 16 rows or fewer) or wants x
+    // repeated; the caching allocator hands out stream-ordered blocks
+    int64_t need = 0;
+    if (k_repeat > 1) need = vqgemm_stages_workspace_bytes_b(d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, (int)k_repeat);
+    else if (variant == VQGEMM_VARIANT_AUTO && d.M > 16)
+        need = vqgemm_workspace_bytes_b(d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, variant);
+    Tensor ws;
+    if (need > 0) ws = at::detail::empty_cuda({need}, at::kByte, x.device(), c10::nullopt);
+    void *ws_p = need > 0 ? ws.data_ptr() : nullptr;
+    const int64_t ws_bytes = need > 0 ? need : 0;
     int rc;
-    if (need > 0) {
-        Tensor ws = at::detail::empty_cuda({need}, at::kByte, x.device(), c10::nullopt);
+    if (k_repeat > 1)
+        rc = vqgemm_e2e_gemm_b_stages(xp, codes_p, cb_p, bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits,
+                                      (int)k_repeat, ws_p, ws_bytes, s);
+    else if (need > 0)
         rc = vqgemm_e2e_gemm_b_ws(xp, codes_p, cb_p, bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, variant,
-                                  ws.data_ptr(), need, s);
-    } else {
+                                  ws_p, ws_bytes, s);
+    else
         rc = vqgemm_e2e_gemm_b_bias(xp, codes_p, cb_p, bias_p, y.data_ptr(), d.M, d.K, d.N, d.vec, d.entries, d.books, d.bits, variant,
                                     nullptr, s);
-    }
     check_rc(rc, "vq_linear");
     return y;
 }

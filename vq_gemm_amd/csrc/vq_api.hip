@@ -222,6 +222,7 @@ ProblemB make_b(const void *x, const void *codes, const void *codebook, void *y,
     p.y = static_cast<half_t *>(y);
     p.bias = nullptr;
     p.M = (int)M; p.K = (int)K; p.N = (int)N;
+    p.k_x = (int)K;
     p.vec = vec; p.entries = entries; p.n_codebooks = n_codebooks; p.code_bits = code_bits;
     p.rows_per_cb = N > 0 ? (int)(N / n_codebooks) : 1;
     if (p.rows_per_cb < 1) p.rows_per_cb = 1;
@@ -497,6 +498,66 @@ int vqgemm_e2e_gemm_b_ws(const void *x, const void *codes, const void *codebook,
                                           nullptr, stream);
     }
     return static_cast<int>(launch_prefill_small_b(p, static_cast<hipStream_t>(stream), sp, workspace));
+}
+
+namespace {
+
+// Additive stages: whether the automatic choice for the whole K reads X as it is, and what it needs as scratch otherwise
+// (the repeated X, then what the product itself wants).
+bool stages_read_x(const ProblemB &p, int stages)
+{
+    ProblemB q = p;
+    q.k_x = p.K / stages;
+    return select_b(p, true) == VQGEMM_VARIANT_DECODE && decode_stages_supports(q);
+}
+int64_t repeated_x_bytes(const ProblemB &p) { return ((int64_t)p.M * p.K * 2 + 255) & ~(int64_t)255; }
+
+}  // namespace
+
+int64_t vqgemm_stages_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks,
+                                        int32_t code_bits, int32_t stages)
+{
+    const DeviceScope device;
+    const int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
+    if (rc != VQGEMM_OK) return rc;
+    if (stages < 1 || K % stages != 0) return VQGEMM_E_SHAPE;
+    if (M == 0 || N == 0 || K == 0) return 0;
+    const ProblemB p = make_b(nullptr, nullptr, nullptr, nullptr, M, K, N, vec, entries, n_codebooks, code_bits);
+    if (stages > 1 && stages_read_x(p, stages)) return 0;
+    return (stages > 1 ? repeated_x_bytes(p) : 0) + (int64_t)workspace_auto(p, true).bytes;
+}
+
+int vqgemm_e2e_gemm_b_stages(const void *x, const void *codes, const void *codebook, const void *bias, void *y, int64_t M, int64_t K,
+                             int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits, int32_t stages,
+                             void *workspace, int64_t workspace_bytes, void *stream)
+{
+    const DeviceScope device;
+    int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
+    if (rc != VQGEMM_OK) return rc;
+    if (stages < 1 || K % stages != 0) return VQGEMM_E_SHAPE;
+    if (workspace_bytes < 0 || (workspace_bytes > 0 && !workspace)) return VQGEMM_E_NULL;
+    if (stages == 1 || M == 0 || N == 0 || K == 0)
+        return vqgemm_e2e_gemm_b_ws(x, codes, codebook, bias, y, M, K, N, vec, entries, n_codebooks, code_bits, VQGEMM_VARIANT_AUTO,
+                                    workspace, workspace_bytes, stream);
+    if (!y || !codebook || !x || !codes) return VQGEMM_E_NULL;
+    if (!aligned(x, 2) || !aligned(y, 2) || !aligned(codebook, 2) || !aligned(codes, code_bits / 8) || !aligned(bias, 2) ||
+        !aligned(workspace, 256))
+        return VQGEMM_E_ALIGN;
+    ProblemB p = make_b(x, codes, codebook, y, M, K, N, vec, entries, n_codebooks, code_bits);
+    p.bias = static_cast<const half_t *>(bias);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool a16 = aligned(x, 16) && aligned(y, 16) && aligned(codebook, 16) && aligned(codes, 16) && aligned(bias, 8);
+    if (a16 && stages_read_x(p, stages)) {
+        p.k_x = p.K / stages;
+        return static_cast<int>(launch_decode_b(p, s));
+    }
+    const int64_t repeated = repeated_x_bytes(p);
+    if (workspace_bytes < repeated) return VQGEMM_E_SCRATCH;
+    const hipError_t e = launch_repeat_columns(p.x, static_cast<half_t *>(workspace), M, K / stages, stages, s);
+    if (e != hipSuccess) return static_cast<int>(e);
+    const int64_t rest = workspace_bytes - repeated;
+    return vqgemm_e2e_gemm_b_ws(workspace, codes, codebook, bias, y, M, K, N, vec, entries, n_codebooks, code_bits, VQGEMM_VARIANT_AUTO,
+                                rest > 0 ? static_cast<uint8_t *>(workspace) + repeated : nullptr, rest, stream);
 }
 
 int vqgemm_e2e_gemm_b_gated(const void *x, const void *codes, const void *codebook, const void *bias, void *y, int64_t M,

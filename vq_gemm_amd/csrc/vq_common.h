@@ -28,6 +28,7 @@ struct ProblemB {
     half_t *y;            // [M,N]
     const half_t *bias;   // [N] added to the fp32 sums before the rounding to fp16, or nullptr
     int M, K, N;
+    int k_x;              // columns of X: K, or K / stages where X repeats along K (the kernel behind decode_stages_supports only)
     int vec, entries, n_codebooks, code_bits;
     int rows_per_cb;      // N / G
     bool packed;          // codes are in the packed layout of the batched decode kernel (launch_pack_codes)
@@ -96,6 +97,7 @@ bool decode_supports(const ProblemB &p);
 // whether the decode path is expected to beat the prefill kernel on a shape it supports
 bool decode_preferred(const ProblemB &p);
 hipError_t launch_decode_b(const ProblemB &p, hipStream_t s);
+bool decode_stages_supports(const ProblemB &p);
 // The packed code layout of the batched decode kernel: the pieces of the code matrix in the order
 // the kernel's lanes load them (same size, codes unchanged).  `inverse` restores the plain matrix.
 bool pack_codes_supports(int64_t N, int64_t K, int vec, int code_bits);
@@ -175,6 +177,9 @@ hipError_t launch_gemm_tiled(const half_t *x, const half_t *w, half_t *y, int M,
 // geometry A, fused: the tiled [K,N] GEMM with its W stages dequantised on the compute unit
 bool fused_a_supports(const ProblemA &p);
 hipError_t launch_fused_a(const ProblemA &p, hipStream_t s);
+
+// out[M, stages * K] = x[M, K] repeated `stages` times along K
+hipError_t launch_repeat_columns(const half_t *x, half_t *out, int64_t M, int64_t K, int stages, hipStream_t s);
 
 // out[M,N] = silu(a[:, :N]) * a[:, N:] for a [M, 2N]
 // (interleaved: gate and up columns alternate in groups of 16 instead of lying in the two halves of a row)

@@ -249,6 +249,10 @@ constexpr int kStageOverTable = 1, kStageOverSlots = 2;
 
 __device__ __forceinline__ const half_t *bias_of() { return nullptr; }
 __device__ __forceinline__ const half_t *bias_of(const half_t *b) { return b; }
+__device__ __forceinline__ const half_t *bias_of(const half_t *b, int) { return b; }
+__device__ __forceinline__ int k_x_of(int K) { return K; }
+__device__ __forceinline__ int k_x_of(int K, const half_t *) { return K; }
+__device__ __forceinline__ int k_x_of(int, const half_t *, int k_x) { return k_x; }
 
 //
 // GATED: the epilogue of a gate/up pair.  The rows of W are gate and up rows interleaved in groups of 16, so an
@@ -269,7 +273,11 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     typedef DecodeCfg<VEC, CodeT> C;
     typedef LaneCodes<VEC, CodeT> Codes;
     // The bias pointer is a kernel argument only in the instantiation that adds one, so that a
-    // launch without bias fetches and tests nothing for it.
+    // launch without bias fetches and tests nothing for it.  The instantiation with a second extra argument, the number of
+    // columns of X, takes what the common shapes do without testing for: K that is no multiple of a slice, N that is none of a
+    // tile, an X that repeats along K, a bias that may be missing.  (A short launch is bound by what its prologue does one
+    // after the other: with those tests in every launch 16 rows of X on K = 4096, N = 1024 took 6.46 us instead of 6.22.)
+    constexpr bool kAny = sizeof...(Bias) == 2;
     constexpr bool kHasBias = sizeof...(Bias) > 0;
     const half_t *bias = bias_of(bias_arg...);
     // All kernel arguments are fetched at once: left to first use, each pointer costs the
@@ -281,7 +289,9 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     const int slab_row = blockIdx.y * kTileN;
     const int M = min(kTileN, m_total - slab_row);
     const int recip_m = M == kTileN ? 65536 / kTileN : recip_tail;
-    x += (int64_t)slab_row * K;
+    // X has k_x columns; where that is less than K (additive stages side by side along K; never gated) they repeat.
+    const int k_x = GATED ? K : k_x_of(K, bias_arg...);
+    x += (int64_t)slab_row * k_x;
     static_assert(!GATED || TB % 2 == 0, "gate and up tiles come in pairs");
     constexpr int kDeal = GATED ? 2 : 1;  // tiles per unit that is dealt to the workgroups
     const int ldy = GATED ? N / 2 : N;
@@ -292,7 +302,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // K goes in n_chunks chunks of (at most) n_waves slices of 256 k: wave w owns slice w of the
     // current chunk; the last chunk may leave the upper waves without one.
     const int n_waves = blockDim.x >> 6;
-    const int total_slices = (K + kSliceK - 1) / kSliceK;  // (the last one may end short: K is a multiple of a lane load's k)
+    const int total_slices = kAny ? (K + kSliceK - 1) / kSliceK : K / kSliceK;  // (the last one may end short: K is a multiple of a lane load's k)
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int r16 = lane & 15;  // W row within the tile (A operand) / X row m (B operand)
@@ -326,18 +336,21 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // lie 4*LB bytes apart in each of 16 rows.  Packed layout (pack_codes_kernel below): the 64 lane
     // loads of a wave load are contiguous, [tile][slice][load][lane], so that a wave instruction
     // reads 64*LB consecutive bytes instead of 16 pieces of 4*LB.
-    constexpr int kLoadPitch = 64 * C::LB;  // packed: bytes between the loads of a slice
+    constexpr int kLoadPitch = PACKED ? 64 * C::LB : 4 * C::LB;  // bytes between the loads of a slice
     // A lane load past the end of K (in a short last slice) reads the chunk's first codes instead, against zeros of X.
-    uint32_t voff[PACKED ? 1 : C::LPT];
+    constexpr bool kOneOffset = PACKED || !kAny;
+    uint32_t voff[kOneOffset ? 1 : C::LPT];
     auto set_voff = [&]() {
         if constexpr (PACKED) {
             voff[0] = (uint32_t)((w * C::LPT * 64 + lane) * C::LB);
+        } else if constexpr (!kAny) {
+            voff[0] = (uint32_t)((r16 * J + (w * kSliceK + kq * C::K_LANE) / VEC) * (int)sizeof(CodeT));
         } else {
 #pragma unroll
             for (int t = 0; t < C::LPT; t++) {
                 const int k = w * kSliceK + t * C::K_WAVE + kq * C::K_LANE;  // inside the chunk
                 voff[t] = (uint32_t)((r16 * J + k / VEC) * (int)sizeof(CodeT));
-                if (K % kSliceK != 0 && chunk * n_waves * kSliceK + k >= K) voff[t] = (uint32_t)(r16 * J * (int)sizeof(CodeT));
+                if (chunk * n_waves * kSliceK + k >= K) voff[t] = (uint32_t)(r16 * J * (int)sizeof(CodeT));
             }
         }
     };
@@ -345,7 +358,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     const int row_bytes = J * (int)sizeof(CodeT);
     // first row of W of a tile: a last tile that N cuts short is moved up to end with N (its first rows are computed twice,
     // with the same result)
-    auto tile_row = [&](int tile) { return min(tile * kTileN, N - kTileN); };
+    auto tile_row = [&](int tile) { return kAny ? min(tile * kTileN, N - kTileN) : tile * kTileN; };
     const int chunk_bytes = n_waves * kSliceK / VEC * (int)sizeof(CodeT) * (PACKED ? kTileN : 1);
     auto load_unit = [&](int q, Codes (&cw)[TB]) {
 #pragma unroll
@@ -353,7 +366,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
             const int tile = tile_begin + q * TB + j;
             if (tile >= tile_end) break;
             const uint8_t *sbase = reinterpret_cast<const uint8_t *>(codes) + (int64_t)tile_row(tile) * row_bytes + chunk * chunk_bytes;
-            if constexpr (PACKED) {
+            if constexpr (kOneOffset) {
                 cw[j].template load_async_s<0>(0, voff[0], sbase);
                 if constexpr (C::LPT >= 2) cw[j].template load_async_s<kLoadPitch>(1, voff[0], sbase);
                 if constexpr (C::LPT >= 3) cw[j].template load_async_s<2 * kLoadPitch>(2, voff[0], sbase);
@@ -432,8 +445,10 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
         const int ln = opaque(lane);
         for (int pc = w; pc < n_blocks * M; pc += n_waves) {
             const int b = pc / M, i = pc - b * M;
-            const int kl = kc0 + b * kStageK + 8 * ln;
-            load_to_lds_16(stage_off + pc * kStagePitch, (uint32_t)((i * K + (kl < K ? kl : 0)) * 2), x);
+            int kl = kc0 + b * kStageK + 8 * ln;
+            kl = kl < K ? kl : 0;
+            if (kAny && !GATED && k_x != K) kl %= k_x;
+            load_to_lds_16(stage_off + pc * kStagePitch, (uint32_t)((i * k_x + kl) * 2), x);
         }
     };
     auto pick_x = [&]() {
@@ -448,9 +463,9 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
             if (active && row < M) v = *reinterpret_cast<const uint4_t *>(smem + win + k * 2);
             xr[s] = as_half8(v);
         }
-        // a slice that K cuts short: zeros behind its end (a branch of its own, so that whole slices test nothing)
+        // a slice that K cuts short: zeros behind its end
         const int k_left = K - chunk * n_waves * kSliceK - k0;
-        if (k_left < kSliceK) {
+        if (kAny && k_left < kSliceK) {
 #pragma unroll
             for (int s = 0; s < kSteps; s++)
                 if ((s / C::SPL) * C::K_WAVE + kg * C::K_LANE + (s % C::SPL) * 8 >= k_left) xr[s] = half8_t{};
@@ -581,9 +596,11 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
             if (!last) {
                 *carry = sum;
             } else if constexpr (kHasBias) {
-                half4_t b;  // (eight bytes at any even address: N may be any number)
-                __builtin_memcpy(&b, bias + n_bias, 8);
-                sum += float4_t{(float)b[0], (float)b[1], (float)b[2], (float)b[3]};
+                if (!kAny || bias) {
+                    half4_t b;  // (eight bytes at any even address: N may be any number)
+                    __builtin_memcpy(&b, bias + n_bias, 8);
+                    sum += float4_t{(float)b[0], (float)b[1], (float)b[2], (float)b[3]};
+                }
             }
             return sum;
         };
@@ -631,11 +648,13 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
         }
         n_act = min(n_waves, total_slices - chunk * n_waves);
         active = w < n_act;
-        if (n_chunks > 1 && K % kSliceK != 0) set_voff();
+        if constexpr (kAny) set_voff();
         // The first codes are requested before the table or X are replaced, to overlap the latencies.
         load_first_units();
         __syncthreads();  // every gather from the old table has been consumed, every slot read
-        if (n_chunks > 1) stage_x();
+        // (a chunk that starts where X repeats has the X of the chunk before it, unless K cuts its last slice short)
+        const bool new_x = n_chunks > 1 && (!kAny || n_waves * kSliceK != k_x || n_act != n_waves);
+        if (new_x) stage_x();
         if (chunk == 0) {
             // (the thread index goes through an empty asm so that nothing derived from it is kept
             // in registers across the tile loop just to be reused here)
@@ -649,7 +668,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
                 if (i1 < cb_slots) cb_lds[i1] = b;
             }
         }
-        if (n_chunks > 1) {
+        if (new_x) {
             wait_vmcnt<0>();
             __syncthreads();  // pieces staged by the other waves, and the new table
             pick_x();
@@ -790,6 +809,20 @@ hipError_t launch_decode_batched(const ProblemB &p, hipStream_t s)
     };
     // a full batch of one tile is the only case with a replicated table and TB = 1
     const int tb = g.full ? C::TB : 1;
+    if constexpr (!PACKED) {
+        // K that is no multiple of a slice, N that is none of a tile, an X that repeats: the instantiations that test for those
+        if (p.K % kSliceK != 0 || p.N % kTileN != 0 || p.k_x != p.K) {
+            if constexpr (C::TB % 2 == 0) {
+                if (p.gated) return g.repl ? launch(decode_batched_kernel<VEC, CodeT, true, C::TB, false, true, const half_t *, int>, p.bias, p.k_x)
+                                           : launch(decode_batched_kernel<VEC, CodeT, false, C::TB, false, true, const half_t *, int>, p.bias, p.k_x);
+            }
+            if (p.gated) return hipErrorInvalidValue;
+            if (g.repl) return tb == 1 ? launch(decode_batched_kernel<VEC, CodeT, true, 1, false, false, const half_t *, int>, p.bias, p.k_x)
+                                       : launch(decode_batched_kernel<VEC, CodeT, true, C::TB, false, false, const half_t *, int>, p.bias, p.k_x);
+            return tb == 1 ? launch(decode_batched_kernel<VEC, CodeT, false, 1, false, false, const half_t *, int>, p.bias, p.k_x)
+                           : launch(decode_batched_kernel<VEC, CodeT, false, C::TB, false, false, const half_t *, int>, p.bias, p.k_x);
+        }
+    }
     if constexpr (!PACKED && C::TB % 2 == 0) {
         if (p.gated) {
             if (p.bias) return g.repl ? launch(decode_batched_kernel<VEC, CodeT, true, C::TB, false, true, const half_t *>, p.bias)
@@ -950,9 +983,12 @@ bool decode_gemv_preferred(const ProblemB &p)
     return (double)p.K <= tn.gemv_max_k;
 }
 
+// Whether launch_decode_b reads an X that repeats along K (the batched kernel does, in every layout of the codes).
+bool decode_stages_supports(const ProblemB &p) { return decode_supports(p) && batched_supports(p) && !decode_stream_preferred(p) && p.k_x % 8 == 0; }
+
 hipError_t launch_decode_b(const ProblemB &p, hipStream_t s)
 {
-    if (!decode_supports(p)) return hipErrorInvalidValue;
+    if (!decode_supports(p) || (p.k_x != p.K && !decode_stages_supports(p))) return hipErrorInvalidValue;
     // long rows of W: the streaming kernel (the batched kernel would walk K in chunks)
     if (decode_stream_preferred(p)) return launch_decode_stream(p, s);
     const bool u8 = p.code_bits == 8;

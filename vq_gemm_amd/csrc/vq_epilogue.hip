@@ -65,4 +65,36 @@ hipError_t launch_silu_mul(const half_t *a, half_t *out, int64_t M, int64_t N, h
     }
 }
 
+namespace {
+
+// X for a product over additive stages side by side along K: every row `stages` times, 16 bytes per thread where rows
+// allow (VEC halves per step).
+template <int VEC>
+__global__ __launch_bounds__(256) void repeat_columns_kernel(const half_t *__restrict__ x, half_t *__restrict__ out, int64_t M,
+                                                             int K, int stages)
+{
+    typedef half_t vec_t __attribute__((ext_vector_type(VEC)));
+    const int row = K / VEC;
+    const int64_t total = M * row;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+        const int64_t m = i / row;
+        const int c = (int)(i - m * row);
+        const vec_t v = reinterpret_cast<const vec_t *>(x)[i];
+        for (int s = 0; s < stages; s++) reinterpret_cast<vec_t *>(out)[(m * stages + s) * row + c] = v;
+    }
+}
+
+}  // namespace
+
+hipError_t launch_repeat_columns(const half_t *x, half_t *out, int64_t M, int64_t K, int stages, hipStream_t s)
+{
+    if (M == 0 || K == 0) return hipSuccess;
+    const bool vec8 = K % 8 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+    int64_t blocks = (M * (vec8 ? K / 8 : K) + 255) / 256;
+    const int64_t cap = (int64_t)device_cu_count() * 16;
+    if (blocks > cap) blocks = cap;
+    if (vec8) return launch_kernel(repeat_columns_kernel<8>, dim3((unsigned)blocks), dim3(256), 0, s, x, out, M, (int)K, stages);
+    return launch_kernel(repeat_columns_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, s, x, out, M, (int)K, stages);
+}
+
 }  // namespace vq

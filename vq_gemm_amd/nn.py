@@ -9,6 +9,7 @@ holds it as one node.  Nothing falls back to the CPU.
 from __future__ import annotations
 
 import torch
+from torch.compiler import is_compiling
 
 from . import cabi
 from .quantize import kmeans_quantize, residual_quantize
@@ -94,7 +95,7 @@ class VQLinear(torch.nn.Module):
         # Called eagerly on an ordinary GPU tensor, the layer is one native call (no dispatch, no autograd bookkeeping:
         # what surrounds a kernel of a few microseconds is most of a decode call's time); under a tracer, a dispatch
         # mode or torch.compile it is the registered operator.
-        if not torch.compiler.is_compiling():
+        if not is_compiling():
             b = self._buffers
             if b["codes_packed"] is None:
                 y = native.linear(x, b["codes"], b["codebook"], b["bias"], self.k_repeat)
@@ -151,7 +152,7 @@ class VQGatedMLP(torch.nn.Module):
         return cls(gu, VQLinear.from_float(down, vec, entries, n_codebooks, None, iters, seed + 1), interleaved=True)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if self.interleaved and not torch.compiler.is_compiling():
+        if self.interleaved and not is_compiling():
             b = self.gate_up._buffers
             h = native.gated(x, b["codes"], b["codebook"], b["bias"])
             if h is not None:
