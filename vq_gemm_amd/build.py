@@ -44,7 +44,7 @@ HIP_FLAGS = ["-O3", f"--offload-arch={ARCH}", "-fPIC", "-std=c++17", "-fno-gpu-r
 # The decode kernels are short launches, and a wave's first instruction there is a fetch of its kernel arguments from a
 # cold scalar cache: gfx950 can hand the first arguments to a wave in scalar registers at launch (at most 14 dwords beside
 # the two of the argument pointer).  The kernels of these sources take their arguments in the order they need them.
-KERNARG_PRELOAD_SOURCES = {"vq_decode_gemv.hip"}
+KERNARG_PRELOAD_SOURCES = {"vq_decode_gemv.hip", "vq_decode.hip"}
 KERNARG_PRELOAD_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=14"]
 
 # variant key -> (VQGEMM_VARIANT_* value, is the hipBLASLt baseline module)
