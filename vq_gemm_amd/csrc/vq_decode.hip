@@ -698,7 +698,7 @@ struct BatchedPlan {
 // LDS must hold the table,
 // the slots, the staged X and, when K goes in chunks, the carried sums of the workgroup's tiles.
 template <int VEC, typename CodeT>
-BatchedPlan plan_batched(const ProblemB &p)
+BatchedPlan plan_batched_chunks(const ProblemB &p, int n_chunks)
 {
     typedef DecodeCfg<VEC, CodeT> C;
     BatchedPlan g = {};
@@ -711,7 +711,8 @@ BatchedPlan plan_batched(const ProblemB &p)
     const int deal = p.gated ? 2 : 1;
     if (p.gated && (p.rows_per_cb % (2 * kTileN) != 0 || C::TB % 2 != 0 || p.packed)) return g;
     const int slices = (p.K + kSliceK - 1) / kSliceK;
-    g.n_chunks = (slices + kMaxWaves - 1) / kMaxWaves;
+    if (n_chunks > slices) return g;
+    g.n_chunks = n_chunks;
     g.n_waves = (slices + g.n_chunks - 1) / g.n_chunks;
     const int m_slab = p.M < kTileN ? p.M : kTileN;  // rows of X one workgroup multiplies
     g.tiles_per_cb = (p.rows_per_cb + kTileN - 1) / kTileN;
@@ -778,6 +779,17 @@ BatchedPlan plan_batched(const ProblemB &p)
         if (g.books_per_wg > 1) g.books_per_wg = 1;  // one codebook per workgroup first
         else g.wgs_per_cb = g.wgs_per_cb * 2 < g.tiles_per_cb / deal ? g.wgs_per_cb * 2 : g.tiles_per_cb / deal;
     }
+}
+
+// As few chunks of K as sixteen waves need; more (with fewer waves each) where the staged X of so many does not fit the LDS beside
+// the table: 4096-entry tables on K beyond 4096.
+template <int VEC, typename CodeT>
+BatchedPlan plan_batched(const ProblemB &p)
+{
+    const int slices = (p.K + kSliceK - 1) / kSliceK, fewest = (slices + kMaxWaves - 1) / kMaxWaves;
+    BatchedPlan g = {};
+    for (int n_chunks = fewest; n_chunks <= 2 * fewest && !g.ok; n_chunks++) g = plan_batched_chunks<VEC, CodeT>(p, n_chunks);
+    return g;
 }
 
 BatchedPlan plan_batched(const ProblemB &p)
