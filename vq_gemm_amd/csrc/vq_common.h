@@ -158,7 +158,6 @@ double prefill_small_cost_us(const ProblemB &p);  // expected time, microseconds
 // n_begin > 0: the W rows [n_begin, N) only (a multiple of 128; the workspace is then sized for those columns)
 hipError_t launch_prefill_small_b(const ProblemB &p, hipStream_t s, int splits = 1, void *workspace = nullptr, int n_begin = 0);
 bool prefill_splitk_supports(const ProblemB &p, int splits);
-size_t prefill_splitk_counter_bytes(int64_t tiles);
 size_t prefill_splitk_workspace_bytes(const ProblemB &p, int splits);
 // slices of K the cost model expects to be fastest with 128x128 tiles and the time it expects (min_splits 1: none is a
 // candidate; 2: the best split); 0 when no split applies
@@ -187,8 +186,6 @@ hipError_t launch_silu_mul(const half_t *a, half_t *out, int64_t M, int64_t N, h
 
 // out[0] = the largest code of codes[0 .. count) (0 when count == 0); out is device memory
 hipError_t launch_max_code(const void *codes, int64_t count, int code_bits, uint32_t *out, hipStream_t s);
-// words[0 .. n) = 0, by a kernel (a launch that may be captured into a graph records no memset)
-hipError_t launch_clear_words(uint32_t *words, int64_t n, hipStream_t s);
 
 // compute units of the current device
 int device_cu_count();
@@ -257,13 +254,13 @@ struct Tuning {
     // whole rounds of large tiles plus the left-over columns in 128x128 tiles with K split: taken with a workspace when
     // expected below this share of the best single plan (0: never; 1000 and more: wherever the plan exists)
     double tail_split_margin = 0.93;
-    // split K over 128x128 tiles: the clearing launch and the last workgroup's extra pass, and the partial sums
-    // written and read once (microseconds per MB of partial sums)
+    // split K over 128x128 tiles: the second launch, and the partial sums written and read once (microseconds per MB of
+    // partial sums)
     double splitk_fixed_us = 4.5;
     double splitk_us_per_partial_mb = 0.15;
-    // 2, 4 or 8: VQGEMM_VARIANT_PREFILL_SPLITK takes this many slices where the shape allows (for measurements); 0: the cost model's
+    // 2 .. 16: VQGEMM_VARIANT_PREFILL_SPLITK takes this many slices where the shape allows (for measurements); 0: the cost model's
     double splitk_force_splits = 0.0;
-    double splitk_validate_fences = 0.0;  // 1: release / acquire fences of device scope around the split-K count (validation)
+    double splitk_validate_fences = 0.0;  // (accepted, without effect: the slices meet in a second launch)
 };
 const Tuning &tuning();
 

@@ -20,10 +20,12 @@
 // ends with one of 64.)
 //
 // Split K.  Where even these tiles are fewer than the compute units, `splits` workgroups share a tile, each
-// multiplying its share of K (whole code tiles).  Nothing waits for anything: a workgroup writes its fp32 sums to a partial
-// buffer with device-scope stores, waits for them, and counts itself in on the tile's counter; the one that
-// finds itself last adds the partial sums up in the order of the slices and runs the epilogue.  The sum is the same whoever comes last, so
-// results do not depend on the order in which the workgroups finish.
+// multiplying its share of K (whole code tiles).  They write their fp32 sums out as their lanes hold them, whole kilobytes
+// per store, and a second launch adds the slices up in order, with the bias or the gate, and rounds: the same bits whatever
+// finishes when, nothing waits for anything inside a kernel, and the additions are spread over the whole device.
+// (With the additions done by the workgroup of a tile that counts itself last, out of 64 KB per slice through device-scope
+// loads and behind a launch that clears the counters, few tiles in many slices are serial: in eight slices M = 128, K = 8192,
+// N = 1024 took 22.4 us and takes 16.2; M = 128, K = 11008, N = 4096 28.5 and 24.4; M = 32, K = N = 4096 21.5 and 12.6.)
 #include "vq_prefill_common.h"
 
 #include <type_traits>
@@ -56,8 +58,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
                                                                     int N, int n_begin, int ldn, int entries,
                                                                     int rows_per_cb, int tiles_m,
                                                                     int tiles_n, int cb_lds_count, int gated,
-                                                                    int splits, float4_t *__restrict__ partials,
-                                                                    unsigned int *__restrict__ counters, int fenced)
+                                                                    int splits, float4_t *__restrict__ partials)
 {
     typedef PrefillCfg<VEC, CodeT> C;
     constexpr int D = NS - 1;                 // loads run D stages ahead
@@ -315,65 +316,19 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     if constexpr (HALF) hold_accumulators(acc);
 
-    // ---- split K: partial sums out, and the workgroup that comes last adds them up -------------------
-    // The partial sums are written and read with device-scope memory instructions (sc1: through the L2 of the
-    // XCD, which is not coherent with the other seven), and the waits are written out: a release / acquire fence
-    // of device scope would write back and invalidate the whole L2 under the workgroups that are still multiplying
-    // (measured: 3 us per MB of partial sums).  A store is complete, and visible device-wide, when the counter
-    // has counted it; the count itself is a relaxed device-scope atomic; the loads of the last workgroup are issued
-    // behind the barrier that follows its count.
-#if !defined(__HIP_DEVICE_COMPILE__) || defined(__gfx942__) || defined(__gfx950__)
-    // (what "sc1" means for a store and a load, and that a counted store is visible device-wide, are properties of
-    // these two targets; another target has to re-establish them or build with the fences below)
-#else
-#error "the split-K exchange relies on the gfx942/gfx950 behaviour of device-scope (sc1) loads and stores"
-#endif
+    // ---- split K: this slice's sums out -------------------------------------------------------------------------
     if (splits > 1) {
-        // partial sums of (tile, slice): half h (two floats) of accumulator (j, i) of thread tid at
-        // [((j * SMP + i) * 2 + h) * 256 + tid], moved as 64-bit words (the widest scoped access there is)
-        constexpr int kPartial = SNP * SMP * 2 * kThreads;  // 64-bit words per tile and slice
-        typedef float float2_t __attribute__((ext_vector_type(2)));
-        uint64_t *tile_partials = reinterpret_cast<uint64_t *>(partials) + (int64_t)wg * splits * kPartial;
-        uint64_t *mine = tile_partials + (int64_t)split * kPartial + tid;
+        // (byte offsets in 32 bits from a uniform base: the accumulators leave few registers for addresses)
+        uint8_t *base = reinterpret_cast<uint8_t *>(partials + (((int64_t)split * n_wg + wg) * 4 + wave) * (SNP * SMP * 64));
+        const uint32_t at = (threadIdx.x & 63) * 16u;
+        const int rows = M - m0 - wm * SWM;  // of the wave tile that exist
 #pragma unroll
-        for (int j = 0; j < SNP; j++)
+        for (int i = 0; i < SMP; i++)
+            if (i * 16 < rows) {
 #pragma unroll
-            for (int i = 0; i < SMP; i++)
-#pragma unroll
-                for (int h = 0; h < 2; h++)
-                    __hip_atomic_store(mine + ((j * SMP + i) * 2 + h) * kThreads,
-                                       __builtin_bit_cast(uint64_t, float2_t{acc[j][i][2 * h], acc[j][i][2 * h + 1]}), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-        // Every partial-sum store of this thread is complete (counted back) here, and the barrier extends that to the
-        // workgroup: nothing may be moved across this wait - not the stores above it, not the count below it.
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        // (validation path, Tuning::splitk_validate_fences: the textbook release / acquire pair of device scope around
-        // the count, as the memory model asks for; same results bit for bit, at the cost of the L2 write-backs)
-        if (fenced) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        __syncthreads();
-        uint32_t *flag = reinterpret_cast<uint32_t *>(smem);
-        if (tid == 0) *flag = __hip_atomic_fetch_add(counters + wg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        const bool last = *flag == (uint32_t)(splits - 1);
-        __syncthreads();  // the flag's word belongs to the epilogue's staging area again
-        if (!last) return;
-        if (fenced) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        // The sum in the order of the slices, whoever is last - this workgroup's own sums are read back like the
-        // others' (the same bits it wrote; its registers are free for the loads that way).
-        for (int sl = 0; sl < splits; sl++) {
-            const uint64_t *src = tile_partials + (int64_t)sl * kPartial + tid;
-#pragma unroll
-            for (int j = 0; j < SNP; j++)
-#pragma unroll
-                for (int i = 0; i < SMP; i++)
-#pragma unroll
-                    for (int h = 0; h < 2; h++) {
-                        const float2_t v = __builtin_bit_cast(
-                            float2_t, __hip_atomic_load(src + ((j * SMP + i) * 2 + h) * kThreads, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-                        acc[j][i][2 * h] = sl == 0 ? v[0] : acc[j][i][2 * h] + v[0];
-                        acc[j][i][2 * h + 1] = sl == 0 ? v[1] : acc[j][i][2 * h + 1] + v[1];
-                    }
-        }
+                for (int j = 0; j < SNP; j++) *reinterpret_cast<float4_t *>(base + (i * SNP + j) * 1024 + at) = acc[j][i];
+            }
+        return;
     }
 
     // ---- epilogue: lane holds Y[m = i*16 + r16][n = j*16 + 4*kg + 0..3] of its 64x64 wave tile ----
@@ -452,8 +407,53 @@ bool small_cfg_supports(const ProblemB &p)
            (int64_t)SBM * p.K * 2 < ((int64_t)1 << 32);
 }
 
-// float4 slots of partial sums per tile and slice, and where the tiles' counters start inside the workspace
-constexpr size_t kPartialBytes = (size_t)SNP * SMP * kThreads * 16;  // 64 KB
+constexpr size_t kPartialBytes = (size_t)SNP * SMP * kThreads * 16;  // of one tile and slice: 64 KB
+
+// The second launch of a split product: the slices' sums of a piece of 16 x 16 in the order of the slices (+ bias), rounded once;
+// GATED: silu(gate) * up of a pair of pieces.  A wave takes a piece (a pair), one workgroup a wave tile of the first launch.
+// Bound by the partial sums' way back (out of the last-level cache) and by its own launch.
+template <bool GATED>
+__global__ __launch_bounds__(SNP *SMP * 64) void splitk_sum_kernel(const float4_t *__restrict__ partials, half_t *__restrict__ y,
+                                                                  const half_t *__restrict__ bias, int M, int N, int n_begin, int ldn,
+                                                                  int tiles_m, int tiles_n, int splits)
+{
+    constexpr int kPer = GATED ? 2 : 1;  // pieces of a wave
+    const int lane = threadIdx.x & 63, r16 = lane & 15, kg = lane >> 4;
+    const int piece = (threadIdx.x >> 6) * kPer, i = piece / SNP, j = piece % SNP;
+    const int tile = blockIdx.x >> 2, wave = blockIdx.x & 3;
+    const int n_wg = tiles_m * tiles_n;
+    const int m = (tile / tiles_n) * SBM + (wave >> 1) * SWM + i * 16 + r16;
+    const int n = n_begin + (tile % tiles_n) * SBN + (wave & 1) * SWN + j * 16 + 4 * kg;
+    if (m >= M || n >= N) return;
+    const float4_t *src = partials + ((int64_t)tile * 4 + wave) * (SNP * SMP * 64) + piece * 64 + lane;
+    const int64_t slice = (int64_t)n_wg * (kPartialBytes / 16);
+    float4_t a[kPer];
+#pragma unroll
+    for (int h = 0; h < kPer; h++) a[h] = src[h * 64];
+    for (int s = 1; s < splits; s++)
+#pragma unroll
+        for (int h = 0; h < kPer; h++) a[h] += src[s * slice + h * 64];
+    if (bias)
+#pragma unroll
+        for (int h = 0; h < kPer; h++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (n + 16 * h + e < N) a[h][e] += (float)bias[n + 16 * h + e];
+    if constexpr (GATED) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) a[0][e] = silu_f32(a[0][e]) * a[1][e];
+    }
+    const half4_t v = {(half_t)a[0][0], (half_t)a[0][1], (half_t)a[0][2], (half_t)a[0][3]};
+    const int first = GATED ? (n >> 5) * 16 + (n & 15) : n, end = GATED ? N / 2 : N;
+    half_t *dst = y + (int64_t)m * (GATED ? ldn / 2 : ldn) + first;
+    if (first + 4 <= end) {
+        __builtin_memcpy(dst, &v, 8);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (first + e < end) dst[e] = v[e];
+    }
+}
 
 // n_begin: the launch covers the W rows [n_begin, N) only (a multiple of the tile's 128 rows)
 template <int VEC, typename CodeT>
@@ -464,15 +464,7 @@ hipError_t launch_small_typed(const ProblemB &p, hipStream_t s, int splits, void
     if (splits < 1 || (splits > 1 && (!workspace || p.K / C::K_SUPER < 2 * splits))) return hipErrorInvalidValue;
     if (n_begin < 0 || n_begin >= p.N || n_begin % SBN != 0) return hipErrorInvalidValue;
     const int tiles_m = (p.M + SBM - 1) / SBM, tiles_n = (p.N - n_begin + SBN - 1) / SBN;
-    // workspace: the tiles' counters (cleared here, by a kernel: the launch may be captured), then the partial sums
-    unsigned int *counters = static_cast<unsigned int *>(workspace);
-    float4_t *partials = nullptr;
-    if (splits > 1) {
-        const size_t counter_bytes = prefill_splitk_counter_bytes(tiles_m * tiles_n);
-        partials = reinterpret_cast<float4_t *>(static_cast<uint8_t *>(workspace) + counter_bytes);
-        const hipError_t e = launch_clear_words(counters, tiles_m * tiles_n, s);
-        if (e != hipSuccess) return e;
-    }
+    float4_t *partials = splits > 1 ? static_cast<float4_t *>(workspace) : nullptr;
     const size_t smem = lds_bytes_small<VEC, CodeT>(p, 4);
     // the split codebook layout is built out of a copy in the last X buffer
     constexpr bool can_split = VEC == 8 && sizeof(CodeT) == 1;
@@ -481,10 +473,12 @@ hipError_t launch_small_typed(const ProblemB &p, hipStream_t s, int splits, void
     const bool half = p.K % C::K_SUPER != 0;
     auto kern = half ? (split ? prefill_small_kernel<VEC, CodeT, 4, can_split, can_half> : prefill_small_kernel<VEC, CodeT, 4, false, can_half>)
                      : (split ? prefill_small_kernel<VEC, CodeT, 4, can_split, false> : prefill_small_kernel<VEC, CodeT, 4, false, false>);
-    return launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(kThreads), smem, s, p.x,
-                       static_cast<const CodeT *>(p.codes), p.cb, p.y, p.bias, p.M, p.K, p.N, n_begin, p.N, p.entries,
-                       p.rows_per_cb, tiles_m, tiles_n, codebooks_per_tile(p, SBN), p.gated ? 1 : 0, splits, partials, counters,
-                       tuning().splitk_validate_fences >= 1.0 ? 1 : 0);
+    const hipError_t e = launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(kThreads), smem, s, p.x,
+                                       static_cast<const CodeT *>(p.codes), p.cb, p.y, p.bias, p.M, p.K, p.N, n_begin, p.N, p.entries,
+                                       p.rows_per_cb, tiles_m, tiles_n, codebooks_per_tile(p, SBN), p.gated ? 1 : 0, splits, partials);
+    if (e != hipSuccess || splits == 1) return e;
+    return launch_kernel(p.gated ? splitk_sum_kernel<true> : splitk_sum_kernel<false>, dim3((unsigned)(tiles_m * tiles_n * 4)),
+                         dim3(SNP * SMP * 64 / (p.gated ? 2 : 1)), 0, s, partials, p.y, p.bias, p.M, p.N, n_begin, p.N, tiles_m, tiles_n, splits);
 }
 
 }  // namespace
@@ -538,24 +532,21 @@ static int small_k_super(const ProblemB &p)
     return kc > kStageK ? kc : kStageK;
 }
 
-size_t prefill_splitk_counter_bytes(int64_t tiles) { return ((size_t)tiles * 4 + 255) & ~(size_t)255; }
-
 size_t prefill_splitk_workspace_bytes(const ProblemB &p, int splits)
 {
     if (splits <= 1) return 0;
-    const int64_t tiles = (int64_t)((p.M + SBM - 1) / SBM) * ((p.N + SBN - 1) / SBN);
-    return prefill_splitk_counter_bytes(tiles) + (size_t)tiles * splits * kPartialBytes;
+    return (size_t)splits * ((p.M + SBM - 1) / SBM) * ((p.N + SBN - 1) / SBN) * kPartialBytes;
 }
 
 // (a slice is at least two code tiles: the loads run that far ahead)
 bool prefill_splitk_supports(const ProblemB &p, int splits)
 {
-    return splits >= 2 && splits <= 8 && prefill_small_supports(p) && p.K / small_k_super(p) >= 2 * splits;
+    return splits >= 2 && splits <= 16 && prefill_small_supports(p) && p.K / small_k_super(p) >= 2 * splits;
 }
 
 // The number of slices of K (1: none) that the cost model expects to be fastest with 128x128 tiles, and its time.
-// A slice is a workgroup of its own: `splits` times the tiles, each over K / splits; on top of that the clearing launch
-// and, per tile, the partial sums written and read once (Tuning::splitk_fixed_us, splitk_us_per_partial_mb).
+// A slice is a workgroup of its own: `splits` times the tiles, each over K / splits; on top of that the second launch
+// and the partial sums written and read once (Tuning::splitk_fixed_us, splitk_us_per_partial_mb).
 int prefill_splitk_choice(const ProblemB &p, double *cost_us, int min_splits)
 {
     int best = min_splits <= 1 ? 1 : 0;
@@ -566,7 +557,7 @@ int prefill_splitk_choice(const ProblemB &p, double *cost_us, int min_splits)
         if (cost_us) *cost_us = 0.0;
         return (int)tn.splitk_force_splits;
     }
-    for (int sp = 2; sp <= 8; sp *= 2) {
+    for (const int sp : {2, 3, 4, 6, 8, 12, 16}) {
         if (!prefill_splitk_supports(p, sp)) break;
         ProblemB q = p;  // the slices as the kernel sees them: sp times the tiles over K / sp
         q.K = p.K / sp;
@@ -576,7 +567,7 @@ int prefill_splitk_choice(const ProblemB &p, double *cost_us, int min_splits)
         const double busy = wgs >= cus ? 1.0 : (double)wgs / cus;
         const double main_us = (double)resident_rounds * tn.prefill_small_tile_fixed_us +
                                (double)rounds * (q.K / 64.0 * (tn.prefill_small_stage_us_idle + (tn.prefill_small_stage_us_busy - tn.prefill_small_stage_us_idle) * busy));
-        const double fix_us = tn.splitk_fixed_us + tn.splitk_us_per_partial_mb * (double)(wgs * kPartialBytes) / 1e6;
+        const double fix_us = tn.splitk_fixed_us + tn.splitk_us_per_partial_mb * (double)sp * p.M * p.N * 4e-6;
         if (main_us + fix_us < best_us) {
             best_us = main_us + fix_us;
             best = sp;
