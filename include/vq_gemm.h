@@ -75,10 +75,12 @@ extern "C" {
                                             VQGEMM_VARIANT_DECODE, the K-sliced MFMA kernels (the limits are constants
                                             of the tuning table below) */
 
-#define VQGEMM_VARIANT_PREFILL_SPLITK 9  /* vqgemm_e2e_gemm_b_ws only: the 128x128 tiles with K split over 2, 4 or 8
+#define VQGEMM_VARIANT_PREFILL_SPLITK 9  /* vqgemm_e2e_gemm_b_ws only: the 128x128 tiles with K split over 2 to 16
                                             workgroups per tile (as many as the cost model expects to be fastest);
                                             medium M on few columns, where whole tiles are fewer than the compute
                                             units; fp32 partial sums through the workspace */
+#define VQGEMM_VARIANT_WAVE_K 10  /* small tiles of Y, K dealt out to the waves of a workgroup: medium M, where the tiles of
+                                     VQGEMM_VARIANT_PREFILL are fewer than the compute units */
 
 /*
  * Fused VQ GEMM, geometry B.

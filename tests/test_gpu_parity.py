@@ -1932,3 +1932,74 @@ def test_stages_multiply_the_same_x_without_a_copy_of_it(M, K, N, v, entries, st
         y = VQLinear(codes, cb, b, k_repeat=stages)(x)
         torch.cuda.synchronize()
         assert torch.equal(y, cabi.e2e_gemm_b_ws(x.repeat(1, stages), codes, cb, bias=b))
+
+
+def _with_wave_tile(tile, call):
+    before = cabi.tuning()
+    try:
+        cabi.set_tuning(wave_k_force=1, wave_k_force_tile=tile)
+        return call()
+    finally:
+        cabi.set_tuning(**{k: before[k] for k in ("wave_k_force", "wave_k_force_tile")})
+
+
+WAVE_K_B = [
+    # M, K, N, vec, E, bits, G: fewer units of K than waves, a last unit shorter than its load, edges of every tile, tiles over
+    # several codebooks, a column more than a tile
+    (1, 128, 16, 8, 256, 8, 1),
+    (17, 192, 32, 8, 256, 8, 1),
+    (65, 1088, 129, 8, 256, 8, 1),
+    (130, 832, 160, 8, 100, 8, 5),
+    (64, 2112, 128, 8, 300, 16, 4),
+    (33, 1216, 65, 4, 256, 8, 1),
+    (100, 704, 192, 4, 256, 8, 6),
+    (48, 960, 96, 4, 1024, 16, 2),
+    (70, 1024, 257, 4, 4096, 16, 1),
+]
+
+
+@pytest.mark.parametrize("row", WAVE_K_B, ids=["x".join(map(str, r)) for r in WAVE_K_B])
+def test_k_dealt_out_to_waves_geometry_b(row):
+    M, K, N, v, E, bits, G = row
+    spec = ProblemSpec("wave_k", GEOM_B, M, K, N, v, E, G, bits, codebook_3d=(G > 1), codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=91, device=DEV)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(4)).half().to(DEV)
+    want = _np(x).astype(np.float64) @ vo.dequant_b(_np(codes), _np(cb)).astype(np.float64).T
+    for tile in (12, 14, 18, 22, 24, 44, 48):
+        _say("wave_k", row, "tile", tile)
+        for b in (None, bias):
+            y = _with_wave_tile(tile, lambda: cabi.e2e_gemm_b(x, codes, cb, variant=cabi.VARIANT_WAVE_K, bias=b))
+            torch.cuda.synchronize()
+            assert vo.rel_err(_np(y), want if b is None else want + _np(b).astype(np.float64))[0] <= TOL, (row, tile)
+        if N % 32 == 0:
+            y = _with_wave_tile(tile, lambda: cabi.e2e_gemm_b_gated(x, codes, cb, variant=cabi.VARIANT_WAVE_K, bias=bias))
+            p = want + _np(bias).astype(np.float64)
+            p = p.reshape(M, N // 32, 2, 16)
+            gated = (p[:, :, 0] / (1 + np.exp(-p[:, :, 0])) * p[:, :, 1]).reshape(M, N // 2)
+            torch.cuda.synchronize()
+            assert vo.rel_err(_np(y), gated)[1] <= TOL, (row, tile, "gated")
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 64, 8), (17, 96, 40), (33, 320, 65), (65, 1056, 2047), (130, 2048, 129), (16, 512, 64)])
+@pytest.mark.parametrize("shift", [0, 1])   # elements by which w is off a 16-byte boundary
+def test_k_dealt_out_to_waves_plain_gemm(M, K, N, shift):
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(M, K, generator=g).half().to(DEV)
+    w = torch.randn(K * N + shift, generator=g).half().to(DEV)[shift:].view(K, N)
+    want = _np(x).astype(np.float64) @ _np(w).astype(np.float64)
+    for tile in (12, 22, 24, 42, 44):
+        _say("wave_k gemm", M, K, N, "shift", shift, "tile", tile)
+        y = _with_wave_tile(tile, lambda: cabi.gemm_f16(x, w))
+        torch.cuda.synchronize()
+        assert vo.rel_err(_np(y), want)[0] <= TOL, tile
+
+
+@pytest.mark.parametrize("M,K,Nc", [(1, 64, 16), (17, 320, 48), (65, 1088, 112), (129, 512, 64)])
+def test_k_dealt_out_to_waves_geometry_a(M, K, Nc):
+    spec = ProblemSpec("A", GEOM_A, M, K, 2 * Nc, 2, 256, Nc // 4, 8, codebook_std=0.05)
+    x, w, cb = make_problem(spec, seed=92, device=DEV)
+    for tile in (12, 22, 24, 42, 44, 84, 86):
+        _say("wave_k geometry A", M, K, Nc, "tile", tile)
+        y = _with_wave_tile(tile, lambda: cabi.e2e_gemm_a(x, w, cb, variant=cabi.VARIANT_PREFILL))
+        torch.cuda.synchronize()
+        _check_gemm(y, x, w, cb, geometry=GEOM_A, what=f"tile {tile}")

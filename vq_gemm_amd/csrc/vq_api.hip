@@ -135,6 +135,8 @@ const TuningEntry kTuningEntries[] = {
     {"splitk_fixed_us", &Tuning::splitk_fixed_us},
     {"splitk_us_per_partial_mb", &Tuning::splitk_us_per_partial_mb},
     {"splitk_force_splits", &Tuning::splitk_force_splits},
+    {"wave_k_force", &Tuning::wave_k_force},
+    {"wave_k_force_tile", &Tuning::wave_k_force_tile},
     {"splitk_validate_fences", &Tuning::splitk_validate_fences},
 };
 constexpr int kTuningCount = (int)(sizeof(kTuningEntries) / sizeof(kTuningEntries[0]));
@@ -193,6 +195,13 @@ bool aligned(const void *p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0;
 // leaves its 128-row tile mostly padding, and the kernel is still an order of magnitude ahead of the
 // scalar one).  Its 4-byte gathers keep the LDS busier than the matrix cores, so once there is more
 // than one round of tiles the two-pass route is faster - when the caller brings the scratch for it.
+// of the two fused geometry-A kernels (both take the same shapes)
+bool wave_k_a_preferred(const ProblemA &p)
+{
+    const int force = (int)tuning().wave_k_force;
+    return wave_k_a_supports(p) && force != 2 && (force == 1 || wave_k_a_cost_us(p) < fused_a_cost_us(p));
+}
+
 bool fused_a_preferred(const ProblemA &p, bool has_workspace)
 {
     if (p.M < 1 || !fused_a_supports(p)) return false;
@@ -240,6 +249,16 @@ int select_b(const ProblemB &p, bool all_aligned16)
         return decode_gemv_preferred(p) ? VQGEMM_VARIANT_DECODE_GEMV : VQGEMM_VARIANT_DECODE;
     if (prefill_ok) return VQGEMM_VARIANT_PREFILL;
     return VQGEMM_VARIANT_GENERIC;
+}
+
+// What the automatic choice launches without a workspace: select_b's kernel, or the wave-K kernel in its place.  (Above 64
+// rows the K-sliced path's model promises more than it keeps: there the prefill kernels' is what the wave-K kernel is held to.)
+int auto_b(const ProblemB &p, bool all_aligned16)
+{
+    const int plain = select_b(p, all_aligned16);
+    if ((plain == VQGEMM_VARIANT_DECODE || plain == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, p.M > 64 ? prefill_cost_us(p) : 0.0))
+        return VQGEMM_VARIANT_WAVE_K;
+    return plain;
 }
 
 }  // namespace
@@ -332,7 +351,7 @@ int vqgemm_e2e_gemm_b_bias(const void *x, const void *codes, const void *codeboo
     const DeviceScope device;
     int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
     if (rc != VQGEMM_OK) return rc;
-    if (variant < VQGEMM_VARIANT_AUTO || variant > VQGEMM_VARIANT_DECODE_GEMV) return VQGEMM_E_VARIANT;
+    if (variant < VQGEMM_VARIANT_AUTO || variant > VQGEMM_VARIANT_WAVE_K || variant == VQGEMM_VARIANT_PREFILL_SPLITK) return VQGEMM_E_VARIANT;
     if (M == 0 || N == 0) return VQGEMM_OK;
     if (!y || !codebook || (K > 0 && (!x || !codes))) return VQGEMM_E_NULL;
     const uintptr_t code_align = code_bits / 8;
@@ -343,7 +362,7 @@ int vqgemm_e2e_gemm_b_bias(const void *x, const void *codes, const void *codeboo
     ProblemB p = make_b(x, codes, codebook, y, M, K, N, vec, entries, n_codebooks, code_bits);
     p.bias = static_cast<const half_t *>(bias);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (variant == VQGEMM_VARIANT_AUTO) variant = select_b(p, a16);
+    if (variant == VQGEMM_VARIANT_AUTO) variant = auto_b(p, a16);
     hipError_t e = hipSuccess;
     switch (variant) {
     case VQGEMM_VARIANT_GENERIC:
@@ -379,6 +398,11 @@ int vqgemm_e2e_gemm_b_bias(const void *x, const void *codes, const void *codeboo
         if (!a16) return VQGEMM_E_ALIGN;
         if (K == 0 || !prefill_small_supports(p)) return VQGEMM_E_VARIANT;
         e = launch_prefill_small_b(p, s);
+        break;
+    case VQGEMM_VARIANT_WAVE_K:
+        if (!a16) return VQGEMM_E_ALIGN;
+        if (!wave_k_b_supports(p)) return VQGEMM_E_VARIANT;
+        e = launch_wave_k_b(p, s);
         break;
     case VQGEMM_VARIANT_TWOPASS:
         if (bias) return VQGEMM_E_VARIANT;  // the plain GEMM of the two-pass route has no bias input
@@ -420,15 +444,16 @@ int splitk_auto(const ProblemB &p, bool all_aligned16, double *t_best = nullptr,
 // of large tiles with the left-over columns in 128x128 tiles and K split there (tail) - whichever the cost models
 // expect to be fastest by a margin.
 struct WorkspaceChoice {
+    bool wave;      // the wave-K kernel, which needs none
     int sp;
     TailSplitPlan tail;
     size_t bytes;
 };
 WorkspaceChoice workspace_auto(const ProblemB &p, bool all_aligned16)
 {
-    WorkspaceChoice c = {0, {false, 0, 0, 0, 1e30, 0}, 0};
+    WorkspaceChoice c = {false, 0, {false, 0, 0, 0, 1e30, 0}, 0};
     double t_best = 1e30;
-    int plain = 0;
+    int plain = VQGEMM_VARIANT_GENERIC;
     c.sp = splitk_auto(p, all_aligned16, &t_best, &plain);
     if (c.sp >= 2) c.bytes = prefill_splitk_workspace_bytes(p, c.sp);
     if (plain == VQGEMM_VARIANT_PREFILL && t_best < 1e29) {
@@ -441,6 +466,11 @@ WorkspaceChoice workspace_auto(const ProblemB &p, bool all_aligned16)
             c.bytes = tail.workspace_bytes;
         }
     }
+    // (a split asked for by the tuning table is not weighed against anything)
+    const bool asked = tuning().splitk_force_splits >= 2.0 || tuning().tail_split_margin >= 1e3;
+    const double t_other = c.tail.ok ? c.tail.cost_us : c.sp >= 2 ? t_best : p.M > 64 ? prefill_cost_us(p) : 0.0;
+    if (!(asked && c.bytes > 0) && (plain == VQGEMM_VARIANT_DECODE || plain == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, t_other))
+        c = {true, 0, {false, 0, 0, 0, 1e30, 0}, 0};
     return c;
 }
 
@@ -489,6 +519,7 @@ int vqgemm_e2e_gemm_b_ws(const void *x, const void *codes, const void *codebook,
         if ((int64_t)prefill_splitk_workspace_bytes(p, sp) > workspace_bytes) return VQGEMM_E_SCRATCH;
     } else {
         const WorkspaceChoice c = workspace_auto(p, a16);
+        if (c.wave) return static_cast<int>(launch_wave_k_b(p, static_cast<hipStream_t>(stream)));
         if (c.tail.ok && (int64_t)c.bytes <= workspace_bytes)
             return static_cast<int>(launch_prefill_tail_split(p, c.tail, static_cast<hipStream_t>(stream), workspace));
         sp = c.tail.ok ? splitk_auto(p, a16) : c.sp;
@@ -502,13 +533,15 @@ int vqgemm_e2e_gemm_b_ws(const void *x, const void *codes, const void *codebook,
 
 namespace {
 
-// Additive stages: whether the automatic choice for the whole K reads X as it is, and what it needs as scratch otherwise
-// (the repeated X, then what the product itself wants).
-bool stages_read_x(const ProblemB &p, int stages)
+// Additive stages: the kernel that the automatic choice for the whole K takes, where that kernel reads an X that repeats along
+// K as it is (VQGEMM_VARIANT_AUTO: it does not, X is repeated in memory)
+int stages_variant(const ProblemB &p, int stages)
 {
     ProblemB q = p;
     q.k_x = p.K / stages;
-    return select_b(p, true) == VQGEMM_VARIANT_DECODE && decode_stages_supports(q);
+    const WorkspaceChoice c = workspace_auto(p, true);
+    if (c.wave) return wave_k_b_supports(q) ? VQGEMM_VARIANT_WAVE_K : VQGEMM_VARIANT_AUTO;
+    return c.bytes == 0 && select_b(p, true) == VQGEMM_VARIANT_DECODE && decode_stages_supports(q) ? VQGEMM_VARIANT_DECODE : VQGEMM_VARIANT_AUTO;
 }
 int64_t repeated_x_bytes(const ProblemB &p) { return ((int64_t)p.M * p.K * 2 + 255) & ~(int64_t)255; }
 
@@ -523,7 +556,7 @@ int64_t vqgemm_stages_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t
     if (stages < 1 || K % stages != 0) return VQGEMM_E_SHAPE;
     if (M == 0 || N == 0 || K == 0) return 0;
     const ProblemB p = make_b(nullptr, nullptr, nullptr, nullptr, M, K, N, vec, entries, n_codebooks, code_bits);
-    if (stages > 1 && stages_read_x(p, stages)) return 0;
+    if (stages > 1 && stages_variant(p, stages) != VQGEMM_VARIANT_AUTO) return 0;
     return (stages > 1 ? repeated_x_bytes(p) : 0) + (int64_t)workspace_auto(p, true).bytes;
 }
 
@@ -547,9 +580,10 @@ int vqgemm_e2e_gemm_b_stages(const void *x, const void *codes, const void *codeb
     p.bias = static_cast<const half_t *>(bias);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool a16 = aligned(x, 16) && aligned(y, 16) && aligned(codebook, 16) && aligned(codes, 16) && aligned(bias, 8);
-    if (a16 && stages_read_x(p, stages)) {
+    const int variant = a16 ? stages_variant(p, stages) : VQGEMM_VARIANT_AUTO;
+    if (variant != VQGEMM_VARIANT_AUTO) {
         p.k_x = p.K / stages;
-        return static_cast<int>(launch_decode_b(p, s));
+        return static_cast<int>(variant == VQGEMM_VARIANT_WAVE_K ? launch_wave_k_b(p, s) : launch_decode_b(p, s));
     }
     const int64_t repeated = repeated_x_bytes(p);
     if (workspace_bytes < repeated) return VQGEMM_E_SCRATCH;
@@ -593,6 +627,8 @@ int vqgemm_e2e_gemm_b_gated(const void *x, const void *codes, const void *codebo
             // resp. per matrix; where one of them refuses, the next in line takes the shape).
             const int plain_variant = select_b(plain, true);
             if (plain_variant == VQGEMM_VARIANT_DECODE_GEMV && decode_gemv_supports(p)) variant = VQGEMM_VARIANT_DECODE_GEMV;
+            else if ((plain_variant == VQGEMM_VARIANT_DECODE || plain_variant == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, p.M > 64 ? prefill_cost_us(plain) : 0.0))
+                variant = VQGEMM_VARIANT_WAVE_K;
             else if ((plain_variant == VQGEMM_VARIANT_DECODE || plain_variant == VQGEMM_VARIANT_DECODE_GEMV) && decode_gated_supports(p))
                 variant = VQGEMM_VARIANT_DECODE;
             else if (prefill_supports(plain)) variant = VQGEMM_VARIANT_PREFILL;
@@ -628,6 +664,11 @@ int vqgemm_e2e_gemm_b_gated(const void *x, const void *codes, const void *codebo
         if (!a16) return VQGEMM_E_ALIGN;
         if (K == 0 || !prefill_small_supports(plain)) return VQGEMM_E_VARIANT;
         e = launch_prefill_small_b(p, s);
+        break;
+    case VQGEMM_VARIANT_WAVE_K:
+        if (!a16) return VQGEMM_E_ALIGN;
+        if (!wave_k_b_supports(p)) return VQGEMM_E_VARIANT;
+        e = launch_wave_k_b(p, s);
         break;
     case VQGEMM_VARIANT_TWOPASS: {
         // (here: the fused product as the automatic choice runs it, then the element-wise pass)
@@ -682,7 +723,7 @@ int vqgemm_e2e_gemm_a(const void *x, const void *w, const void *codebook, void *
         break;
     case VQGEMM_VARIANT_PREFILL:
         if (!fused_a_supports(p)) return aligned(x, 16) && aligned(w, 16) && aligned(codebook, 16) ? VQGEMM_E_VARIANT : VQGEMM_E_ALIGN;
-        e = launch_fused_a(p, s);
+        e = wave_k_a_preferred(p) ? launch_wave_k_a(p, s) : launch_fused_a(p, s);
         break;
     case VQGEMM_VARIANT_TWOPASS:
         if (!workspace) return VQGEMM_E_NULL;

@@ -128,6 +128,7 @@ hipError_t launch_decode_stream(const ProblemB &p, hipStream_t s);
 bool decode_gated_supports(const ProblemB &p);
 // expected microseconds of the batched decode kernel for tall X (more rows than the general kernel serves); 1e30 otherwise
 double decode_cost_us(const ProblemB &p);
+double decode_slab_cost_us(const ProblemB &p);   // of up to 64 rows of X
 
 bool prefill_supports(const ProblemB &p);
 // whether the 256x128 tile of the prefill kernel can serve the shape (a subset of prefill_supports)
@@ -170,12 +171,27 @@ hipError_t launch_gemm_nt(const half_t *x, const half_t *w, half_t *y, int M, in
 // the tiled kernel behind the two above (w_is_kn: w is [K,N], else [N,K]) and the shapes it takes;
 // tile: 0 = the width expected to be faster, 1 = 256x256, 2 = 256x128
 bool gemm_tiled_supports(const half_t *x, const half_t *w, int M, int K, int N, bool w_is_kn);
+double gemm_tiled_cost_us(int M, int K, int N);  // of the tile it would take
 hipError_t launch_gemm_tiled(const half_t *x, const half_t *w, half_t *y, int M, int K, int N, bool w_is_kn, hipStream_t s,
                              int tile = 0);
 
 // geometry A, fused: the tiled [K,N] GEMM with its W stages dequantised on the compute unit
 bool fused_a_supports(const ProblemA &p);
+double fused_a_cost_us(const ProblemA &p);
 hipError_t launch_fused_a(const ProblemA &p, hipStream_t s);
+
+// small tiles, K dealt out to the waves of a workgroup (vq_wave_k.hip): the plain [K,N] GEMM and geometry A
+bool gemm_wave_k_supports(const half_t *x, const half_t *w, int M, int K, int N);
+double gemm_wave_k_cost_us(const half_t *w, int M, int K, int N);
+hipError_t launch_gemm_wave_k(const half_t *x, const half_t *w, half_t *y, int M, int K, int N, hipStream_t s);
+bool wave_k_a_supports(const ProblemA &p);
+double wave_k_a_cost_us(const ProblemA &p);
+hipError_t launch_wave_k_a(const ProblemA &p, hipStream_t s);
+bool wave_k_b_supports(const ProblemB &p);
+double wave_k_b_cost_us(const ProblemB &p);
+// whether the automatic choice takes this kernel (`t_other`: what the best of the others is expected to take, by their cost models)
+bool wave_k_b_preferred(const ProblemB &p, double t_other);
+hipError_t launch_wave_k_b(const ProblemB &p, hipStream_t s);
 
 // out[M, stages * K] = x[M, K] repeated `stages` times along K
 hipError_t launch_repeat_columns(const half_t *x, half_t *out, int64_t M, int64_t K, int stages, hipStream_t s);
@@ -260,6 +276,10 @@ struct Tuning {
     double splitk_us_per_partial_mb = 0.15;
     // 2 .. 16: VQGEMM_VARIANT_PREFILL_SPLITK takes this many slices where the shape allows (for measurements); 0: the cost model's
     double splitk_force_splits = 0.0;
+    // (for measurements and tests) the kernels that deal K out to waves: 0 where the cost model expects them to be fastest,
+    // 1 wherever they apply, 2 never; and their tile as 10 * (rows / 16) + columns / 16 (0: the cost model's)
+    double wave_k_force = 0.0;
+    double wave_k_force_tile = 0.0;
     double splitk_validate_fences = 0.0;  // (accepted, without effect: the slices meet in a second launch)
 };
 const Tuning &tuning();

@@ -950,7 +950,9 @@ static double batched_cost_us(const ProblemB &p)
     const int rounds_d = (per_slab * g.n_slabs + cus * g.per_cu - 1) / (cus * g.per_cu);
     const bool shared = g.per_cu > 1;
     const Tuning &tn = tuning();
-    const double t_tile = (g.n_chunks == 1 ? tn.decode_tile_us : tn.decode_tile_chunked_us) * g.n_waves / kMaxWaves * g.per_cu * (shared ? 1.35 : 1.0);
+    // (4-vectors: two gathers per operand, and with 16-bit codes out of tables whose entries collide more)
+    const double format = p.vec == 8 ? 1.0 : p.code_bits == 8 ? 1.15 : 1.65;
+    const double t_tile = (g.n_chunks == 1 ? tn.decode_tile_us : tn.decode_tile_chunked_us) * g.n_waves / kMaxWaves * g.per_cu * (shared ? 1.35 : 1.0) * format;
     const int passes = g.books_per_wg * g.n_chunks;
     return rounds_d * ((shared ? tn.decode_prologue_shared_cu_us : tn.decode_prologue_us) + passes * g.tiles_per_wg * t_tile +
                        (passes - 1) * tn.decode_pass_change_us);
@@ -968,6 +970,26 @@ double decode_cost_us(const ProblemB &p)
 {
     if (!decode_supports(p) || p.M <= kGeneralMaxM || !batched_supports(p)) return 1e30;
     return batched_cost_us(p);
+}
+
+// Microseconds the batched kernel is expected to take with up to 64 rows of X, closer than the above (which only has to
+// tell it from the tiled kernels): per round of workgroups 3.0 (1.1 more per chunk of K beyond the first), 1.8 per 64 K
+// elements of X staged on a compute unit, and per tile and 4096 k 1.1 (8-vectors), 1.4 (4-vectors) or 1.9 (4-vectors with
+// 16-bit codes, whose tables collide more) - a tenth off the measured times either way, over 400 shapes.  1e30: another
+// kernel of the decode path takes the shape.
+double decode_slab_cost_us(const ProblemB &p)
+{
+    if (p.M > kGeneralMaxM || !decode_supports(p) || decode_stream_preferred(p)) return 1e30;
+    const BatchedPlan g = plan_batched(p);
+    if (!g.ok) return 1e30;
+    const int cus = device_cu_count(), by_lds = (int)(kDecodeLdsLimit / g.smem);
+    const int resident = by_lds < 1 ? 1 : (by_lds < g.per_cu ? by_lds : g.per_cu);
+    const int per_slab = g.books_per_wg > 1 ? (p.n_codebooks + g.books_per_wg - 1) / g.books_per_wg : g.wgs_per_cb * p.n_codebooks;
+    const int wgs = per_slab * g.n_slabs, rounds = (wgs + cus * resident - 1) / (cus * resident);
+    const int on_unit = (wgs + cus - 1) / cus < resident ? (wgs + cus - 1) / cus : resident;
+    const double tile_us = p.code_bits == 16 && p.vec < 8 ? 1.9 : p.vec < 8 ? 1.4 : 1.1;
+    return 1.2 + rounds * (3.0 + 1.1 * (g.n_chunks - 1) + on_unit * (1.8 * (p.M < kTileN ? p.M : kTileN) * p.K / 65536.0 +
+                                                                    (double)g.books_per_wg * g.tiles_per_wg * p.K / 4096.0 * tile_us));
 }
 
 // The GEMV kernels have no work shared between their waves.  One row of X in the first format

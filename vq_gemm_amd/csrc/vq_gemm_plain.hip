@@ -149,6 +149,10 @@ hipError_t launch_plain(const half_t *x, const half_t *w, half_t *y, int M, int 
 
 hipError_t launch_gemm_nn(const half_t *x, const half_t *w, half_t *y, int M, int K, int N, hipStream_t s)
 {
+    const int force = (int)tuning().wave_k_force;
+    if (force != 2 && gemm_wave_k_supports(x, w, M, K, N) &&
+        (force == 1 || !gemm_tiled_supports(x, w, M, K, N, true) || gemm_wave_k_cost_us(w, M, K, N) < gemm_tiled_cost_us(M, K, N)))
+        return launch_gemm_wave_k(x, w, y, M, K, N, s);
     if (M >= VQ_TILED_MIN_M && gemm_tiled_supports(x, w, M, K, N, true)) return launch_gemm_tiled(x, w, y, M, K, N, true, s);
     return launch_plain<true>(x, w, y, M, K, N, s);
 }

@@ -636,26 +636,37 @@ bool gemm_tiled_supports(const half_t *x, const half_t *w, int M, int K, int N, 
     return (int64_t)BM * K * 2 < (int64_t)1 << 31;
 }
 
+// Rounds of tiles over the compute units.  A tile costs K/64 times a per-stage time that grows with the share of the
+// units at work (the clock drops under load): fitted to measurements, 1.2 us for the 256x256 tile, 0.68 us for 256x128
+// and 0.40 us for 128x128 on an idle device, 1.6 times that on a full one.
+static int tiled_choice(int M, int K, int N, double *cost_us)
+{
+    const int cus = device_cu_count();
+    auto cost = [&](int bm, int bn, double per_stage) {
+        const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        const int64_t rounds = (tiles + cus - 1) / cus;
+        const double busy = (double)tiles / (double)(rounds * cus);
+        return (double)rounds * (5.0 + K / 64.0 * per_stage * (1.0 + 0.6 * busy));
+    };
+    const double t1 = cost(256, 256, 1.2), t2 = cost(256, 128, 0.68), t3 = cost(128, 128, 0.40);
+    const int tile = t3 < t2 && t3 < t1 ? 3 : (t2 < t1 ? 2 : 1);
+    if (cost_us) *cost_us = tile == 3 ? t3 : tile == 2 ? t2 : t1;
+    return tile;
+}
+
+double gemm_tiled_cost_us(int M, int K, int N)
+{
+    double t;
+    tiled_choice(M, K, N, &t);
+    return t;
+}
+
 // tile: 0 = the tile expected to be fastest, 1 = 256x256, 2 = 256x128, 3 = 128x128
 hipError_t launch_gemm_tiled(const half_t *x, const half_t *w, half_t *y, int M, int K, int N, bool w_is_kn, hipStream_t s,
                              int tile)
 {
     if (!gemm_tiled_supports(x, w, M, K, N, w_is_kn)) return hipErrorInvalidValue;
-    if (tile == 0) {
-        // Rounds of tiles over the compute units.  A tile costs K/64 times a per-stage time that
-        // grows with the share of the units at work (the clock drops under load): fitted to
-        // measurements, 1.2 us for the 256x256 tile, 0.68 us for 256x128 and 0.40 us for 128x128 on
-        // an idle device, 1.6 times that on a full one.
-        const int cus = device_cu_count();
-        auto cost = [&](int bm, int bn, double per_stage) {
-            const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-            const int64_t rounds = (tiles + cus - 1) / cus;
-            const double busy = (double)tiles / (double)(rounds * cus);
-            return (double)rounds * (5.0 + K / 64.0 * per_stage * (1.0 + 0.6 * busy));
-        };
-        const double t1 = cost(256, 256, 1.2), t2 = cost(256, 128, 0.68), t3 = cost(128, 128, 0.40);
-        tile = t3 < t2 && t3 < t1 ? 3 : (t2 < t1 ? 2 : 1);
-    }
+    if (tile == 0) tile = tiled_choice(M, K, N, nullptr);
     if (tile == 3) return w_is_kn ? launch_tiled<true, 4, 4>(x, w, y, M, K, N, s) : launch_tiled<false, 4, 4>(x, w, y, M, K, N, s);
     if (tile == 2) return w_is_kn ? launch_tiled<true, 4, 8>(x, w, y, M, K, N, s) : launch_tiled<false, 4, 8>(x, w, y, M, K, N, s);
     return w_is_kn ? launch_tiled<true, 8, 8>(x, w, y, M, K, N, s) : launch_tiled<false, 8, 8>(x, w, y, M, K, N, s);
@@ -671,21 +682,33 @@ bool fused_a_supports(const ProblemA &p)
     return (int64_t)BM * p.K * 2 < (int64_t)1 << 31 && (int64_t)2 * kStepK * p.Nc < (int64_t)1 << 31;
 }
 
+// 256x128 tiles, or 128x128 where those go over the compute units in fewer rounds at four fifths of the
+// time per round (measured at one round each: 48 against 60 us per 4096 k)
+static bool fused_a_tall(const ProblemA &p)
+{
+    const int cus = device_cu_count(), tiles_n = (2 * p.Nc + kABN - 1) / kABN;
+    const int64_t n_tall = (int64_t)((p.M + 255) / 256) * tiles_n, n_short = (int64_t)((p.M + 127) / 128) * tiles_n;
+    return (double)((n_tall + cus - 1) / cus) <= 0.8 * (double)((n_short + cus - 1) / cus);
+}
+
+double fused_a_cost_us(const ProblemA &p)
+{
+    const int cus = device_cu_count();
+    const bool tall = fused_a_tall(p);
+    const int64_t tiles = (int64_t)((p.M + (tall ? 255 : 127)) / (tall ? 256 : 128)) * ((2 * p.Nc + kABN - 1) / kABN);
+    return (double)((tiles + cus - 1) / cus) * (4.0 + p.K * (tall ? 0.0132 : 0.0102));
+}
+
 hipError_t launch_fused_a(const ProblemA &p, hipStream_t s)
 {
     if (!fused_a_supports(p)) return hipErrorInvalidValue;
     const int tiles_n = (2 * p.Nc + kABN - 1) / kABN;
-    // 256x128 tiles, or 128x128 where those go over the compute units in fewer rounds at four fifths of the
-    // time per round (measured at one round each: 48 against 60 us per 4096 k)
-    const int cus = device_cu_count();
-    const int64_t n_tall = (int64_t)((p.M + 255) / 256) * tiles_n, n_short = (int64_t)((p.M + 127) / 128) * tiles_n;
-    const bool tall = (double)((n_tall + cus - 1) / cus) <= 0.8 * (double)((n_short + cus - 1) / cus);
     auto launch = [&](auto kern, int bm, size_t lds) {
         const int tiles_m = (p.M + bm - 1) / bm;
         return launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads), lds, s, p.x, p.w, p.cb, p.y, p.M, p.K,
                            p.Nc, tiles_m, tiles_n);
     };
-    return tall ? launch(gemm_a_fused_kernel<8>, 256, FusedACfg<8>::kLdsBytes) : launch(gemm_a_fused_kernel<4>, 128, FusedACfg<4>::kLdsBytes);
+    return fused_a_tall(p) ? launch(gemm_a_fused_kernel<8>, 256, FusedACfg<8>::kLdsBytes) : launch(gemm_a_fused_kernel<4>, 128, FusedACfg<4>::kLdsBytes);
 }
 
 }  // namespace vq

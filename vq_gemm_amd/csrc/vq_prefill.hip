@@ -855,13 +855,14 @@ size_t lds_bytes_narrow(const ProblemB &p)
 // Microseconds a launch over `cols` tile columns of `bn` W rows is expected to take, fitted to
 // measurements: a tile costs 5 us of prologue and epilogue plus K/64 stages of 1.0 us (256x256) or
 // 0.56 us (256x128) when the device is mostly idle, up to 1.6 times that when every compute unit
-// works (the clock the device holds under load); the tiles go over the compute units in rounds.
+// works (the clock the device holds under load), and 1.18 times that with 4-vectors, whose operands are two gathers; the tiles
+// go over the compute units in rounds.
 double tile_cost_us(const ProblemB &p, int bn, int cols)
 {
     const int64_t tiles = (int64_t)((p.M + BM - 1) / BM) * cols;
     const int cus = device_cu_count();
     const Tuning &tn = tuning();
-    const double stages = p.K / 64.0 * (bn == BN ? tn.prefill_stage_us_256x256 : tn.prefill_stage_us_256x128);
+    const double stages = p.K / 64.0 * (bn == BN ? tn.prefill_stage_us_256x256 : tn.prefill_stage_us_256x128) * (p.vec == 8 ? 1.0 : 1.18);
     const int64_t full = tiles / cus, rem = tiles % cus;
     double t = (double)full * (tn.prefill_tile_fixed_us + stages * tn.prefill_full_device_factor);
     if (rem) t += tn.prefill_tile_fixed_us + stages * (1.0 + (tn.prefill_full_device_factor - 1.0) * (double)rem / cus);

@@ -496,21 +496,26 @@ bool prefill_small_supports(const ProblemB &p)
     }
 }
 
-// Microseconds the kernel is expected to take, fitted to measurements: the tiles go over the
+// Microseconds `wgs` workgroups are expected to take over K, fitted to measurements: they go over the
 // compute units in rounds (a second workgroup on a unit shares its LDS bandwidth, which is what
 // bounds this tile, and gains nothing in the main loop; it does overlap its prologue and epilogue
 // with the other's work); a tile costs 4 us plus K/64 stages of 0.46 us on an idle device, 0.56 us
-// when every unit works.
+// when every unit works - with 4-vectors, whose operands are two gathers, 1.18 times that.
+static double small_tiles_us(const ProblemB &p, int64_t wgs, int K)
+{
+    const int cus = device_cu_count();
+    const bool two = codebooks_per_tile(p, SBN) * (int64_t)p.entries * p.vec * 2 <= 8 * 1024;   // workgroups on a unit: by the LDS
+    const int64_t rounds = (wgs + cus - 1) / cus, resident_rounds = two ? (wgs + 2 * cus - 1) / (2 * cus) : rounds;
+    const double busy = wgs >= cus ? 1.0 : (double)wgs / cus;
+    const Tuning &tn = tuning();
+    const double stage_us = tn.prefill_small_stage_us_idle + (tn.prefill_small_stage_us_busy - tn.prefill_small_stage_us_idle) * busy;
+    return (double)resident_rounds * tn.prefill_small_tile_fixed_us + (double)rounds * (K / 64.0 * stage_us) * (p.vec == 8 ? 1.0 : 1.18);
+}
+
 double prefill_small_cost_us(const ProblemB &p)
 {
     if (!prefill_small_supports(p)) return 1e30;
-    const int cus = device_cu_count();
-    const int64_t tiles = (int64_t)((p.M + SBM - 1) / SBM) * ((p.N + SBN - 1) / SBN);
-    const int64_t rounds = (tiles + cus - 1) / cus, resident_rounds = (tiles + 2 * cus - 1) / (2 * cus);
-    const double busy = tiles >= cus ? 1.0 : (double)tiles / cus;
-    const Tuning &tn = tuning();
-    return (double)resident_rounds * tn.prefill_small_tile_fixed_us +
-           (double)rounds * (p.K / 64.0 * (tn.prefill_small_stage_us_idle + (tn.prefill_small_stage_us_busy - tn.prefill_small_stage_us_idle) * busy));
+    return small_tiles_us(p, (int64_t)((p.M + SBM - 1) / SBM) * ((p.N + SBN - 1) / SBN), p.K);
 }
 
 hipError_t launch_prefill_small_b(const ProblemB &p, hipStream_t s, int splits, void *workspace, int n_begin)
@@ -559,14 +564,7 @@ int prefill_splitk_choice(const ProblemB &p, double *cost_us, int min_splits)
     }
     for (const int sp : {2, 3, 4, 6, 8, 12, 16}) {
         if (!prefill_splitk_supports(p, sp)) break;
-        ProblemB q = p;  // the slices as the kernel sees them: sp times the tiles over K / sp
-        q.K = p.K / sp;
-        const int cus = device_cu_count();
-        const int64_t wgs = tiles * sp;
-        const int64_t rounds = (wgs + cus - 1) / cus, resident_rounds = (wgs + 2 * cus - 1) / (2 * cus);
-        const double busy = wgs >= cus ? 1.0 : (double)wgs / cus;
-        const double main_us = (double)resident_rounds * tn.prefill_small_tile_fixed_us +
-                               (double)rounds * (q.K / 64.0 * (tn.prefill_small_stage_us_idle + (tn.prefill_small_stage_us_busy - tn.prefill_small_stage_us_idle) * busy));
+        const double main_us = small_tiles_us(p, tiles * sp, p.K / sp);   // the slices: sp times the tiles over K / sp
         const double fix_us = tn.splitk_fixed_us + tn.splitk_us_per_partial_mb * (double)sp * p.M * p.N * 4e-6;
         if (main_us + fix_us < best_us) {
             best_us = main_us + fix_us;

@@ -1,0 +1,140 @@
+// The kernels of vq_wave_k.h for geometry B.
+#include "vq_wave_k.h"
+
+namespace vq {
+
+namespace {
+
+// A format, and what its kernels' units are: two steps of K - whole 128-byte lines of X, the codes of both steps in one
+// read - where the LDS holds two such units of eight waves beside the codebooks, one step for the larger tiles and the
+// larger tables.
+template <int VEC_, typename CodeT_>
+struct Format {
+    static constexpr int VEC = VEC_, CSZ = (int)sizeof(CodeT_);
+    template <int MP, int NP>
+    using Wave = WaveB<VEC_, CodeT_, ((MP * NP > 16 || (CSZ == 2 && MP >= 4)) ? 1 : 2)>;
+};
+
+// calls f with the pieces of the tile (10 * rows + columns), as types
+template <class F>
+void with_tile(int tile, F f)
+{
+    using std::integral_constant;
+    switch (tile) {
+    case 12: f(integral_constant<int, 1>{}, integral_constant<int, 2>{}); break;
+    case 14: f(integral_constant<int, 1>{}, integral_constant<int, 4>{}); break;
+    case 18: f(integral_constant<int, 1>{}, integral_constant<int, 8>{}); break;
+    case 22: f(integral_constant<int, 2>{}, integral_constant<int, 2>{}); break;
+    case 24: f(integral_constant<int, 2>{}, integral_constant<int, 4>{}); break;
+    case 44: f(integral_constant<int, 4>{}, integral_constant<int, 4>{}); break;
+    case 48: f(integral_constant<int, 4>{}, integral_constant<int, 8>{}); break;
+    default: break;
+    }
+}
+
+template <class F>
+bool fits(const ProblemB &p, int tile)
+{
+    bool ok = false;
+    with_tile(tile, [&](auto mp, auto np) {
+        typedef WaveKCfg<typename F::template Wave<mp(), np()>, mp(), np()> C;
+        if constexpr (C::kExists) ok = C::lds_bytes((size_t)codebooks_per_tile(p, C::TN) * p.entries * p.vec * 2) <= 160 * 1024;
+    });
+    return ok;
+}
+
+template <class F>
+WaveKPlan plan_b(const ProblemB &p)
+{
+    const int forced = (int)tuning().wave_k_force_tile;
+    // (16-bit codes bring tables whose entries collide more often)
+    constexpr WaveKTile kTiles8[] = {{12, 2.2, 39, 14}, {14, 2.5, 65, 28}, {18, 3.2, 118, 62}, {22, 2.4, 44, 19}, {24, 3.0, 68, 29}, {44, 4.0, 95, 68}, {48, 6.1, 180, 165}};
+    constexpr WaveKTile kTiles16[] = {{12, 2.6, 45, 19}, {14, 2.8, 79, 59}, {18, 3.0, 169, 200}, {22, 2.7, 52, 24}, {24, 3.0, 91, 45}, {44, 3.5, 124, 112}, {48, 5.9, 214, 182}};
+    WaveKPlan best = {0, 0, 1e30};
+    for (const WaveKTile &t : F::CSZ == 1 ? kTiles8 : kTiles16) {
+        if (forced > 0 && forced != t.tile) continue;
+        if (!fits<F>(p, t.tile)) continue;
+        const double bytes = (double)p.K * p.N * F::CSZ / F::VEC + 2.0 * (double)p.M * (p.K + p.N);
+        const double us = wave_k_tile_cost_us(t, p.M, p.K, p.N, bytes);
+        if (us < best.cost_us) best = {t.tile / 10, t.tile % 10, us};
+    }
+    return best;
+}
+
+template <class F>
+hipError_t launch_b(const ProblemB &p, hipStream_t s)
+{
+    const WaveKPlan plan = plan_b<F>(p);
+    const WaveKArgs a = {p.x, p.codes, p.cb, p.y, p.bias, p.M, p.K, p.N, p.k_x, 0, 0, p.entries, p.rows_per_cb, codebooks_per_tile(p, plan.np * 16), p.gated ? 1 : 0};
+    hipError_t e = hipErrorInvalidValue;
+    with_tile(plan.mp * 10 + plan.np, [&](auto mp, auto np) {
+        typedef typename F::template Wave<mp(), np()> P;
+        if constexpr (WaveKCfg<P, mp(), np()>::kExists) e = launch_tile<P, mp(), np()>(a, s);
+    });
+    return e;
+}
+
+// calls f with the format's type; false where there is none
+template <class F>
+bool with_format(const ProblemB &p, F f)
+{
+    const bool u8 = p.code_bits == 8;
+    if (p.vec == 8) {
+        if (u8) f(Format<8, uint8_t>{});
+        else f(Format<8, uint16_t>{});
+    } else if (p.vec == 4) {
+        if (u8) f(Format<4, uint8_t>{});
+        else f(Format<4, uint16_t>{});
+    } else {
+        return false;
+    }
+    return true;
+}
+
+}  // namespace
+
+bool wave_k_b_supports(const ProblemB &p)
+{
+    if (!wave_k_shape(p.x, p.M, p.K, p.N) || p.K % 64 != 0 || p.K < 128 || p.packed || p.k_x % 64 != 0) return false;
+    if (((size_t)p.entries * p.vec * 2) % 16 != 0) return false;
+    if ((int64_t)128 * (p.K / p.vec) * (p.code_bits / 8) >= (int64_t)1 << 31) return false;
+    bool ok = false;
+    with_format(p, [&](auto format) { ok = fits<decltype(format)>(p, 22); });
+    return ok;
+}
+
+double wave_k_b_cost_us(const ProblemB &p)
+{
+    double t = 1e30;
+    if (wave_k_b_supports(p)) with_format(p, [&](auto format) { t = plan_b<decltype(format)>(p).cost_us; });
+    return t;
+}
+
+// The rule.  Up to two rows of X are the GEMV kernels' or the decode path's.  Up to 16 the decode path is about as fast: this
+// kernel where it is expected to be a tenth faster (long K or many columns, where the decode path walks K in chunks or fills
+// its tables several times; over 300 shapes 8 to 11 % of the time).  Up to 64 rows this kernel, except on the shortest products
+// in 8-bit codes (K <= 2048, one 16 x 16 tile of Y per compute unit at most), which the decode path has done 5 to 10 %
+// earlier.  Above, where it is
+// expected to be faster than the others by more than the models' error.  (us, before -> now: M = 44, K = 704, N = 21888, 4-vectors 32.3 ->
+// 11.0; M = 100, K = 1408, N = 3500 11.9 -> 6.5; M = 256, K = N = 4096, 16-bit codes 26.5 -> 17.6; M = 451, K = 1152,
+// N = 1376 18.2 -> 8.0.)
+bool wave_k_b_preferred(const ProblemB &p, double t_other)
+{
+    const int force = (int)tuning().wave_k_force;
+    if (force == 2 || !wave_k_b_supports(p)) return false;
+    if (force == 1) return true;
+    if (p.M <= 2) return false;
+    if (p.M <= 16) return wave_k_b_cost_us(p) < 0.9 * decode_slab_cost_us(p) && decode_slab_cost_us(p) < 1e29;
+    if (p.M <= 64) return !(p.code_bits == 8 && p.K <= 2048 && (int64_t)((p.M + 15) / 16) * ((p.N + 15) / 16) <= device_cu_count());
+    return wave_k_b_cost_us(p) < 0.95 * t_other;
+}
+
+hipError_t launch_wave_k_b(const ProblemB &p, hipStream_t s)
+{
+    if (!wave_k_b_supports(p)) return hipErrorInvalidValue;
+    hipError_t e = hipErrorInvalidValue;
+    with_format(p, [&](auto format) { e = launch_b<decltype(format)>(p, s); });
+    return e;
+}
+
+}  // namespace vq
