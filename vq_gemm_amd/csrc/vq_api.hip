@@ -143,6 +143,7 @@ constexpr int kTuningCount = (int)(sizeof(kTuningEntries) / sizeof(kTuningEntrie
 
 std::mutex g_tuning_mu;
 Tuning g_tuning;             // written under the mutex; read without it (plain doubles, set before the launches that use them)
+std::atomic<uint32_t> g_tuning_version{0};   // of the table: a plan made under another one is made again
 std::atomic<bool> g_tuning_file_read{false};  // (acquire/release: a reader that sees true also sees what the file set)
 
 const TuningEntry *find_tuning(const char *name)
@@ -183,6 +184,7 @@ int read_tuning_file(const char *path)
         const TuningEntry *e = find_tuning(key.c_str());
         if (e && v == v && v >= 0.0 && v < 1e9) {
             g_tuning.*(e->field) = v;
+            g_tuning_version.fetch_add(1, std::memory_order_release);
             set++;
         }
     }
@@ -251,14 +253,110 @@ int select_b(const ProblemB &p, bool all_aligned16)
     return VQGEMM_VARIANT_GENERIC;
 }
 
-// What the automatic choice launches without a workspace: select_b's kernel, or the wave-K kernel in its place.  (Above 64
-// rows the K-sliced path's model promises more than it keeps: there the prefill kernels' is what the wave-K kernel is held to.)
-int auto_b(const ProblemB &p, bool all_aligned16)
+// Split K with the cost model's number of slices when that is expected to beat what the automatic choice would
+// launch otherwise by a margin (and then at least two slices); 0: do not split.
+int splitk_auto(const ProblemB &p, double *t_best, int *plain_variant)
 {
-    const int plain = select_b(p, all_aligned16);
-    if ((plain == VQGEMM_VARIANT_DECODE || plain == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, p.M > 64 ? prefill_cost_us(p) : 0.0))
-        return VQGEMM_VARIANT_WAVE_K;
-    return plain;
+    *t_best = 1e30;
+    const int plain = select_b(p, true);
+    *plain_variant = plain;
+    double t_plain;
+    if (plain == VQGEMM_VARIANT_PREFILL) t_plain = prefill_cost_us(p);
+    else if (plain == VQGEMM_VARIANT_DECODE) t_plain = decode_cost_us(p);
+    else return 0;
+    if (t_plain >= 1e29) return 0;  // (short X: the decode path is taken without a comparison, and stays)
+    double t_split = 1e30;
+    const int sp = prefill_splitk_choice(p, &t_split, 2);
+    const bool take = sp >= 2 && t_split < 0.9 * t_plain;
+    *t_best = take ? t_split : t_plain;
+    return take ? sp : 0;
+}
+
+// What the automatic choice does with a workspace: nothing, K split over every 128x128 tile (sp slices), or whole rounds
+// of large tiles with the left-over columns in 128x128 tiles and K split there (tail) - whichever the cost models
+// expect to be fastest by a margin.
+struct WorkspaceChoice {
+    bool wave;      // the wave-K kernel, which needs none
+    int sp;
+    TailSplitPlan tail;
+    size_t bytes;
+};
+WorkspaceChoice workspace_auto(const ProblemB &p)
+{
+    WorkspaceChoice c = {false, 0, {false, 0, 0, 0, 1e30, 0}, 0};
+    double t_best = 1e30;
+    int plain = VQGEMM_VARIANT_GENERIC;
+    c.sp = splitk_auto(p, &t_best, &plain);
+    if (c.sp >= 2) c.bytes = prefill_splitk_workspace_bytes(p, c.sp);
+    if (plain == VQGEMM_VARIANT_PREFILL && t_best < 1e29) {
+        const TailSplitPlan tail = prefill_tail_split_plan(p);
+        // (a margin of 1000 and more: wherever the plan exists - for measurements and tests)
+        const double margin = tuning().tail_split_margin;
+        if (tail.ok && (margin >= 1e3 || tail.cost_us < margin * t_best)) {
+            c.sp = 0;
+            c.tail = tail;
+            c.bytes = tail.workspace_bytes;
+        }
+    }
+    // (a split asked for by the tuning table is not weighed against anything)
+    const bool asked = tuning().splitk_force_splits >= 2.0 || tuning().tail_split_margin >= 1e3;
+    const double t_other = c.tail.ok ? c.tail.cost_us : c.sp >= 2 ? t_best : prefill_cost_us(p);
+    if (!(asked && c.bytes > 0) && (plain == VQGEMM_VARIANT_DECODE || plain == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, t_other))
+        c = {true, 0, {false, 0, 0, 0, 1e30, 0}, 0};
+    return c;
+}
+
+// What the automatic choice launches: without a workspace, and with one.  wave_tile: the wave-K kernel's tile where it is taken.
+struct AutoPlan {
+    int variant;
+    WorkspaceChoice ws;
+    int wave_tile;
+};
+
+// (Above 64 rows the K-sliced path's model promises more than it keeps: there the prefill kernels' is what the wave-K kernel
+// is held to.  The gated product takes what the plain one would run on: every tiled kernel carries the gated epilogue itself;
+// the GEMV kernels and the K-sliced decode kernels want whole groups of 32 interleaved rows per codebook resp. per matrix,
+// and where one of them refuses, the next in line takes the shape.)
+AutoPlan make_plan(const ProblemB &p)
+{
+    AutoPlan plan = {VQGEMM_VARIANT_GENERIC, {false, 0, {false, 0, 0, 0, 1e30, 0}, 0}, 0};
+    if (p.K == 0) return plan;
+    ProblemB plain = p;
+    plain.gated = false;
+    const int v = p.gated && decode_gemv_wide_preferred(p) ? VQGEMM_VARIANT_DECODE_GEMV : select_b(plain, true);
+    const bool tiled = v == VQGEMM_VARIANT_DECODE || v == VQGEMM_VARIANT_PREFILL;
+    const bool wave = tiled && wave_k_b_preferred(p, p.M > 64 ? prefill_cost_us(plain) : 0.0);
+    if (wave) plan.variant = VQGEMM_VARIANT_WAVE_K;
+    else if (!p.gated) plan.variant = v;
+    else if (v == VQGEMM_VARIANT_DECODE_GEMV && decode_gemv_supports(p)) plan.variant = v;
+    else if ((v == VQGEMM_VARIANT_DECODE || v == VQGEMM_VARIANT_DECODE_GEMV) && decode_gated_supports(p)) plan.variant = VQGEMM_VARIANT_DECODE;
+    else if (prefill_supports(plain)) plan.variant = VQGEMM_VARIANT_PREFILL;
+    if (!p.gated && tiled) plan.ws = p.M > 64 ? workspace_auto(p) : WorkspaceChoice{wave, 0, {false, 0, 0, 0, 1e30, 0}, 0};
+    if (wave || plan.ws.wave) plan.wave_tile = wave_k_b_tile(p);
+    return plan;
+}
+
+// The plan of a shape, kept per thread for the shapes it has met last: a serving thread multiplies by the same few weights
+// again and again, and the cost models are a microsecond of arithmetic.
+const AutoPlan &auto_plan(const ProblemB &p)
+{
+    struct Entry {
+        uint64_t key[4];
+        AutoPlan plan;
+    };
+    constexpr int kEntries = 64;
+    thread_local Entry entries[kEntries];
+    (void)tuning();   // (a file is read before its version is)
+    const uint64_t key[4] = {(uint64_t)(uint32_t)p.M << 32 | (uint32_t)p.K, (uint64_t)(uint32_t)p.N << 32 | (uint32_t)p.entries,
+                             (uint64_t)(uint32_t)p.n_codebooks << 32 | (uint32_t)(p.vec << 8 | p.code_bits << 1 | (p.gated ? 1 : 0)),
+                             ((uint64_t)g_tuning_version.load(std::memory_order_acquire) << 32 | (uint32_t)current_device()) + 1};
+    uint64_t h = key[0] * 0x9e3779b97f4a7c15ull ^ key[1] * 0xc2b2ae3d27d4eb4full ^ key[2] * 0x165667b19e3779f9ull;
+    Entry &e = entries[(h ^ h >> 32) >> 8 & (kEntries - 1)];
+    if (e.key[3] != key[3] || e.key[0] != key[0] || e.key[1] != key[1] || e.key[2] != key[2]) {
+        e.plan = make_plan(p);
+        for (int i = 0; i < 4; i++) e.key[i] = key[i];
+    }
+    return e.plan;
 }
 
 }  // namespace
@@ -306,6 +404,7 @@ int vqgemm_tuning_set(const char *name, double value)
     (void)tuning();  // (a file is read before, not after, an explicit setting)
     std::lock_guard<std::mutex> lock(g_tuning_mu);
     g_tuning.*(e->field) = value;
+    g_tuning_version.fetch_add(1, std::memory_order_release);
     return VQGEMM_OK;
 }
 
@@ -362,7 +461,13 @@ int vqgemm_e2e_gemm_b_bias(const void *x, const void *codes, const void *codeboo
     ProblemB p = make_b(x, codes, codebook, y, M, K, N, vec, entries, n_codebooks, code_bits);
     p.bias = static_cast<const half_t *>(bias);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (variant == VQGEMM_VARIANT_AUTO) variant = auto_b(p, a16);
+    int wave_tile = 0;
+    if (variant == VQGEMM_VARIANT_AUTO) {
+        const AutoPlan none = {VQGEMM_VARIANT_GENERIC, {}, 0};
+        const AutoPlan &plan = a16 ? auto_plan(p) : none;
+        variant = plan.variant;
+        wave_tile = plan.wave_tile;
+    }
     hipError_t e = hipSuccess;
     switch (variant) {
     case VQGEMM_VARIANT_GENERIC:
@@ -402,7 +507,7 @@ int vqgemm_e2e_gemm_b_bias(const void *x, const void *codes, const void *codeboo
     case VQGEMM_VARIANT_WAVE_K:
         if (!a16) return VQGEMM_E_ALIGN;
         if (!wave_k_b_supports(p)) return VQGEMM_E_VARIANT;
-        e = launch_wave_k_b(p, s);
+        e = launch_wave_k_b(p, s, wave_tile);
         break;
     case VQGEMM_VARIANT_TWOPASS:
         if (bias) return VQGEMM_E_VARIANT;  // the plain GEMM of the two-pass route has no bias input
@@ -418,64 +523,6 @@ int vqgemm_e2e_gemm_b_bias(const void *x, const void *codes, const void *codeboo
     return static_cast<int>(e);
 }
 
-namespace {
-
-// Split K with the cost model's number of slices when that is expected to beat what the automatic choice would
-// launch otherwise by a margin (and then at least two slices); 0: do not split.
-int splitk_auto(const ProblemB &p, bool all_aligned16, double *t_best = nullptr, int *plain_variant = nullptr)
-{
-    if (t_best) *t_best = 1e30;
-    if (p.K == 0 || !all_aligned16 || p.gated) return 0;
-    const int plain = select_b(p, all_aligned16);
-    if (plain_variant) *plain_variant = plain;
-    double t_plain;
-    if (plain == VQGEMM_VARIANT_PREFILL) t_plain = prefill_cost_us(p);
-    else if (plain == VQGEMM_VARIANT_DECODE) t_plain = decode_cost_us(p);
-    else return 0;
-    if (t_plain >= 1e29) return 0;  // (short X: the decode path is taken without a comparison, and stays)
-    double t_split = 1e30;
-    const int sp = prefill_splitk_choice(p, &t_split, 2);
-    const bool take = sp >= 2 && t_split < 0.9 * t_plain;
-    if (t_best) *t_best = take ? t_split : t_plain;
-    return take ? sp : 0;
-}
-
-// What the automatic choice does with a workspace: nothing, K split over every 128x128 tile (sp slices), or whole rounds
-// of large tiles with the left-over columns in 128x128 tiles and K split there (tail) - whichever the cost models
-// expect to be fastest by a margin.
-struct WorkspaceChoice {
-    bool wave;      // the wave-K kernel, which needs none
-    int sp;
-    TailSplitPlan tail;
-    size_t bytes;
-};
-WorkspaceChoice workspace_auto(const ProblemB &p, bool all_aligned16)
-{
-    WorkspaceChoice c = {false, 0, {false, 0, 0, 0, 1e30, 0}, 0};
-    double t_best = 1e30;
-    int plain = VQGEMM_VARIANT_GENERIC;
-    c.sp = splitk_auto(p, all_aligned16, &t_best, &plain);
-    if (c.sp >= 2) c.bytes = prefill_splitk_workspace_bytes(p, c.sp);
-    if (plain == VQGEMM_VARIANT_PREFILL && t_best < 1e29) {
-        const TailSplitPlan tail = prefill_tail_split_plan(p);
-        // (a margin of 1000 and more: wherever the plan exists - for measurements and tests)
-        const double margin = tuning().tail_split_margin;
-        if (tail.ok && (margin >= 1e3 || tail.cost_us < margin * t_best)) {
-            c.sp = 0;
-            c.tail = tail;
-            c.bytes = tail.workspace_bytes;
-        }
-    }
-    // (a split asked for by the tuning table is not weighed against anything)
-    const bool asked = tuning().splitk_force_splits >= 2.0 || tuning().tail_split_margin >= 1e3;
-    const double t_other = c.tail.ok ? c.tail.cost_us : c.sp >= 2 ? t_best : p.M > 64 ? prefill_cost_us(p) : 0.0;
-    if (!(asked && c.bytes > 0) && (plain == VQGEMM_VARIANT_DECODE || plain == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, t_other))
-        c = {true, 0, {false, 0, 0, 0, 1e30, 0}, 0};
-    return c;
-}
-
-}  // namespace
-
 int64_t vqgemm_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks,
                                  int32_t code_bits, int32_t variant)
 {
@@ -485,7 +532,7 @@ int64_t vqgemm_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t vec, i
     if (M == 0 || N == 0 || K == 0) return 0;
     const ProblemB p = make_b(nullptr, nullptr, nullptr, nullptr, M, K, N, vec, entries, n_codebooks, code_bits);
     if (variant == VQGEMM_VARIANT_TWOPASS) return N * K * 2;
-    if (variant == VQGEMM_VARIANT_AUTO) return (int64_t)workspace_auto(p, true).bytes;
+    if (variant == VQGEMM_VARIANT_AUTO) return (int64_t)auto_plan(p).ws.bytes;
     int sp = 0;
     if (variant == VQGEMM_VARIANT_PREFILL_SPLITK) sp = prefill_splitk_choice(p, nullptr, 2);
     return sp >= 2 ? (int64_t)prefill_splitk_workspace_bytes(p, sp) : 0;
@@ -518,13 +565,15 @@ int vqgemm_e2e_gemm_b_ws(const void *x, const void *codes, const void *codebook,
         if (sp < 2) return VQGEMM_E_VARIANT;
         if ((int64_t)prefill_splitk_workspace_bytes(p, sp) > workspace_bytes) return VQGEMM_E_SCRATCH;
     } else {
-        const WorkspaceChoice c = workspace_auto(p, a16);
-        if (c.wave) return static_cast<int>(launch_wave_k_b(p, static_cast<hipStream_t>(stream)));
+        const AutoPlan none = {VQGEMM_VARIANT_GENERIC, {}, 0};
+        const AutoPlan &plan = a16 && K > 0 ? auto_plan(p) : none;
+        const WorkspaceChoice &c = plan.ws;
+        if (c.wave) return static_cast<int>(launch_wave_k_b(p, static_cast<hipStream_t>(stream), plan.wave_tile));
         if (c.tail.ok && (int64_t)c.bytes <= workspace_bytes)
             return static_cast<int>(launch_prefill_tail_split(p, c.tail, static_cast<hipStream_t>(stream), workspace));
-        sp = c.tail.ok ? splitk_auto(p, a16) : c.sp;
         // (a workspace that is too small is not an error for the automatic choice: it does without)
-        if (sp < 2 || (int64_t)prefill_splitk_workspace_bytes(p, sp) > workspace_bytes)
+        sp = c.sp;
+        if (sp < 2 || (int64_t)c.bytes > workspace_bytes)
             return vqgemm_e2e_gemm_b_bias(x, codes, codebook, bias, y, M, K, N, vec, entries, n_codebooks, code_bits, VQGEMM_VARIANT_AUTO,
                                           nullptr, stream);
     }
@@ -539,7 +588,7 @@ int stages_variant(const ProblemB &p, int stages)
 {
     ProblemB q = p;
     q.k_x = p.K / stages;
-    const WorkspaceChoice c = workspace_auto(p, true);
+    const WorkspaceChoice &c = auto_plan(p).ws;
     if (c.wave) return wave_k_b_supports(q) ? VQGEMM_VARIANT_WAVE_K : VQGEMM_VARIANT_AUTO;
     return c.bytes == 0 && select_b(p, true) == VQGEMM_VARIANT_DECODE && decode_stages_supports(q) ? VQGEMM_VARIANT_DECODE : VQGEMM_VARIANT_AUTO;
 }
@@ -557,7 +606,7 @@ int64_t vqgemm_stages_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t
     if (M == 0 || N == 0 || K == 0) return 0;
     const ProblemB p = make_b(nullptr, nullptr, nullptr, nullptr, M, K, N, vec, entries, n_codebooks, code_bits);
     if (stages > 1 && stages_variant(p, stages) != VQGEMM_VARIANT_AUTO) return 0;
-    return (stages > 1 ? repeated_x_bytes(p) : 0) + (int64_t)workspace_auto(p, true).bytes;
+    return (stages > 1 ? repeated_x_bytes(p) : 0) + (int64_t)auto_plan(p).ws.bytes;
 }
 
 int vqgemm_e2e_gemm_b_stages(const void *x, const void *codes, const void *codebook, const void *bias, void *y, int64_t M, int64_t K,
@@ -618,21 +667,13 @@ int vqgemm_e2e_gemm_b_gated(const void *x, const void *codes, const void *codebo
     ProblemB plain = p;
     plain.gated = false;
     plain.y = static_cast<half_t *>(workspace);
+    int wave_tile = 0;
     if (variant == VQGEMM_VARIANT_AUTO) {
-        if (K == 0 || !a16) variant = VQGEMM_VARIANT_GENERIC;
-        else if (decode_gemv_wide_preferred(p)) variant = VQGEMM_VARIANT_DECODE_GEMV;
-        else {
-            // What the plain product would run on decides: every tiled kernel carries the gated epilogue itself (the
-            // GEMV kernels and the K-sliced decode kernels want whole groups of 32 interleaved rows per codebook
-            // resp. per matrix; where one of them refuses, the next in line takes the shape).
-            const int plain_variant = select_b(plain, true);
-            if (plain_variant == VQGEMM_VARIANT_DECODE_GEMV && decode_gemv_supports(p)) variant = VQGEMM_VARIANT_DECODE_GEMV;
-            else if ((plain_variant == VQGEMM_VARIANT_DECODE || plain_variant == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, p.M > 64 ? prefill_cost_us(plain) : 0.0))
-                variant = VQGEMM_VARIANT_WAVE_K;
-            else if ((plain_variant == VQGEMM_VARIANT_DECODE || plain_variant == VQGEMM_VARIANT_DECODE_GEMV) && decode_gated_supports(p))
-                variant = VQGEMM_VARIANT_DECODE;
-            else if (prefill_supports(plain)) variant = VQGEMM_VARIANT_PREFILL;
-            else variant = VQGEMM_VARIANT_GENERIC;
+        variant = VQGEMM_VARIANT_GENERIC;
+        if (a16 && K > 0) {
+            const AutoPlan &plan = auto_plan(p);
+            variant = plan.variant;
+            wave_tile = plan.wave_tile;
         }
     }
     hipError_t e = hipSuccess;
@@ -668,7 +709,7 @@ int vqgemm_e2e_gemm_b_gated(const void *x, const void *codes, const void *codebo
     case VQGEMM_VARIANT_WAVE_K:
         if (!a16) return VQGEMM_E_ALIGN;
         if (!wave_k_b_supports(p)) return VQGEMM_E_VARIANT;
-        e = launch_wave_k_b(p, s);
+        e = launch_wave_k_b(p, s, wave_tile);
         break;
     case VQGEMM_VARIANT_TWOPASS: {
         // (here: the fused product as the automatic choice runs it, then the element-wise pass)

@@ -191,7 +191,8 @@ bool wave_k_b_supports(const ProblemB &p);
 double wave_k_b_cost_us(const ProblemB &p);
 // whether the automatic choice takes this kernel (`t_other`: what the best of the others is expected to take, by their cost models)
 bool wave_k_b_preferred(const ProblemB &p, double t_other);
-hipError_t launch_wave_k_b(const ProblemB &p, hipStream_t s);
+int wave_k_b_tile(const ProblemB &p);   // the tile its cost model expects to be fastest
+hipError_t launch_wave_k_b(const ProblemB &p, hipStream_t s, int tile = 0);   // (0: that one)
 
 // out[M, stages * K] = x[M, K] repeated `stages` times along K
 hipError_t launch_repeat_columns(const half_t *x, half_t *out, int64_t M, int64_t K, int stages, hipStream_t s);

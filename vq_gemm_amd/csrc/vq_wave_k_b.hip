@@ -62,12 +62,15 @@ WaveKPlan plan_b(const ProblemB &p)
 }
 
 template <class F>
-hipError_t launch_b(const ProblemB &p, hipStream_t s)
+hipError_t launch_b(const ProblemB &p, hipStream_t s, int tile)
 {
-    const WaveKPlan plan = plan_b<F>(p);
-    const WaveKArgs a = {p.x, p.codes, p.cb, p.y, p.bias, p.M, p.K, p.N, p.k_x, 0, 0, p.entries, p.rows_per_cb, codebooks_per_tile(p, plan.np * 16), p.gated ? 1 : 0};
+    if (tile == 0) {
+        const WaveKPlan plan = plan_b<F>(p);
+        tile = plan.mp * 10 + plan.np;
+    }
+    const WaveKArgs a = {p.x, p.codes, p.cb, p.y, p.bias, p.M, p.K, p.N, p.k_x, 0, 0, p.entries, p.rows_per_cb, codebooks_per_tile(p, tile % 10 * 16), p.gated ? 1 : 0};
     hipError_t e = hipErrorInvalidValue;
-    with_tile(plan.mp * 10 + plan.np, [&](auto mp, auto np) {
+    with_tile(tile, [&](auto mp, auto np) {
         typedef typename F::template Wave<mp(), np()> P;
         if constexpr (WaveKCfg<P, mp(), np()>::kExists) e = launch_tile<P, mp(), np()>(a, s);
     });
@@ -110,6 +113,16 @@ double wave_k_b_cost_us(const ProblemB &p)
     return t;
 }
 
+int wave_k_b_tile(const ProblemB &p)
+{
+    int tile = 0;
+    with_format(p, [&](auto format) {
+        const WaveKPlan plan = plan_b<decltype(format)>(p);
+        tile = plan.mp * 10 + plan.np;
+    });
+    return tile;
+}
+
 // The rule.  Up to two rows of X are the GEMV kernels' or the decode path's.  Up to 16 the decode path is about as fast: this
 // kernel where it is expected to be a tenth faster (long K or many columns, where the decode path walks K in chunks or fills
 // its tables several times; over 300 shapes 8 to 11 % of the time).  Up to 64 rows this kernel, except on the shortest products
@@ -124,16 +137,19 @@ bool wave_k_b_preferred(const ProblemB &p, double t_other)
     if (force == 2 || !wave_k_b_supports(p)) return false;
     if (force == 1) return true;
     if (p.M <= 2) return false;
-    if (p.M <= 16) return wave_k_b_cost_us(p) < 0.9 * decode_slab_cost_us(p) && decode_slab_cost_us(p) < 1e29;
+    if (p.M <= 16) {
+        const double t_decode = decode_slab_cost_us(p);
+        return t_decode < 1e29 && wave_k_b_cost_us(p) < 0.9 * t_decode;
+    }
     if (p.M <= 64) return !(p.code_bits == 8 && p.K <= 2048 && (int64_t)((p.M + 15) / 16) * ((p.N + 15) / 16) <= device_cu_count());
     return wave_k_b_cost_us(p) < 0.95 * t_other;
 }
 
-hipError_t launch_wave_k_b(const ProblemB &p, hipStream_t s)
+hipError_t launch_wave_k_b(const ProblemB &p, hipStream_t s, int tile)
 {
     if (!wave_k_b_supports(p)) return hipErrorInvalidValue;
     hipError_t e = hipErrorInvalidValue;
-    with_format(p, [&](auto format) { e = launch_b<decltype(format)>(p, s); });
+    with_format(p, [&](auto format) { e = launch_b<decltype(format)>(p, s, tile); });
     return e;
 }
 
