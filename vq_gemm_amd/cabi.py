@@ -364,7 +364,23 @@ def e2e_gemm_a_noalloc(x, w, codebook, out, variant=VARIANT_AUTO):
     return out
 
 
+_native = None  # the compiled extension's calls, once one of the functions below has loaded it
+
+
+def _extension():
+    global _native
+    if _native is None:
+        lib()
+        from .torch_ops import native
+        _native = native
+    return _native
+
+
 def dequant_b(codes, codebook, out=None):
+    if out is None and codes.is_cuda:
+        w = (_native or _extension()).dequant(codes, codebook)
+        if w is not None:
+            return w
     import torch
     _require(codes.dim() == 2, "codes must be [N, K/vec]")
     N, J = codes.shape
@@ -384,6 +400,10 @@ def dequant_b(codes, codebook, out=None):
 
 def encode_b(w, codebook, code_bits=None, out=None):
     """Nearest-codeword codes [N, K/vec] of W [N,K] fp16 for the given codebook(s)."""
+    if out is None and code_bits is None and w.is_cuda:
+        codes = (_native or _extension()).encode(w, codebook)
+        if codes is not None:
+            return codes
     import torch
     _require(w.dim() == 2, "w must be [N, K]")
     N, K = w.shape

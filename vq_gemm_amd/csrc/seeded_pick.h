@@ -9,7 +9,7 @@
 #pragma once
 
 #include <cstdint>
-#include <unordered_map>
+#include <vector>
 
 namespace vq {
 
@@ -53,7 +53,7 @@ private:
         at_ = 0;
     }
     // (element i needs i + 1 and i + 397, old or already new: every loop reads at least 227 elements away from what it writes)
-    __attribute__((optimize("O3"), target_clones("avx2", "default"))) static void twist(uint32_t *s)
+    __attribute__((optimize("O3"), target_clones("avx512f", "avx2", "default"))) static void twist(uint32_t *s)
     {
         for (int i = 0; i < kN - kM; i++) s[i] = s[i + kM] ^ mix(s[i], s[i + 1]);
         for (int i = kN - kM; i < kN - 1; i++) s[i] = s[i + kM - kN] ^ mix(s[i], s[i + 1]);
@@ -67,16 +67,28 @@ private:
 // which then moves on by the whole permutation's draws
 inline void first_of_permutation(Mt19937 &gen, int64_t n, int64_t count, bool another, int32_t *out)
 {
-    std::unordered_map<int64_t, int32_t> moved;  // elements that are not where they started
-    moved.reserve((size_t)count * 2);
+    // elements that are not where they started: open addressing, at most half full (as a node-based map, four fifths of the
+    // time: 256 draws 9.5 us)
+    size_t slots = 16;
+    while (slots < 4 * (size_t)count) slots *= 2;
+    std::vector<int64_t> where(slots, -1);
+    std::vector<int32_t> what(slots);
+    auto find = [&](int64_t i) {
+        size_t at = (size_t)((uint64_t)i * 0x9e3779b97f4a7c15ull >> 32) & (slots - 1);
+        while (where[at] >= 0 && where[at] != i) at = (at + 1) & (slots - 1);
+        return at;
+    };
     auto value = [&](int64_t i) {
-        const auto it = moved.find(i);
-        return it == moved.end() ? (int32_t)i : it->second;
+        const size_t at = find(i);
+        return where[at] < 0 ? (int32_t)i : what[at];
     };
     for (int64_t i = 0; i < count; i++) {
-        const int64_t j = i < n - 1 ? i + (int64_t)(gen.next() % (uint64_t)(n - i)) : i;
-        out[i] = value(j);
-        moved[j] = value(i);
+        const int64_t j = i < n - 1 ? i + (int64_t)(gen.next() % (uint32_t)(n - i)) : i;
+        const int32_t mine = value(i);
+        const size_t at = find(j);
+        out[i] = where[at] < 0 ? (int32_t)j : what[at];
+        where[at] = j;
+        what[at] = mine;
     }
     if (another) gen.skip(n - 1 - (count < n - 1 ? count : n - 1));
 }

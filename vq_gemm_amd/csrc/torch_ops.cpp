@@ -253,6 +253,42 @@ py::object gated(const Tensor &x, const Tensor &codes, const Tensor &codebook, c
     return py::cast(gated_impl(x, codes, codebook, bias));
 }
 
+// ---- the codec ------------------------------------------------------------------------------------------------
+
+// What cabi.encode_b and cabi.dequant_b do on well-formed operands of the current device, without their checks one by one in
+// Python (11 of the 12 us of a call on a small matrix); None sends the caller down that path, which says what is wrong.
+bool codec_operands(const Tensor &m, const Tensor &codebook, int64_t per_column)
+{
+    return plain_call(m) && m.dim() == 2 && m.is_contiguous() && codebook.is_cuda() && codebook.device() == m.device() && codebook.is_contiguous() &&
+           codebook.scalar_type() == at::kHalf && (codebook.dim() == 2 || codebook.dim() == 3) && codebook.size(-1) > 0 &&
+           m.device().index() == c10::hip::current_device() && (m.size(1) * per_column) % codebook.size(-1) == 0 &&
+           (codebook.dim() == 2 || (codebook.size(0) > 0 && m.size(0) % codebook.size(0) == 0));
+}
+
+py::object encode(const Tensor &w, const Tensor &codebook)
+{
+    if (!codec_operands(w, codebook, 1) || w.scalar_type() != at::kHalf) return py::none();
+    const int64_t N = w.size(0), K = w.size(1), vec = codebook.size(-1), entries = codebook.size(-2);
+    const int bits = entries <= 256 ? 8 : 16;
+    Tensor codes = at::detail::empty_cuda({N, K / vec}, bits == 8 ? at::kByte : at::kUInt16, w.device(), c10::nullopt);
+    if (vqgemm_encode_b(w.data_ptr(), codebook.data_ptr(), codes.data_ptr(), N, K, (int)vec, (int)entries,
+                        codebook.dim() == 3 ? (int)codebook.size(0) : 1, bits, stream_of(w)) != 0)
+        return py::none();
+    return py::cast(codes);
+}
+
+py::object dequant(const Tensor &codes, const Tensor &codebook)
+{
+    const bool u8 = codes.scalar_type() == at::kByte;
+    if ((!u8 && codes.scalar_type() != at::kUInt16) || !codec_operands(codes, codebook, codebook.dim() > 0 ? codebook.size(-1) : 1)) return py::none();
+    const int64_t N = codes.size(0), vec = codebook.size(-1), K = codes.size(1) * vec;
+    Tensor w = at::detail::empty_cuda({N, K}, at::kHalf, codes.device(), c10::nullopt);
+    if (vqgemm_dequant_b(codes.data_ptr(), codebook.data_ptr(), w.data_ptr(), N, K, (int)vec, (int)codebook.size(-2),
+                         codebook.dim() == 3 ? (int)codebook.size(0) : 1, u8 ? 8 : 16, stream_of(codes)) != 0)
+        return py::none();
+    return py::cast(w);
+}
+
 // ---- the quantiser --------------------------------------------------------------------------------------------
 
 // int32 [books, count] on the host: row g is the start of the g-th permutation of 0 .. n-1 that a generator seeded with `seed` makes
@@ -319,5 +355,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("linear", &linear, "x @ W.T (+ bias) on plain GPU tensors; None where the registered operator is to be called instead");
     m.def("first_of_permutations", &first_of_permutations, "the first elements of seeded random permutations");
     m.def("kmeans", &kmeans, "Lloyd iterations on the device; None where the codebook is too large for them");
+    m.def("encode", &encode, "nearest-codeword codes; None where cabi.encode_b is to check the operands one by one");
+    m.def("dequant", &dequant, "codes and codebook to fp16 likewise");
     m.def("gated", &gated, "silu(gate) * up likewise");
 }

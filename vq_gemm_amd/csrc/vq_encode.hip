@@ -93,11 +93,9 @@ __global__ __launch_bounds__(kEncThreads) void encode_b_kernel(const half_t *__r
 // vector unit one instruction: of a group of eight scores four to fold them to their minimum and four to keep the best
 // two groups (0.75 in groups of sixteen).  4096 x 4096, 8-vectors, 256 entries: 230 -> 32 us.
 //
-// A wave takes 128 vectors as four batches of 32, so that an entry tile read from the LDS (its halves and its
+// A wave takes 128 vectors as four batches of 32 (64 as two, where there are too few for a workgroup on every other unit), so that an entry tile read from the LDS (its halves and its
 // half norms) meets four MFMAs.  A lane of the result holds 16 scores of one vector - two groups of eight entries, or one -, and
 // the lane 32 further on the other 16.
-constexpr int kScanBatches = 4;                 // batches of 32 vectors per wave
-constexpr int kScanVectors = 32 * kScanBatches;
 // Scores per group: a larger one costs the scan less and the rule more; they meet at about this many entries.
 constexpr int kScanWideGroupEntries = 768;
 
@@ -161,7 +159,7 @@ __device__ __forceinline__ HalfWaves swap_half_waves(uint32_t a, uint32_t b)
 // both leave as the workgroup's row of `partials`: entries * (VEC + 1) sums and counts, then the error.  The sums are kept in
 // double: an LDS addition of doubles takes a fifth of the time of one of floats on this device (2.1 M vectors of 8 elements:
 // 19 against 99 us), and is exact for weights of any usual range.
-template <int VEC, typename CodeT, int GROUP, bool ACCUMULATE>
+template <int VEC, typename CodeT, int GROUP, bool ACCUMULATE, int kScanBatches>
 __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t *__restrict__ w, const half_t *__restrict__ cb,
                                                                    CodeT *__restrict__ codes, int64_t vectors_per_cb, int entries,
                                                                    int wgs_per_cb, float *__restrict__ partials)
@@ -169,6 +167,7 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ float reduce[kScanThreads / 64];
     constexpr int DW = VEC / 2;                       // dwords of a vector
+    constexpr int kScanVectors = 32 * kScanBatches;   // of a wave
     // An entry's place in the table: one is left out after every 256 bytes of them, or the entries of all best groups, which
     // start at multiples of sixteen entries, would lie in the same few banks.
     constexpr int kRow = 128 / VEC;
@@ -395,14 +394,19 @@ size_t scan_lds_bytes(const ProblemB &p, bool accumulate)
     return scan_table_bytes(p.entries, p.vec) + padded * 4 + (accumulate ? (size_t)p.entries * (p.vec + 1) * 8 : 0);
 }
 
-// Workgroups per codebook: as many as are resident together (two of eight waves per unit while the LDS allows), none without work.
-int scan_workgroups(const ProblemB &p, bool accumulate)
+// Batches of a wave and workgroups per codebook: as many as are resident together (two of eight waves per unit while the LDS
+// allows), none without work.
+struct ScanPlan {
+    int batches, wgs_per_cb;
+};
+ScanPlan scan_plan(const ProblemB &p, bool accumulate)
 {
     const int64_t vectors = (int64_t)p.rows_per_cb * (p.K / p.vec);
     const int per_cu = scan_lds_bytes(p, accumulate) <= 72 * 1024 ? 2 : 1;
     const int64_t want = ((int64_t)device_cu_count() * per_cu + p.n_codebooks - 1) / p.n_codebooks;
-    const int64_t have = (vectors + kScanThreads / 64 * kScanVectors - 1) / (kScanThreads / 64 * kScanVectors);
-    return (int)(want < have ? want : have);
+    auto have = [&](int batches) { return (vectors + kScanThreads / 2 * batches - 1) / (kScanThreads / 2 * batches); };
+    const int batches = have(4) * p.n_codebooks * 2 <= device_cu_count() ? 2 : 4;
+    return {batches, (int)(want < have(batches) ? want : have(batches))};
 }
 
 bool scan_supports(const half_t *w, const ProblemB &p, bool accumulate)
@@ -416,11 +420,13 @@ hipError_t launch_scan(const half_t *w, const ProblemB &p, void *codes_out, floa
 {
     const int64_t vectors_per_cb = (int64_t)p.rows_per_cb * (p.K / VEC);
     if (vectors_per_cb == 0) return hipSuccess;
-    const int wgs_per_cb = scan_workgroups(p, ACCUMULATE);
+    const ScanPlan plan = scan_plan(p, ACCUMULATE);
     const size_t smem = scan_lds_bytes(p, ACCUMULATE);
-    auto kern = p.entries < kScanWideGroupEntries ? encode_scan_kernel<VEC, CodeT, 8, ACCUMULATE> : encode_scan_kernel<VEC, CodeT, 16, ACCUMULATE>;
-    return launch_kernel(kern, dim3((unsigned)(wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem, s, w, p.cb,
-                       static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, wgs_per_cb, partials);
+    const bool narrow = p.entries < kScanWideGroupEntries;
+    auto kern = plan.batches == 4 ? (narrow ? encode_scan_kernel<VEC, CodeT, 8, ACCUMULATE, 4> : encode_scan_kernel<VEC, CodeT, 16, ACCUMULATE, 4>)
+                                  : (narrow ? encode_scan_kernel<VEC, CodeT, 8, ACCUMULATE, 2> : encode_scan_kernel<VEC, CodeT, 16, ACCUMULATE, 2>);
+    return launch_kernel(kern, dim3((unsigned)(plan.wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem, s, w, p.cb,
+                       static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, plan.wgs_per_cb, partials);
 }
 
 template <int VEC, typename CodeT>
@@ -454,7 +460,7 @@ hipError_t launch_encode_b(const half_t *w, const ProblemB &p, void *codes_out, 
 
 bool lloyd_supports(const ProblemB &p) { return encode_supports(p) && scan_lds_bytes(p, true) <= 128 * 1024; }
 
-int lloyd_assign_rows(const ProblemB &p) { return scan_workgroups(p, true); }
+int lloyd_assign_rows(const ProblemB &p) { return scan_plan(p, true).wgs_per_cb; }
 
 hipError_t launch_lloyd_assign(const half_t *w, const ProblemB &p, void *codes_out, float *partials, hipStream_t s)
 {

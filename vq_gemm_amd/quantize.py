@@ -46,7 +46,7 @@ def kmeans_quantize(w, vec: int, entries: int, n_codebooks: int = 1, iters: int 
         done = native.kmeans(w, pick, vec, entries, G, code_bits, iters)
         if done is not None:
             codes, codebook, errors = done
-            return codes, codebook, (errors / w.numel()).tolist()
+            return codes, codebook, [e / w.numel() for e in errors.tolist()]
     vectors = w.view(G, per_cb, vec)
     pick = pick.to(w.device).to(torch.int64)
     codebook = torch.gather(vectors, 1, pick[:, :, None].expand(G, entries, vec)).contiguous()
