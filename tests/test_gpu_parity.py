@@ -2003,3 +2003,27 @@ def test_k_dealt_out_to_waves_geometry_a(M, K, Nc):
         y = _with_wave_tile(tile, lambda: cabi.e2e_gemm_a(x, w, cb, variant=cabi.VARIANT_PREFILL))
         torch.cuda.synchronize()
         _check_gemm(y, x, w, cb, geometry=GEOM_A, what=f"tile {tile}")
+
+
+@pytest.mark.parametrize("N,K,v", [(1024, 1032, 8), (1032, 1024, 8), (700, 768, 4)])   # the last and first sizes of a wave's 64 and 128 vectors
+def test_encoder_on_both_sides_of_the_line_between_its_wave_sizes(N, K, v):
+    g = torch.Generator(device="cpu").manual_seed(6)
+    cb, w = torch.randn(1, 256, v, generator=g).half(), torch.randn(N, K, generator=g).half()
+    _say("encode", N, K, v)
+    codes = cabi.encode_b(w.to(DEV), cb.to(DEV))
+    torch.cuda.synchronize()
+    assert np.array_equal(_np(codes), c_oracle.encode_b(w.numpy(), cb.numpy(), 8))
+
+
+@pytest.mark.parametrize("M,K,N", [(257, 192, 263), (130, 448, 129), (40, 256, 300)])
+def test_rows_of_y_that_begin_anywhere(M, K, N):
+    spec = ProblemSpec("odd_rows", GEOM_B, M, K, N, 8, 256, 1, 8, codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=93, device=DEV)
+    want = _np(x).astype(np.float64) @ vo.dequant_b(_np(codes), _np(cb)).astype(np.float64).T
+    for variant in (cabi.VARIANT_PREFILL, cabi.VARIANT_PREFILL_NARROW, cabi.VARIANT_PREFILL_SMALL):
+        _say("rows of", N, "columns", cabi.VARIANT_NAMES[variant])
+        guard = torch.full((M * N + 8,), 7.0, dtype=torch.float16, device=DEV)
+        cabi.e2e_gemm_b(x, codes, cb, variant=variant, out=guard[:M * N].view(M, N))
+        torch.cuda.synchronize()
+        assert vo.rel_err(_np(guard[:M * N].view(M, N)), want)[0] <= TOL, variant
+        assert bool((guard[M * N:] == 7.0).all())

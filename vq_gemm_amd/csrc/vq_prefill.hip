@@ -463,48 +463,27 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
                 const int n = n0 + wn * WN + j * 16 + 4 * kg + e;
                 bj[j][e] = HB && n < N ? (float)bias[n] : 0.f;
             }
-        if ((ldn & 7) == 0) {
-            // Through the LDS: each wave transposes its 128x128 fp16 block, 64 rows at a time, in a
-            // private region (row pitch 272 bytes) and stores 256-byte row segments.
-            constexpr int kPitch = 272;
-            uint8_t *stage_out = smem + wave * (64 * kPitch);
+        // Through the LDS: each wave transposes its 128x128 fp16 block, 64 rows at a time, in a
+        // private region (row pitch 272 bytes) and stores 256-byte row segments.
+        constexpr int kPitch = 272;
+        uint8_t *stage_out = smem + wave * (64 * kPitch);
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < 2; h++) {
 #pragma unroll
-                for (int ii = 0; ii < 4; ii++) {
-                    const int i = 4 * h + ii;
+            for (int ii = 0; ii < 4; ii++) {
+                const int i = 4 * h + ii;
 #pragma unroll
-                    for (int j = 0; j < NP; j++)
-                        *reinterpret_cast<half4_t *>(stage_out + (ii * 16 + r16) * kPitch + (j * 16 + 4 * kg) * 2) =
-                            round4<HB>(acc[j][i], bj[j]);
-                }
-#pragma unroll
-                for (int it = 0; it < 16; it++) {
-                    const int row = it * 4 + (lane >> 4), c = lane & 15;
-                    const uint4_t v = *reinterpret_cast<const uint4_t *>(stage_out + row * kPitch + c * 16);
-                    const int m = m0 + wm * WM + h * 64 + row;
-                    const int n = n0 + wn * WN + c * 8;
-                    if (m < M && n < N) st_global_16_streaming(y + (int64_t)m * ldn + n, v);
-                }
+                for (int j = 0; j < NP; j++)
+                    *reinterpret_cast<half4_t *>(stage_out + (ii * 16 + r16) * kPitch + (j * 16 + 4 * kg) * 2) =
+                        round4<HB>(acc[j][i], bj[j]);
             }
-        } else {
 #pragma unroll
-            for (int i = 0; i < MP; i++) {
-                const int m = m0 + wm * WM + i * 16 + r16;
-                if (m >= M) continue;
-#pragma unroll
-                for (int j = 0; j < NP; j++) {
-                    const int n = n0 + wn * WN + j * 16 + 4 * kg;
-                    half_t *dst = y + (int64_t)m * ldn + n;
-                    const half4_t hv = round4<HB>(acc[j][i], bj[j]);
-                    if ((ldn & 3) == 0 && n + 3 < N) {
-                        *reinterpret_cast<half4_t *>(dst) = hv;
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (n + e < N) dst[e] = hv[e];
-                    }
-                }
+            for (int it = 0; it < 16; it++) {
+                const int row = it * 4 + (lane >> 4), c = lane & 15;
+                const uint4_t v = *reinterpret_cast<const uint4_t *>(stage_out + row * kPitch + c * 16);
+                const int m = m0 + wm * WM + h * 64 + row;
+                const int n = n0 + wn * WN + c * 8;
+                if (m < M) store_eight(y + (int64_t)m * ldn + n, v, N - n, (ldn & 7) == 0);
             }
         }
     };
@@ -791,42 +770,21 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
                 const int n = n0 + wn * WNN + j * 16 + 4 * kg + e;
                 bj[j][e] = HB && n < N ? (float)bias[n] : 0.f;
             }
-        if ((ldn & 7) == 0) {
-            constexpr int kPitch = 144;  // 64 fp16 + 16 bytes: rows land in different banks
-            uint8_t *stage_out = smem + wave * (128 * kPitch);
+        constexpr int kPitch = 144;  // 64 fp16 + 16 bytes: rows land in different banks
+        uint8_t *stage_out = smem + wave * (128 * kPitch);
 #pragma unroll
-            for (int i = 0; i < MP; i++)
+        for (int i = 0; i < MP; i++)
 #pragma unroll
-                for (int j = 0; j < NPN; j++)
-                    *reinterpret_cast<half4_t *>(stage_out + (i * 16 + r16) * kPitch + (j * 16 + 4 * kg) * 2) =
-                        round4<HB>(acc[j][i], bj[j]);
+            for (int j = 0; j < NPN; j++)
+                *reinterpret_cast<half4_t *>(stage_out + (i * 16 + r16) * kPitch + (j * 16 + 4 * kg) * 2) =
+                    round4<HB>(acc[j][i], bj[j]);
 #pragma unroll
-            for (int it = 0; it < 16; it++) {
-                const int row = it * 8 + (lane >> 3), c = lane & 7;
-                const uint4_t v = *reinterpret_cast<const uint4_t *>(stage_out + row * kPitch + c * 16);
-                const int m = m0 + wm * WM + row;
-                const int n = n0 + wn * WNN + c * 8;
-                if (m < M && n < N) st_global_16_streaming(y + (int64_t)m * ldn + n, v);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < MP; i++) {
-                const int m = m0 + wm * WM + i * 16 + r16;
-                if (m >= M) continue;
-#pragma unroll
-                for (int j = 0; j < NPN; j++) {
-                    const int n = n0 + wn * WNN + j * 16 + 4 * kg;
-                    half_t *dst = y + (int64_t)m * ldn + n;
-                    const half4_t hv = round4<HB>(acc[j][i], bj[j]);
-                    if ((ldn & 3) == 0 && n + 3 < N) {
-                        *reinterpret_cast<half4_t *>(dst) = hv;
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (n + e < N) dst[e] = hv[e];
-                    }
-                }
-            }
+        for (int it = 0; it < 16; it++) {
+            const int row = it * 8 + (lane >> 3), c = lane & 7;
+            const uint4_t v = *reinterpret_cast<const uint4_t *>(stage_out + row * kPitch + c * 16);
+            const int m = m0 + wm * WM + row;
+            const int n = n0 + wn * WNN + c * 8;
+            if (m < M) store_eight(y + (int64_t)m * ldn + n, v, N - n, (ldn & 7) == 0);
         }
     };
     if (gated) {

@@ -342,42 +342,21 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_small_kernel(const half_t
                 const int n = n0 + wn * SWN + j * 16 + 4 * kg + e;
                 bj[j][e] = HB && n < N ? (float)bias[n] : 0.f;
             }
-        if ((ldn & 7) == 0) {
-            constexpr int kPitch = 144;  // 64 fp16 + 16 bytes: rows land in different banks
-            uint8_t *stage_out = smem + wave * (SWM * kPitch);
+        constexpr int kPitch = 144;  // 64 fp16 + 16 bytes: rows land in different banks
+        uint8_t *stage_out = smem + wave * (SWM * kPitch);
 #pragma unroll
-            for (int i = 0; i < SMP; i++)
+        for (int i = 0; i < SMP; i++)
 #pragma unroll
-                for (int j = 0; j < SNP; j++)
-                    *reinterpret_cast<half4_t *>(stage_out + (i * 16 + r16) * kPitch + (j * 16 + 4 * kg) * 2) =
-                        round4<HB>(acc[j][i], bj[j]);
+            for (int j = 0; j < SNP; j++)
+                *reinterpret_cast<half4_t *>(stage_out + (i * 16 + r16) * kPitch + (j * 16 + 4 * kg) * 2) =
+                    round4<HB>(acc[j][i], bj[j]);
 #pragma unroll
-            for (int it = 0; it < SWM / 8; it++) {
-                const int row = it * 8 + (lane >> 3), c = lane & 7;
-                const uint4_t v = *reinterpret_cast<const uint4_t *>(stage_out + row * kPitch + c * 16);
-                const int m = m0 + wm * SWM + row;
-                const int n = n0 + wn * SWN + c * 8;
-                if (m < M && n < N) st_global_16_streaming(y + (int64_t)m * ldn + n, v);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < SMP; i++) {
-                const int m = m0 + wm * SWM + i * 16 + r16;
-                if (m >= M) continue;
-#pragma unroll
-                for (int j = 0; j < SNP; j++) {
-                    const int n = n0 + wn * SWN + j * 16 + 4 * kg;
-                    half_t *dst = y + (int64_t)m * ldn + n;
-                    const half4_t hv = round4<HB>(acc[j][i], bj[j]);
-                    if ((ldn & 3) == 0 && n + 3 < N) {
-                        *reinterpret_cast<half4_t *>(dst) = hv;
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (n + e < N) dst[e] = hv[e];
-                    }
-                }
-            }
+        for (int it = 0; it < SWM / 8; it++) {
+            const int row = it * 8 + (lane >> 3), c = lane & 7;
+            const uint4_t v = *reinterpret_cast<const uint4_t *>(stage_out + row * kPitch + c * 16);
+            const int m = m0 + wm * SWM + row;
+            const int n = n0 + wn * SWN + c * 8;
+            if (m < M) store_eight(y + (int64_t)m * ldn + n, v, N - n, (ldn & 7) == 0);
         }
     };
     if (gated) {

@@ -33,6 +33,23 @@ __device__ __forceinline__ void st_global_16_streaming(void *p, uint4_t v)
     __builtin_nontemporal_store(v, reinterpret_cast<uint4_t *>(p));
 }
 
+// Eight results of a row; `left`: columns up to the row's end.  Rows that are no multiple of 16 bytes (aligned false) begin
+// anywhere: still one store, the memory takes any address, and only the row's last piece goes element by element.
+__device__ __forceinline__ void store_eight(half_t *dst, uint4_t v, int left, bool aligned)
+{
+    if (left <= 0) return;
+    if (aligned) {
+        st_global_16_streaming(dst, v);
+    } else if (left >= 8) {
+        __builtin_memcpy(dst, &v, 16);
+    } else {
+        const half8_t h = __builtin_bit_cast(half8_t, v);
+#pragma unroll
+        for (int e = 0; e < 7; e++)
+            if (e < left) dst[e] = h[e];
+    }
+}
+
 // Holds the accumulators where they are (the AGPRs) up to here.  Called behind the wait for the last MFMAs: the compiler
 // does not see what an inline-assembly MFMA is still writing, and where a loop's last pass is peeled off it would copy
 // each accumulator out right behind its last MFMA.
