@@ -2027,3 +2027,16 @@ def test_rows_of_y_that_begin_anywhere(M, K, N):
         torch.cuda.synchronize()
         assert vo.rel_err(_np(guard[:M * N].view(M, N)), want)[0] <= TOL, variant
         assert bool((guard[M * N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("M,K,N", [(3914, 1024, 4616), (1800, 1024, 10240)])   # 16 x 19 and 8 x 40 large tiles: whole rounds and a few more
+def test_plain_gemm_with_the_left_over_columns_in_a_second_launch(M, K, N):
+    g = torch.Generator().manual_seed(7)
+    x, w = torch.randn(M, K, generator=g).half().to(DEV), torch.randn(K, N, generator=g).half().to(DEV)
+    _say("gemm", M, K, N)
+    guard = torch.full((M * N + 8,), 7.0, dtype=torch.float16, device=DEV)
+    y = cabi.gemm_f16(x, w, out=guard[:M * N].view(M, N))
+    want = x.float() @ w.float()
+    torch.cuda.synchronize()
+    assert ((y.float() - want).norm() / want.norm()).item() <= TOL and bool((guard[M * N:] == 7.0).all())
+    assert ((y.float() - want).abs().max() / want.abs().max()).item() <= TOL

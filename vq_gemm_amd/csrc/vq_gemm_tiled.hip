@@ -75,7 +75,7 @@ __device__ __forceinline__ int kmajor_swizzle(int k) { return 2 * ((k & 3) | (((
 template <bool W_IS_KN, int NP, int MPW>
 __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const half_t *__restrict__ x,
                                                                  const half_t *__restrict__ w,
-                                                                 half_t *__restrict__ y, int M, int K, int N,
+                                                                 half_t *__restrict__ y, int M, int K, int N, int ldn,
                                                                  int tiles_m, int tiles_n)
 {
     typedef TileCfg<NP, MPW> C;
@@ -111,12 +111,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const half_t *_
         if (W_IS_KN && i < C::kWLoads) {
             const int k = slot / C::kChunksPerK;
             const int c = (slot % C::kChunksPerK) ^ kmajor_swizzle(k);
-            w_voff[i] = (uint32_t)(((int64_t)k * N + (min(n0 + c * 8, N - 8) - n0)) * 2);
+            w_voff[i] = (uint32_t)(((int64_t)k * ldn + (min(n0 + c * 8, N - 8) - n0)) * 2);
         }
     }
     // Where the loads of the stage NS ahead of the current one read (the last stage again once K is
     // used up: harmless, and every stage so brings the same number of loads); moved on once per step.
-    const int64_t w_step = W_IS_KN ? (int64_t)kStepK * N : kStepK;
+    const int64_t w_step = W_IS_KN ? (int64_t)kStepK * ldn : kStepK;
     const int first_ahead = min(NS, n_stage - 1);
     const half_t *x_ahead = x + (int64_t)m0 * K + first_ahead * kStepK;
     const half_t *w_ahead = (W_IS_KN ? w + n0 : w + (int64_t)n0 * K) + first_ahead * w_step;
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const half_t *_
 
     // ---- epilogue: lane holds Y[m = i*16 + r16][n = j*16 + 4*kg + 0..3] of its wave tile ----------
     auto round4 = [](const float4_t &a) { return half4_t{(half_t)a[0], (half_t)a[1], (half_t)a[2], (half_t)a[3]}; };
-    if ((N & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
+    if ((ldn & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
         // Through the LDS: each wave transposes its fp16 block, 64 rows at a time, in a
         // private region (padded rows) and stores whole row segments.
         constexpr int kPitch = WN * 2 + 16;
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const half_t *_
                 const uint4_t v = *reinterpret_cast<const uint4_t *>(stage_out + row * kPitch + c * 16);
                 const int m = m0 + wm * WM + h * 64 + row;
                 const int n = n0 + wn * WN + c * 8;
-                if (m < M && n < N) st_global_16_streaming(y + (int64_t)m * N + n, v);
+                if (m < M && n < N) st_global_16_streaming(y + (int64_t)m * ldn + n, v);
             }
         }
     } else {
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const half_t *_
 #pragma unroll
             for (int j = 0; j < NP; j++) {
                 const int n = n0 + wn * WN + j * 16 + 4 * kg;
-                half_t *dst = y + (int64_t)m * N + n;
+                half_t *dst = y + (int64_t)m * ldn + n;
                 const half4_t hv = round4(acc[j][i]);
 #pragma unroll
                 for (int e = 0; e < 4; e++)
@@ -616,12 +616,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_a_fused_kernel(const half_t 
 }
 
 template <bool W_IS_KN, int NP, int MPW>
-hipError_t launch_tiled(const half_t *x, const half_t *w, half_t *y, int M, int K, int N, hipStream_t s)
+hipError_t launch_tiled(const half_t *x, const half_t *w, half_t *y, int M, int K, int N, int ldn, hipStream_t s)
 {
     typedef TileCfg<NP, MPW> C;
     const int tiles_m = (M + C::BM - 1) / C::BM, tiles_n = (N + C::BN - 1) / C::BN;
     auto kern = gemm_tiled_kernel<W_IS_KN, NP, MPW>;
-    return launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads), C::kLdsBytes, s, x, w, y, M, K, N,
+    return launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads), C::kLdsBytes, s, x, w, y, M, K, N, ldn,
                        tiles_m, tiles_n);
 }
 
@@ -636,40 +636,64 @@ bool gemm_tiled_supports(const half_t *x, const half_t *w, int M, int K, int N, 
     return (int64_t)BM * K * 2 < (int64_t)1 << 31;
 }
 
+// Which tiles a launch takes: `tile` (1 = 256x256, 2 = 256x128, 3 = 128x128) on the columns before n_split, `tail` on the rest.
+//
 // Rounds of tiles over the compute units.  A tile costs K/64 times a per-stage time that grows with the share of the
 // units at work (the clock drops under load): fitted to measurements, 1.2 us for the 256x256 tile, 0.68 us for 256x128
-// and 0.40 us for 128x128 on an idle device, 1.6 times that on a full one.
-static int tiled_choice(int M, int K, int N, double *cost_us)
+// and 0.40 us for 128x128 on an idle device, 1.6 times that on a full one.  Where the large tiles are a few more than whole
+// rounds, the columns left over go to a second launch in tiles small enough for one more short round.
+struct TiledPlan {
+    int tile, n_split, tail;
+    double cost_us;
+};
+static TiledPlan tiled_plan(int M, int K, int N)
 {
     const int cus = device_cu_count();
-    auto cost = [&](int bm, int bn, double per_stage) {
-        const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    constexpr int kBm[4] = {0, 256, 256, 128}, kBn[4] = {0, 256, 128, 128};
+    constexpr double kStageUs[4] = {0.0, 1.2, 0.68, 0.40};
+    auto cost = [&](int t, int n) {
+        const int64_t tiles = (int64_t)((M + kBm[t] - 1) / kBm[t]) * ((n + kBn[t] - 1) / kBn[t]);
         const int64_t rounds = (tiles + cus - 1) / cus;
         const double busy = (double)tiles / (double)(rounds * cus);
-        return (double)rounds * (5.0 + K / 64.0 * per_stage * (1.0 + 0.6 * busy));
+        return (double)rounds * (5.0 + K / 64.0 * kStageUs[t] * (1.0 + 0.6 * busy));
     };
-    const double t1 = cost(256, 256, 1.2), t2 = cost(256, 128, 0.68), t3 = cost(128, 128, 0.40);
-    const int tile = t3 < t2 && t3 < t1 ? 3 : (t2 < t1 ? 2 : 1);
-    if (cost_us) *cost_us = tile == 3 ? t3 : tile == 2 ? t2 : t1;
-    return tile;
+    auto single = [&](int n) {
+        const double t1 = cost(1, n), t2 = cost(2, n), t3 = cost(3, n);
+        const int t = t3 < t2 && t3 < t1 ? 3 : (t2 < t1 ? 2 : 1);
+        return TiledPlan{t, n, t, t == 3 ? t3 : t == 2 ? t2 : t1};
+    };
+    const TiledPlan one = single(N);
+    TiledPlan best = one;
+    for (int t = 1; t <= 2; t++) {
+        const int tiles_m = (M + kBm[t] - 1) / kBm[t], cols = (N + kBn[t] - 1) / kBn[t];
+        const int64_t rounds = (int64_t)tiles_m * cols / cus;
+        const int head = (int)(rounds * cus / tiles_m);
+        if (rounds < 1 || head < 1 || head >= cols) continue;
+        const TiledPlan rest = single(N - head * kBn[t]);
+        const double us = cost(t, head * kBn[t]) + rest.cost_us + 2.0;
+        if (us < 0.95 * one.cost_us && us < best.cost_us) best = {t, head * kBn[t], rest.tile, us};
+    }
+    return best;
 }
 
-double gemm_tiled_cost_us(int M, int K, int N)
-{
-    double t;
-    tiled_choice(M, K, N, &t);
-    return t;
-}
+double gemm_tiled_cost_us(int M, int K, int N) { return tiled_plan(M, K, N).cost_us; }
 
-// tile: 0 = the tile expected to be fastest, 1 = 256x256, 2 = 256x128, 3 = 128x128
+// tile: 0 = the plan expected to be fastest, 1 = 256x256, 2 = 256x128, 3 = 128x128
 hipError_t launch_gemm_tiled(const half_t *x, const half_t *w, half_t *y, int M, int K, int N, bool w_is_kn, hipStream_t s,
                              int tile)
 {
     if (!gemm_tiled_supports(x, w, M, K, N, w_is_kn)) return hipErrorInvalidValue;
-    if (tile == 0) tile = tiled_choice(M, K, N, nullptr);
-    if (tile == 3) return w_is_kn ? launch_tiled<true, 4, 4>(x, w, y, M, K, N, s) : launch_tiled<false, 4, 4>(x, w, y, M, K, N, s);
-    if (tile == 2) return w_is_kn ? launch_tiled<true, 4, 8>(x, w, y, M, K, N, s) : launch_tiled<false, 4, 8>(x, w, y, M, K, N, s);
-    return w_is_kn ? launch_tiled<true, 8, 8>(x, w, y, M, K, N, s) : launch_tiled<false, 8, 8>(x, w, y, M, K, N, s);
+    const TiledPlan plan = tile == 0 ? tiled_plan(M, K, N) : TiledPlan{tile, N, tile, 0.0};
+    auto launch = [&](int t, int n0, int n) {
+        const half_t *ws = w + (w_is_kn ? (int64_t)n0 : (int64_t)n0 * K);
+        half_t *ys = y + n0;
+        if (t == 3) return w_is_kn ? launch_tiled<true, 4, 4>(x, ws, ys, M, K, n, N, s) : launch_tiled<false, 4, 4>(x, ws, ys, M, K, n, N, s);
+        if (t == 2) return w_is_kn ? launch_tiled<true, 4, 8>(x, ws, ys, M, K, n, N, s) : launch_tiled<false, 4, 8>(x, ws, ys, M, K, n, N, s);
+        return w_is_kn ? launch_tiled<true, 8, 8>(x, ws, ys, M, K, n, N, s) : launch_tiled<false, 8, 8>(x, ws, ys, M, K, n, N, s);
+    };
+    const hipError_t e = launch(plan.tile, 0, plan.n_split);
+    if (e != hipSuccess || plan.n_split >= N) return e;
+    return launch(plan.tail, plan.n_split, N - plan.n_split);
 }
 
 // Nc in whole 16-byte pieces of code bytes, K in whole pairs of stages, 16-byte aligned operands.
