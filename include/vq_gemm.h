@@ -302,8 +302,9 @@ int vqgemm_gemm_f16(const void *x, const void *w, void *y, int64_t M, int64_t K,
                     void *stream);
 
 /*
- * Which kernel VQGEMM_VARIANT_AUTO resolves to for a geometry-B shape (host only, no GPU
- * call): returns a VQGEMM_VARIANT_* value, or a negative error for an invalid shape.
+ * Which family of kernels a geometry-B shape belongs to (host only, no GPU call): returns a VQGEMM_VARIANT_* value, or
+ * a negative error for an invalid shape.  VQGEMM_VARIANT_AUTO launches that kernel, or VQGEMM_VARIANT_WAVE_K (or, above
+ * 64 rows of X, VQGEMM_VARIANT_PREFILL) in its place where the cost models expect that to be faster.
  */
 int vqgemm_select_variant_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries,
                             int32_t n_codebooks, int32_t code_bits);

@@ -253,12 +253,21 @@ int select_b(const ProblemB &p, bool all_aligned16)
     return VQGEMM_VARIANT_GENERIC;
 }
 
+// select_b's kernel for an aligned operand set, or - above 64 rows of X, where the K-sliced path's model promises more than
+// it keeps (65 rows, K = 1024, N = 11904, 4-vectors: 24 us, the prefill kernels 13) - the prefill kernels in that path's place
+// wherever the wave-K kernel stands by for what they are slow at.
+int plain_b(const ProblemB &p)
+{
+    const int v = select_b(p, true);
+    return v == VQGEMM_VARIANT_DECODE && p.M > 64 && prefill_supports(p) && wave_k_b_supports(p) ? VQGEMM_VARIANT_PREFILL : v;
+}
+
 // Split K with the cost model's number of slices when that is expected to beat what the automatic choice would
 // launch otherwise by a margin (and then at least two slices); 0: do not split.
 int splitk_auto(const ProblemB &p, double *t_best, int *plain_variant)
 {
     *t_best = 1e30;
-    const int plain = select_b(p, true);
+    const int plain = plain_b(p);
     *plain_variant = plain;
     double t_plain;
     if (plain == VQGEMM_VARIANT_PREFILL) t_plain = prefill_cost_us(p);
@@ -313,8 +322,7 @@ struct AutoPlan {
     int wave_tile;
 };
 
-// (Above 64 rows the K-sliced path's model promises more than it keeps: there the prefill kernels' is what the wave-K kernel
-// is held to.  The gated product takes what the plain one would run on: every tiled kernel carries the gated epilogue itself;
+// (The gated product takes what the plain one would run on: every tiled kernel carries the gated epilogue itself;
 // the GEMV kernels and the K-sliced decode kernels want whole groups of 32 interleaved rows per codebook resp. per matrix,
 // and where one of them refuses, the next in line takes the shape.)
 AutoPlan make_plan(const ProblemB &p)
@@ -323,7 +331,7 @@ AutoPlan make_plan(const ProblemB &p)
     if (p.K == 0) return plan;
     ProblemB plain = p;
     plain.gated = false;
-    const int v = p.gated && decode_gemv_wide_preferred(p) ? VQGEMM_VARIANT_DECODE_GEMV : select_b(plain, true);
+    const int v = p.gated && decode_gemv_wide_preferred(p) ? VQGEMM_VARIANT_DECODE_GEMV : plain_b(plain);
     const bool tiled = v == VQGEMM_VARIANT_DECODE || v == VQGEMM_VARIANT_PREFILL;
     const bool wave = tiled && wave_k_b_preferred(p, p.M > 64 ? prefill_cost_us(plain) : 0.0);
     if (wave) plan.variant = VQGEMM_VARIANT_WAVE_K;
@@ -590,7 +598,7 @@ int stages_variant(const ProblemB &p, int stages)
     q.k_x = p.K / stages;
     const WorkspaceChoice &c = auto_plan(p).ws;
     if (c.wave) return wave_k_b_supports(q) ? VQGEMM_VARIANT_WAVE_K : VQGEMM_VARIANT_AUTO;
-    return c.bytes == 0 && select_b(p, true) == VQGEMM_VARIANT_DECODE && decode_stages_supports(q) ? VQGEMM_VARIANT_DECODE : VQGEMM_VARIANT_AUTO;
+    return c.bytes == 0 && plain_b(p) == VQGEMM_VARIANT_DECODE && decode_stages_supports(q) ? VQGEMM_VARIANT_DECODE : VQGEMM_VARIANT_AUTO;
 }
 int64_t repeated_x_bytes(const ProblemB &p) { return ((int64_t)p.M * p.K * 2 + 255) & ~(int64_t)255; }
 

@@ -822,8 +822,9 @@ double tile_cost_us(const ProblemB &p, int bn, int cols)
     const Tuning &tn = tuning();
     const double stages = p.K / 64.0 * (bn == BN ? tn.prefill_stage_us_256x256 : tn.prefill_stage_us_256x128) * (p.vec == 8 ? 1.0 : 1.18);
     const int64_t full = tiles / cus, rem = tiles % cus;
-    double t = (double)full * (tn.prefill_tile_fixed_us + stages * tn.prefill_full_device_factor);
-    if (rem) t += tn.prefill_tile_fixed_us + stages * (1.0 + (tn.prefill_full_device_factor - 1.0) * (double)rem / cus);
+    const double fixed = tn.prefill_tile_fixed_us + ((int64_t)p.entries * p.vec > 4096 ? 5.0 : 0.0);   // (a table of more than 8 KB to fill)
+    double t = (double)full * (fixed + stages * tn.prefill_full_device_factor);
+    if (rem) t += fixed + stages * (1.0 + (tn.prefill_full_device_factor - 1.0) * (double)rem / cus);
     return t;
 }
 
@@ -959,8 +960,8 @@ bool prefill_narrow_supports(const ProblemB &p)
     return what.narrow;
 }
 
-// 128x128 tiles are taken when they are expected to be clearly faster than the best cut into large tiles
-constexpr double kSmallTileMargin = 0.95;
+// 128x128 tiles are taken when they are expected to be faster than the best cut into large tiles
+constexpr double kSmallTileMargin = 0.99;
 
 double prefill_cost_us(const ProblemB &p)
 {

@@ -479,7 +479,7 @@ bool prefill_small_supports(const ProblemB &p)
 // compute units in rounds (a second workgroup on a unit shares its LDS bandwidth, which is what
 // bounds this tile, and gains nothing in the main loop; it does overlap its prologue and epilogue
 // with the other's work); a tile costs 4 us plus K/64 stages of 0.46 us on an idle device, 0.56 us
-// when every unit works - with 4-vectors, whose operands are two gathers, 1.18 times that.
+// when every unit works - with 4-vectors, whose operands are two gathers, 1.08 times that.
 static double small_tiles_us(const ProblemB &p, int64_t wgs, int K)
 {
     const int cus = device_cu_count();
@@ -488,7 +488,10 @@ static double small_tiles_us(const ProblemB &p, int64_t wgs, int K)
     const double busy = wgs >= cus ? 1.0 : (double)wgs / cus;
     const Tuning &tn = tuning();
     const double stage_us = tn.prefill_small_stage_us_idle + (tn.prefill_small_stage_us_busy - tn.prefill_small_stage_us_idle) * busy;
-    return (double)resident_rounds * tn.prefill_small_tile_fixed_us + (double)rounds * (K / 64.0 * stage_us) * (p.vec == 8 ? 1.0 : 1.18);
+    // (with two on a unit a last round that is not full costs about half of what is missing, and later prologues are hidden)
+    const double rounds_us = two && rounds > 1 ? 0.5 * ((double)rounds + (double)wgs / cus) : (double)rounds;
+    const double fixed = two ? 1.0 + 0.375 * (double)(resident_rounds - 1) : (double)rounds;
+    return fixed * tn.prefill_small_tile_fixed_us + rounds_us * (K / 64.0 * stage_us) * (p.vec == 8 ? 1.0 : 1.08);
 }
 
 double prefill_small_cost_us(const ProblemB &p)

@@ -123,25 +123,23 @@ int wave_k_b_tile(const ProblemB &p)
     return tile;
 }
 
-// The rule.  Up to two rows of X are the GEMV kernels' or the decode path's.  Up to 16 the decode path is about as fast: this
-// kernel where it is expected to be a tenth faster (long K or many columns, where the decode path walks K in chunks or fills
-// its tables several times; over 300 shapes 8 to 11 % of the time).  Up to 64 rows this kernel, except on the shortest products
-// in 8-bit codes (K <= 2048, one 16 x 16 tile of Y per compute unit at most), which the decode path has done 5 to 10 %
-// earlier.  Above, where it is
-// expected to be faster than the others by more than the models' error.  (us, before -> now: M = 44, K = 704, N = 21888, 4-vectors 32.3 ->
-// 11.0; M = 100, K = 1408, N = 3500 11.9 -> 6.5; M = 256, K = N = 4096, 16-bit codes 26.5 -> 17.6; M = 451, K = 1152,
-// N = 1376 18.2 -> 8.0.)
+// The rule: whichever is expected to be faster.  Up to 64 rows of X the other is the decode path, whose model is as close as this
+// one's (with these margins the choice is 1 to 3 % from the better one over 540 measured shapes); where that
+// path would take its streaming or its general kernel it keeps up to 16 rows.  Above, the tiled kernels, by more than the models' error.
+// (us, before -> now: M = 8, K = 640, N = 22912 23.8 -> 6.1; M = 44, K = 704, N = 21888, 4-vectors 32.3 -> 11.0; M = 100,
+// K = 1408, N = 3500 11.9 -> 6.5; M = 256, K = N = 4096, 16-bit codes 26.5 -> 17.6; M = 451, K = 1152, N = 1376 18.2 -> 8.0.)
 bool wave_k_b_preferred(const ProblemB &p, double t_other)
 {
     const int force = (int)tuning().wave_k_force;
     if (force == 2 || !wave_k_b_supports(p)) return false;
     if (force == 1) return true;
-    if (p.M <= 2) return false;
-    if (p.M <= 16) {
+    if (p.M <= 64) {
         const double t_decode = decode_slab_cost_us(p);
-        return t_decode < 1e29 && wave_k_b_cost_us(p) < 0.9 * t_decode;
+        if (t_decode > 1e29) return p.M > 16;
+        // (the gated decode kernels deal tiles in pairs, which their model does not see; up to 16 rows near ties stay where the packed
+        // code layout, which only the decode path reads, gives the same bits)
+        return wave_k_b_cost_us(p) < (p.gated ? 1.15 : p.M <= 16 ? 0.89 : 0.97) * t_decode;
     }
-    if (p.M <= 64) return !(p.code_bits == 8 && p.K <= 2048 && (int64_t)((p.M + 15) / 16) * ((p.N + 15) / 16) <= device_cu_count());
     return wave_k_b_cost_us(p) < 0.95 * t_other;
 }
 
