@@ -193,3 +193,38 @@ def test_start_of_a_seeded_permutation_is_torch_randperm_s(n, count, books, seed
     want = torch.stack([torch.randperm(n, generator=gen)[:count] for _ in range(books)]).to(torch.int32)
     assert torch.equal(native.first_of_permutations(n, count, books, seed), want)
     assert torch.equal(_initial_vectors(n, count, books, seed), want)
+
+
+def test_launches_of_the_wave_k_kernel_hold_what_the_copy_of_their_codebooks_writes(tmp_path):
+    """The codebooks go into the LDS in wave loads of 1 KB: a launch asks for the LDS up to the end of the last one, whatever the
+    tables' size.  Checked by the compiler (host pass, nothing is linked) for every tile and format, on the kernel's own
+    configuration: tables of every size from one 16-byte chunk to just over four wave loads."""
+    import subprocess
+    from vq_gemm_amd import build
+    src = tmp_path / "lds.hip"
+    src.write_text("""
+#include "vq_wave_k_b.hip"
+namespace vq {
+template <class C> constexpr bool holds_every_table()
+{
+    for (size_t chunks = 1; chunks <= 260; chunks++)   // 16-byte chunks; 64 lanes of 16 bytes a load
+        if (C::lds_bytes(chunks * 16) < C::kRing + (chunks + 63) / 64 * 64 * 16) return false;
+    return true;
+}
+template <class F, int MP, int NP> constexpr bool holds()
+{
+    typedef WaveKCfg<typename F::template Wave<MP, NP>, MP, NP> C;
+    if constexpr (C::kExists) return holds_every_table<C>();
+    else return true;
+}
+template <class F> constexpr bool every_tile()
+{
+    return holds<F, 1, 2>() && holds<F, 1, 4>() && holds<F, 1, 8>() && holds<F, 2, 2>() && holds<F, 2, 4>() && holds<F, 4, 4>() && holds<F, 4, 8>();
+}
+static_assert(every_tile<Format<8, uint8_t>>() && every_tile<Format<8, uint16_t>>(), "8-vectors");
+static_assert(every_tile<Format<4, uint8_t>>() && every_tile<Format<4, uint16_t>>(), "4-vectors");
+}
+""")
+    res = subprocess.run([build.HIPCC, "-x", "hip", "--offload-host-only", f"--offload-arch={build.ARCH}", "-std=c++17", "-fsyntax-only",
+                          "-fconstexpr-steps=10000000", f"-I{build.CSRC}", str(src)], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout + res.stderr

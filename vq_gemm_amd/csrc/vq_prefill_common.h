@@ -189,10 +189,14 @@ inline int codebooks_per_tile(const ProblemB &p, int bn)
     return n < p.n_codebooks ? n : p.n_codebooks;
 }
 
+// LDS that a copy of `bytes` bytes writes: a wave load brings 1 KB, all 64 lanes on, so that a table of no whole kilobyte is
+// followed by up to 1008 bytes of what lies behind it (or of its end again)
+constexpr size_t copied_bytes(size_t bytes) { return (bytes + 1023) & ~(size_t)1023; }
+
 // codebooks of a tile, padded to the 1 KB steps they are copied in, plus 16 zero bytes
 inline size_t books_bytes(const ProblemB &p, int bn)
 {
-    return (((size_t)codebooks_per_tile(p, bn) * p.entries * p.vec * 2 + 1023) & ~(size_t)1023) + 16;
+    return copied_bytes((size_t)codebooks_per_tile(p, bn) * p.entries * p.vec * 2) + 16;
 }
 
 }  // namespace

@@ -86,7 +86,12 @@ struct WaveKCfg {
     static constexpr int kSumBytes = kWaves * kPassMP * NP * 1024;
     static constexpr bool kExists = D >= 2;   // the LDS holds two units of every wave
     static_assert(D * kLoads < 64 && kPassMP >= 1 && MP % kPassMP == 0 && kSumBytes <= 160 * 1024, "counts of loads, passes of the sum");
-    static size_t lds_bytes(size_t books) { return kRing + books > (size_t)kSumBytes ? kRing + books : (size_t)kSumBytes; }
+    // (`books` bytes of codebooks, copied in steps of a wave load)
+    static constexpr size_t lds_bytes(size_t books)
+    {
+        const size_t use = kRing + copied_bytes(books);
+        return use > (size_t)kSumBytes ? use : (size_t)kSumBytes;
+    }
 };
 
 // X in a unit of one step: 64-byte rows, four to a 256-byte bank row, XOR-swizzled; of two steps: x_offset.
