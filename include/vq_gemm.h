@@ -130,9 +130,11 @@ int64_t vqgemm_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t vec, i
 /*
  * The product over additive ("residual") stages: codes [N, K/vec] hold `stages` blocks of K/stages columns of W side by side, all of
  * which multiply the same x [M, K/stages]: y = sum over the stages of x . W_s^T, in one fp32 sum.  The kernel is the automatic
- * choice's for K; the decode kernel reads x as it is, the others from a copy repeated along K in the workspace
+ * choice's for K; the decode and the wave-K kernel read x as it is, the others from a copy repeated along K in the workspace
  * (vqgemm_stages_workspace_bytes_b bytes, 256-byte aligned; what is beyond the copy serves split K as in
- * vqgemm_e2e_gemm_b_ws).  VQGEMM_E_SCRATCH when the workspace does not hold a copy that is needed.  No counterpart in the reference.
+ * vqgemm_e2e_gemm_b_ws).  That many bytes suffice wherever the operands begin: those that are not 16-byte aligned (bias: 8) go to
+ * the scalar kernel, which reads x as it is where the others do.  VQGEMM_E_SCRATCH when the workspace does not hold a copy that
+ * is needed.  No counterpart in the reference.
  */
 int64_t vqgemm_stages_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t vec,
                                         int32_t entries, int32_t n_codebooks, int32_t code_bits,

@@ -1934,6 +1934,35 @@ def test_stages_multiply_the_same_x_without_a_copy_of_it(M, K, N, v, entries, st
         assert torch.equal(y, cabi.e2e_gemm_b_ws(x.repeat(1, stages), codes, cb, bias=b))
 
 
+# shapes whose stages need no copy of x (decode kernel, wave-K kernel), and one that needs it (tall X); every operand begins off
+# its alignment in turn, codes and codebook as slices of larger tensors like the bias
+@pytest.mark.parametrize("M,K,N,v,entries,stages,bits", [(5, 4096, 80, 8, 128, 2, 8), (20, 2048, 64, 4, 256, 4, 16), (130, 512, 72, 8, 128, 2, 8)])
+@pytest.mark.parametrize("which", ["bias", "codes", "codebook"])
+def test_stages_take_operands_that_begin_anywhere(M, K, N, v, entries, stages, bits, which):
+    from vq_gemm_amd.nn import VQLinear
+    _say("stages, unaligned", which, M, K, N, v, entries, stages)
+    spec = ProblemSpec("stages", GEOM_B, M, stages * K, N, v, stages * entries, 1, bits, codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=18, device=DEV)
+    x = x[:, :K].contiguous()
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(1)).half().to(DEV)
+
+    def shifted(t):
+        big = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+        big[1:] = t.reshape(-1)
+        return big[1:].view(t.shape)
+
+    operands = {"codes": codes, "codebook": cb, "bias": bias}
+    operands[which] = shifted(operands[which])
+    layer = VQLinear(operands["codes"], operands["codebook"], operands["bias"], k_repeat=stages)
+    assert getattr(layer, which).data_ptr() % 8 != 0
+    y = layer(x)
+    torch.cuda.synchronize()
+    want = _np(x.repeat(1, stages)).astype(np.float64) @ vo.dequant_b(_np(codes), _np(cb)).astype(np.float64).T + _np(bias).astype(np.float64)
+    assert vo.rel_err(_np(y), want)[0] <= TOL
+    # the scalar kernel on a copy: the same sums in the same order
+    assert torch.equal(y, cabi.e2e_gemm_b(x.repeat(1, stages), codes, cb, variant=cabi.VARIANT_GENERIC, bias=bias))
+
+
 def _with_wave_tile(tile, call):
     before = cabi.tuning()
     try:

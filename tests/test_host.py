@@ -228,3 +228,21 @@ static_assert(every_tile<Format<4, uint8_t>>() && every_tile<Format<4, uint16_t>
     res = subprocess.run([build.HIPCC, "-x", "hip", "--offload-host-only", f"--offload-arch={build.ARCH}", "-std=c++17", "-fsyntax-only",
                           "-fconstexpr-steps=10000000", f"-I{build.CSRC}", str(src)], capture_output=True, text=True)
     assert res.returncode == 0, res.stdout + res.stderr
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="made-up addresses: only where no kernel can be launched")
+def test_stages_need_no_more_scratch_than_they_ask_for_wherever_the_operands_begin():
+    lib = cabi.lib()
+    ptr = ctypes.c_void_p
+    base = 1 << 20
+    checked = 0
+    for M, K, N, vec, entries, bits in ((5, 8192, 4096, 8, 256, 8), (20, 8192, 64, 4, 1024, 16), (3, 8320, 33, 8, 256, 8), (16, 960, 50, 8, 300, 16)):
+        for stages in (2, 3):
+            if K % stages or lib.vqgemm_stages_workspace_bytes_b(M, K, N, vec, entries, 1, bits, stages) != 0:
+                continue
+            for shift in ((0, 0, 0, 0, 0), (2, 0, 0, 0, 0), (0, 2, 0, 0, 0), (0, 0, 2, 0, 0), (0, 0, 0, 2, 0), (0, 0, 0, 0, 2)):
+                x, codes, cb, bias, y = (ptr(base + s) for s in shift)
+                rc = lib.vqgemm_e2e_gemm_b_stages(x, codes, cb, bias, y, M, K, N, vec, entries, 1, bits, stages, None, 0, None)
+                assert rc > 0, (M, K, N, stages, shift, rc)   # as far as the launch, which finds no device
+                checked += 1
+    assert checked >= 18

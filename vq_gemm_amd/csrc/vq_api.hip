@@ -590,10 +590,12 @@ int vqgemm_e2e_gemm_b_ws(const void *x, const void *codes, const void *codebook,
 
 namespace {
 
-// Additive stages: the kernel that the automatic choice for the whole K takes, where that kernel reads an X that repeats along
-// K as it is (VQGEMM_VARIANT_AUTO: it does not, X is repeated in memory)
-int stages_variant(const ProblemB &p, int stages)
+// Additive stages: the kernel that the automatic choice for the whole K takes on aligned operands, where that kernel reads an X
+// that repeats along K as it is (VQGEMM_VARIANT_AUTO: it does not, X is repeated in memory).  A matter of the sizes only: the
+// question for a workspace is asked before there are operands.
+int stages_variant(ProblemB p, int stages)
 {
+    p.x = nullptr;
     ProblemB q = p;
     q.k_x = p.K / stages;
     const WorkspaceChoice &c = auto_plan(p).ws;
@@ -637,12 +639,15 @@ int vqgemm_e2e_gemm_b_stages(const void *x, const void *codes, const void *codeb
     p.bias = static_cast<const half_t *>(bias);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool a16 = aligned(x, 16) && aligned(y, 16) && aligned(codebook, 16) && aligned(codes, 16) && aligned(bias, 8);
-    const int variant = a16 ? stages_variant(p, stages) : VQGEMM_VARIANT_AUTO;
-    if (variant != VQGEMM_VARIANT_AUTO) {
+    const int64_t repeated = repeated_x_bytes(p);
+    const int variant = stages_variant(p, stages);
+    // (operands that begin anywhere, and no room for a copy because for these sizes none is asked for: the scalar kernel, which
+    // such operands go to in any case, reads X as it is too; whole vectors, since both kernels above want K / stages % 8 == 0)
+    if (variant != VQGEMM_VARIANT_AUTO && (a16 || workspace_bytes < repeated)) {
         p.k_x = p.K / stages;
+        if (!a16) return static_cast<int>(launch_generic_b(p, s));
         return static_cast<int>(variant == VQGEMM_VARIANT_WAVE_K ? launch_wave_k_b(p, s) : launch_decode_b(p, s));
     }
-    const int64_t repeated = repeated_x_bytes(p);
     if (workspace_bytes < repeated) return VQGEMM_E_SCRATCH;
     const hipError_t e = launch_repeat_columns(p.x, static_cast<half_t *>(workspace), M, K / stages, stages, s);
     if (e != hipSuccess) return static_cast<int>(e);

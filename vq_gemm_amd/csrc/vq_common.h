@@ -28,7 +28,7 @@ struct ProblemB {
     half_t *y;            // [M,N]
     const half_t *bias;   // [N] added to the fp32 sums before the rounding to fp16, or nullptr
     int M, K, N;
-    int k_x;              // columns of X: K, or K / stages where X repeats along K (the kernel behind decode_stages_supports only)
+    int k_x;              // columns of X: K, or K / stages where X repeats along K (wave-K, the kernel behind decode_stages_supports, the scalar one)
     int vec, entries, n_codebooks, code_bits;
     int rows_per_cb;      // N / G
     bool packed;          // codes are in the packed layout of the batched decode kernel (launch_pack_codes)

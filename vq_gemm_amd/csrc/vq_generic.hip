@@ -12,23 +12,26 @@ __global__ __launch_bounds__(256) void generic_b_kernel(const half_t *__restrict
                                                         const half_t *__restrict__ cb,
                                                         half_t *__restrict__ y,
                                                         const half_t *__restrict__ bias, int M, int K, int N,
-                                                        int vec, int entries, int rows_per_cb)
+                                                        int k_x, int vec, int entries, int rows_per_cb)
 {
+    // X has k_x columns, whole vectors; where that is less than K (additive stages side by side along K) they repeat.
     // blockDim = (64, 4): x index -> n (coalesced y stores), y index -> m.
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
-    const int J = K / vec;
+    const int J = K / vec, J_x = k_x / vec;
     const half_t *book = cb + (int64_t)(n / rows_per_cb) * entries * vec;
     const CodeT *crow = codes + (int64_t)n * J;
     const float b = bias ? (float)bias[n] : 0.0f;
     for (int m = blockIdx.y * blockDim.y + threadIdx.y; m < M; m += gridDim.y * blockDim.y) {
-        const half_t *xrow = x + (int64_t)m * K;
+        const half_t *xrow = x + (int64_t)m * k_x;
         float acc = 0.0f;
-        for (int j = 0; j < J; j++) {
-            uint32_t c = crow[j];
-            c = c < (uint32_t)entries ? c : (uint32_t)entries - 1;  // memory safety only
-            const half_t *cw = book + (int64_t)c * vec;
-            for (int t = 0; t < vec; t++) acc += (float)xrow[j * vec + t] * (float)cw[t];
+        for (int j0 = 0; j0 < J; j0 += J_x) {
+            for (int j = 0; j < J_x; j++) {
+                uint32_t c = crow[j0 + j];
+                c = c < (uint32_t)entries ? c : (uint32_t)entries - 1;  // memory safety only
+                const half_t *cw = book + (int64_t)c * vec;
+                for (int t = 0; t < vec; t++) acc += (float)xrow[j * vec + t] * (float)cw[t];
+            }
         }
         y[(int64_t)m * N + n] = (half_t)(acc + b);
     }
@@ -73,6 +76,7 @@ __global__ __launch_bounds__(256) void generic_b_gated_kernel(const half_t *__re
 hipError_t launch_generic_b(const ProblemB &p, hipStream_t s)
 {
     if (p.M == 0 || p.N == 0) return hipSuccess;
+    if (p.k_x != p.K && (p.gated || p.k_x < p.vec || p.k_x % p.vec != 0 || p.K % p.k_x != 0)) return hipErrorInvalidValue;
     if (p.gated) {
         dim3 block(64, 4);
         dim3 grid((p.N / 2 + 63) / 64, (unsigned)(((p.M + 3) / 4) < 32768 ? (p.M + 3) / 4 : 32768));
@@ -87,10 +91,10 @@ hipError_t launch_generic_b(const ProblemB &p, hipStream_t s)
     dim3 grid((p.N + 63) / 64, (unsigned)(((p.M + 3) / 4) < 32768 ? (p.M + 3) / 4 : 32768));
     if (p.code_bits == 8)
         return launch_kernel((generic_b_kernel<uint8_t>), grid, block, 0, s, p.x, static_cast<const uint8_t *>(p.codes),
-                           p.cb, p.y, p.bias, p.M, p.K, p.N, p.vec, p.entries, p.rows_per_cb);
+                           p.cb, p.y, p.bias, p.M, p.K, p.N, p.k_x, p.vec, p.entries, p.rows_per_cb);
     else
         return launch_kernel((generic_b_kernel<uint16_t>), grid, block, 0, s, p.x, static_cast<const uint16_t *>(p.codes),
-                           p.cb, p.y, p.bias, p.M, p.K, p.N, p.vec, p.entries, p.rows_per_cb);
+                           p.cb, p.y, p.bias, p.M, p.K, p.N, p.k_x, p.vec, p.entries, p.rows_per_cb);
 }
 
 // Geometry A: out[m, 2n + r] = sum_k x[m,k] * cb[n/4][w[k,n]][r].  One thread per code
