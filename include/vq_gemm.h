@@ -282,6 +282,15 @@ int vqgemm_decode_packed_supports(int64_t M, int64_t K, int64_t N, int32_t vec, 
                                   int32_t n_codebooks, int32_t code_bits);
 
 /*
+ * 1 where a caller that holds the codes in both layouts does best with the packed one: VQGEMM_VARIANT_AUTO (with or without a
+ * workspace) launches the K-sliced MFMA kernel on the plain matrix, and VQGEMM_VARIANT_DECODE_PACKED is that kernel with the
+ * same result bit for bit.  0 where AUTO takes another kernel (VQGEMM_VARIANT_WAVE_K, the GEMV kernels, the streaming kernel, the
+ * prefill kernels) or the packed layout is not served; a negative error for an invalid shape.  Host only, no GPU call.
+ */
+int vqgemm_packed_preferred_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries,
+                              int32_t n_codebooks, int32_t code_bits);
+
+/*
  * The code-range contract, and the check for it.  Every code must be below `entries` (geometry A:
  * any byte is valid, its codebooks have 256 entries).  The fused kernels do not test codes: they
  * gather at code * entry size inside the workgroup's own LDS allocation (the GEMV kernel of 8-bit

@@ -1483,6 +1483,29 @@ def test_vqlinear_repacks_after_its_codes_change():
     assert torch.equal(layer(x), cabi.e2e_gemm_b(x, codes, cb))
 
 
+# K-sliced kernel, wave-K kernel, streaming kernel, GEMV kernel, prefill kernels; two additive stages
+@pytest.mark.parametrize("M,K,N,v,entries,bits,stages", [(4, 4096, 8192, 8, 256, 8, 1), (64, 8192, 512, 4, 4096, 16, 1), (16, 14336, 512, 8, 256, 8, 1),
+                                                         (1, 4096, 512, 8, 256, 8, 1), (300, 512, 256, 4, 256, 8, 1), (8, 1024, 512, 8, 256, 8, 2)])
+def test_packed_layer_takes_the_native_call_and_gives_the_plain_layers_bits(M, K, N, v, entries, bits, stages, monkeypatch):
+    from vq_gemm_amd.nn import VQLinear
+    _say("packed layer", M, K, N, v, entries, bits, stages)
+    spec = ProblemSpec("packed", GEOM_B, M, stages * K, N, v, entries, 1, bits, codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=19, device=DEV)
+    x = x[:, :K].contiguous()
+    bias = torch.randn(N + 1, generator=torch.Generator().manual_seed(2)).half().to(DEV)
+    for b in (None, bias[:N], bias[1:]):   # (the last one begins off 8 bytes: no kernel but the scalar one takes it)
+        plain = VQLinear(codes, cb, b, k_repeat=stages)
+        packed = VQLinear(codes, cb, b, k_repeat=stages).prepack_for_decode()
+        want = plain(x)
+        with monkeypatch.context() as m:
+            m.setattr(VQLinear, "_forward_op", lambda self, x: pytest.fail("a plain call went through the dispatcher"))
+            y = packed(x)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+        if b is None or b.data_ptr() % 8 == 0:
+            assert torch.equal(packed._forward_op(x), want) or stages > 1
+
+
 def test_ctypes_wrappers_check_dtypes_and_shapes_before_the_gpu_sees_them():
     spec = CONFIGS["C1"]
     x, codes, cb = make_problem(spec, seed=42, device=DEV)

@@ -246,3 +246,13 @@ def test_stages_need_no_more_scratch_than_they_ask_for_wherever_the_operands_beg
                 assert rc > 0, (M, K, N, stages, shift, rc)   # as far as the launch, which finds no device
                 checked += 1
     assert checked >= 18
+
+
+def test_the_packed_layout_is_taken_where_the_automatic_choice_takes_its_kernel():
+    # the K-sliced kernel's shapes; the wave-K kernel's (which serves the packed layout too, slower); the streaming kernel's; tall X
+    assert cabi.packed_preferred_b(4, 4096, 8192, 8, 256, 1, 8)
+    for dims in ((64, 8192, 14336, 4, 4096, 1, 16), (64, 4096, 4096, 8, 256, 1, 8), (16, 14336, 4096, 8, 256, 1, 8), (512, 4096, 4096, 8, 256, 1, 8)):
+        assert cabi.decode_packed_supports(*dims) and not cabi.packed_preferred_b(*dims), dims
+    assert not cabi.packed_preferred_b(4, 320, 8192, 8, 256, 1, 8)   # no packed layout for this K
+    assert not cabi.packed_preferred_b(0, 4096, 8192, 8, 256, 1, 8)
+    assert cabi.lib().vqgemm_packed_preferred_b(4, 60, 8, 8, 256, 1, 8) < 0

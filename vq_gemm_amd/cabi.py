@@ -38,6 +38,7 @@ _SIGNATURES = {
     "vqgemm_kmeans_b": (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _P, _I64, _P]),
     "vqgemm_pack_codes_b": (ctypes.c_int, [_P, _P, _I64, _I64, _I32, _I32, _I32, _P]),
     "vqgemm_decode_packed_supports": (ctypes.c_int, [_I64, _I64, _I64, _I32, _I32, _I32, _I32]),
+    "vqgemm_packed_preferred_b": (ctypes.c_int, [_I64, _I64, _I64, _I32, _I32, _I32, _I32]),
     "vqgemm_gemm_f16": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _I64, _P]),
     "vqgemm_silu_mul": (ctypes.c_int, [_P, _P, _I64, _I64, _P]),
     "vqgemm_max_code": (ctypes.c_int, [_P, _I64, _I32, _P, _P]),
@@ -457,6 +458,12 @@ def max_code(codes) -> int:
 
 def decode_packed_supports(M, K, N, vec, entries, n_codebooks, code_bits) -> bool:
     return lib().vqgemm_decode_packed_supports(M, K, N, vec, entries, n_codebooks, code_bits) == 1
+
+
+def packed_preferred_b(M, K, N, vec, entries, n_codebooks, code_bits) -> bool:
+    """Whether a caller that holds both layouts of the codes hands the packed one over (`VARIANT_DECODE_PACKED`): the automatic
+    choice would launch the same kernel on the plain matrix."""
+    return lib().vqgemm_packed_preferred_b(M, K, N, vec, entries, n_codebooks, code_bits) == 1
 
 
 def dequant_a(w, codebook, out=None):

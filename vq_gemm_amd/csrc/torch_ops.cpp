@@ -239,11 +239,26 @@ constexpr char kLinear[] = "vq_gemm_amd::vq_linear", kLinearPacked[] = "vq_gemm_
 
 // ---- the layers' direct calls ---------------------------------------------------------------------------------
 
-py::object linear(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias, int64_t k_repeat)
+// packed: `codes` are in the packed layout (a single stage)
+py::object linear(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias, int64_t k_repeat, bool packed)
 {
     if (!plain_call(x)) return py::none();
+    TORCH_CHECK_VALUE(!packed || k_repeat == 1, "linear: additive stages have no packed layout");
     RECORD_FUNCTION("vq_gemm_amd::vq_linear", c10::ArrayRef<const c10::IValue>());
-    return py::cast(linear_impl(x, codes, codebook, bias, k_repeat));
+    return py::cast(linear_impl(x, codes, codebook, bias, k_repeat, packed ? VQGEMM_VARIANT_DECODE_PACKED : VQGEMM_VARIANT_AUTO));
+}
+
+// Whether a layer that holds both layouts of its codes hands the packed one over for x (what is wrong with x the call itself says;
+// the kernel of the packed layout takes no operands that begin anywhere).
+bool takes_packed(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
+{
+    if (!plain_call(x) || x.dim() < 1 || codes.dim() != 2 || (codebook.dim() != 2 && codebook.dim() != 3) || !aligned16(codebook)) return false;
+    if (bias.has_value() && bias->defined() && (reinterpret_cast<uintptr_t>(bias->data_ptr()) & 7) != 0) return false;
+    const int64_t vec = codebook.size(-1), K = codes.size(1) * vec;
+    if (K == 0 || x.size(-1) != K) return false;
+    const c10::OptionalDeviceGuard guard(x.device());
+    return vqgemm_packed_preferred_b(x.numel() / K, K, codes.size(0), (int)vec, (int)codebook.size(-2),
+                                     codebook.dim() == 3 ? (int)codebook.size(0) : 1, codes.scalar_type() == at::kByte ? 8 : 16) == 1;
 }
 
 py::object gated(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
@@ -353,6 +368,7 @@ TORCH_LIBRARY_IMPL(vq_gemm_amd, AutogradCUDA, m)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.def("linear", &linear, "x @ W.T (+ bias) on plain GPU tensors; None where the registered operator is to be called instead");
+    m.def("takes_packed", &takes_packed, "whether `linear` does best with the packed layout of the codes");
     m.def("first_of_permutations", &first_of_permutations, "the first elements of seeded random permutations");
     m.def("kmeans", &kmeans, "Lloyd iterations on the device; None where the codebook is too large for them");
     m.def("encode", &encode, "nearest-codeword codes; None where cabi.encode_b is to check the operands one by one");

@@ -843,6 +843,18 @@ int vqgemm_decode_packed_supports(int64_t M, int64_t K, int64_t N, int32_t vec, 
     return decode_packed_supports(p) ? 1 : 0;
 }
 
+int vqgemm_packed_preferred_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks,
+                              int32_t code_bits)
+{
+    const DeviceScope device;
+    const int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
+    if (rc != VQGEMM_OK) return rc;
+    if (M == 0 || N == 0 || K == 0) return 0;
+    const ProblemB p = make_b(nullptr, nullptr, nullptr, nullptr, M, K, N, vec, entries, n_codebooks, code_bits);
+    const AutoPlan &plan = auto_plan(p);
+    return plan.variant == VQGEMM_VARIANT_DECODE && !plan.ws.wave && plan.ws.bytes == 0 && decode_packed_preferred(p) ? 1 : 0;
+}
+
 int vqgemm_encode_b(const void *w, const void *codebook, void *codes_out, int64_t N, int64_t K, int32_t vec,
                     int32_t entries, int32_t n_codebooks, int32_t code_bits, void *stream)
 {

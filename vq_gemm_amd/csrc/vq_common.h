@@ -105,6 +105,8 @@ hipError_t launch_pack_codes(const void *src, void *dst, int64_t N, int64_t K, i
                              hipStream_t s);
 // whether launch_decode_b takes the shape with p.packed set (the batched kernel only)
 bool decode_packed_supports(const ProblemB &p);
+// whether the packed matrix is the same kernel's faster input where the automatic choice takes launch_decode_b
+bool decode_packed_preferred(const ProblemB &p);
 // the GEMV kernel behind launch_decode_b (vq_decode_gemv.hip): one row of X, 8-vectors, 8-bit codes,
 // whole rows of W per wave; the automatic choice takes it while a compute unit has few rows to do
 bool decode_gemv_supports(const ProblemB &p);

@@ -906,6 +906,9 @@ bool decode_packed_supports(const ProblemB &p)
     return p.M >= 1 && p.M <= kBatchedMaxM && decode_general_supports(p) && batched_supports(q);
 }
 
+// where launch_decode_b takes the batched kernel on the plain matrix (not the streaming kernel, which adds up in another order)
+bool decode_packed_preferred(const ProblemB &p) { return decode_packed_supports(p) && !decode_stream_preferred(p); }
+
 bool pack_codes_supports(int64_t N, int64_t K, int vec, int code_bits)
 {
     return (vec == 2 || vec == 4 || vec == 8) && (code_bits == 8 || code_bits == 16) && K % kSliceK == 0 && N % kTileN == 0;

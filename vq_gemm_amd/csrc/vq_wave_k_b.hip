@@ -136,8 +136,9 @@ bool wave_k_b_preferred(const ProblemB &p, double t_other)
     if (p.M <= 64) {
         const double t_decode = decode_slab_cost_us(p);
         if (t_decode > 1e29) return p.M > 16;
-        // (the gated decode kernels deal tiles in pairs, which their model does not see; up to 16 rows near ties stay where the packed
-        // code layout, which only the decode path reads, gives the same bits)
+        // (the gated decode kernels deal tiles in pairs, which their model does not see; up to 16 rows the decode kernel is ahead near
+        // ties on codes out of HBM: over 145 shapes this line is 1.0 % from the better kernel there, 0.97 is 1.8 %, and on codes that
+        // the caches hold, where it is the other way round, they are 3.8 and 2.1 %)
         return wave_k_b_cost_us(p) < (p.gated ? 1.15 : p.M <= 16 ? 0.89 : 0.97) * t_decode;
     }
     return wave_k_b_cost_us(p) < 0.95 * t_other;

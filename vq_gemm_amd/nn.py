@@ -46,10 +46,11 @@ class VQLinear(torch.nn.Module):
 
     def prepack_for_decode(self) -> "VQLinear":
         """Keep a second copy of the codes in the decode kernel's packed layout (`cabi.pack_codes_b`;
-        as large as the codes, 1/16 of the fp16 weight for 8-vectors with 8-bit codes).  Inputs short
-        enough for the decode kernel then read that copy: one contiguous run per wave load instead
-        of sixteen row pieces, 10-25 % less time once a workgroup has several tiles, the same result
-        bit for bit.  Taller inputs keep using the plain matrix."""
+        as large as the codes, 1/16 of the fp16 weight for 8-vectors with 8-bit codes).  Inputs that the
+        automatic choice gives to the K-sliced decode kernel then read that copy: one contiguous run
+        per wave load instead of sixteen row pieces, the same result bit for bit.  All others - taller
+        inputs, one or two rows, the shapes of the wave-K kernel, additive stages - keep using the
+        plain matrix (`cabi.packed_preferred_b`)."""
         try:
             self.codes_packed = cabi.pack_codes_b(self.codes, self.codebook.shape[-1])
         except cabi.VqGemmError as e:
@@ -97,10 +98,12 @@ class VQLinear(torch.nn.Module):
         # mode or torch.compile it is the registered operator.
         if not is_compiling():
             b = self._buffers
-            if b["codes_packed"] is None:
-                y = native.linear(x, b["codes"], b["codebook"], b["bias"], self.k_repeat)
-                if y is not None:
-                    return y
+            codes, packed = b["codes"], False
+            if b["codes_packed"] is not None and self.k_repeat == 1 and native.takes_packed(x, codes, b["codebook"], b["bias"]):
+                codes, packed = self._fresh_packed_codes(), True
+            y = native.linear(x, codes, b["codebook"], b["bias"], self.k_repeat, packed)
+            if y is not None:
+                return y
         return self._forward_op(x)
 
     @torch.no_grad()
@@ -112,7 +115,7 @@ class VQLinear(torch.nn.Module):
         if self.codes_packed is not None:
             g, e, v = cabi._cb_dims(self.codebook)
             dims = (x.numel() // x.shape[-1], x.shape[-1], self.out_features, v, e, g, 8 * self.codes.element_size())
-            if cabi.select_variant_b(*dims) == cabi.VARIANT_DECODE and cabi.decode_packed_supports(*dims):
+            if cabi.packed_preferred_b(*dims):
                 return vq_linear_packed(x, self._fresh_packed_codes(), self.codebook, self.bias)
         return vq_linear(x, self.codes, self.codebook, self.bias)
 
