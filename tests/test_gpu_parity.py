@@ -1896,6 +1896,40 @@ def test_widths_that_are_no_multiple_of_a_tile_or_a_slice(row):
         assert e2 <= TOL and e1 <= 2 * TOL, (name, "gated", e1, e2)
 
 
+# K that ends inside a slice, a code tile or a unit, in every format; fewer than 16 columns and K % 64 = 32, which the general decode kernel takes
+@pytest.mark.parametrize("M,K,N,v,entries,bits,G", [(5, 320, 48, 8, 256, 8, 1), (16, 2240, 33, 8, 100, 8, 1), (40, 4160, 80, 8, 256, 8, 1), (9, 448, 50, 8, 700, 16, 1),
+                                                    (12, 832, 61, 4, 256, 8, 1), (16, 4288, 77, 4, 1024, 16, 1), (7, 576, 40, 2, 256, 8, 1), (3, 320, 32, 2, 300, 16, 1),
+                                                    (5, 384, 8, 8, 256, 8, 1), (16, 1120, 48, 4, 300, 16, 3), (20, 4384, 33, 4, 300, 16, 1), (130, 1984, 160, 8, 256, 8, 1), (70, 416, 96, 4, 256, 8, 1)])
+def test_infinite_codewords_reach_their_own_rows_only_and_as_infinities(M, K, N, v, entries, bits, G):
+    """Entry 0 is infinite and selected nowhere, entry 1 by the first code of every third row: with positive X those rows are +inf, as
+    the definition has them, and all others finite.  What a kernel multiplies beyond K must not bring either in."""
+    spec = ProblemSpec("inf", GEOM_B, M, K, N, v, entries, G, bits, codebook_3d=(G > 1), codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=96, device=DEV)
+    x = (x.float().abs() + 0.1).half()
+    c = codes.to(torch.int32)
+    c = torch.where(c < 2, torch.full_like(c, 2), c)
+    c[::3, 0] = 1
+    codes = c.to(codes.dtype)
+    cb[..., :2, :] = float("inf")
+    w = vo.dequant_b(_np(codes), _np(cb)).astype(np.float64)
+    hit = np.zeros(N, bool)
+    hit[::3] = True
+    want = _np(x).astype(np.float64) @ w[~hit].T
+    ran = []
+    for variant in (cabi.VARIANT_AUTO, cabi.VARIANT_GENERIC, cabi.VARIANT_DECODE, cabi.VARIANT_PREFILL, cabi.VARIANT_PREFILL_NARROW,
+                    cabi.VARIANT_PREFILL_SMALL, cabi.VARIANT_PREFILL_SPLITK, cabi.VARIANT_WAVE_K):
+        _say("infinite codewords", M, K, N, v, entries, bits, G, cabi.VARIANT_NAMES[variant])
+        try:
+            y = _np(cabi.e2e_gemm_b_ws(x, codes, cb, variant=variant))
+        except cabi.VqGemmError as e:
+            assert e.code == -4
+            continue
+        assert np.isposinf(y[:, hit]).all(), (variant, int(np.isnan(y[:, hit]).sum()))
+        assert vo.rel_err(y[:, ~hit], want)[0] <= TOL, variant
+        ran.append(variant)
+    assert cabi.VARIANT_GENERIC in ran and (M > 64 or cabi.VARIANT_DECODE in ran)
+
+
 LLOYD_B = [
     # N, K, vec, entries, G: codebooks in several workgroups, entries nothing is assigned to, a last tile of entries cut short
     (512, 1024, 8, 256, 2),

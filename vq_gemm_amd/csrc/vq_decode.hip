@@ -196,14 +196,49 @@ __device__ __forceinline__ uint32_t codeword_addr(const LaneCodes<VEC, CodeT> &c
     }
 }
 
-// Issue the gathers of the operand of MFMA step s: codewords s*CPO .. s*CPO + CPO-1 of the slice.
+// Where a lane gathers from.  CUT: K may end inside a slice; the lane loads past its end then gather 16 zero bytes at LDS address
+// `zeros` whatever codes they hold, since against X's zeros a codeword that is infinite would make NaN of an infinite sum.  Which
+// lane loads these are is in registers, a mask that goes beside the shift and a base that is or-ed in, so that the loop has no test.
+template <int VEC, typename CodeT, bool REPL, bool CUT>
+struct GatherFrom {
+    uint32_t base;
+    __device__ __forceinline__ void set(uint32_t b, uint32_t, int, int) { base = b; }
+    __device__ __forceinline__ uint32_t addr(const LaneCodes<VEC, CodeT> &cw, int c) const { return codeword_addr<VEC, CodeT, REPL>(cw, c, base); }
+};
+
 template <int VEC, typename CodeT, bool REPL>
-__device__ __forceinline__ void gather_issue(Operand<VEC> &o, const LaneCodes<VEC, CodeT> &cw, int s, uint32_t base)
+struct GatherFrom<VEC, CodeT, REPL, true> {
+    typedef DecodeCfg<VEC, CodeT> C;
+    static constexpr int kBits = 8 * (int)sizeof(CodeT), kPerWord = 32 / kBits;
+    static constexpr int kShift = REPL ? 8 : VEC == 8 ? 4 : VEC == 4 ? 3 : 2;  // log2 of the LDS bytes of an entry
+    uint32_t base[C::LPT], mask[C::LPT];
+
+    // k: of the lane's first load
+    __device__ __forceinline__ void set(uint32_t b, uint32_t zeros, int k, int K)
+    {
+#pragma unroll
+        for (int t = 0; t < C::LPT; t++) {
+            const bool past = k + t * C::K_WAVE >= K;
+            base[t] = past ? zeros : b;
+            mask[t] = past ? 0u : ((1u << kBits) - 1) << kShift;
+        }
+    }
+    __device__ __forceinline__ uint32_t addr(const LaneCodes<VEC, CodeT> &cw, int c) const
+    {
+        const int t = c / C::CPL, ci = c % C::CPL, bit = (ci % kPerWord) * kBits;
+        const uint32_t word = cw.w[t][ci / kPerWord];
+        return ((bit < kShift ? word << (kShift - bit) : word >> (bit - kShift)) & mask[t]) | base[t];
+    }
+};
+
+// Issue the gathers of the operand of MFMA step s: codewords s*CPO .. s*CPO + CPO-1 of the slice.
+template <int VEC, typename CodeT, bool REPL, bool CUT>
+__device__ __forceinline__ void gather_issue(Operand<VEC> &o, const LaneCodes<VEC, CodeT> &cw, int s, const GatherFrom<VEC, CodeT, REPL, CUT> &from)
 {
     typedef DecodeCfg<VEC, CodeT> C;
 #pragma unroll
     for (int i = 0; i < Operand<VEC>::kPieces; i++)
-        lds_read_async(o.p[i], codeword_addr<VEC, CodeT, REPL>(cw, s * C::CPO + i, base));
+        lds_read_async(o.p[i], from.addr(cw, s * C::CPO + i));
 }
 
 // s_waitcnt for the vector-memory counter only (gfx9 encoding: vmcnt = simm16[15:14]:[3:0]).
@@ -310,8 +345,12 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     const int J = K / VEC;
     const int cb_slots = REPL ? entries * 16 : entries * kEntryBytes / 16;  // 16-byte slots of the LDS table
     uint4_t *cb_lds = reinterpret_cast<uint4_t *>(smem);
-    const uint32_t gather_base = REPL ? (lane % (256 / kEntryBytes)) * kEntryBytes : 0;
     const uint32_t red_base = red_off;
+    // zeros for the lane loads past the end of K: the pad of the first slot, which nothing else is written to but staged X
+    const uint32_t zeros = red_base + kSlotPitch - 16;
+    auto store_zeros = [&]() {
+        if (kAny && w == 0) reinterpret_cast<uint32_t *>(smem + zeros)[opaque(lane) & 3] = (uint32_t)opaque(0);
+    };
 
     // blockIdx.x picks the codebooks.  Either wgs_per_cb workgroups share the tiles_per_cb tiles
     // of one codebook (a contiguous range each: tiles_q, one more for the first tiles_r; quotient
@@ -337,7 +376,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // loads of a wave load are contiguous, [tile][slice][load][lane], so that a wave instruction
     // reads 64*LB consecutive bytes instead of 16 pieces of 4*LB.
     constexpr int kLoadPitch = PACKED ? 64 * C::LB : 4 * C::LB;  // bytes between the loads of a slice
-    // A lane load past the end of K (in a short last slice) reads the chunk's first codes instead, against zeros of X.
+    // A lane load past the end of K (in a short last slice) reads the row's first codes of the chunk instead and gathers zeros.
     constexpr bool kOneOffset = PACKED || !kAny;
     uint32_t voff[kOneOffset ? 1 : C::LPT];
     auto set_voff = [&]() {
@@ -360,6 +399,10 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // with the same result)
     auto tile_row = [&](int tile) { return kAny ? min(tile * kTileN, N - kTileN) : tile * kTileN; };
     const int chunk_bytes = n_waves * kSliceK / VEC * (int)sizeof(CodeT) * (PACKED ? kTileN : 1);
+    GatherFrom<VEC, CodeT, REPL, kAny> from;
+    auto set_gathers = [&]() {
+        from.set(REPL ? (lane % (256 / kEntryBytes)) * kEntryBytes : 0, zeros, (chunk * n_waves + w) * kSliceK + kq * C::K_LANE, K);
+    };
     auto load_unit = [&](int q, Codes (&cw)[TB]) {
 #pragma unroll
         for (int j = 0; j < TB; j++) {
@@ -473,16 +516,17 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     };
     stage_x();
     if (!codes_first) first_code_loads = load_first_units();
+    set_gathers();
     if (!(stage_over & kStageOverTable)) store_codebook();
+    if (!stage_over) store_zeros();
     wait_vmcnt_upto(first_code_loads);  // X staged (and everything older); the codes may still be in flight
     __syncthreads();  // pieces staged by the other waves
     pick_x();
     if (stage_over) {
         __syncthreads();  // every wave has picked up its X before the staging area is written again
-        if (stage_over & kStageOverTable) {
-            store_codebook();
-            __syncthreads();
-        }
+        if (stage_over & kStageOverTable) store_codebook();
+        store_zeros();
+        if (kAny || (stage_over & kStageOverTable)) __syncthreads();
     }
 
     // Partial results: slot (j, kq, m) = (j*4 + kq)*M + m for tile j of the unit; this lane writes
@@ -511,7 +555,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
                 // tile, and each is replaced by the next tile's as soon as it has been multiplied.
                 Operand<VEC> ops[kSteps];
 #pragma unroll
-                for (int s = 0; s < kSteps; s++) gather_issue<VEC, CodeT, REPL>(ops[s], cur[0], s, gather_base);
+                for (int s = 0; s < kSteps; s++) gather_issue(ops[s], cur[0], s, from);
 #pragma unroll
                 for (int i = 0; i < TB * kSteps; i++) {
                     const int j = i / kSteps, s = i % kSteps;
@@ -522,7 +566,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
                     acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.value(), xr[s], s == 0 ? c0 : acc[j], 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                     const int t = i + kSteps;
-                    if (t < TB * kSteps) gather_issue<VEC, CodeT, REPL>(o, cur[t / kSteps], t % kSteps, gather_base);
+                    if (t < TB * kSteps) gather_issue(o, cur[t / kSteps], t % kSteps, from);
                     // All gather addresses of the unit are computed: its ring slot takes the unit after next.
                     if (t == TB * kSteps - 1 || (TB == 1 && i == 0))
                         if (q + 2 < n_units) load_unit(q + 2, cur);
@@ -536,7 +580,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
                     if (j < nt) {
                         Operand<VEC> ops[kSteps];
 #pragma unroll
-                        for (int s = 0; s < kSteps; s++) gather_issue<VEC, CodeT, REPL>(ops[s], cur[j], s, gather_base);
+                        for (int s = 0; s < kSteps; s++) gather_issue(ops[s], cur[j], s, from);
 #pragma unroll
                         for (int s = 0; s < kSteps; s++) {
                             wait_lgkmcnt_upto((kSteps - 1 - s) * kPieces);
@@ -651,6 +695,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
         if constexpr (kAny) set_voff();
         // The first codes are requested before the table or X are replaced, to overlap the latencies.
         load_first_units();
+        if constexpr (kAny) set_gathers();
         __syncthreads();  // every gather from the old table has been consumed, every slot read
         // (a chunk that starts where X repeats has the X of the chunk before it, unless K cuts its last slice short)
         const bool new_x = n_chunks > 1 && (!kAny || n_waves * kSliceK != k_x || n_act != n_waves);
@@ -674,6 +719,10 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
             pick_x();
         }
         __syncthreads();  // X picked up before the slots (which the staging area may lie over) are written
+        if (kAny && new_x) {
+            store_zeros();
+            __syncthreads();
+        }
     }
 }
 

@@ -129,8 +129,13 @@ __global__ __launch_bounds__(512) void decode_general_kernel(const half_t *__res
     const int cb_lds_bytes = REPL ? entries * 256 : ((cb_bytes + 15) & ~15);
     uint8_t *cb_lds = smem;
     // Lane's copy of the entries in the replicated layout (0 in the plain one).
-    const uint8_t *cb_gather = smem + (REPL ? (lane % (256 / kEntryBytes)) * kEntryBytes : 0);
-    float4_t *red = reinterpret_cast<float4_t *>(smem + cb_lds_bytes);
+    const uint32_t copy_off = REPL ? (lane % (256 / kEntryBytes)) * kEntryBytes : 0;
+    // 16 zero bytes behind the table: what a lane gathers past the end of K (its codes are 0 there, and entry 0 against X's zeros
+    // would be NaN if it is infinite)
+    float4_t *red = reinterpret_cast<float4_t *>(smem + cb_lds_bytes + 16);
+    auto store_zeros = [&]() {
+        if (threadIdx.x == 0) *reinterpret_cast<uint4_t *>(cb_lds + cb_lds_bytes) = uint4_t{0u, 0u, 0u, 0u};
+    };
 
     // Balanced contiguous split of the tiles over the workgroups: tiles_q each, one more for the
     // first tiles_r (quotient and remainder of tiles / workgroups, computed by the host).
@@ -165,6 +170,7 @@ __global__ __launch_bounds__(512) void decode_general_kernel(const half_t *__res
         }
     };
     auto load_codebook = [&](int g) {
+        store_zeros();
         if constexpr (REPL) {
             // 16-byte slot i of the table belongs to entry i / 16; it holds 16 / entry_bytes copies.
             // All loads are issued before the first write so that their latencies overlap.
@@ -221,6 +227,7 @@ __global__ __launch_bounds__(512) void decode_general_kernel(const half_t *__res
         }
     };
     auto store_codebook = [&]() {
+        store_zeros();
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int i = threadIdx.x + j * blockDim.x;
@@ -295,10 +302,15 @@ __global__ __launch_bounds__(512) void decode_general_kernel(const half_t *__res
 #pragma unroll
             for (int t = 0; t < C::LPT; t++) cw[t] = cwq[u][t];
             if (q + PF < q_end) load_unit(q + PF, cwq[u]);
-            if (n_chunks > 1) load_x(chunk * chunk_k + wave * kSliceK);
+            const int k0 = chunk * chunk_k + wave * kSliceK;
+            if (n_chunks > 1) load_x(k0);
+            uint32_t k_gather = (uint32_t)k0, gather_base[C::LPT];
+            asm volatile("" : "+s"(k_gather));  // (the bases are computed here and not kept from unit to unit)
+#pragma unroll
+            for (int t = 0; t < C::LPT; t++) gather_base[t] = step_k((int)k_gather, t * C::SPL) < K ? copy_off : (uint32_t)cb_lds_bytes;
 #pragma unroll
             for (int s = 0; s < kSteps; s++) {
-                const half8_t a = gather_operand<VEC, CodeT, kStride>(cb_gather, cw[s / C::SPL], (s % C::SPL) * C::CPO);
+                const half8_t a = gather_operand<VEC, CodeT, kStride>(smem + gather_base[s / C::SPL], cw[s / C::SPL], (s % C::SPL) * C::CPO);
                 acc[s & 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, xr[s], acc[s & 3], 0, 0, 0);
                 // Bound how far the scheduler hoists gathers ahead of their MFMAs (register pressure).
                 if (STEPS > 16 && (s & 7) == 7) __builtin_amdgcn_sched_barrier(0);
@@ -377,7 +389,7 @@ hipError_t launch_decode_steps(const ProblemB &p, hipStream_t s)
     // Replicated codebook (one 256-byte bank row per entry, <= 64 KB): worth its fill time only
     // when the workgroup gathers from it for several tiles.
     const bool repl = p.entries <= 256 && tiles_per_wg >= 4;
-    const size_t base = (repl ? (size_t)p.entries * 256 : (size_t)((cb_bytes + 15) & ~15)) +
+    const size_t base = (repl ? (size_t)p.entries * 256 : (size_t)((cb_bytes + 15) & ~15)) + 16 +
                         (size_t)2 * n_waves * 64 * sizeof(float4_t);
     const size_t stage = (size_t)n_waves * p.M * (kSliceK * 2 + 16);
     size_t smem = base;
