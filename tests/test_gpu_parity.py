@@ -789,6 +789,53 @@ def test_registered_op_traces_and_matches_eager():
     assert torch.equal(got, want)
 
 
+def test_layer_calls_are_seen_by_subclasses_and_function_modes(monkeypatch):
+    """The layers' direct calls step aside for whatever overrides __torch_function__: a mode and a subclass see the registered
+    operator, a subclass comes back as one.  A default device is no reason to leave them."""
+    from torch.overrides import TorchFunctionMode
+    from vq_gemm_amd.nn import VQGatedMLP, VQLinear
+
+    class Sub(torch.Tensor):
+        pass
+
+    class Off(torch.Tensor):
+        __torch_function__ = torch._C._disabled_torch_function_impl
+
+    class Seen(TorchFunctionMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    x, codes, cb = make_problem(ProblemSpec("s", GEOM_B, 5, 512, 768, 8, 256, 1, 8), seed=4, device=DEV)
+    _, dcodes, _ = make_problem(ProblemSpec("s", GEOM_B, 5, 384, 512, 8, 256, 1, 8), seed=5, device=DEV)
+    lin, mlp = VQLinear(codes, cb), VQGatedMLP(VQLinear(codes, cb), VQLinear(dcodes, cb), interleaved=True)
+    packed = VQLinear(codes, cb).prepack_for_decode()
+    for layer, op in ((lin, "vq_linear"), (packed, "vq_linear"), (mlp, "vq_gated_linear")):
+        _say("watched layer calls", op)
+        want = layer(x)
+        assert type(want) is torch.Tensor and type(layer(x.as_subclass(Off))) is torch.Tensor
+        y = layer(x.as_subclass(Sub))
+        assert type(y) is Sub and torch.equal(y.as_subclass(torch.Tensor), want)
+        with Seen() as mode:
+            y = layer(x)
+        assert type(y) is torch.Tensor and torch.equal(y, want) and any(op in n for n in mode.names), mode.names
+    lin.codes = codes.as_subclass(Sub)
+    assert type(lin(x)) is Sub
+    lin.codes = codes
+    def not_here(x):
+        raise AssertionError("a default device sent the layer to the operator")
+    monkeypatch.setattr(lin, "_forward_op", not_here)
+    with torch.device(DEV):
+        assert torch.equal(lin(x), packed(x))
+    with Seen() as mode:
+        decoded = cabi.dequant_b(codes, cb)
+    assert mode.names and torch.equal(decoded, cabi.dequant_b(codes, cb))
+
+
 def test_random_shapes_agree_across_kernels():
     """Seeded random shapes (ragged M and N, rows per codebook that are no multiple of anything, one
     to many K stages, with and without bias): the scalar kernel and the automatic choice against the

@@ -6,8 +6,12 @@
 // costs: as a Python custom operator over ctypes it took 26 us per call on 4096 x 4096 with one row of X (the kernel:
 // 3.7).  The operators are therefore registered here, and the layers (vq_gemm_amd/nn.py) call `linear` and `gated` below
 // without going through the dispatcher at all; those two step aside (return None) whenever something else is to see
-// the call - a fake or wrapped tensor, a dispatch mode, a tracer - and the layer then calls the registered operator.
+// the call - a fake or wrapped tensor, a tensor subclass, a dispatch or function mode, a tracer - and the layer then calls
+// the registered operator.
 #include <torch/extension.h>
+#include <torch/csrc/PyInterpreter.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
@@ -239,20 +243,59 @@ constexpr char kLinear[] = "vq_gemm_amd::vq_linear", kLinearPacked[] = "vq_gemm_
 
 // ---- the layers' direct calls ---------------------------------------------------------------------------------
 
+// Whether a function mode is to see the call.  A default device (torch.set_default_device, `with torch.device(...)`) is such
+// a mode too, but looks at factory functions only.
+PyObject *default_device_mode = nullptr, *no_torch_function = nullptr;  // its class, and what a class without an override has; set on loading
+bool function_mode_watches()
+{
+    if (!at::impl::torch_function_mode_enabled()) return false;
+    for (int64_t i = 0; i < at::impl::PythonTorchFunctionTLS::stack_len(); i++)
+        if ((PyObject *)Py_TYPE(at::impl::PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter())) != default_device_mode) return true;
+    return false;
+}
+
+// A tensor whose class overrides __torch_function__.
+bool subclass_watches(const Tensor &t)
+{
+    const py::object o = py::cast(t);
+    if (THPVariable_CheckTypeExact(Py_TYPE(o.ptr()))) return false;
+    if (at::impl::PythonTorchFunctionTLS::get_disabled_state() != at::impl::TorchFunctionDisabledState::ENABLED) return false;
+    return py::object(o.attr("__torch_function__")).ptr() != no_torch_function;
+}
+
+// `plain_call` for a call from Python on these operands (those that are there at all).
+bool plain_python_call(std::initializer_list<const Tensor *> operands)
+{
+    if (function_mode_watches()) return false;
+    for (const Tensor *t : operands)
+        if (t->defined() && (!plain_call(*t) || subclass_watches(*t))) return false;
+    return (*operands.begin())->defined();
+}
+
+const Tensor &given(const OptTensor &t)
+{
+    static const Tensor none;
+    return t.has_value() ? *t : none;
+}
+
 // packed: `codes` are in the packed layout (a single stage)
 py::object linear(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias, int64_t k_repeat, bool packed)
 {
-    if (!plain_call(x)) return py::none();
+    if (!plain_python_call({&x, &codes, &codebook, &given(bias)})) return py::none();
     TORCH_CHECK_VALUE(!packed || k_repeat == 1, "linear: additive stages have no packed layout");
-    RECORD_FUNCTION("vq_gemm_amd::vq_linear", c10::ArrayRef<const c10::IValue>());
-    return py::cast(linear_impl(x, codes, codebook, bias, k_repeat, packed ? VQGEMM_VARIANT_DECODE_PACKED : VQGEMM_VARIANT_AUTO));
+    Tensor y;
+    {
+        RECORD_FUNCTION("vq_gemm_amd::vq_linear", c10::ArrayRef<const c10::IValue>());
+        y = linear_impl(x, codes, codebook, bias, k_repeat, packed ? VQGEMM_VARIANT_DECODE_PACKED : VQGEMM_VARIANT_AUTO);
+    }
+    return py::cast(y);
 }
 
 // Whether a layer that holds both layouts of its codes hands the packed one over for x (what is wrong with x the call itself says;
 // the kernel of the packed layout takes no operands that begin anywhere).
 bool takes_packed(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
 {
-    if (!plain_call(x) || x.dim() < 1 || codes.dim() != 2 || (codebook.dim() != 2 && codebook.dim() != 3) || !aligned16(codebook)) return false;
+    if (!plain_python_call({&x, &codes, &codebook, &given(bias)}) || x.dim() < 1 || codes.dim() != 2 || (codebook.dim() != 2 && codebook.dim() != 3) || !aligned16(codebook)) return false;
     if (bias.has_value() && bias->defined() && (reinterpret_cast<uintptr_t>(bias->data_ptr()) & 7) != 0) return false;
     const int64_t vec = codebook.size(-1), K = codes.size(1) * vec;
     if (K == 0 || x.size(-1) != K) return false;
@@ -263,9 +306,13 @@ bool takes_packed(const Tensor &x, const Tensor &codes, const Tensor &codebook, 
 
 py::object gated(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
 {
-    if (!plain_call(x)) return py::none();
-    RECORD_FUNCTION("vq_gemm_amd::vq_gated_linear", c10::ArrayRef<const c10::IValue>());
-    return py::cast(gated_impl(x, codes, codebook, bias));
+    if (!plain_python_call({&x, &codes, &codebook, &given(bias)})) return py::none();
+    Tensor y;
+    {
+        RECORD_FUNCTION("vq_gemm_amd::vq_gated_linear", c10::ArrayRef<const c10::IValue>());
+        y = gated_impl(x, codes, codebook, bias);
+    }
+    return py::cast(y);
 }
 
 // ---- the codec ------------------------------------------------------------------------------------------------
@@ -274,7 +321,7 @@ py::object gated(const Tensor &x, const Tensor &codes, const Tensor &codebook, c
 // Python (11 of the 12 us of a call on a small matrix); None sends the caller down that path, which says what is wrong.
 bool codec_operands(const Tensor &m, const Tensor &codebook, int64_t per_column)
 {
-    return plain_call(m) && m.dim() == 2 && m.is_contiguous() && codebook.is_cuda() && codebook.device() == m.device() && codebook.is_contiguous() &&
+    return plain_python_call({&m, &codebook}) && m.dim() == 2 && m.is_contiguous() && codebook.is_cuda() && codebook.device() == m.device() && codebook.is_contiguous() &&
            codebook.scalar_type() == at::kHalf && (codebook.dim() == 2 || codebook.dim() == 3) && codebook.size(-1) > 0 &&
            m.device().index() == c10::hip::current_device() && (m.size(1) * per_column) % codebook.size(-1) == 0 &&
            (codebook.dim() == 2 || (codebook.size(0) > 0 && m.size(0) % codebook.size(0) == 0));
@@ -285,10 +332,14 @@ py::object encode(const Tensor &w, const Tensor &codebook)
     if (!codec_operands(w, codebook, 1) || w.scalar_type() != at::kHalf) return py::none();
     const int64_t N = w.size(0), K = w.size(1), vec = codebook.size(-1), entries = codebook.size(-2);
     const int bits = entries <= 256 ? 8 : 16;
-    Tensor codes = at::detail::empty_cuda({N, K / vec}, bits == 8 ? at::kByte : at::kUInt16, w.device(), c10::nullopt);
-    if (vqgemm_encode_b(w.data_ptr(), codebook.data_ptr(), codes.data_ptr(), N, K, (int)vec, (int)entries,
-                        codebook.dim() == 3 ? (int)codebook.size(0) : 1, bits, stream_of(w)) != 0)
-        return py::none();
+    Tensor codes;
+    int rc;
+    {
+        codes = at::detail::empty_cuda({N, K / vec}, bits == 8 ? at::kByte : at::kUInt16, w.device(), c10::nullopt);
+        rc = vqgemm_encode_b(w.data_ptr(), codebook.data_ptr(), codes.data_ptr(), N, K, (int)vec, (int)entries,
+                             codebook.dim() == 3 ? (int)codebook.size(0) : 1, bits, stream_of(w));
+    }
+    if (rc != 0) return py::none();
     return py::cast(codes);
 }
 
@@ -297,10 +348,14 @@ py::object dequant(const Tensor &codes, const Tensor &codebook)
     const bool u8 = codes.scalar_type() == at::kByte;
     if ((!u8 && codes.scalar_type() != at::kUInt16) || !codec_operands(codes, codebook, codebook.dim() > 0 ? codebook.size(-1) : 1)) return py::none();
     const int64_t N = codes.size(0), vec = codebook.size(-1), K = codes.size(1) * vec;
-    Tensor w = at::detail::empty_cuda({N, K}, at::kHalf, codes.device(), c10::nullopt);
-    if (vqgemm_dequant_b(codes.data_ptr(), codebook.data_ptr(), w.data_ptr(), N, K, (int)vec, (int)codebook.size(-2),
-                         codebook.dim() == 3 ? (int)codebook.size(0) : 1, u8 ? 8 : 16, stream_of(codes)) != 0)
-        return py::none();
+    Tensor w;
+    int rc;
+    {
+        w = at::detail::empty_cuda({N, K}, at::kHalf, codes.device(), c10::nullopt);
+        rc = vqgemm_dequant_b(codes.data_ptr(), codebook.data_ptr(), w.data_ptr(), N, K, (int)vec, (int)codebook.size(-2),
+                              codebook.dim() == 3 ? (int)codebook.size(0) : 1, u8 ? 8 : 16, stream_of(codes));
+    }
+    if (rc != 0) return py::none();
     return py::cast(w);
 }
 
@@ -326,16 +381,22 @@ py::object kmeans(const Tensor &w, const Tensor &pick, int64_t vec, int64_t entr
     TORCH_CHECK_VALUE(w.is_cuda() && w.scalar_type() == at::kHalf && w.is_contiguous() && pick.scalar_type() == at::kInt &&
                           pick.numel() == books * entries && pick.is_contiguous() && vec > 0 && K % vec == 0 && books > 0 && N % books == 0,
                       "kmeans: w fp16 [N, K] on the GPU, pick int32 [books, entries]");
+    if (!plain_python_call({&w})) return py::none();
     const int64_t need = vqgemm_kmeans_workspace_bytes_b(N, K, (int)vec, (int)entries, (int)books, (int)code_bits);
     if (need < 0 || (reinterpret_cast<uintptr_t>(w.data_ptr()) & 7) != 0) return py::none();
     const c10::OptionalDeviceGuard guard(w.device());
-    const Tensor pick_d = pick.to(w.device());
     auto on_device = [&](at::IntArrayRef shape, at::ScalarType t) { return at::detail::empty_cuda(shape, t, w.device(), c10::nullopt); };
-    Tensor codes = on_device({N, K / vec}, code_bits == 8 ? at::kByte : at::kUInt16);
-    Tensor codebook = on_device({books, entries, vec}, at::kHalf), errors = on_device({iters + 1}, at::kDouble), ws = on_device({need}, at::kByte);
-    check_rc(vqgemm_kmeans_b(w.data_ptr(), pick_d.data_ptr<int32_t>(), codes.data_ptr(), codebook.data_ptr(), errors.data_ptr<double>(), N, K,
-                             (int)vec, (int)entries, (int)books, (int)code_bits, (int)iters, ws.data_ptr(), need, stream_of(w)),
-             "kmeans");
+    Tensor codes, codebook, errors;
+    {
+        const Tensor pick_d = pick.to(w.device());
+        codes = on_device({N, K / vec}, code_bits == 8 ? at::kByte : at::kUInt16);
+        codebook = on_device({books, entries, vec}, at::kHalf);
+        errors = on_device({iters + 1}, at::kDouble);
+        const Tensor ws = on_device({need}, at::kByte);
+        check_rc(vqgemm_kmeans_b(w.data_ptr(), pick_d.data_ptr<int32_t>(), codes.data_ptr(), codebook.data_ptr(), errors.data_ptr<double>(), N, K,
+                                 (int)vec, (int)entries, (int)books, (int)code_bits, (int)iters, ws.data_ptr(), need, stream_of(w)),
+                 "kmeans");
+    }
     return py::make_tuple(codes, codebook, errors);
 }
 
@@ -367,6 +428,8 @@ TORCH_LIBRARY_IMPL(vq_gemm_amd, AutogradCUDA, m)
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
+    no_torch_function = py::object(py::module_::import("torch._C").attr("_disabled_torch_function_impl")).release().ptr();
+    default_device_mode = py::object(py::module_::import("torch.utils._device").attr("DeviceContext")).release().ptr();
     m.def("linear", &linear, "x @ W.T (+ bias) on plain GPU tensors; None where the registered operator is to be called instead");
     m.def("takes_packed", &takes_packed, "whether `linear` does best with the packed layout of the codes");
     m.def("first_of_permutations", &first_of_permutations, "the first elements of seeded random permutations");
