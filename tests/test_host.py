@@ -256,3 +256,30 @@ def test_the_packed_layout_is_taken_where_the_automatic_choice_takes_its_kernel(
     assert not cabi.packed_preferred_b(4, 320, 8192, 8, 256, 1, 8)   # no packed layout for this K
     assert not cabi.packed_preferred_b(0, 4096, 8192, 8, 256, 1, 8)
     assert cabi.lib().vqgemm_packed_preferred_b(4, 60, 8, 8, 256, 1, 8) < 0
+
+
+def test_native_calls_let_other_threads_run():
+    """A long call of the compiled extension (the starts of twelve permutations of 2^24) works without the GIL."""
+    import threading
+    import time
+    from vq_gemm_amd.torch_ops import native
+    ran, stop = [], threading.Event()
+
+    def beat():
+        while not stop.is_set():
+            ran.append(time.perf_counter())
+            time.sleep(0.001)
+
+    other = threading.Thread(target=beat)
+    other.start()
+    try:
+        while not ran:
+            time.sleep(0.001)
+        t0 = time.perf_counter()
+        native.first_of_permutations(1 << 24, 16, 12, 7)
+        t1 = time.perf_counter()
+    finally:
+        stop.set()
+        other.join()
+    # (with the GIL held the other thread can run right at the edges of the call, not between)
+    assert any(t0 + 0.25 * (t1 - t0) < t < t0 + 0.75 * (t1 - t0) for t in ran), (t1 - t0, len(ran))

@@ -7,7 +7,8 @@
 // 3.7).  The operators are therefore registered here, and the layers (vq_gemm_amd/nn.py) call `linear` and `gated` below
 // without going through the dispatcher at all; those two step aside (return None) whenever something else is to see
 // the call - a fake or wrapped tensor, a tensor subclass, a dispatch or function mode, a tracer - and the layer then calls
-// the registered operator.
+// the registered operator.  The direct calls work without the GIL, as the operators do: a launch that waits on a full
+// queue must not hold up the other threads.
 #include <torch/extension.h>
 #include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -285,6 +286,7 @@ py::object linear(const Tensor &x, const Tensor &codes, const Tensor &codebook, 
     TORCH_CHECK_VALUE(!packed || k_repeat == 1, "linear: additive stages have no packed layout");
     Tensor y;
     {
+        const py::gil_scoped_release no_gil;
         RECORD_FUNCTION("vq_gemm_amd::vq_linear", c10::ArrayRef<const c10::IValue>());
         y = linear_impl(x, codes, codebook, bias, k_repeat, packed ? VQGEMM_VARIANT_DECODE_PACKED : VQGEMM_VARIANT_AUTO);
     }
@@ -309,6 +311,7 @@ py::object gated(const Tensor &x, const Tensor &codes, const Tensor &codebook, c
     if (!plain_python_call({&x, &codes, &codebook, &given(bias)})) return py::none();
     Tensor y;
     {
+        const py::gil_scoped_release no_gil;
         RECORD_FUNCTION("vq_gemm_amd::vq_gated_linear", c10::ArrayRef<const c10::IValue>());
         y = gated_impl(x, codes, codebook, bias);
     }
@@ -335,6 +338,7 @@ py::object encode(const Tensor &w, const Tensor &codebook)
     Tensor codes;
     int rc;
     {
+        const py::gil_scoped_release no_gil;
         codes = at::detail::empty_cuda({N, K / vec}, bits == 8 ? at::kByte : at::kUInt16, w.device(), c10::nullopt);
         rc = vqgemm_encode_b(w.data_ptr(), codebook.data_ptr(), codes.data_ptr(), N, K, (int)vec, (int)entries,
                              codebook.dim() == 3 ? (int)codebook.size(0) : 1, bits, stream_of(w));
@@ -351,6 +355,7 @@ py::object dequant(const Tensor &codes, const Tensor &codebook)
     Tensor w;
     int rc;
     {
+        const py::gil_scoped_release no_gil;
         w = at::detail::empty_cuda({N, K}, at::kHalf, codes.device(), c10::nullopt);
         rc = vqgemm_dequant_b(codes.data_ptr(), codebook.data_ptr(), w.data_ptr(), N, K, (int)vec, (int)codebook.size(-2),
                               codebook.dim() == 3 ? (int)codebook.size(0) : 1, u8 ? 8 : 16, stream_of(codes));
@@ -388,6 +393,7 @@ py::object kmeans(const Tensor &w, const Tensor &pick, int64_t vec, int64_t entr
     auto on_device = [&](at::IntArrayRef shape, at::ScalarType t) { return at::detail::empty_cuda(shape, t, w.device(), c10::nullopt); };
     Tensor codes, codebook, errors;
     {
+        const py::gil_scoped_release no_gil;
         const Tensor pick_d = pick.to(w.device());
         codes = on_device({N, K / vec}, code_bits == 8 ? at::kByte : at::kUInt16);
         codebook = on_device({books, entries, vec}, at::kHalf);
@@ -432,7 +438,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     default_device_mode = py::object(py::module_::import("torch.utils._device").attr("DeviceContext")).release().ptr();
     m.def("linear", &linear, "x @ W.T (+ bias) on plain GPU tensors; None where the registered operator is to be called instead");
     m.def("takes_packed", &takes_packed, "whether `linear` does best with the packed layout of the codes");
-    m.def("first_of_permutations", &first_of_permutations, "the first elements of seeded random permutations");
+    m.def("first_of_permutations", &first_of_permutations, py::call_guard<py::gil_scoped_release>(), "the first elements of seeded random permutations");
     m.def("kmeans", &kmeans, "Lloyd iterations on the device; None where the codebook is too large for them");
     m.def("encode", &encode, "nearest-codeword codes; None where cabi.encode_b is to check the operands one by one");
     m.def("dequant", &dequant, "codes and codebook to fp16 likewise");
