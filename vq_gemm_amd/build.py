@@ -88,9 +88,10 @@ def _newer(target: str, deps) -> bool:
 # budget the rest by hand; a spill there means the budget was missed.  No kernel of this library
 # has a reason to spill or to use scratch memory, so every kernel of every source is checked:
 # zero VGPR spills and zero bytes of private segment.  (A scalar register that the compiler parks in a lane
-# of a vector register - an "SGPR spill" that never touches memory - is tolerated in small numbers: it costs
-# one lane write and read outside the hand-scheduled loops.)
-MAX_SGPR_SPILLS = 8
+# of a vector register - an "SGPR spill" that never touches memory - costs one lane write and read outside the
+# hand-scheduled loops.  Only the instances of the batched decode kernel that take a cut K, a cut N or a repeated X
+# have any: 20 kernels, 6 at most.)
+MAX_SGPR_SPILLS = 6
 
 
 def _check_no_spills(asm_path: str) -> None:
