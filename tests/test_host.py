@@ -283,3 +283,12 @@ def test_native_calls_let_other_threads_run():
         other.join()
     # (with the GIL held the other thread can run right at the edges of the call, not between)
     assert any(t0 + 0.25 * (t1 - t0) < t < t0 + 0.75 * (t1 - t0) for t in ran), (t1 - t0, len(ran))
+
+
+def test_split_k_is_asked_for_where_it_was_measured_faster():
+    """The workspace the automatic choice asks for: none where the wave-K kernel was measured at 0.75 to 0.85 of split K's time, slices
+    of K where it was the other way round (short K with a middling M here, few columns of a long K there)."""
+    for M, K, N, v, e, bits in ((203, 2816, 7040, 8, 256, 8), (489, 3072, 3328, 8, 256, 8), (72, 2304, 8832, 4, 4096, 16), (438, 2944, 3072, 4, 4096, 16)):
+        assert cabi.workspace_bytes_b(M, K, N, v, e, 1, bits) == 0, (M, K, N)
+    for M, K, N, v, e, bits in ((3028, 11264, 640, 8, 256, 8), (954, 14080, 1920, 8, 256, 8), (657, 13376, 1040, 8, 256, 8), (118, 11008, 14080, 4, 4096, 16)):
+        assert cabi.workspace_bytes_b(M, K, N, v, e, 1, bits) > 0, (M, K, N)

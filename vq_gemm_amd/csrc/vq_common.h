@@ -192,7 +192,7 @@ hipError_t launch_wave_k_a(const ProblemA &p, hipStream_t s);
 bool wave_k_b_supports(const ProblemB &p);
 double wave_k_b_cost_us(const ProblemB &p);
 // whether the automatic choice takes this kernel (`t_other`: what the best of the others is expected to take, by their cost models)
-bool wave_k_b_preferred(const ProblemB &p, double t_other);
+bool wave_k_b_preferred(const ProblemB &p, double t_other, double margin);
 int wave_k_b_tile(const ProblemB &p);   // the tile its cost model expects to be fastest
 hipError_t launch_wave_k_b(const ProblemB &p, hipStream_t s, int tile = 0);   // (0: that one)
 
@@ -274,8 +274,8 @@ struct Tuning {
     // expected below this share of the best single plan (0: never; 1000 and more: wherever the plan exists)
     double tail_split_margin = 0.93;
     // split K over 128x128 tiles: the second launch, and the partial sums written and read once (microseconds per MB of
-    // partial sums)
-    double splitk_fixed_us = 4.5;
+    // partial sums): 4 % off either way over 193 launches of 2 to 12 slices
+    double splitk_fixed_us = 7.5;
     double splitk_us_per_partial_mb = 0.15;
     // 2 .. 16: VQGEMM_VARIANT_PREFILL_SPLITK takes this many slices where the shape allows (for measurements); 0: the cost model's
     double splitk_force_splits = 0.0;

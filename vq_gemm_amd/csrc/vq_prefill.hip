@@ -1001,7 +1001,8 @@ TailSplitPlan prefill_tail_split_plan(const ProblemB &p)
         // (Tuning::splitk_force_splits, for measurements and tests: that many slices where the shape allows)
         const int forced = (int)tuning().splitk_force_splits;
         if (forced >= 2 && prefill_splitk_supports(tail, forced)) sp = forced;
-        const double t = tile_cost_us(p, bn, cols_head) + t_tail + 3.0;
+        // (the further launch: 3 us, where K is split in splitk_fixed_us already)
+        const double t = tile_cost_us(p, bn, cols_head) + t_tail + (sp > 1 ? 0.0 : 3.0);
         if (t < best.cost_us) best = {true, head_tile, n_split, sp, t, sp > 1 ? prefill_splitk_workspace_bytes(tail, sp) : 0};
     }
     return best;

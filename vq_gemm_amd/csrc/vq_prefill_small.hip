@@ -533,7 +533,8 @@ bool prefill_splitk_supports(const ProblemB &p, int splits)
 
 // The number of slices of K (1: none) that the cost model expects to be fastest with 128x128 tiles, and its time.
 // A slice is a workgroup of its own: `splits` times the tiles, each over K / splits; on top of that the second launch
-// and the partial sums written and read once (Tuning::splitk_fixed_us, splitk_us_per_partial_mb).
+// and the partial sums written and read once (Tuning::splitk_fixed_us, splitk_us_per_partial_mb).  A stage of a slice takes
+// 0.87 (8-bit codes) or 0.97 of what small_tiles_us has for it, the whole 4 % off either way over 193 measured launches.
 int prefill_splitk_choice(const ProblemB &p, double *cost_us, int min_splits)
 {
     int best = min_splits <= 1 ? 1 : 0;
@@ -546,7 +547,8 @@ int prefill_splitk_choice(const ProblemB &p, double *cost_us, int min_splits)
     }
     for (const int sp : {2, 3, 4, 6, 8, 12, 16}) {
         if (!prefill_splitk_supports(p, sp)) break;
-        const double main_us = small_tiles_us(p, tiles * sp, p.K / sp);   // the slices: sp times the tiles over K / sp
+        const double ends_us = small_tiles_us(p, tiles * sp, 0);   // the slices: sp times the tiles over K / sp
+        const double main_us = ends_us + (p.code_bits == 8 ? 0.87 : 0.97) * (small_tiles_us(p, tiles * sp, p.K / sp) - ends_us);
         const double fix_us = tn.splitk_fixed_us + tn.splitk_us_per_partial_mb * (double)sp * p.M * p.N * 4e-6;
         if (main_us + fix_us < best_us) {
             best_us = main_us + fix_us;

@@ -517,13 +517,14 @@ struct WaveKTile {
 };
 
 // Microseconds a launch is expected to take (a tenth off, either way): the tiles go over the compute units in rounds.
-inline double wave_k_tile_cost_us(const WaveKTile &t, int M, int K, int N, double bytes)
+// wait: how much longer a unit takes than fitted.
+inline double wave_k_tile_cost_us(const WaveKTile &t, int M, int K, int N, double bytes, double wait = 1.0)
 {
     const int cus = device_cu_count(), tm = t.tile / 10 * 16, tn = t.tile % 10 * 16;
     const int64_t tiles = (int64_t)((M + tm - 1) / tm) * ((N + tn - 1) / tn);
     const int64_t rounds = (tiles + cus - 1) / cus;
     const double busy = (double)tiles / (double)(rounds * cus);
-    const double tiles_us = (double)rounds * (t.fixed_us + (K / (double)kStepK) * (t.idle_clk + t.busy_clk * busy) / 2100.0);
+    const double tiles_us = (double)rounds * (t.fixed_us + (K / (double)kStepK) * (t.idle_clk + t.busy_clk * busy) * wait / 2100.0);
     const double memory_us = bytes / 4e6;
     return 2.0 + (tiles_us > memory_us ? tiles_us : memory_us);
 }

@@ -1,6 +1,8 @@
 // The kernels of vq_wave_k.h for geometry B.
 #include "vq_wave_k.h"
 
+#include <cmath>
+
 namespace vq {
 
 namespace {
@@ -50,13 +52,24 @@ WaveKPlan plan_b(const ProblemB &p)
     // (16-bit codes bring tables whose entries collide more often)
     constexpr WaveKTile kTiles8[] = {{12, 2.2, 39, 14}, {14, 2.5, 65, 28}, {18, 3.2, 118, 62}, {22, 2.4, 44, 19}, {24, 3.0, 68, 29}, {44, 4.0, 95, 68}, {48, 6.1, 180, 165}};
     constexpr WaveKTile kTiles16[] = {{12, 2.6, 45, 19}, {14, 2.8, 79, 59}, {18, 3.0, 169, 200}, {22, 2.7, 52, 24}, {24, 3.0, 91, 45}, {44, 3.5, 124, 112}, {48, 5.9, 214, 182}};
+    // An X of more than the 4 MB of an XCD's L2 keeps the units waiting, 15 % longer from 16 MB on whatever the tile, and tiles of
+    // 64 x 64 in several rounds another 30 % from 1500 rows on: M = 2168, K = 7808, N = 1024 takes 95 us, M = 3028, K = 11264, N = 640
+    // 98 us, expected 64 without the two.  Over 192 shapes of M 66 to 4002 measured and expected time differ by 10 % (15 % without).
+    const double octaves = std::log2(2.0 * p.M * p.K / 2e6);
+    const double wait = 1.0 + 0.15 * (octaves < 0.0 ? 0.0 : octaves > 3.0 ? 1.0 : octaves / 3.0);
+    const double wait_rows = 1.0 + 0.3 * (p.M < 1000 ? 0.0 : p.M > 1500 ? 1.0 : (p.M - 1000) / 500.0);
+    const bool rounds = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) > device_cu_count();
+    const double bytes = (double)p.K * p.N * F::CSZ / F::VEC + 2.0 * (double)p.M * (p.K + p.N);
     WaveKPlan best = {0, 0, 1e30};
+    double best_us = 1e30;
     for (const WaveKTile &t : F::CSZ == 1 ? kTiles8 : kTiles16) {
         if (forced > 0 && forced != t.tile) continue;
         if (!fits<F>(p, t.tile)) continue;
-        const double bytes = (double)p.K * p.N * F::CSZ / F::VEC + 2.0 * (double)p.M * (p.K + p.N);
-        const double us = wave_k_tile_cost_us(t, p.M, p.K, p.N, bytes);
-        if (us < best.cost_us) best = {t.tile / 10, t.tile % 10, us};
+        const double w = t.tile == 44 && rounds ? wait_rows : 1.0, us = wave_k_tile_cost_us(t, p.M, p.K, p.N, bytes, w);
+        if (us < best_us) {
+            best_us = us;
+            best = {t.tile / 10, t.tile % 10, wave_k_tile_cost_us(t, p.M, p.K, p.N, bytes, w * wait)};
+        }
     }
     return best;
 }
@@ -128,7 +141,7 @@ int wave_k_b_tile(const ProblemB &p)
 // path would take its streaming or its general kernel it keeps up to 16 rows.  Above, the tiled kernels, by more than the models' error.
 // (us, before -> now: M = 8, K = 640, N = 22912 23.8 -> 6.1; M = 44, K = 704, N = 21888, 4-vectors 32.3 -> 11.0; M = 100,
 // K = 1408, N = 3500 11.9 -> 6.5; M = 256, K = N = 4096, 16-bit codes 26.5 -> 17.6; M = 451, K = 1152, N = 1376 18.2 -> 8.0.)
-bool wave_k_b_preferred(const ProblemB &p, double t_other)
+bool wave_k_b_preferred(const ProblemB &p, double t_other, double margin)
 {
     const int force = (int)tuning().wave_k_force;
     if (force == 2 || !wave_k_b_supports(p)) return false;
@@ -141,7 +154,7 @@ bool wave_k_b_preferred(const ProblemB &p, double t_other)
         // the caches hold, where it is the other way round, they are 3.8 and 2.1 %)
         return wave_k_b_cost_us(p) < (p.gated ? 1.15 : p.M <= 16 ? 0.89 : 0.97) * t_decode;
     }
-    return wave_k_b_cost_us(p) < 0.95 * t_other;
+    return wave_k_b_cost_us(p) < margin * t_other;
 }
 
 hipError_t launch_wave_k_b(const ProblemB &p, hipStream_t s, int tile)
