@@ -310,8 +310,7 @@ def main():
         res = {
             "M": spec.M, "K": spec.K, "N": spec.N, "vec": spec.vec, "code_bits": spec.code_bits,
             "entries": spec.entries, "n_codebooks": spec.n_codebooks,
-            "variant": cabi.VARIANT_NAMES[cabi.select_variant_b(spec.M, spec.K, spec.N, spec.vec, spec.entries,
-                                                                 spec.n_codebooks, spec.code_bits)],
+            "variant": cabi.auto_variant_name_b(spec.M, spec.K, spec.N, spec.vec, spec.entries, spec.n_codebooks, spec.code_bits),
             "us": t_cold * 1e6, "us_warm_cache": t_warm * 1e6,
             "tflops": spec.flops / t_cold / 1e12,
             "tflops_2p40": spec.flops / t_cold / 1024 ** 4,   # the reference's own divisor (strategy_1/src.cu:396)
@@ -379,7 +378,7 @@ def main():
             report[name] = {"M": M, "K": K, "H": H, "n_codebooks": G,
                             "product_then_elementwise_us": t_before * 1e6, "product_alone_us": t_plain * 1e6,
                             "gated_entry_point_us": t_after * 1e6, "speedup": t_before / t_after,
-                            "plain_variant": cabi.VARIANT_NAMES[cabi.select_variant_b(M, K, 2 * H, 8, 256, G, 8)],
+                            "plain_variant": cabi.auto_variant_name_b(M, K, 2 * H, 8, 256, G, 8),
                             "cold_code_buffers": n_bufs}
             del pool, prod, y
             torch.cuda.empty_cache()
@@ -410,12 +409,11 @@ def main():
                 t_both = t_prod
             report[f"slices_{S}"] = {"K_per_slice": spec.K // S, "rows": spec.N * S, "product_us": t_prod * 1e6,
                                      "with_summing_pass_us": t_both * 1e6,
-                                     "variant": cabi.VARIANT_NAMES[cabi.select_variant_b(spec.M, spec.K // S, spec.N * S, spec.vec,
-                                                                                         spec.entries, 1, spec.code_bits)]}
+                                     "variant": cabi.auto_variant_name_b(spec.M, spec.K // S, spec.N * S, spec.vec, spec.entries, 1, spec.code_bits)}
             del pool, part, ysum
             torch.cuda.empty_cache()
-        # The tiles of medium M: split K is built there (vqgemm_e2e_gemm_b_ws: 128x128 tiles, 2-8 workgroups per tile, the
-        # last one sums the partial products).  The automatic choice without and with a workspace, and the baselines.
+        # The tiles of medium M: split K is built there (vqgemm_e2e_gemm_b_ws: 128x128 tiles, 2 to 16 slices of K, a
+        # second launch sums the partial products).  The automatic choice without and with a workspace, and the baselines.
         tiles = {}
         for M, K, N, G in ((256, 4096, 4096, 32), (384, 4096, 4096, 32), (512, 4096, 4096, 32), (768, 4096, 4096, 32),
                            (256, 8192, 8192, 1), (512, 8192, 8192, 1), (256, 11008, 4096, 1), (2048, 4096, 1024, 8),
@@ -431,8 +429,9 @@ def main():
             t_blas = time_launches(lambda i: cabi.ref_gemm_f16(x, wd, w_is_nk=True, out=y), 1, 40, 10, min_launches=1)[0]
             t_torch = time_launches(lambda i: torch.nn.functional.linear(x, wd), 1, 40, 10, min_launches=1)[0]
             tiles[tspec.name] = {"n_codebooks": G, "without_workspace_us": t_plain * 1e6,
-                                 "without_workspace_variant": cabi.VARIANT_NAMES[cabi.select_variant_b(M, K, N, 8, 256, G, 8)],
-                                 "workspace_bytes_wanted": need, "with_workspace_us": t_ws * 1e6,
+                                 "without_workspace_variant": cabi.auto_variant_name_b(M, K, N, 8, 256, G, 8),
+                                 "workspace_bytes_wanted": need, "with_workspace_variant": cabi.auto_variant_name_b(M, K, N, 8, 256, G, 8, need),
+                                 "with_workspace_us": t_ws * 1e6,
                                  "hipblaslt_us": t_blas * 1e6, "torch_linear_us": t_torch * 1e6}
             del x, codes, cb, y, ws, wd
             torch.cuda.empty_cache()

@@ -321,6 +321,15 @@ int vqgemm_select_variant_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_
                             int32_t n_codebooks, int32_t code_bits);
 
 /*
+ * What VQGEMM_VARIANT_AUTO launches on a geometry-B shape with aligned operands - vqgemm_e2e_gemm_b (workspace_bytes 0) or
+ * vqgemm_e2e_gemm_b_ws with a workspace of that many bytes - for reports (host only, no GPU call): a VQGEMM_VARIANT_* value, VQGEMM_PLAN_TAIL_SPLIT (whole rounds of large tiles, the columns that
+ * are left in 128x128 tiles with K split; no variant to ask for), or a negative error for an invalid shape.
+ */
+#define VQGEMM_PLAN_TAIL_SPLIT 32
+int vqgemm_auto_variant_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks,
+                          int32_t code_bits, int64_t workspace_bytes);
+
+/*
  * The constants of the cost models behind VQGEMM_VARIANT_AUTO (host only).  The compiled-in values were fitted
  * to measurements on one 256-CU MI355X; `python -m vq_gemm_amd.tune --fit` measures the box at hand and writes
  * a flat JSON object {"name": number, ...} that vqgemm_tuning_load reads (and that the library reads by itself,

@@ -1103,11 +1103,28 @@ def test_gated_mlp_module():
         assert e2 <= TOL and e1 <= 0.1, (e1, e2)
 
 
+@pytest.mark.parametrize("dims", [(1, 4096, 4096, 8, 256, 1, 8), (16, 4096, 4096, 8, 256, 1, 8), (16, 2048, 11008, 8, 16, 1, 8), (64, 4096, 2048, 4, 4096, 1, 16),
+                                  (203, 2816, 7040, 8, 256, 1, 8), (954, 14080, 1920, 8, 256, 1, 8), (600, 1024, 2048, 8, 256, 1, 8)])
+def test_the_automatic_choice_launches_what_the_report_names(dims):
+    """Bit for bit (every kernel has its own order of sums), without a workspace and with the one asked for."""
+    M, K, N, v, e, g, bits = dims
+    x, codes, cb = make_problem(ProblemSpec("named", GEOM_B, *dims), seed=3, device=DEV)
+    need = cabi.workspace_bytes_b(*dims)
+    for ws_bytes in (0, max(need, 256)):
+        name = cabi.auto_variant_name_b(*dims, ws_bytes)
+        _say("named by the report", dims, ws_bytes, name)
+        variant = {n: i for i, n in cabi.VARIANT_NAMES.items()}[name]
+        ws = torch.empty(max(ws_bytes, cabi.workspace_bytes_b(*dims, variant)), dtype=torch.uint8, device=DEV)
+        y = cabi.e2e_gemm_b_ws(x, codes, cb, workspace=ws) if ws_bytes else cabi.e2e_gemm_b(x, codes, cb)
+        assert torch.equal(y, cabi.e2e_gemm_b_ws(x, codes, cb, variant=variant, workspace=ws)), name
+
+
 def test_tune_reports_every_variant_and_the_automatic_choice():
     from vq_gemm_amd import tune
     _say("tune 300 512 520")
     r = tune.tune(300, 512, 520, 8, 256, 4, 8, verbose=False)
     assert {"prefill", "prefill_small", "twopass", "auto"} <= set(r["times_us"])
+    assert "wave_k" in r["times_us"] and "wave_k" in tune.tune_cold(100, 512, 520, 8, 256, 4, 8, verbose=False)["times_us"]
     assert r["auto_picks"] in r["times_us"] and r["hipblaslt_us"] > 0
     # (how close the automatic choice comes to the fastest variant is a figure of the report, r["auto_over_fastest"]:
     # a timing, not a parity property, and not asserted here)

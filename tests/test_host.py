@@ -292,3 +292,16 @@ def test_split_k_is_asked_for_where_it_was_measured_faster():
         assert cabi.workspace_bytes_b(M, K, N, v, e, 1, bits) == 0, (M, K, N)
     for M, K, N, v, e, bits in ((3028, 11264, 640, 8, 256, 8), (954, 14080, 1920, 8, 256, 8), (657, 13376, 1040, 8, 256, 8), (118, 11008, 14080, 4, 4096, 16)):
         assert cabi.workspace_bytes_b(M, K, N, v, e, 1, bits) > 0, (M, K, N)
+
+
+def test_the_report_of_the_automatic_choice_names_what_it_launches():
+    """Host only; that the kernels named are the ones launched is held bit for bit on the GPU."""
+    name = cabi.auto_variant_name_b
+    assert name(1, 4096, 4096, 8, 256, 1, 8) == "decode_gemv" and name(16, 4096, 4096, 8, 256, 1, 8) == "decode"
+    assert name(64, 8192, 14336, 4, 4096, 1, 16) == "wave_k" and cabi.select_variant_b(64, 8192, 14336, 4, 4096, 1, 16) == cabi.VARIANT_DECODE
+    assert name(4096, 4096, 4096, 8, 256, 32, 8) == "prefill" and name(4, 60, 20, 4, 256, 1, 8) == "generic"
+    for dims, plan in (((954, 14080, 1920, 8, 256, 1, 8), "prefill_splitk"), ((1536, 4096, 11008, 8, 256, 43, 8), "prefill_tail_split")):
+        need = cabi.workspace_bytes_b(*dims)
+        assert need > 0 and name(*dims, need) == plan and name(*dims, need - 1) == name(*dims) != plan
+    with pytest.raises(cabi.VqGemmError):
+        name(4, 60, 8, 8, 256, 1, 8)

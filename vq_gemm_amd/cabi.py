@@ -38,6 +38,7 @@ _SIGNATURES = {
     "vqgemm_kmeans_b": (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _P, _I64, _P]),
     "vqgemm_pack_codes_b": (ctypes.c_int, [_P, _P, _I64, _I64, _I32, _I32, _I32, _P]),
     "vqgemm_decode_packed_supports": (ctypes.c_int, [_I64, _I64, _I64, _I32, _I32, _I32, _I32]),
+    "vqgemm_auto_variant_b": (ctypes.c_int, [_I64, _I64, _I64, _I32, _I32, _I32, _I32, _I64]),
     "vqgemm_packed_preferred_b": (ctypes.c_int, [_I64, _I64, _I64, _I32, _I32, _I32, _I32]),
     "vqgemm_gemm_f16": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _I64, _P]),
     "vqgemm_silu_mul": (ctypes.c_int, [_P, _P, _I64, _I64, _P]),
@@ -552,4 +553,13 @@ def select_variant_a(M, K, Nc, has_workspace=False) -> int:
 
 
 def select_variant_b(M, K, N, vec, entries, n_codebooks, code_bits) -> int:
+    """The family of kernels of a shape; what `VARIANT_AUTO` launches is `auto_variant_name_b`."""
     return lib().vqgemm_select_variant_b(M, K, N, vec, entries, n_codebooks, code_bits)
+
+
+def auto_variant_name_b(M, K, N, vec, entries, n_codebooks, code_bits, workspace_bytes=0) -> str:
+    """The name of what `VARIANT_AUTO` launches, without a workspace or with one of that many bytes."""
+    v = lib().vqgemm_auto_variant_b(M, K, N, vec, entries, n_codebooks, code_bits, workspace_bytes)
+    if v < 0:
+        raise VqGemmError(v, "vqgemm_auto_variant_b")
+    return "prefill_tail_split" if v == 32 else VARIANT_NAMES[v]

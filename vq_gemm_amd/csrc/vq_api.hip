@@ -553,6 +553,21 @@ int64_t vqgemm_workspace_bytes_b(int64_t M, int64_t K, int64_t N, int32_t vec, i
     return sp >= 2 ? (int64_t)prefill_splitk_workspace_bytes(p, sp) : 0;
 }
 
+int vqgemm_auto_variant_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits,
+                          int64_t workspace_bytes)
+{
+    const DeviceScope device;
+    const int rc = check_b(M, K, N, vec, entries, n_codebooks, code_bits);
+    if (rc != VQGEMM_OK) return rc;
+    const ProblemB p = make_b(nullptr, nullptr, nullptr, nullptr, M, K, N, vec, entries, n_codebooks, code_bits);
+    if (M == 0 || N == 0 || K == 0) return VQGEMM_VARIANT_GENERIC;
+    const AutoPlan &plan = auto_plan(p);
+    if (workspace_bytes <= 0) return plan.variant;
+    if (plan.ws.wave) return VQGEMM_VARIANT_WAVE_K;
+    if ((int64_t)plan.ws.bytes > workspace_bytes) return plan.variant;
+    return plan.ws.tail.ok ? VQGEMM_PLAN_TAIL_SPLIT : plan.ws.sp >= 2 ? VQGEMM_VARIANT_PREFILL_SPLITK : plan.variant;
+}
+
 int vqgemm_e2e_gemm_b_ws(const void *x, const void *codes, const void *codebook, const void *bias, void *y, int64_t M,
                          int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits,
                          int32_t variant, void *workspace, int64_t workspace_bytes, void *stream)

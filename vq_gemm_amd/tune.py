@@ -26,7 +26,7 @@ per-kernel durations behind every figure.
 
 The choice between the kernels rests on cost models fitted to measurements on one MI355X; this
 prints, for the box at hand, the time of each variant that accepts the shape (launches replayed
-from a HIP graph), the variant `VQGEMM_VARIANT_AUTO` resolves to, its distance from the fastest,
+from a HIP graph), what `VQGEMM_VARIANT_AUTO` launches (with the workspace it asks for), its distance from the fastest,
 and the hipBLASLt fp16 GEMM on the dequantised weights beside them.  Inputs are synthetic
 (X ~ N(0,1), uniform codes, codebooks ~ N(0, 0.02)), as in the bench.
 """
@@ -69,11 +69,11 @@ def tune_cold(M: int, K: int, N: int, vec: int = 8, entries: int = 256, n_codebo
     """Microseconds per launch of every variant that takes the shape, on codes that come from HBM."""
     times = {}
     for variant in (cabi.VARIANT_AUTO, cabi.VARIANT_DECODE, cabi.VARIANT_DECODE_GEMV, cabi.VARIANT_PREFILL, cabi.VARIANT_PREFILL_NARROW,
-                    cabi.VARIANT_PREFILL_SMALL):
+                    cabi.VARIANT_PREFILL_SMALL, cabi.VARIANT_WAVE_K):
         t = _cold_us(M, K, N, variant, vec=vec, entries=entries, n_codebooks=n_codebooks, code_bits=code_bits, device=device)
         if t is not None:
             times[cabi.VARIANT_NAMES[variant]] = t
-    picked = cabi.VARIANT_NAMES[cabi.select_variant_b(M, K, N, vec, entries, n_codebooks, code_bits)]
+    picked = cabi.auto_variant_name_b(M, K, N, vec, entries, n_codebooks, code_bits)
     if verbose:
         print(f"M={M} K={K} N={N} vec={vec} entries={entries} codebooks={n_codebooks} code_bits={code_bits}, cold code matrices")
         for v, t in times.items():
@@ -93,34 +93,35 @@ def tune(M: int, K: int, N: int, vec: int = 8, entries: int = 256, n_codebooks: 
     cabi.e2e_gemm_b(x, codes, cb, out=y, variant=cabi.VARIANT_TWOPASS, workspace=workspace)
     torch.cuda.synchronize()
     for variant in (cabi.VARIANT_DECODE, cabi.VARIANT_DECODE_GEMV, cabi.VARIANT_PREFILL, cabi.VARIANT_PREFILL_NARROW, cabi.VARIANT_PREFILL_SMALL,
-                    cabi.VARIANT_TWOPASS, cabi.VARIANT_AUTO):
+                    cabi.VARIANT_WAVE_K, cabi.VARIANT_TWOPASS, cabi.VARIANT_AUTO):
         try:
-            times[variant] = time_graph(lambda: cabi.e2e_gemm_b(x, codes, cb, out=y, variant=variant, workspace=workspace))
+            times[cabi.VARIANT_NAMES[variant]] = time_graph(lambda: cabi.e2e_gemm_b(x, codes, cb, out=y, variant=variant, workspace=workspace))
         except cabi.VqGemmError as e:
             if e.code != -4:   # anything but "this variant does not take the shape"
                 raise
-    # split K over the 128x128 tiles, and the automatic choice when it is given a workspace to split K with
+    # split K over the 128x128 tiles, and the automatic choice when it is given the workspace it asks for
     need = cabi.workspace_bytes_b(M, K, N, vec, entries, n_codebooks, code_bits, cabi.VARIANT_PREFILL_SPLITK)
     if need > 0:
         ws = torch.empty(need, dtype=torch.uint8, device=device)
-        times[cabi.VARIANT_PREFILL_SPLITK] = time_graph(
+        times["prefill_splitk"] = time_graph(
             lambda: cabi.e2e_gemm_b_ws(x, codes, cb, out=y, variant=cabi.VARIANT_PREFILL_SPLITK, workspace=ws))
     auto_need = cabi.workspace_bytes_b(M, K, N, vec, entries, n_codebooks, code_bits)
+    picked = cabi.auto_variant_name_b(M, K, N, vec, entries, n_codebooks, code_bits, 2 ** 62)
+    # (a size that asks for none can still be planned otherwise with one: any workspace says so)
+    ws = torch.empty(max(auto_need, 256), dtype=torch.uint8, device=device)
+    times["auto"] = time_graph(lambda: cabi.e2e_gemm_b_ws(x, codes, cb, out=y, workspace=ws))
+    if picked == "prefill_tail_split":   # (nothing but the automatic choice takes it)
+        times[picked] = times["auto"]
     w = cabi.dequant_b(codes, cb)
     t_lib = time_graph(lambda: cabi.ref_gemm_f16(x, w, w_is_nk=True, out=y))
-    picked = cabi.select_variant_b(M, K, N, vec, entries, n_codebooks, code_bits)
-    forced = {v: t for v, t in times.items() if v != cabi.VARIANT_AUTO}
+    forced = {v: t for v, t in times.items() if v != "auto"}
     fastest = min(forced, key=forced.get)
-    if auto_need > 0:   # with a workspace the automatic choice splits K here
-        picked = cabi.VARIANT_PREFILL_SPLITK
-        times[cabi.VARIANT_AUTO] = times[cabi.VARIANT_PREFILL_SPLITK]
-    result = {"times_us": {cabi.VARIANT_NAMES[v]: t for v, t in times.items()}, "auto_picks": cabi.VARIANT_NAMES[picked],
-              "fastest": cabi.VARIANT_NAMES[fastest], "auto_over_fastest": times[cabi.VARIANT_AUTO] / forced[fastest],
+    result = {"times_us": times, "auto_picks": picked, "fastest": fastest, "auto_over_fastest": times["auto"] / forced[fastest],
               "hipblaslt_us": t_lib}
     if verbose:
         print(f"M={M} K={K} N={N} vec={vec} entries={entries} codebooks={n_codebooks} code_bits={code_bits}")
         for v, t in times.items():
-            print(f"  {cabi.VARIANT_NAMES[v]:15s} {t:9.1f} us  {spec.flops / t / 1e6:8.1f} TFLOP/s")
+            print(f"  {v:15s} {t:9.1f} us  {spec.flops / t / 1e6:8.1f} TFLOP/s")
         print(f"  {'hipBLASLt fp16':15s} {t_lib:9.1f} us  (on the dequantised weights)")
         print(f"  automatic choice: {result['auto_picks']} (the prefill variant chooses its tile itself); fastest forced "
               f"variant: {result['fastest']}; automatic / fastest = {result['auto_over_fastest']:.2f}")
