@@ -137,7 +137,6 @@ const TuningEntry kTuningEntries[] = {
     {"splitk_force_splits", &Tuning::splitk_force_splits},
     {"wave_k_force", &Tuning::wave_k_force},
     {"wave_k_force_tile", &Tuning::wave_k_force_tile},
-    {"splitk_validate_fences", &Tuning::splitk_validate_fences},
 };
 constexpr int kTuningCount = (int)(sizeof(kTuningEntries) / sizeof(kTuningEntries[0]));
 

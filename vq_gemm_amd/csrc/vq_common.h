@@ -283,7 +283,6 @@ struct Tuning {
     // 1 wherever they apply, 2 never; and their tile as 10 * (rows / 16) + columns / 16 (0: the cost model's)
     double wave_k_force = 0.0;
     double wave_k_force_tile = 0.0;
-    double splitk_validate_fences = 0.0;  // (accepted, without effect: the slices meet in a second launch)
 };
 const Tuning &tuning();
 
