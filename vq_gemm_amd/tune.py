@@ -211,7 +211,7 @@ def fit(device: str = "cuda:0", verbose: bool = True) -> dict:
             break
     out["gemv_max_tiles_per_cu"] = best
     # split K over the 128x128 tiles: what two slices cost beyond their multiplying (the same tiles as an unsplit problem
-    # of half the K and twice the columns), at two sizes of partial sums
+    # of half the K and twice the columns, whose stages the model has at 0.87 in a slice), at two sizes of partial sums
     def split_extra(M, K, N):
         cabi.set_tuning(splitk_force_splits=2)
         try:
@@ -226,7 +226,10 @@ def fit(device: str = "cuda:0", verbose: bool = True) -> dict:
         finally:
             cabi.set_tuning(splitk_force_splits=cur["splitk_force_splits"])
         t_main = _t(M, K // 2, 2 * N, cabi.VARIANT_PREFILL_SMALL)
-        return None if t_main is None else (t_split - t_main, need / 1e6)
+        if t_main is None:
+            return None
+        ends = min(t_main, out["prefill_small_tile_fixed_us"])
+        return t_split - (ends + 0.87 * (t_main - ends)), need / 1e6
     small, large = split_extra(128, 4096, 4096), split_extra(512, 4096, 4096)
     if small and large and large[1] > small[1]:
         per_mb = max((large[0] - small[0]) / (large[1] - small[1]), 0.05)
