@@ -2147,6 +2147,32 @@ def test_k_dealt_out_to_waves_geometry_a(M, K, Nc):
         _check_gemm(y, x, w, cb, geometry=GEOM_A, what=f"tile {tile}")
 
 
+@pytest.mark.parametrize("what", ["weights", "entries", "entry 0 is NaN", "both", "equal vectors and entries", "all zero"])
+@pytest.mark.parametrize("N,K,v,E,G", [(64, 256, 8, 256, 2), (48, 520, 8, 100, 1), (40, 128, 4, 4096, 1), (50, 64, 2, 77, 1), (24, 64, 8, 5000, 1)])
+def test_encoder_keeps_the_rule_where_nothing_is_finite_or_everything_is_equal(N, K, v, E, G, what):
+    """A NaN distance never wins and entry 0 is taken as it is; among equals the lowest index is kept."""
+    g = torch.Generator(device="cpu").manual_seed(17)
+    cb, w = torch.randn(G, E, v, generator=g).half(), torch.randn(N, K, generator=g).half()
+    odd = torch.tensor([float("inf"), float("-inf"), float("nan"), 65504.0, -65504.0, 0.0, -0.0]).half()
+    some = lambda t, share: torch.where(torch.rand(t.shape, generator=g) < share, odd[torch.randint(0, 7, t.shape, generator=g)], t)
+    if what in ("weights", "both"):
+        w = some(w, 0.03)
+    if what in ("entries", "both"):
+        cb = some(cb, 0.01)
+    if what == "entry 0 is NaN":
+        cb[:, 0, v - 1] = float("nan")
+    if what == "equal vectors and entries":
+        cb[:, E // 2:] = cb[:, :E - E // 2].clone()
+        w.view(N, K // v, v)[:, ::2] = cb[0, E // 3]
+    if what == "all zero":
+        cb[:], w[:] = 0.0, 0.0
+    bits = 8 if E <= 256 else 16
+    _say("encode", N, K, v, E, what)
+    codes = cabi.encode_b(w.to(DEV), cb.to(DEV), bits)
+    torch.cuda.synchronize()
+    assert np.array_equal(_np(codes), c_oracle.encode_b(w.numpy(), cb.numpy(), bits))
+
+
 @pytest.mark.parametrize("N,K,v", [(1024, 1032, 8), (1032, 1024, 8), (700, 768, 4)])   # the last and first sizes of a wave's 64 and 128 vectors
 def test_encoder_on_both_sides_of_the_line_between_its_wave_sizes(N, K, v):
     g = torch.Generator(device="cpu").manual_seed(6)

@@ -192,17 +192,17 @@ int read_tuning_file(const char *path)
 
 bool aligned(const void *p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
 
-// Whether the automatic choice takes the fused geometry-A kernel: at every height (a short X
-// leaves its 128-row tile mostly padding, and the kernel is still an order of magnitude ahead of the
-// scalar one).  Its 4-byte gathers keep the LDS busier than the matrix cores, so once there is more
-// than one round of tiles the two-pass route is faster - when the caller brings the scratch for it.
-// of the two fused geometry-A kernels (both take the same shapes)
+// Of the two fused geometry-A kernels (both take the same shapes), whether the wave-K kernel is expected to be the faster one.
 bool wave_k_a_preferred(const ProblemA &p)
 {
     const int force = (int)tuning().wave_k_force;
     return wave_k_a_supports(p) && force != 2 && (force == 1 || wave_k_a_cost_us(p) < fused_a_cost_us(p));
 }
 
+// Whether the automatic choice takes a fused geometry-A kernel: at every height (a short X
+// leaves its 128-row tile mostly padding, and the kernel is still an order of magnitude ahead of the
+// scalar one).  Its 4-byte gathers keep the LDS busier than the matrix cores, so once there is more
+// than one round of tiles the two-pass route is faster - when the caller brings the scratch for it.
 bool fused_a_preferred(const ProblemA &p, bool has_workspace)
 {
     if (p.M < 1 || !fused_a_supports(p)) return false;

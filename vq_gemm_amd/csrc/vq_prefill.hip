@@ -378,7 +378,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
 #undef C_WLO_N
 #undef C_WHI_N
             buf = buf_next;
-            };
+        };
         int super = 0;
         do {
             stage_body(super, std::integral_constant<int, 0>{}, std::false_type{});
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(const half_t *__re
 #undef L_WLO_N
 #undef L_WLO_N2
             buf = buf_next;
-            };
+        };
         int super = 0;
         do {
             stage_body(super, std::integral_constant<int, 0>{}, std::false_type{});
@@ -744,7 +744,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_narrow_kernel(const half_
 #undef LC_N_23
 #undef LC_NB_01
         buf = buf_next;
-        };
+    };
     int super = 0;
     do {
         stage_body(super, std::integral_constant<int, 0>{});

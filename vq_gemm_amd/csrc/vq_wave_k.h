@@ -1,5 +1,5 @@
 // Products whose tiles of the large kernels are fewer than the compute units: a workgroup takes a small tile of Y
-// (16 to 128 rows by 32 or 64 columns) and its eight waves deal K out among themselves.
+// (16 to 128 rows by 32 to 128 columns) and its waves, eight in nearly all tiles, deal K out among themselves.
 //
 //   NN:        y[M,N] = x[M,K] . w[K,N], fp16 w
 //   geometry A: out[M, 2*Nc] = x[M,K] . W_dec, W_dec[k, 2n + r] = codebook[n/4][w[k,n]][r] (reference
