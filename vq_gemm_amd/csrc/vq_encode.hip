@@ -128,6 +128,9 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c)
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, a), __builtin_bit_cast(half2_t, b), c, false);
 }
 
+// two halves with both zeros as one (-0 + 0 is 0)
+__device__ __forceinline__ uint32_t one_zero(uint32_t v) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) + half2_t{}); }
+
 template <int DW>
 __device__ __forceinline__ void read_entry(const uint32_t *table, int e, uint32_t (&c)[DW])
 {
@@ -153,7 +156,7 @@ __device__ __forceinline__ HalfWaves swap_half_waves(uint32_t a, uint32_t b)
 }
 
 // LDS: entries padded to whole tiles of 32: halves with flipped signs, then |c|^2 / 2 (infinity behind the last entry),
-// then with ACCUMULATE the sums of the vectors assigned to each entry and their number, [entry][VEC + 1].
+// then with ACCUMULATE the sums of the vectors assigned to each entry and their number, [entry][VEC + 1], then n_buckets words.
 //
 // ACCUMULATE (a Lloyd iteration): every vector is added to its entry's sums, its distance to the workgroup's error, and
 // both leave as the workgroup's row of `partials`: entries * (VEC + 1) sums and counts, then the error.  The sums are kept in
@@ -162,7 +165,8 @@ __device__ __forceinline__ HalfWaves swap_half_waves(uint32_t a, uint32_t b)
 template <int VEC, typename CodeT, int GROUP, bool ACCUMULATE, int kScanBatches>
 __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t *__restrict__ w, const half_t *__restrict__ cb,
                                                                    CodeT *__restrict__ codes, int64_t vectors_per_cb, int entries,
-                                                                   int wgs_per_cb, float *__restrict__ partials)
+                                                                   int wgs_per_cb, float *__restrict__ partials, int bucket_off,
+                                                                   int n_buckets)
 {
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ float reduce[kScanThreads / 64];
@@ -179,6 +183,7 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
     uint32_t *table = reinterpret_cast<uint32_t *>(smem);                         // [n_tiles * 32][DW]
     float *norms = reinterpret_cast<float *>(smem + scan_table_bytes(entries, VEC));
     double *sums = reinterpret_cast<double *>(norms + n_tiles * 32);
+    uint32_t *bucket = reinterpret_cast<uint32_t *>(smem + bucket_off);
     const int g = blockIdx.x / wgs_per_cb, part = blockIdx.x % wgs_per_cb;
     const half_t *wg_w = w + (int64_t)g * vectors_per_cb * VEC;
     CodeT *wg_codes = codes + (int64_t)g * vectors_per_cb;
@@ -186,20 +191,46 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
     // table, half norms, whether all of them are finite (else every vector of the codebook is decided by the rule)
     bool book_finite;
     {
-        float largest = 0.f;
-        const uint32_t *book = reinterpret_cast<const uint32_t *>(cb + (int64_t)g * entries * VEC);
-        for (int e = tid; e < n_tiles * 32; e += kScanThreads) {
-            float n2 = 0.f;
+        // An entry that equals an earlier one is never chosen, but beside it no vector would be clear below, and a vector by the rule
+        // takes as long as twenty others: it gets an infinite norm.  The entries' hashes deal them out to buckets, and an entry looks
+        // at the first one in its bucket.  (What meets another entry there, and so stays, costs time, not the result.)  A codebook
+        // half of whose entries equal the other half, 4096 x 4096 8-vectors: 749 -> 125 us, two equal ones and half of the weights
+        // that value 435 -> 40; none equal 41.3 and 41.2.
+        auto bucket_of = [&](const uint32_t (&c)[DW]) {
+            uint32_t h = 0;
 #pragma unroll
             for (int i = 0; i < DW; i++) {
-                const uint32_t v = e < entries ? book[(int64_t)e * DW + i] : 0u;
-                const half2_t c = __builtin_bit_cast(half2_t, v);
-                n2 = __builtin_fmaf((float)c[0], (float)c[0], n2);
-                n2 = __builtin_fmaf((float)c[1], (float)c[1], n2);
-                table[at(e) * DW + i] = v ^ 0x80008000u;
+                const uint32_t v = one_zero(c[i]);
+                h ^= i ? v << (7 * i) | v >> (32 - 7 * i) : v;
+            }
+            return (int)__umulhi(h * 0x9e3779b1u, (uint32_t)n_buckets);
+        };
+        float largest = 0.f;
+        const uint32_t *book = reinterpret_cast<const uint32_t *>(cb + (int64_t)g * entries * VEC);
+        uint32_t own[DW];   // the thread's first entry, on its way while the buckets are cleared
+        auto load = [&](int e) {
+#pragma unroll
+            for (int i = 0; i < DW; i++) own[i] = book[(int64_t)min(e, entries - 1) * DW + i];
+#pragma unroll
+            for (int i = 0; i < DW; i++) own[i] = (e < entries ? own[i] : 0u) ^ 0x80008000u;
+        };
+        load(tid);
+        for (int i = tid; i < n_buckets; i += kScanThreads) bucket[i] = ~0u;
+        if (n_buckets) __syncthreads();
+        for (int e = tid; e < n_tiles * 32; e += kScanThreads) {
+            if (e != tid) load(e);
+            float n2 = 0.f;
+            uint32_t c[DW];
+#pragma unroll
+            for (int i = 0; i < DW; i++) {
+                const half2_t f = __builtin_bit_cast(half2_t, own[i]);
+                n2 = __builtin_fmaf((float)f[0], (float)f[0], n2);
+                n2 = __builtin_fmaf((float)f[1], (float)f[1], n2);
+                table[at(e) * DW + i] = c[i] = own[i];
             }
             norms[e] = e < entries ? 0.5f * n2 : __builtin_inff();
             largest = n2 < __builtin_inff() ? fmaxf(largest, n2) : __builtin_inff();
+            if (n_buckets && e < entries) atomicMin(&bucket[bucket_of(c)], (uint32_t)e);
         }
         if constexpr (ACCUMULATE)
             for (int i = tid; i < entries * (VEC + 1); i += kScanThreads) sums[i] = 0.0;
@@ -210,6 +241,19 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
 #pragma unroll
         for (int i = 0; i < kScanThreads / 64; i++) largest = fmaxf(largest, reduce[i]);
         book_finite = largest < __builtin_inff();
+        if (n_buckets) {
+            for (int e = tid; e < entries; e += kScanThreads) {
+                uint32_t c[DW], other[DW];
+                read_entry<DW>(table, at(e), c);
+                const int first = (int)bucket[bucket_of(c)];
+                read_entry<DW>(table, at(first), other);
+                uint32_t differ = first < e ? 0u : 1u;
+#pragma unroll
+                for (int i = 0; i < DW; i++) differ |= one_zero(c[i]) ^ one_zero(other[i]);
+                if (!differ) norms[e] = __builtin_inff();
+            }
+            __syncthreads();
+        }
     }
 
     // Infinities the compiler takes for any numbers: a minimum that starts from one folds two scores per instruction, and
@@ -394,6 +438,17 @@ size_t scan_lds_bytes(const ProblemB &p, bool accumulate)
     return scan_table_bytes(p.entries, p.vec) + padded * 4 + (accumulate ? (size_t)p.entries * (p.vec + 1) * 8 : 0);
 }
 
+constexpr size_t kScanLdsTwoPerUnit = 72 * 1024, kScanLds = 128 * 1024;
+
+// Buckets for finding equal entries: four per entry where the LDS has room that neither keeps a second workgroup off the unit nor the
+// codebook off this kernel; none where not even one per two entries fits.
+int scan_buckets(const ProblemB &p, bool accumulate)
+{
+    const size_t bytes = scan_lds_bytes(p, accumulate), room = ((bytes <= kScanLdsTwoPerUnit ? kScanLdsTwoPerUnit : kScanLds) - bytes) / 4;
+    const size_t want = 4 * (size_t)p.entries;
+    return room >= want ? (int)want : 2 * room >= (size_t)p.entries ? (int)room : 0;
+}
+
 // Batches of a wave and workgroups per codebook: as many as are resident together (two of eight waves per unit while the LDS
 // allows), none without work.
 struct ScanPlan {
@@ -402,7 +457,7 @@ struct ScanPlan {
 ScanPlan scan_plan(const ProblemB &p, bool accumulate)
 {
     const int64_t vectors = (int64_t)p.rows_per_cb * (p.K / p.vec);
-    const int per_cu = scan_lds_bytes(p, accumulate) <= 72 * 1024 ? 2 : 1;
+    const int per_cu = scan_lds_bytes(p, accumulate) <= kScanLdsTwoPerUnit ? 2 : 1;
     const int64_t want = ((int64_t)device_cu_count() * per_cu + p.n_codebooks - 1) / p.n_codebooks;
     auto have = [&](int batches) { return (vectors + kScanThreads / 2 * batches - 1) / (kScanThreads / 2 * batches); };
     const int batches = have(4) * p.n_codebooks * 2 <= device_cu_count() ? 2 : 4;
@@ -412,7 +467,7 @@ ScanPlan scan_plan(const ProblemB &p, bool accumulate)
 bool scan_supports(const half_t *w, const ProblemB &p, bool accumulate)
 {
     const uintptr_t align = p.vec * 2 < 8 ? p.vec * 2 : 8;
-    return ((uintptr_t)w & (align - 1)) == 0 && ((uintptr_t)p.cb & 3) == 0 && scan_lds_bytes(p, accumulate) <= 128 * 1024;
+    return ((uintptr_t)w & (align - 1)) == 0 && ((uintptr_t)p.cb & 3) == 0 && scan_lds_bytes(p, accumulate) <= kScanLds;
 }
 
 template <int VEC, typename CodeT, bool ACCUMULATE>
@@ -422,11 +477,12 @@ hipError_t launch_scan(const half_t *w, const ProblemB &p, void *codes_out, floa
     if (vectors_per_cb == 0) return hipSuccess;
     const ScanPlan plan = scan_plan(p, ACCUMULATE);
     const size_t smem = scan_lds_bytes(p, ACCUMULATE);
+    const int buckets = scan_buckets(p, ACCUMULATE);
     const bool narrow = p.entries < kScanWideGroupEntries;
     auto kern = plan.batches == 4 ? (narrow ? encode_scan_kernel<VEC, CodeT, 8, ACCUMULATE, 4> : encode_scan_kernel<VEC, CodeT, 16, ACCUMULATE, 4>)
                                   : (narrow ? encode_scan_kernel<VEC, CodeT, 8, ACCUMULATE, 2> : encode_scan_kernel<VEC, CodeT, 16, ACCUMULATE, 2>);
-    return launch_kernel(kern, dim3((unsigned)(plan.wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem, s, w, p.cb,
-                       static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, plan.wgs_per_cb, partials);
+    return launch_kernel(kern, dim3((unsigned)(plan.wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem + 4 * (size_t)buckets, s, w, p.cb,
+                       static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, plan.wgs_per_cb, partials, (int)smem, buckets);
 }
 
 template <int VEC, typename CodeT>
@@ -458,7 +514,7 @@ hipError_t launch_encode_b(const half_t *w, const ProblemB &p, void *codes_out, 
     }
 }
 
-bool lloyd_supports(const ProblemB &p) { return encode_supports(p) && scan_lds_bytes(p, true) <= 128 * 1024; }
+bool lloyd_supports(const ProblemB &p) { return encode_supports(p) && scan_lds_bytes(p, true) <= kScanLds; }
 
 int lloyd_assign_rows(const ProblemB &p) { return scan_plan(p, true).wgs_per_cb; }
 
