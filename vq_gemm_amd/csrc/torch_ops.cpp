@@ -192,15 +192,18 @@ Tensor no_gradient(Tensor y, std::initializer_list<const Tensor *> inputs)
 
 // Whether nothing but this library is to see a call on `x`: an ordinary tensor in GPU memory, no dispatch mode, no
 // functional transform, no tracer.
-bool plain_call(const Tensor &x)
+bool plain_tensor(const Tensor &x)
 {
     if (!x.defined() || !x.is_cuda()) return false;
     constexpr c10::DispatchKeySet wrappers({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::Functionalize,
                                             c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
                                             c10::DispatchKey::BatchedNestedTensor, c10::DispatchKey::NestedTensor});
-    if (x.key_set().has_any(wrappers)) return false;
-    return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
+    return !x.key_set().has_any(wrappers);
 }
+
+bool plain_thread() { return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty(); }
+
+bool plain_call(const Tensor &x) { return plain_tensor(x) && plain_thread(); }
 
 // The autograd kernels call the device implementation directly (one dispatch per call instead of two), unless the tensors
 // only stand for data: then the call goes on to whoever wrapped them.
@@ -255,49 +258,56 @@ bool function_mode_watches()
     return false;
 }
 
-// A tensor whose class overrides __torch_function__.
-bool subclass_watches(const Tensor &t)
+// Whether the tensor's class overrides __torch_function__.
+bool subclass_watches(PyObject *tensor)
 {
-    const py::object o = py::cast(t);
-    if (THPVariable_CheckTypeExact(Py_TYPE(o.ptr()))) return false;
+    if (THPVariable_CheckTypeExact(Py_TYPE(tensor))) return false;
     if (at::impl::PythonTorchFunctionTLS::get_disabled_state() != at::impl::TorchFunctionDisabledState::ENABLED) return false;
-    return py::object(o.attr("__torch_function__")).ptr() != no_torch_function;
+    return py::object(py::handle(tensor).attr("__torch_function__")).ptr() != no_torch_function;
 }
 
-// `plain_call` for a call from Python on these operands (those that are there at all).
-bool plain_python_call(std::initializer_list<const Tensor *> operands)
+// The tensor behind an argument, without a reference of its own: the caller's arguments live as long as the call.
+const Tensor &tensor_of(py::handle h)
 {
-    if (function_mode_watches()) return false;
-    for (const Tensor *t : operands)
-        if (t->defined() && (!plain_call(*t) || subclass_watches(*t))) return false;
-    return (*operands.begin())->defined();
+    if (!THPVariable_Check(h.ptr())) throw py::type_error("expected a tensor");
+    return THPVariable_Unpack(h.ptr());
 }
 
-const Tensor &given(const OptTensor &t)
+// `plain_call` for a call from Python on these operands (None is none).
+bool plain_python_call(std::initializer_list<py::handle> operands)
 {
-    static const Tensor none;
-    return t.has_value() ? *t : none;
+    if (function_mode_watches() || !plain_thread()) return false;
+    for (const py::handle h : operands)
+        if (!h.is_none() && (!plain_tensor(tensor_of(h)) || subclass_watches(h.ptr()))) return false;
+    return true;
 }
+
+OptTensor optional_of(py::handle h) { return h.is_none() ? OptTensor() : OptTensor(tensor_of(h)); }
 
 // packed: `codes` are in the packed layout (a single stage)
-py::object linear(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias, int64_t k_repeat, bool packed)
+py::object linear(py::handle x, py::handle codes, py::handle codebook, py::handle bias, int64_t k_repeat, bool packed)
 {
-    if (!plain_python_call({&x, &codes, &codebook, &given(bias)})) return py::none();
+    if (!plain_python_call({x, codes, codebook, bias})) return py::none();
     TORCH_CHECK_VALUE(!packed || k_repeat == 1, "linear: additive stages have no packed layout");
+    const Tensor &x_t = tensor_of(x), &codes_t = tensor_of(codes), &codebook_t = tensor_of(codebook);
+    const OptTensor bias_t = optional_of(bias);
     Tensor y;
     {
         const py::gil_scoped_release no_gil;
         RECORD_FUNCTION("vq_gemm_amd::vq_linear", c10::ArrayRef<const c10::IValue>());
-        y = linear_impl(x, codes, codebook, bias, k_repeat, packed ? VQGEMM_VARIANT_DECODE_PACKED : VQGEMM_VARIANT_AUTO);
+        y = linear_impl(x_t, codes_t, codebook_t, bias_t, k_repeat, packed ? VQGEMM_VARIANT_DECODE_PACKED : VQGEMM_VARIANT_AUTO);
     }
     return py::cast(y);
 }
 
 // Whether a layer that holds both layouts of its codes hands the packed one over for x (what is wrong with x the call itself says;
 // the kernel of the packed layout takes no operands that begin anywhere).
-bool takes_packed(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
+bool takes_packed(py::handle x_h, py::handle codes_h, py::handle codebook_h, py::handle bias_h)
 {
-    if (!plain_python_call({&x, &codes, &codebook, &given(bias)}) || x.dim() < 1 || codes.dim() != 2 || (codebook.dim() != 2 && codebook.dim() != 3) || !aligned16(codebook)) return false;
+    if (!plain_python_call({x_h, codes_h, codebook_h, bias_h})) return false;
+    const Tensor &x = tensor_of(x_h), &codes = tensor_of(codes_h), &codebook = tensor_of(codebook_h);
+    const OptTensor bias = optional_of(bias_h);
+    if (x.dim() < 1 || codes.dim() != 2 || (codebook.dim() != 2 && codebook.dim() != 3) || !aligned16(codebook)) return false;
     if (bias.has_value() && bias->defined() && (reinterpret_cast<uintptr_t>(bias->data_ptr()) & 7) != 0) return false;
     const int64_t vec = codebook.size(-1), K = codes.size(1) * vec;
     if (K == 0 || x.size(-1) != K) return false;
@@ -306,14 +316,16 @@ bool takes_packed(const Tensor &x, const Tensor &codes, const Tensor &codebook, 
                                      codebook.dim() == 3 ? (int)codebook.size(0) : 1, codes.scalar_type() == at::kByte ? 8 : 16) == 1;
 }
 
-py::object gated(const Tensor &x, const Tensor &codes, const Tensor &codebook, const OptTensor &bias)
+py::object gated(py::handle x, py::handle codes, py::handle codebook, py::handle bias)
 {
-    if (!plain_python_call({&x, &codes, &codebook, &given(bias)})) return py::none();
+    if (!plain_python_call({x, codes, codebook, bias})) return py::none();
+    const Tensor &x_t = tensor_of(x), &codes_t = tensor_of(codes), &codebook_t = tensor_of(codebook);
+    const OptTensor bias_t = optional_of(bias);
     Tensor y;
     {
         const py::gil_scoped_release no_gil;
         RECORD_FUNCTION("vq_gemm_amd::vq_gated_linear", c10::ArrayRef<const c10::IValue>());
-        y = gated_impl(x, codes, codebook, bias);
+        y = gated_impl(x_t, codes_t, codebook_t, bias_t);
     }
     return py::cast(y);
 }
@@ -322,17 +334,20 @@ py::object gated(const Tensor &x, const Tensor &codes, const Tensor &codebook, c
 
 // What cabi.encode_b and cabi.dequant_b do on well-formed operands of the current device, without their checks one by one in
 // Python (11 of the 12 us of a call on a small matrix); None sends the caller down that path, which says what is wrong.
-bool codec_operands(const Tensor &m, const Tensor &codebook, int64_t per_column)
+bool codec_operands(py::handle m_h, py::handle codebook_h, int64_t per_column)
 {
-    return plain_python_call({&m, &codebook}) && m.dim() == 2 && m.is_contiguous() && codebook.is_cuda() && codebook.device() == m.device() && codebook.is_contiguous() &&
+    if (!plain_python_call({m_h, codebook_h})) return false;
+    const Tensor &m = tensor_of(m_h), &codebook = tensor_of(codebook_h);
+    return m.dim() == 2 && m.is_contiguous() && codebook.is_cuda() && codebook.device() == m.device() && codebook.is_contiguous() &&
            codebook.scalar_type() == at::kHalf && (codebook.dim() == 2 || codebook.dim() == 3) && codebook.size(-1) > 0 &&
            m.device().index() == c10::hip::current_device() && (m.size(1) * per_column) % codebook.size(-1) == 0 &&
            (codebook.dim() == 2 || (codebook.size(0) > 0 && m.size(0) % codebook.size(0) == 0));
 }
 
-py::object encode(const Tensor &w, const Tensor &codebook)
+py::object encode(py::handle w_h, py::handle codebook_h)
 {
-    if (!codec_operands(w, codebook, 1) || w.scalar_type() != at::kHalf) return py::none();
+    const Tensor &w = tensor_of(w_h), &codebook = tensor_of(codebook_h);
+    if (!codec_operands(w_h, codebook_h, 1) || w.scalar_type() != at::kHalf) return py::none();
     const int64_t N = w.size(0), K = w.size(1), vec = codebook.size(-1), entries = codebook.size(-2);
     const int bits = entries <= 256 ? 8 : 16;
     Tensor codes;
@@ -347,10 +362,11 @@ py::object encode(const Tensor &w, const Tensor &codebook)
     return py::cast(codes);
 }
 
-py::object dequant(const Tensor &codes, const Tensor &codebook)
+py::object dequant(py::handle codes_h, py::handle codebook_h)
 {
+    const Tensor &codes = tensor_of(codes_h), &codebook = tensor_of(codebook_h);
     const bool u8 = codes.scalar_type() == at::kByte;
-    if ((!u8 && codes.scalar_type() != at::kUInt16) || !codec_operands(codes, codebook, codebook.dim() > 0 ? codebook.size(-1) : 1)) return py::none();
+    if ((!u8 && codes.scalar_type() != at::kUInt16) || !codec_operands(codes_h, codebook_h, codebook.dim() > 0 ? codebook.size(-1) : 1)) return py::none();
     const int64_t N = codes.size(0), vec = codebook.size(-1), K = codes.size(1) * vec;
     Tensor w;
     int rc;
@@ -380,13 +396,14 @@ Tensor first_of_permutations(int64_t n, int64_t count, int64_t books, int64_t se
 
 // (codes, codebook, squared errors [iters + 1] on the device) of Lloyd iterations from the vectors `pick`, or None where the library
 // has no kernel for the codebook's size.  The caller has checked w: fp16 [N, K] on the GPU, contiguous.
-py::object kmeans(const Tensor &w, const Tensor &pick, int64_t vec, int64_t entries, int64_t books, int64_t code_bits, int64_t iters)
+py::object kmeans(py::handle w_h, const Tensor &pick, int64_t vec, int64_t entries, int64_t books, int64_t code_bits, int64_t iters)
 {
+    const Tensor &w = tensor_of(w_h);
     const int64_t N = w.size(0), K = w.size(1);
     TORCH_CHECK_VALUE(w.is_cuda() && w.scalar_type() == at::kHalf && w.is_contiguous() && pick.scalar_type() == at::kInt &&
                           pick.numel() == books * entries && pick.is_contiguous() && vec > 0 && K % vec == 0 && books > 0 && N % books == 0,
                       "kmeans: w fp16 [N, K] on the GPU, pick int32 [books, entries]");
-    if (!plain_python_call({&w})) return py::none();
+    if (!plain_python_call({w_h})) return py::none();
     const int64_t need = vqgemm_kmeans_workspace_bytes_b(N, K, (int)vec, (int)entries, (int)books, (int)code_bits);
     if (need < 0 || (reinterpret_cast<uintptr_t>(w.data_ptr()) & 7) != 0) return py::none();
     const c10::OptionalDeviceGuard guard(w.device());
