@@ -285,9 +285,11 @@ constexpr int kStageOverTable = 1, kStageOverSlots = 2;
 __device__ __forceinline__ const half_t *bias_of() { return nullptr; }
 __device__ __forceinline__ const half_t *bias_of(const half_t *b) { return b; }
 __device__ __forceinline__ const half_t *bias_of(const half_t *b, int) { return b; }
+__device__ __forceinline__ const half_t *bias_of(const half_t *b, int, int) { return b; }
 __device__ __forceinline__ int k_x_of(int K) { return K; }
 __device__ __forceinline__ int k_x_of(int K, const half_t *) { return K; }
 __device__ __forceinline__ int k_x_of(int, const half_t *, int k_x) { return k_x; }
+__device__ __forceinline__ int k_x_of(int, const half_t *, int k_x, int) { return k_x; }
 
 //
 // GATED: the epilogue of a gate/up pair.  The rows of W are gate and up rows interleaved in groups of 16, so an
@@ -309,10 +311,13 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     typedef LaneCodes<VEC, CodeT> Codes;
     // The bias pointer is a kernel argument only in the instantiation that adds one, so that a
     // launch without bias fetches and tests nothing for it.  The instantiation with a second extra argument, the number of
-    // columns of X, takes what the common shapes do without testing for: K that is no multiple of a slice, N that is none of a
-    // tile, an X that repeats along K, a bias that may be missing.  (A short launch is bound by what its prologue does one
-    // after the other: with those tests in every launch 16 rows of X on K = 4096, N = 1024 took 6.46 us instead of 6.22.)
-    constexpr bool kAny = sizeof...(Bias) == 2;
+    // columns of X, takes what the common shapes do without testing for: N that is no multiple of a
+    // tile, an X that repeats along K, a bias that may be missing; with a third one (unused) also K that is none of a slice.
+    // (A short launch is bound by what its prologue does one
+    // after the other: with those tests in every launch 16 rows of X on K = 4096, N = 1024 took 6.46 us instead of 6.22.  And
+    // every instruction of a gather counts: two additive stages, 5 rows of X, K = 8192, N = 4096 take 6.84 us, with the masks of
+    // a cut K 7.03.)
+    constexpr bool kAny = sizeof...(Bias) >= 2, kCut = sizeof...(Bias) == 3;
     constexpr bool kHasBias = sizeof...(Bias) > 0;
     const half_t *bias = bias_of(bias_arg...);
     // All kernel arguments are fetched at once: left to first use, each pointer costs the
@@ -337,7 +342,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // K goes in n_chunks chunks of (at most) n_waves slices of 256 k: wave w owns slice w of the
     // current chunk; the last chunk may leave the upper waves without one.
     const int n_waves = blockDim.x >> 6;
-    const int total_slices = kAny ? (K + kSliceK - 1) / kSliceK : K / kSliceK;  // (the last one may end short: K is a multiple of a lane load's k)
+    const int total_slices = kCut ? (K + kSliceK - 1) / kSliceK : K / kSliceK;  // (the last one may end short: K is a multiple of a lane load's k)
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int r16 = lane & 15;  // W row within the tile (A operand) / X row m (B operand)
@@ -349,7 +354,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // zeros for the lane loads past the end of K: the pad of the first slot, which nothing else is written to but staged X
     const uint32_t zeros = red_base + kSlotPitch - 16;
     auto store_zeros = [&]() {
-        if (kAny && w == 0) reinterpret_cast<uint32_t *>(smem + zeros)[opaque(lane) & 3] = (uint32_t)opaque(0);
+        if (kCut && w == 0) reinterpret_cast<uint32_t *>(smem + zeros)[opaque(lane) & 3] = (uint32_t)opaque(0);
     };
 
     // blockIdx.x picks the codebooks.  Either wgs_per_cb workgroups share the tiles_per_cb tiles
@@ -377,12 +382,12 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // reads 64*LB consecutive bytes instead of 16 pieces of 4*LB.
     constexpr int kLoadPitch = PACKED ? 64 * C::LB : 4 * C::LB;  // bytes between the loads of a slice
     // A lane load past the end of K (in a short last slice) reads the row's first codes of the chunk instead and gathers zeros.
-    constexpr bool kOneOffset = PACKED || !kAny;
+    constexpr bool kOneOffset = PACKED || !kCut;
     uint32_t voff[kOneOffset ? 1 : C::LPT];
     auto set_voff = [&]() {
         if constexpr (PACKED) {
             voff[0] = (uint32_t)((w * C::LPT * 64 + lane) * C::LB);
-        } else if constexpr (!kAny) {
+        } else if constexpr (!kCut) {
             voff[0] = (uint32_t)((r16 * J + (w * kSliceK + kq * C::K_LANE) / VEC) * (int)sizeof(CodeT));
         } else {
 #pragma unroll
@@ -399,7 +404,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
     // with the same result)
     auto tile_row = [&](int tile) { return kAny ? min(tile * kTileN, N - kTileN) : tile * kTileN; };
     const int chunk_bytes = n_waves * kSliceK / VEC * (int)sizeof(CodeT) * (PACKED ? kTileN : 1);
-    GatherFrom<VEC, CodeT, REPL, kAny> from;
+    GatherFrom<VEC, CodeT, REPL, kCut> from;
     auto set_gathers = [&]() {
         from.set(REPL ? (lane % (256 / kEntryBytes)) * kEntryBytes : 0, zeros, (chunk * n_waves + w) * kSliceK + kq * C::K_LANE, K);
     };
@@ -508,7 +513,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
         }
         // a slice that K cuts short: zeros behind its end
         const int k_left = K - chunk * n_waves * kSliceK - k0;
-        if (kAny && k_left < kSliceK) {
+        if (kCut && k_left < kSliceK) {
 #pragma unroll
             for (int s = 0; s < kSteps; s++)
                 if ((s / C::SPL) * C::K_WAVE + kg * C::K_LANE + (s % C::SPL) * 8 >= k_left) xr[s] = half8_t{};
@@ -526,7 +531,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
         __syncthreads();  // every wave has picked up its X before the staging area is written again
         if (stage_over & kStageOverTable) store_codebook();
         store_zeros();
-        if (kAny || (stage_over & kStageOverTable)) __syncthreads();
+        if (kCut || (stage_over & kStageOverTable)) __syncthreads();
     }
 
     // Partial results: slot (j, kq, m) = (j*4 + kq)*M + m for tile j of the unit; this lane writes
@@ -692,10 +697,10 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
         }
         n_act = min(n_waves, total_slices - chunk * n_waves);
         active = w < n_act;
-        if constexpr (kAny) set_voff();
+        if constexpr (kCut) set_voff();
         // The first codes are requested before the table or X are replaced, to overlap the latencies.
         load_first_units();
-        if constexpr (kAny) set_gathers();
+        if constexpr (kCut) set_gathers();
         __syncthreads();  // every gather from the old table has been consumed, every slot read
         // (a chunk that starts where X repeats has the X of the chunk before it, unless K cuts its last slice short)
         const bool new_x = n_chunks > 1 && (!kAny || n_waves * kSliceK != k_x || n_act != n_waves);
@@ -719,7 +724,7 @@ __global__ __launch_bounds__(1024) void decode_batched_kernel(const half_t *__re
             pick_x();
         }
         __syncthreads();  // X picked up before the slots (which the staging area may lie over) are written
-        if (kAny && new_x) {
+        if (kCut && new_x) {
             store_zeros();
             __syncthreads();
         }
@@ -851,6 +856,24 @@ BatchedPlan plan_batched(const ProblemB &p)
     }
 }
 
+// The batched kernel's instance with the tests of `any`: bias and columns of X, and one more where K is no multiple of a slice.
+template <int VEC, typename CodeT, typename Launch, typename... Any>
+hipError_t launch_decode_any(const ProblemB &p, const BatchedPlan &g, Launch launch, Any... any)
+{
+    typedef DecodeCfg<VEC, CodeT> C;
+    // (gate and up rows come in whole tiles and meet one X: only K can be what brings a gated product here)
+    if constexpr (C::TB % 2 == 0 && sizeof...(Any) == 3) {
+        if (p.gated) return g.repl ? launch(decode_batched_kernel<VEC, CodeT, true, C::TB, false, true, Any...>, any...)
+                                   : launch(decode_batched_kernel<VEC, CodeT, false, C::TB, false, true, Any...>, any...);
+    }
+    if (p.gated) return hipErrorInvalidValue;
+    const bool one = !g.full || C::TB == 1;
+    if (g.repl) return one ? launch(decode_batched_kernel<VEC, CodeT, true, 1, false, false, Any...>, any...)
+                           : launch(decode_batched_kernel<VEC, CodeT, true, C::TB, false, false, Any...>, any...);
+    return one ? launch(decode_batched_kernel<VEC, CodeT, false, 1, false, false, Any...>, any...)
+               : launch(decode_batched_kernel<VEC, CodeT, false, C::TB, false, false, Any...>, any...);
+}
+
 template <int VEC, typename CodeT, bool PACKED>
 hipError_t launch_decode_batched(const ProblemB &p, hipStream_t s)
 {
@@ -872,17 +895,8 @@ hipError_t launch_decode_batched(const ProblemB &p, hipStream_t s)
     const int tb = g.full ? C::TB : 1;
     if constexpr (!PACKED) {
         // K that is no multiple of a slice, N that is none of a tile, an X that repeats: the instantiations that test for those
-        if (p.K % kSliceK != 0 || p.N % kTileN != 0 || p.k_x != p.K) {
-            if constexpr (C::TB % 2 == 0) {
-                if (p.gated) return g.repl ? launch(decode_batched_kernel<VEC, CodeT, true, C::TB, false, true, const half_t *, int>, p.bias, p.k_x)
-                                           : launch(decode_batched_kernel<VEC, CodeT, false, C::TB, false, true, const half_t *, int>, p.bias, p.k_x);
-            }
-            if (p.gated) return hipErrorInvalidValue;
-            if (g.repl) return tb == 1 ? launch(decode_batched_kernel<VEC, CodeT, true, 1, false, false, const half_t *, int>, p.bias, p.k_x)
-                                       : launch(decode_batched_kernel<VEC, CodeT, true, C::TB, false, false, const half_t *, int>, p.bias, p.k_x);
-            return tb == 1 ? launch(decode_batched_kernel<VEC, CodeT, false, 1, false, false, const half_t *, int>, p.bias, p.k_x)
-                           : launch(decode_batched_kernel<VEC, CodeT, false, C::TB, false, false, const half_t *, int>, p.bias, p.k_x);
-        }
+        if (p.K % kSliceK != 0) return launch_decode_any<VEC, CodeT>(p, g, launch, p.bias, p.k_x, 0);
+        if (p.N % kTileN != 0 || p.k_x != p.K) return launch_decode_any<VEC, CodeT>(p, g, launch, p.bias, p.k_x);
     }
     if constexpr (!PACKED && C::TB % 2 == 0) {
         if (p.gated) {
