@@ -1986,6 +1986,31 @@ def test_infinite_codewords_reach_their_own_rows_only_and_as_infinities(M, K, N,
     assert cabi.VARIANT_GENERIC in ran and (M > 64 or cabi.VARIANT_DECODE in ran)
 
 
+@pytest.mark.parametrize("M,K,N,G", [(1, 2080, 48, 1), (2, 2080, 33, 1), (1, 8224, 64, 1), (2, 6176, 4096, 1), (1, 14336, 40, 1), (2, 14336, 2048, 1), (1, 4096, 32, 1)])
+def test_a_row_that_ends_in_an_infinite_codeword_is_infinite_in_the_gemv_kernels(M, K, N, G):
+    """The long form reads a row's last codes once more where K ends inside a piece of it."""
+    spec = ProblemSpec("inf", GEOM_B, M, K, N, 8, 256, G, 8, codebook_3d=(G > 1), codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=97, device=DEV)
+    x = (x.float().abs() + 0.1).half()
+    c = codes.to(torch.int32)
+    c = torch.where(c < 2, torch.full_like(c, 2), c)
+    c[::3, -1] = 1
+    c[1, 0], c[1, 1] = 0, 1                    # plus and minus infinity meet: NaN by the definition
+    codes = c.to(codes.dtype)
+    cb[..., 0, :], cb[..., 1, :] = -float("inf"), float("inf")
+    w = vo.dequant_b(_np(codes), _np(cb)).astype(np.float64)
+    hit, plain = np.zeros(N, bool), np.ones(N, bool)
+    hit[::3] = True
+    plain[::3] = plain[1] = False
+    want = _np(x).astype(np.float64) @ w[plain].T
+    bias = torch.ones(N, dtype=torch.float16, device=DEV)
+    for variant in (cabi.VARIANT_DECODE_GEMV, cabi.VARIANT_AUTO, cabi.VARIANT_GENERIC):
+        _say("infinite last codewords", M, K, N, G, cabi.VARIANT_NAMES[variant])
+        y = _np(cabi.e2e_gemm_b(x, codes, cb, variant=variant, bias=bias))
+        assert np.isposinf(y[:, hit]).all() and np.isnan(y[:, 1]).all(), (variant, int(np.isnan(y[:, hit]).sum()))
+        assert vo.rel_err(y[:, plain], want + 1.0)[0] <= TOL, variant
+
+
 LLOYD_B = [
     # N, K, vec, entries, G: codebooks in several workgroups, entries nothing is assigned to, a last tile of entries cut short
     (512, 1024, 8, 256, 2),
