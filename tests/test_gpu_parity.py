@@ -2147,6 +2147,54 @@ def test_k_dealt_out_to_waves_geometry_b(row):
             assert vo.rel_err(_np(y), gated)[1] <= TOL, (row, tile, "gated")
 
 
+@pytest.mark.parametrize("row", WAVE_K_B + [(81, 192, 80, 8, 256, 8, 1), (97, 1088, 66, 4, 16, 8, 1), (31, 128, 130, 8, 300, 16, 1)],
+                         ids=lambda r: "x".join(map(str, r)))
+def test_k_dealt_out_to_waves_tall_and_wide_tiles(row):
+    """32 x 128, 48, 80 and 96 x 64: an odd number of rows of pieces, one step a unit and two, edges on both sides."""
+    M, K, N, v, E, bits, G = row
+    spec = ProblemSpec("wave_k", GEOM_B, M, K, N, v, E, G, bits, codebook_3d=(G > 1), codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=93, device=DEV)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(6)).half().to(DEV)
+    want = _np(x).astype(np.float64) @ vo.dequant_b(_np(codes), _np(cb)).astype(np.float64).T + _np(bias).astype(np.float64)
+    ran = 0
+    for tile in (28, 34, 54, 64):
+        _say("wave_k", row, "tile", tile)
+        try:
+            y = _with_wave_tile(tile, lambda: cabi.e2e_gemm_b(x, codes, cb, variant=cabi.VARIANT_WAVE_K, bias=bias))
+        except cabi.VqGemmError:
+            continue   # no room for this tile's units beside the tables
+        torch.cuda.synchronize()
+        assert vo.rel_err(_np(y), want)[0] <= TOL, (row, tile)
+        ran += 1
+        if N % 32 == 0:
+            y = _with_wave_tile(tile, lambda: cabi.e2e_gemm_b_gated(x, codes, cb, variant=cabi.VARIANT_WAVE_K, bias=bias))
+            p = want.reshape(M, N // 32, 2, 16)
+            gated = (p[:, :, 0] / (1 + np.exp(-p[:, :, 0])) * p[:, :, 1]).reshape(M, N // 2)
+            torch.cuda.synchronize()
+            assert vo.rel_err(_np(y), gated)[1] <= TOL, (row, tile, "gated")
+    assert ran == (2 if v == 4 and bits == 16 else 4)   # (32 bytes of codes a row and unit: 80 and 96 x 64 only)
+
+
+@pytest.mark.parametrize("vec", [4, 8])
+@pytest.mark.parametrize("M,K,N,E", [(1, 128, 6, 256), (16, 192, 258, 1 << 7), (33, 1088, 130, 254), (40, 4160, 34, 8), (32, 2048, 642, 256)])
+def test_copies_of_the_codebook_change_no_bit(vec, M, K, N, E):
+    """One codebook: a table of copies, where the tile has one.  The same codebook twice, each for half of the columns, such that
+    tiles meet both: the plain table.  The same operands meet in the same order.  Infinite and NaN entries too."""
+    spec = ProblemSpec("wave_k", GEOM_B, M, K, N, vec, E, 1, 8, codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=94, device=DEV)
+    for special in (False, True):
+        if special:
+            cb[E - 1, 0], cb[E // 2, vec - 1], cb[0, 1] = float("inf"), float("nan"), float("-inf")
+        twice = torch.stack([cb, cb]).contiguous()
+        for tile in (12, 14, 18, 22, 24, 28):
+            _say("copies", vec, M, K, N, E, special, "tile", tile)
+            assert (N // 2) % (tile % 10 * 16) != 0
+            one = _with_wave_tile(tile, lambda: cabi.e2e_gemm_b(x, codes, cb, variant=cabi.VARIANT_WAVE_K))
+            two = _with_wave_tile(tile, lambda: cabi.e2e_gemm_b(x, codes, twice, variant=cabi.VARIANT_WAVE_K))
+            torch.cuda.synchronize()
+            assert torch.equal(one.view(torch.int16), two.view(torch.int16)), tile
+
+
 @pytest.mark.parametrize("M,K,N", [(1, 64, 8), (17, 96, 40), (33, 320, 65), (65, 1056, 2047), (130, 2048, 129), (16, 512, 64)])
 @pytest.mark.parametrize("shift", [0, 1])   # elements by which w is off a 16-byte boundary
 def test_k_dealt_out_to_waves_plain_gemm(M, K, N, shift):

@@ -290,11 +290,11 @@ struct WorkspaceChoice {
     size_t bytes;
 };
 // Above 64 rows of X the wave-K kernel is taken below this share of what the other plan is expected to take: the tiled kernels by
-// more than the models' error, split K (whose model is as close as the wave-K kernel's) at even odds.  Over 260 shapes of M 65 to
+// more than the models' error, split K (whose model is as close as the wave-K kernel's) at nearly even odds.  Over 260 shapes of M 65 to
 // 4002, 100 of them where split K stood to be taken, the choice is 1.7 % from the best plan measured; at 0.95 for both, with split K's
 // second launch at 4.5 us and no wait for a large X it was 8.7 % (M = 203, K = 2816, N = 7040: 24.9 us split, 20.2 now; M = 657,
 // K = 13376, N = 1040: 39.2 us, split 35.3 now).
-constexpr double kWaveOverTiles = 0.95, kWaveOverSplit = 1.0;
+constexpr double kWaveOverTiles = 0.95, kWaveOverSplit = 0.97;
 
 WorkspaceChoice workspace_auto(const ProblemB &p)
 {

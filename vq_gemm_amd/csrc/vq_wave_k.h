@@ -35,25 +35,29 @@ namespace vq {
 namespace {
 
 constexpr int kStepK = 32;                // k of one MFMA step
+constexpr int kCopiesEntries = 256, kCopiesBytes = kCopiesEntries * 256;   // a table of copies: a row of banks per entry
 
 // What W is and how a unit of it is laid out.  S: MFMA steps of a unit.
 struct WaveDense {       // fp16 [K,N], rows of whole 16-byte chunks
     static constexpr int S = 1;
-    static constexpr bool kDense = true, kAnyN = false, kA = false, kB = false;
+    static constexpr bool kDense = true, kAnyN = false, kA = false, kB = false, kCopies = false;
     static constexpr int VEC = 0, CSZ = 2;
 };
 struct WaveDenseAnyN {   // fp16 [K,N], any N, elements aligned to 2 bytes
     static constexpr int S = 1;
-    static constexpr bool kDense = false, kAnyN = true, kA = false, kB = false;
+    static constexpr bool kDense = false, kAnyN = true, kA = false, kB = false, kCopies = false;
     static constexpr int VEC = 0, CSZ = 2;
 };
 struct WaveA {           // geometry A
     static constexpr int S = 1;
-    static constexpr bool kDense = false, kAnyN = false, kA = true, kB = false;
+    static constexpr bool kDense = false, kAnyN = false, kA = true, kB = false, kCopies = false;
     static constexpr int VEC = 2, CSZ = 1;
 };
-template <int VEC_, typename CodeT_, int S_>
+// COPIES: the table holds one codebook of at most 256 entries, each as often as fills a row of the 64 banks (16 copies of
+// an 8-vector, 32 of a 4-vector), and a lane gathers its own copy: no two lanes of a gather meet in a bank.
+template <int VEC_, typename CodeT_, int S_, bool COPIES_ = false>
 struct WaveB {           // geometry B
+    static constexpr bool kCopies = COPIES_;
     static constexpr int S = S_;
     static constexpr bool kDense = false, kAnyN = false, kA = false, kB = true;
     static constexpr int VEC = VEC_, CSZ = (int)sizeof(CodeT_);
@@ -61,6 +65,14 @@ struct WaveB {           // geometry B
 
 // Waves of a workgroup: two on every SIMD, one's MFMAs beside the other's reads, where their accumulators leave room for two.
 constexpr int wave_count(int mp, int np) { return mp * np > 32 ? 4 : 8; }
+
+// Rows of pieces whose partial sums, `per_row` KB of them each, fit the LDS together: the most that divide the tile's.
+constexpr int pass_rows(int mp, int per_row)
+{
+    int rows = mp;
+    while (rows > 1 && (mp % rows != 0 || rows * per_row > 160)) rows--;
+    return rows;
+}
 
 // MP x NP pieces of 16 x 16: the tile.
 template <class P, int MP, int NP>
@@ -78,18 +90,18 @@ struct WaveKCfg {
     static constexpr int kUnitBytes = kXBytes + kWLoads * 1024;
     static constexpr int kLoads = S * MP + kWLoads;                                        // direct loads of a wave and unit
     static constexpr int kBooks = P::kA ? TN / 8 * 1024 : 0;                                 // bytes of codebooks known here
-    static constexpr int kRoom = 160 * 1024 - (P::kB ? (P::CSZ == 2 ? 33 : 5) * 1024 : kBooks);
+    static constexpr int kRoom = 160 * 1024 - (P::kCopies ? kCopiesBytes : P::kB ? (P::CSZ == 2 ? 33 : 5) * 1024 : kBooks);
     static constexpr int kFit = kRoom / (kWaves * kUnitBytes);
     static constexpr int D = kFit > 6 ? 6 : kFit;                                           // units in the LDS per wave
     static constexpr int kRing = kWaves * D * kUnitBytes;
-    static constexpr int kPassMP = MP * NP * kWaves <= 128 ? MP : MP * NP * kWaves <= 256 ? MP / 2 : MP / 4;   // rows of pieces summed in one pass
+    static constexpr int kPassMP = pass_rows(MP, NP * kWaves);                              // rows of pieces summed in one pass
     static constexpr int kSumBytes = kWaves * kPassMP * NP * 1024;
     static constexpr bool kExists = D >= 2;   // the LDS holds two units of every wave
     static_assert(D * kLoads < 64 && kPassMP >= 1 && MP % kPassMP == 0 && kSumBytes <= 160 * 1024, "counts of loads, passes of the sum");
     // (`books` bytes of codebooks, copied in steps of a wave load)
     static constexpr size_t lds_bytes(size_t books)
     {
-        const size_t use = kRing + copied_bytes(books);
+        const size_t use = kRing + (P::kCopies ? (size_t)kCopiesBytes : copied_bytes(books));
         return use > (size_t)kSumBytes ? use : (size_t)kSumBytes;
     }
 };
@@ -126,6 +138,28 @@ struct WaveKArgs {
     int entries, rows_per_cb, books;   // (geometry B) books: codebooks of a tile
     int gated;
 };
+
+// The entry of a table of copies by a load that the compiler does not count, beside the direct loads, which it does not either:
+// it would wait for all of them.  The registers are not to be read ahead of loaded_entry, behind the wait.
+template <int DW>
+__device__ __forceinline__ void load_entry(uint32_t (&entry)[DW], const half_t *src)
+{
+    typedef uint32_t entry_t __attribute__((ext_vector_type(DW)));
+    entry_t v;
+    if constexpr (DW == 4) asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(v) : "v"(src) : "memory");
+    else asm volatile("global_load_dwordx2 %0, %1, off" : "=&v"(v) : "v"(src) : "memory");
+#pragma unroll
+    for (int i = 0; i < DW; i++) entry[i] = v[i];
+}
+
+// sixteen bytes of a row of copies: the entry, or two side by side
+template <int DW>
+__device__ __forceinline__ uint4_t loaded_entry(uint32_t (&entry)[DW])
+{
+#pragma unroll
+    for (int i = 0; i < DW; i++) asm volatile("" : "+v"(entry[i]));
+    return uint4_t{entry[0], entry[1], entry[DW == 4 ? 2 : 0], entry[DW == 4 ? 3 : 1]};
+}
 
 template <class P, int MP, int NP>
 __global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) void wave_k_kernel(const WaveKArgs a)
@@ -240,11 +274,11 @@ __global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) vo
         for (int j = 0; j < NP; j++)
             w_rd[j] = ring + C::kXBytes + k * (kRowChunks * 16) + (r16 & 1) * 8 + ((2 * j + ((r16 & 3) >> 1)) ^ wave_w_swizzle<NP>(k)) * 16;
     } else {
-        // codebook of the piece's row
+        // codebook of the piece's row, or the lane's copy in it
         const int g_first = n0 / a.rows_per_cb;
 #pragma unroll
         for (int j = 0; j < NP; j++)
-            w_rd[j] = kBookBase + (uint32_t)((min(n0 + j * 16 + r16, N - 1) / a.rows_per_cb - g_first) * a.entries * (P::VEC * 2));
+            w_rd[j] = P::kCopies ? kBookBase + (uint32_t)(lane * (P::VEC * 2) & 255) : kBookBase + (uint32_t)((min(n0 + j * 16 + r16, N - 1) / a.rows_per_cb - g_first) * a.entries * (P::VEC * 2));
     }
     const uint32_t code_rd = ring + C::kXBytes + (C::kCodeBytes == 32 ? (kg >> 1) * (C::kRows * 16) + (kg & 1) * 8 : kg * (C::kCodeBytes / 4)) + r16 * 16;
     typedef short short4_t __attribute__((__vector_size__(4 * sizeof(short))));
@@ -304,16 +338,17 @@ __global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) vo
                 ws[set][2 * q + 1] = __builtin_bit_cast(half8_t, odd);
             }
         } else if constexpr (P::kB) {
+            constexpr int kEntry = P::kCopies ? 256 : P::VEC * 2;   // bytes from entry to entry
 #pragma unroll
             for (int j = 0; j < NP; j++) {
                 if constexpr (P::VEC == 8) {
                     const uint32_t c = P::CSZ == 1 ? (code_b[j][0] >> (8 * s)) & 0xffu : (code_b[j][0] >> (16 * s)) & 0xffffu;
-                    ws[set][j] = *reinterpret_cast<const half8_t *>(smem + w_rd[j] + c * 16);
+                    ws[set][j] = *reinterpret_cast<const half8_t *>(smem + w_rd[j] + c * kEntry);
                 } else {
                     const uint32_t pair = P::CSZ == 1 ? (code_b[j][0] >> (16 * s)) & 0xffffu : code_b[j][C::kCodeBytes == 32 ? s : 0];
                     const uint32_t c_lo = P::CSZ == 1 ? pair & 0xffu : pair & 0xffffu, c_hi = P::CSZ == 1 ? pair >> 8 : pair >> 16;
-                    const half4_t lo = *reinterpret_cast<const half4_t *>(smem + w_rd[j] + c_lo * 8);
-                    const half4_t hi = *reinterpret_cast<const half4_t *>(smem + w_rd[j] + c_hi * 8);
+                    const half4_t lo = *reinterpret_cast<const half4_t *>(smem + w_rd[j] + c_lo * kEntry);
+                    const half4_t hi = *reinterpret_cast<const half4_t *>(smem + w_rd[j] + c_hi * kEntry);
                     ws[set][j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
                 }
             }
@@ -358,7 +393,12 @@ __global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) vo
     };
 
     // ---- codebooks, first units -------------------------------------------------------------------
-    if constexpr (P::kA || P::kB) {
+    uint32_t entry[P::VEC == 4 ? 2 : 4];   // (copies) the thread's, on its way until the wait below
+    if constexpr (P::kCopies) {
+        static_assert(P::VEC == 8 || P::VEC == 4, "entries of 16 or 8 bytes");
+        const half_t *src = a.cb + ((int64_t)(n0 / a.rows_per_cb) * a.entries + min(tid & (kCopiesEntries - 1), a.entries - 1)) * P::VEC;
+        load_entry(entry, src);
+    } else if constexpr (P::kA || P::kB) {
         const int book_bytes = P::kA ? 1024 : a.entries * (P::VEC * 2);
         const int g_first = P::kA ? n0 / 8 : n0 / a.rows_per_cb;
         const int n16 = (P::kA ? C::TN / 8 : a.books) * book_bytes / 16;
@@ -371,7 +411,18 @@ __global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) vo
 #pragma unroll
     for (int d = 0; d < D; d++)
         if (d < n_unit) issue(d, d);
-    if constexpr (P::kA || P::kB) {
+    if constexpr (P::kCopies) {
+        // (the entry is the oldest load)
+        if (n_unit >= D) wait_vmcnt<D * C::kLoads>();
+        else wait_vmcnt<0>();
+        // two threads an entry, eight pieces of 16 bytes each, neighbouring entries in another order
+        static_assert(kWaves * 64 == 2 * kCopiesEntries, "two threads an entry");
+        const uint4_t piece = loaded_entry(entry);
+        const uint32_t at = kBookBase + (tid & (kCopiesEntries - 1)) * 256 + (tid >> 8) * 128 + (tid & 7) * 16;
+#pragma unroll
+        for (int i = 0; i < 8; i++) *reinterpret_cast<uint4_t *>(smem + (at ^ (i * 16))) = piece;
+        __syncthreads();
+    } else if constexpr (P::kA || P::kB) {
         // (the codebooks are the oldest loads of the waves that brought them)
         if (n_unit >= D) wait_vmcnt<D * C::kLoads>();
         else wait_vmcnt<0>();
@@ -509,11 +560,11 @@ hipError_t launch_tile(WaveKArgs a, hipStream_t s)
 }
 
 // What a tile of mp x np pieces (10 * mp + np) costs, fitted to measurements: microseconds besides its units of 32 k (their
-// first latency, the sum over the waves, the stores), cycles per unit on an idle device, and how many more when every compute
-// unit works.
+// first latency, the sum over the waves, the stores), cycles per unit on an idle device, how many more when every compute
+// unit works, and by which share a unit takes longer with every doubling of X beyond 2 MB (geometry B).
 struct WaveKTile {
     int tile;
-    double fixed_us, idle_clk, busy_clk;
+    double fixed_us, idle_clk, busy_clk, wait = 0.05;
 };
 
 // Microseconds a launch is expected to take (a tenth off, either way): the tiles go over the compute units in rounds.

@@ -15,6 +15,14 @@ struct Format {
     static constexpr int VEC = VEC_, CSZ = (int)sizeof(CodeT_);
     template <int MP, int NP>
     using Wave = WaveB<VEC_, CodeT_, ((MP * NP > 16 || (CSZ == 2 && MP >= 4)) ? 1 : 2)>;
+    // Tiles of up to 32 rows gather more than they read of X: with a table of copies, 64 KB of the LDS that their units leave,
+    // the gathers' bank conflicts go, M = 128, K = N = 4096 9.5 -> 9.0 us, M = 16, K = 2048, N = 11008 6.7 -> 6.0, tiles of
+    // 32 x 128 14.5 -> 12.0.  Taller ones read X twice as long as they gather and would keep half the units in flight: 64 x 64
+    // with 32 KB of copies 13.7 -> 15.0.
+    template <int MP, int NP>
+    static constexpr bool kHasCopies = CSZ == 1 && MP <= 2;
+    template <int MP, int NP>
+    using Copies = WaveB<VEC_, CodeT_, Wave<MP, NP>::S, true>;
 };
 
 // calls f with the pieces of the tile (10 * rows + columns), as types
@@ -30,8 +38,19 @@ void with_tile(int tile, F f)
     case 24: f(integral_constant<int, 2>{}, integral_constant<int, 4>{}); break;
     case 44: f(integral_constant<int, 4>{}, integral_constant<int, 4>{}); break;
     case 48: f(integral_constant<int, 4>{}, integral_constant<int, 8>{}); break;
+    case 34: f(integral_constant<int, 3>{}, integral_constant<int, 4>{}); break;
+    case 54: f(integral_constant<int, 5>{}, integral_constant<int, 4>{}); break;
+    case 64: f(integral_constant<int, 6>{}, integral_constant<int, 4>{}); break;
+    case 28: f(integral_constant<int, 2>{}, integral_constant<int, 8>{}); break;
     default: break;
     }
+}
+
+// Whether the tile's kernel with a table of copies serves the problem: 8-bit codes, tiles that meet one codebook.
+template <class F, int MP, int NP>
+bool takes_copies(const ProblemB &p)
+{
+    return F::template kHasCopies<MP, NP> && codebooks_per_tile(p, NP * 16) == 1;
 }
 
 template <class F>
@@ -49,27 +68,34 @@ template <class F>
 WaveKPlan plan_b(const ProblemB &p)
 {
     const int forced = (int)tuning().wave_k_force_tile;
-    // (16-bit codes bring tables whose entries collide more often)
-    constexpr WaveKTile kTiles8[] = {{12, 2.2, 39, 14}, {14, 2.5, 65, 28}, {18, 3.2, 118, 62}, {22, 2.4, 44, 19}, {24, 3.0, 68, 29}, {44, 4.0, 95, 68}, {48, 6.1, 180, 165}};
-    constexpr WaveKTile kTiles16[] = {{12, 2.6, 45, 19}, {14, 2.8, 79, 59}, {18, 3.0, 169, 200}, {22, 2.7, 52, 24}, {24, 3.0, 91, 45}, {44, 3.5, 124, 112}, {48, 5.9, 214, 182}};
-    // An X of more than the 4 MB of an XCD's L2 keeps the units waiting, 15 % longer from 16 MB on whatever the tile, and tiles of
-    // 64 x 64 in several rounds another 30 % from 1500 rows on: M = 2168, K = 7808, N = 1024 takes 95 us, M = 3028, K = 11264, N = 640
-    // 98 us, expected 64 without the two.  Over 192 shapes of M 66 to 4002 measured and expected time differ by 10 % (15 % without).
-    const double octaves = std::log2(2.0 * p.M * p.K / 2e6);
-    const double wait = 1.0 + 0.15 * (octaves < 0.0 ? 0.0 : octaves > 3.0 ? 1.0 : octaves / 3.0);
+    // Fitted to 1700 launches of both vector lengths, K 512 to 12288, 24 to 700 tiles (a twentieth off; the tiles whose units are
+    // one step, 64 x 128, 80 x 64 and 96 x 64 - with 16-bit codes 64 x 64 too - a tenth, and 80 and 96 x 64, of which one launch in
+    // ten took half as long again, are set a tenth above their fit).  (16-bit codes bring tables whose entries collide more often)
+    constexpr WaveKTile kTiles8[] = {{12, 2.0, 40, 13}, {14, 2.3, 63, 22}, {18, 2.9, 116, 45}, {22, 2.2, 47, 21}, {24, 2.8, 70, 33}, {28, 4.4, 120, 57, 0.08},
+                                     {34, 3.5, 81, 31, 0.15}, {44, 4.3, 94, 47, 0.08}, {48, 7.0, 160, 100, 0.27}, {54, 5.3, 110, 85, 0.45}, {64, 5.7, 120, 100, 0.45}};
+    constexpr WaveKTile kTiles16[] = {{12, 2.6, 45, 19}, {14, 2.8, 79, 59}, {18, 3.0, 169, 200}, {22, 2.7, 52, 24}, {24, 3.0, 91, 45}, {28, 4.1, 124, 41, 0.11},
+                                      {34, 3.6, 75, 32, 0.17}, {44, 4.2, 92, 92, 0.20}, {48, 6.4, 200, 140, 0.15}, {54, 5.3, 130, 110, 0.45}, {64, 5.7, 140, 120, 0.45}};
+    constexpr WaveKTile kTilesCopies[] = {{12, 2.1, 34, 12}, {14, 2.4, 45, 17}, {18, 2.7, 76, 38}, {22, 2.4, 41, 17}, {24, 2.7, 58, 38}, {28, 3.9, 103, 30, 0.19}};
+    // An X that does not fit the 4 MB of an XCD's L2 beside the rest keeps the units waiting, the longer the larger it is, and most where
+    // a unit of one step takes half a 128-byte line at a time.
+    const double octaves = std::fmin(3.0, std::fmax(0.0, std::log2(2.0 * p.M * p.K / 2e6)));
+    // Tiles of 64 x 64 in several rounds take another 30 % from 1500 rows on: M = 2168, K = 7808, N = 1024 takes 95 us, M = 3028, K = 11264,
+    // N = 640 98 us, expected 64 without the two.
     const double wait_rows = 1.0 + 0.3 * (p.M < 1000 ? 0.0 : p.M > 1500 ? 1.0 : (p.M - 1000) / 500.0);
     const bool rounds = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) > device_cu_count();
     const double bytes = (double)p.K * p.N * F::CSZ / F::VEC + 2.0 * (double)p.M * (p.K + p.N);
     WaveKPlan best = {0, 0, 1e30};
-    double best_us = 1e30;
-    for (const WaveKTile &t : F::CSZ == 1 ? kTiles8 : kTiles16) {
-        if (forced > 0 && forced != t.tile) continue;
-        if (!fits<F>(p, t.tile)) continue;
-        const double w = t.tile == 44 && rounds ? wait_rows : 1.0, us = wave_k_tile_cost_us(t, p.M, p.K, p.N, bytes, w);
-        if (us < best_us) {
-            best_us = us;
-            best = {t.tile / 10, t.tile % 10, wave_k_tile_cost_us(t, p.M, p.K, p.N, bytes, w * wait)};
-        }
+    for (const WaveKTile &plain : F::CSZ == 1 ? kTiles8 : kTiles16) {
+        if (forced > 0 && forced != plain.tile) continue;
+        if (!fits<F>(p, plain.tile)) continue;
+        WaveKTile t = plain;
+        with_tile(t.tile, [&](auto mp, auto np) {
+            if (!takes_copies<F, mp(), np()>(p)) return;
+            for (const WaveKTile &c : kTilesCopies)
+                if (c.tile == t.tile) t = c;
+        });
+        const double us = wave_k_tile_cost_us(t, p.M, p.K, p.N, bytes, (1.0 + t.wait * octaves) * (t.tile == 44 && rounds ? wait_rows : 1.0));
+        if (us < best.cost_us) best = {t.tile / 10, t.tile % 10, us};
     }
     return best;
 }
@@ -81,9 +107,15 @@ hipError_t launch_b(const ProblemB &p, hipStream_t s, int tile)
         const WaveKPlan plan = plan_b<F>(p);
         tile = plan.mp * 10 + plan.np;
     }
+    if (tile == 0) return hipErrorInvalidValue;   // (the one tile asked for does not fit)
     const WaveKArgs a = {p.x, p.codes, p.cb, p.y, p.bias, p.M, p.K, p.N, p.k_x, 0, 0, p.entries, p.rows_per_cb, codebooks_per_tile(p, tile % 10 * 16), p.gated ? 1 : 0};
     hipError_t e = hipErrorInvalidValue;
     with_tile(tile, [&](auto mp, auto np) {
+        if constexpr (F::template kHasCopies<mp(), np()>)
+            if (takes_copies<F, mp(), np()>(p)) {
+                e = launch_tile<typename F::template Copies<mp(), np()>, mp(), np()>(a, s);
+                return;
+            }
         typedef typename F::template Wave<mp(), np()> P;
         if constexpr (WaveKCfg<P, mp(), np()>::kExists) e = launch_tile<P, mp(), np()>(a, s);
     });
