@@ -45,7 +45,8 @@ extern "C" {
                                      through the streaming kernel of this path: K dealt to the waves in pieces, no
                                      chunks of K */
 #define VQGEMM_VARIANT_PREFILL 3  /* large M: 256x256 tiles of 16x16x32 MFMAs, codewords gathered into operands;
-                                     256x128 tiles when those put more compute units to work */
+                                     256x128 tiles when those put more compute units to work, tiles of 128 to 224
+                                     rows by 128 columns where they go over the units in one round or two */
 #define VQGEMM_VARIANT_TWOPASS 4  /* dequantise to HBM scratch, then the plain fp16 GEMM */
 #define VQGEMM_VARIANT_PREFILL_NARROW 5  /* the prefill kernel with 256x128 tiles, whatever the shape */
 #define VQGEMM_VARIANT_PREFILL_SMALL 6   /* the prefill kernel with 128x128 tiles, two workgroups per compute unit
@@ -109,7 +110,7 @@ int vqgemm_e2e_gemm_b_bias(const void *x, const void *codes, const void *codeboo
 /*
  * vqgemm_e2e_gemm_b_bias with a workspace whose size the library is told, so that the automatic choice may use
  * kernels that need scratch memory: split K over every 128x128 tile (VQGEMM_VARIANT_PREFILL_SPLITK), which
- * VQGEMM_VARIANT_AUTO takes where its cost model expects at least 5 % over what it would launch otherwise, and -
+ * VQGEMM_VARIANT_AUTO takes where its cost models expect it to be ahead of what it would launch otherwise, and -
  * where the large tiles of a shape are a few more than whole rounds over the compute units - those whole rounds as
  * one launch and the columns of W that are left over as a second one, in 128x128 tiles with K split there; either
  * only when `workspace_bytes` suffices (a workspace that is too small, or NULL, is no error for AUTO: it does without).  vqgemm_workspace_bytes_b says

@@ -2110,6 +2110,51 @@ def _with_wave_tile(tile, call):
         cabi.set_tuning(**{k: before[k] for k in ("wave_k_force", "wave_k_force_tile")})
 
 
+@pytest.mark.parametrize("row", [
+    # M, K, N, v, E, bits, G: one row, a row more and less than a tile, K of one and two code tiles and a half one, ragged columns,
+    # a short codebook, tiles that meet several codebooks
+    (1, 128, 8, 8, 256, 8, 1),
+    (129, 192, 129, 8, 256, 8, 1),
+    (160, 1088, 131, 8, 100, 8, 1),
+    (161, 320, 288, 8, 256, 8, 3),
+    (225, 704, 192, 8, 200, 8, 6),
+    (193, 64, 160, 4, 256, 8, 1),
+    (223, 448, 257, 4, 30, 8, 1),
+    (192, 576, 96, 4, 256, 8, 3),
+    (131, 64, 33, 8, 512, 16, 1),
+    (257, 832, 160, 8, 700, 16, 2),
+    (159, 128, 130, 4, 4096, 16, 1),
+    (224, 960, 256, 4, 1024, 16, 2),
+], ids=lambda r: "x".join(map(str, r)))
+def test_prefill_tiles_with_a_compute_unit_to_themselves(row):
+    M, K, N, v, E, bits, G = row
+    spec = ProblemSpec("mid", GEOM_B, M, K, N, v, E, G, bits, codebook_3d=(G > 1), codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=95, device=DEV)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(7)).half().to(DEV)
+    want = _np(x).astype(np.float64) @ vo.dequant_b(_np(codes), _np(cb)).astype(np.float64).T
+    before = cabi.tuning()
+    calls = {"plain": lambda v: cabi.e2e_gemm_b(x, codes, cb, variant=v), "bias": lambda v: cabi.e2e_gemm_b(x, codes, cb, variant=v, bias=bias)}
+    if N % 32 == 0:
+        calls["gated"] = lambda v: cabi.e2e_gemm_b_gated(x, codes, cb, variant=v, bias=bias)
+    for special in (False, True):
+        if special:   # what is not finite goes where the sums of the other tiles take it
+            flat = cb.view(-1, v)
+            flat[E - 1, 0], flat[E // 2, v - 1], flat[0, 1] = float("inf"), float("nan"), float("-inf")
+        for what, call in calls.items():
+            other = call(cabi.VARIANT_PREFILL_SMALL)   # the 128x128 tiles: the same sums in the same order
+            for rows in (128, 160, 192, 224):
+                _say("mid", row, special, what, "rows", rows)
+                try:
+                    cabi.set_tuning(prefill_mid_force=rows)
+                    y = call(cabi.VARIANT_PREFILL)
+                finally:
+                    cabi.set_tuning(prefill_mid_force=before["prefill_mid_force"])
+                torch.cuda.synchronize()
+                assert torch.equal(y.view(torch.int16), other.view(torch.int16)), (row, rows, what)
+                if not special and what == "plain":
+                    assert vo.rel_err(_np(y), want)[0] <= TOL, (row, rows)
+
+
 WAVE_K_B = [
     # M, K, N, vec, E, bits, G: fewer units of K than waves, a last unit shorter than its load, edges of every tile, tiles over
     # several codebooks, a column more than a tile

@@ -137,6 +137,7 @@ const TuningEntry kTuningEntries[] = {
     {"splitk_force_splits", &Tuning::splitk_force_splits},
     {"wave_k_force", &Tuning::wave_k_force},
     {"wave_k_force_tile", &Tuning::wave_k_force_tile},
+    {"prefill_mid_force", &Tuning::prefill_mid_force},
 };
 constexpr int kTuningCount = (int)(sizeof(kTuningEntries) / sizeof(kTuningEntries[0]));
 
@@ -275,7 +276,9 @@ int splitk_auto(const ProblemB &p, double *t_best, int *plain_variant)
     if (t_plain >= 1e29) return 0;  // (short X: the decode path is taken without a comparison, and stays)
     double t_split = 1e30;
     const int sp = prefill_splitk_choice(p, &t_split, 2);
-    const bool take = sp >= 2 && t_split < 0.95 * t_plain;
+    // (at even odds with the tiles that have a unit to themselves, whose model is as close as split K's: of 20 shapes above 200 rows
+    // where the two were measured within 10 % of each other 9 were faster split, and they differ by 5 % on average)
+    const bool take = sp >= 2 && t_split < (plain == VQGEMM_VARIANT_PREFILL && prefill_mid_plan(p).cost_us <= t_plain ? 1.005 : 0.95) * t_plain;
     *t_best = take ? t_split : t_plain;
     return take ? sp : 0;
 }
@@ -289,12 +292,10 @@ struct WorkspaceChoice {
     TailSplitPlan tail;
     size_t bytes;
 };
-// Above 64 rows of X the wave-K kernel is taken below this share of what the other plan is expected to take: the tiled kernels by
-// more than the models' error, split K (whose model is as close as the wave-K kernel's) at nearly even odds.  Over 260 shapes of M 65 to
-// 4002, 100 of them where split K stood to be taken, the choice is 1.7 % from the best plan measured; at 0.95 for both, with split K's
-// second launch at 4.5 us and no wait for a large X it was 8.7 % (M = 203, K = 2816, N = 7040: 24.9 us split, 20.2 now; M = 657,
-// K = 13376, N = 1040: 39.2 us, split 35.3 now).
-constexpr double kWaveOverTiles = 0.95, kWaveOverSplit = 0.97;
+// Above 64 rows of X the wave-K kernel is taken below this share of what the other plan is expected to take, the models being 3 to 7 %
+// off.  Over 300 shapes of M 65 to 3000 the choice takes 0.951 of the time that it took before the tiles with a compute unit to
+// themselves and the wave-K kernel's last four tile shapes.
+constexpr double kWaveMargin = 0.95;
 
 WorkspaceChoice workspace_auto(const ProblemB &p)
 {
@@ -316,7 +317,7 @@ WorkspaceChoice workspace_auto(const ProblemB &p)
     // (a split asked for by the tuning table is not weighed against anything)
     const bool asked = tuning().splitk_force_splits >= 2.0 || tuning().tail_split_margin >= 1e3;
     const double t_other = c.tail.ok ? c.tail.cost_us : c.sp >= 2 ? t_best : prefill_cost_us(p);
-    if (!(asked && c.bytes > 0) && (plain == VQGEMM_VARIANT_DECODE || plain == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, t_other, c.sp >= 2 ? kWaveOverSplit : kWaveOverTiles))
+    if (!(asked && c.bytes > 0) && (plain == VQGEMM_VARIANT_DECODE || plain == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, t_other, kWaveMargin))
         c = {true, 0, {false, 0, 0, 0, 1e30, 0}, 0};
     return c;
 }
@@ -339,7 +340,7 @@ AutoPlan make_plan(const ProblemB &p)
     plain.gated = false;
     const int v = p.gated && decode_gemv_wide_preferred(p) ? VQGEMM_VARIANT_DECODE_GEMV : plain_b(plain);
     const bool tiled = v == VQGEMM_VARIANT_DECODE || v == VQGEMM_VARIANT_PREFILL;
-    const bool wave = tiled && wave_k_b_preferred(p, p.M > 64 ? prefill_cost_us(plain) : 0.0, kWaveOverTiles);
+    const bool wave = tiled && wave_k_b_preferred(p, p.M > 64 ? prefill_cost_us(plain) : 0.0, kWaveMargin);
     if (wave) plan.variant = VQGEMM_VARIANT_WAVE_K;
     else if (!p.gated) plan.variant = v;
     else if (v == VQGEMM_VARIANT_DECODE_GEMV && decode_gemv_supports(p)) plan.variant = v;

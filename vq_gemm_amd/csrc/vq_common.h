@@ -154,6 +154,15 @@ struct TailSplitPlan {
 TailSplitPlan prefill_tail_split_plan(const ProblemB &p);
 hipError_t launch_prefill_tail_split(const ProblemB &p, const TailSplitPlan &plan, hipStream_t s, void *workspace);
 
+// the prefill kernel with tiles of 128 to 224 rows by 128 columns, one to a compute unit (vq_prefill_mid.hip): the rows of the tile
+// that is expected to be fastest (0: not served) and its time
+struct MidPlan {
+    int rows;
+    double cost_us;
+};
+MidPlan prefill_mid_plan(const ProblemB &p);
+hipError_t launch_prefill_mid_b(const ProblemB &p, hipStream_t s, int rows);
+
 // the prefill kernel with 128x128 tiles (vq_prefill_small.hip), for medium M
 bool prefill_small_supports(const ProblemB &p);
 double prefill_small_cost_us(const ProblemB &p);  // expected time, microseconds (1e30: not supported)
@@ -283,6 +292,8 @@ struct Tuning {
     // 1 wherever they apply, 2 never; and their tile as 10 * (rows / 16) + columns / 16 (0: the cost model's)
     double wave_k_force = 0.0;
     double wave_k_force_tile = 0.0;
+    // (likewise) the prefill tiles that have a compute unit to themselves: 0 where expected to be fastest, 1 never, or their rows
+    double prefill_mid_force = 0.0;
 };
 const Tuning &tuning();
 

@@ -960,17 +960,34 @@ bool prefill_narrow_supports(const ProblemB &p)
     return what.narrow;
 }
 
-// 128x128 tiles are taken when they are expected to be faster than the best cut into large tiles
+namespace {
+
+// The tiles that are expected to be fastest: 128x128 two to a compute unit, or 128 to 224 rows by 128 columns (mid_rows) with a
+// unit to themselves, where they are ahead of the best cut into large tiles.  (Over 500 shapes of M 90 to 2500 the latter take
+// 0.917 of the time of the best of the others.)
+struct TileChoice {
+    bool wide, small;
+    int mid_rows;
+    double cost_us;
+};
 constexpr double kSmallTileMargin = 0.99;
 
-double prefill_cost_us(const ProblemB &p)
+TileChoice choose_tiles(const ProblemB &p)
 {
     PrefillQuery what;
     prefill_query(p, what);
-    if (!what.wide) return what.cost_us;
+    TileChoice c = {what.wide, false, 0, what.cost_us};
+    if (!what.wide) return c;
     const double small = prefill_small_cost_us(p);
-    return small < kSmallTileMargin * what.cost_us ? small : what.cost_us;
+    if (small < kSmallTileMargin * c.cost_us) c = {true, true, 0, small};
+    const MidPlan mid = prefill_mid_plan(p);
+    if (mid.rows > 0 && (mid.cost_us < kSmallTileMargin * c.cost_us || tuning().prefill_mid_force > 1.0)) c = {true, false, mid.rows, mid.cost_us};
+    return c;
 }
+
+}  // namespace
+
+double prefill_cost_us(const ProblemB &p) { return choose_tiles(p).cost_us; }
 
 // ---- whole rounds of large tiles, then the columns that are left in 128x128 tiles with K split ------------------
 // A launch whose large tiles are a few more than a multiple of the compute units pays a whole further round for them.
@@ -1026,9 +1043,9 @@ hipError_t launch_prefill_b(const ProblemB &p, hipStream_t s, int tile)
 {
     if (!prefill_supports(p)) return hipErrorInvalidValue;
     if (tile == 0) {
-        PrefillQuery what;
-        prefill_query(p, what);
-        if (prefill_small_cost_us(p) < kSmallTileMargin * what.cost_us) return launch_prefill_small_b(p, s);
+        const TileChoice c = choose_tiles(p);
+        if (c.mid_rows > 0) return launch_prefill_mid_b(p, s, c.mid_rows);
+        if (c.small) return launch_prefill_small_b(p, s);
     }
     const bool u8 = p.code_bits == 8;
     switch (p.vec) {

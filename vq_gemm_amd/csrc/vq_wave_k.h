@@ -563,8 +563,8 @@ hipError_t launch_tile(WaveKArgs a, hipStream_t s)
 // first latency, the sum over the waves, the stores), cycles per unit on an idle device, how many more when every compute
 // unit works, and by which share a unit takes longer with every doubling of X beyond 2 MB (geometry B).
 struct WaveKTile {
-    int tile;
-    double fixed_us, idle_clk, busy_clk, wait = 0.05;
+    int tile = 0;
+    double fixed_us = 0.0, idle_clk = 0.0, busy_clk = 0.0, wait = 0.05;
 };
 
 // Microseconds a launch is expected to take (a tenth off, either way): the tiles go over the compute units in rounds.

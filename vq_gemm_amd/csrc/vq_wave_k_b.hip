@@ -64,18 +64,28 @@ bool fits(const ProblemB &p, int tile)
     return ok;
 }
 
+// Costs of the tiles, by code size and vector length, fitted to 1700 launches, K 512 to 12288, 24 to 700 tiles: 4 % off; the tiles
+// whose units are one step, 64 x 128, 80 x 64 and 96 x 64 - with 16-bit codes 64 x 64 too - 7 %, and 80 and 96 x 64, of which one
+// launch in ten took half as long again, are set a tenth above their fit.
+constexpr WaveKTile kTileCosts[2][2][11] = {
+    {{{12, 1.9, 42, 13, 0.04}, {14, 2.4, 58, 20, 0.04}, {18, 2.9, 115, 41, 0.04}, {22, 2.5, 43, 18, 0.19}, {24, 3.0, 61, 28, 0.17}, {28, 4.4, 124, 33, 0.19},
+      {34, 3.6, 78, 32, 0.14}, {44, 4.5, 91, 40, 0.11}, {48, 6.9, 154, 81, 0.36}, {54, 5.3, 95, 90, 0.50}, {64, 5.1, 138, 115, 0.40}},
+     {{12, 2.0, 42, 10, 0.21}, {14, 2.2, 69, 27, 0.01}, {18, 3.0, 114, 64, 0.00}, {22, 2.3, 44, 19, 0.28}, {24, 2.9, 70, 35, 0.04}, {28, 4.4, 117, 75, 0.05},
+      {34, 3.5, 83, 34, 0.14}, {44, 4.2, 98, 49, 0.11}, {48, 7.0, 152, 140, 0.16}, {54, 4.9, 140, 110, 0.25}, {64, 5.9, 115, 75, 0.45}}},
+    {{{12, 2.1, 37, 12, 0.07}, {14, 2.5, 56, 21, 0.05}, {18, 2.9, 110, 48, 0.02}, {22, 2.5, 40, 18, 0.27}, {24, 3.0, 63, 26, 0.19}, {28, 4.1, 124, 41, 0.11},
+      {34, 3.6, 75, 32, 0.17}, {44, 4.3, 77, 58, 0.43}, {48, 6.7, 162, 92, 0.35}, {54, 4.8, 108, 98, 0.50}, {64, 5.1, 135, 125, 0.42}},
+     // (no 32 x 128 and 48 x 64 here)
+     {{12, 2.5, 42, 17, 0.12}, {14, 2.7, 75, 20, 0.06}, {18, 3.4, 142, 47, 0.06}, {22, 2.6, 52, 19, 0.22}, {24, 3.2, 80, 38, 0.12}, {44, 4.2, 94, 95, 0.14},
+      {48, 6.4, 192, 132, 0.11}, {54, 4.8, 132, 125, 0.30}, {64, 5.9, 128, 102, 0.40}}}};
+// with a table of copies
+constexpr WaveKTile kCopiesCosts[2][6] = {
+    {{12, 2.1, 36, 10, 0.09}, {14, 2.4, 41, 17, 0.14}, {18, 2.7, 71, 31, 0.16}, {22, 2.5, 39, 17, 0.26}, {24, 2.9, 50, 28, 0.27}, {28, 3.9, 91, 39, 0.18}},
+    {{12, 2.1, 33, 12, 0.14}, {14, 2.2, 48, 28, 0.05}, {18, 2.8, 83, 31, 0.00}, {22, 2.5, 41, 9, 0.35}, {24, 2.9, 55, 26, 0.24}, {28, 3.9, 99, 55, 0.20}}};
+
 template <class F>
 WaveKPlan plan_b(const ProblemB &p)
 {
     const int forced = (int)tuning().wave_k_force_tile;
-    // Fitted to 1700 launches of both vector lengths, K 512 to 12288, 24 to 700 tiles (a twentieth off; the tiles whose units are
-    // one step, 64 x 128, 80 x 64 and 96 x 64 - with 16-bit codes 64 x 64 too - a tenth, and 80 and 96 x 64, of which one launch in
-    // ten took half as long again, are set a tenth above their fit).  (16-bit codes bring tables whose entries collide more often)
-    constexpr WaveKTile kTiles8[] = {{12, 2.0, 40, 13}, {14, 2.3, 63, 22}, {18, 2.9, 116, 45}, {22, 2.2, 47, 21}, {24, 2.8, 70, 33}, {28, 4.4, 120, 57, 0.08},
-                                     {34, 3.5, 81, 31, 0.15}, {44, 4.3, 94, 47, 0.08}, {48, 7.0, 160, 100, 0.27}, {54, 5.3, 110, 85, 0.45}, {64, 5.7, 120, 100, 0.45}};
-    constexpr WaveKTile kTiles16[] = {{12, 2.6, 45, 19}, {14, 2.8, 79, 59}, {18, 3.0, 169, 200}, {22, 2.7, 52, 24}, {24, 3.0, 91, 45}, {28, 4.1, 124, 41, 0.11},
-                                      {34, 3.6, 75, 32, 0.17}, {44, 4.2, 92, 92, 0.20}, {48, 6.4, 200, 140, 0.15}, {54, 5.3, 130, 110, 0.45}, {64, 5.7, 140, 120, 0.45}};
-    constexpr WaveKTile kTilesCopies[] = {{12, 2.1, 34, 12}, {14, 2.4, 45, 17}, {18, 2.7, 76, 38}, {22, 2.4, 41, 17}, {24, 2.7, 58, 38}, {28, 3.9, 103, 30, 0.19}};
     // An X that does not fit the 4 MB of an XCD's L2 beside the rest keeps the units waiting, the longer the larger it is, and most where
     // a unit of one step takes half a 128-byte line at a time.
     const double octaves = std::fmin(3.0, std::fmax(0.0, std::log2(2.0 * p.M * p.K / 2e6)));
@@ -85,13 +95,12 @@ WaveKPlan plan_b(const ProblemB &p)
     const bool rounds = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) > device_cu_count();
     const double bytes = (double)p.K * p.N * F::CSZ / F::VEC + 2.0 * (double)p.M * (p.K + p.N);
     WaveKPlan best = {0, 0, 1e30};
-    for (const WaveKTile &plain : F::CSZ == 1 ? kTiles8 : kTiles16) {
-        if (forced > 0 && forced != plain.tile) continue;
-        if (!fits<F>(p, plain.tile)) continue;
-        WaveKTile t = plain;
+    for (WaveKTile t : kTileCosts[F::CSZ - 1][F::VEC == 8 ? 0 : 1]) {
+        if (forced > 0 && forced != t.tile) continue;
+        if (!fits<F>(p, t.tile)) continue;
         with_tile(t.tile, [&](auto mp, auto np) {
             if (!takes_copies<F, mp(), np()>(p)) return;
-            for (const WaveKTile &c : kTilesCopies)
+            for (const WaveKTile &c : kCopiesCosts[F::VEC == 8 ? 0 : 1])
                 if (c.tile == t.tile) t = c;
         });
         const double us = wave_k_tile_cost_us(t, p.M, p.K, p.N, bytes, (1.0 + t.wait * octaves) * (t.tile == 44 && rounds ? wait_rows : 1.0));
