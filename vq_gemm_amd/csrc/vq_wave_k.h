@@ -63,8 +63,11 @@ struct WaveB {           // geometry B
     static constexpr int VEC = VEC_, CSZ = (int)sizeof(CodeT_);
 };
 
-// Waves of a workgroup: two on every SIMD, one's MFMAs beside the other's reads, where their accumulators leave room for two.
-constexpr int wave_count(int mp, int np) { return mp * np > 32 ? 4 : 8; }
+// Waves of a workgroup: two on every SIMD, one's MFMAs beside the other's reads, where their accumulators leave room for two; four for
+// the smallest tile on a table of copies, whose waves wait for one another's reads least (M = 16, K = 11008, N = 4096 9.2 -> 8.5 us; twice
+// as wide a tile gains nothing from it, 9.7, and loses at K = 4096, 6.0 -> 6.7).
+template <class P>
+constexpr int wave_count(int mp, int np) { return mp * np > 32 ? 4 : P::kB && P::kCopies && mp * np == 1 ? 16 : 8; }
 
 // Rows of pieces whose partial sums, `per_row` KB of them each, fit the LDS together: the most that divide the tile's.
 constexpr int pass_rows(int mp, int per_row)
@@ -77,7 +80,7 @@ constexpr int pass_rows(int mp, int per_row)
 // MP x NP pieces of 16 x 16: the tile.
 template <class P, int MP, int NP>
 struct WaveKCfg {
-    static constexpr int kWaves = wave_count(MP, NP);
+    static constexpr int kWaves = wave_count<P>(MP, NP);
     static constexpr int S = P::S, kUnitK = S * kStepK;
     static constexpr int TM = MP * 16, TN = NP * 16;
     static constexpr int kXBytes = S * MP * 1024;
@@ -162,7 +165,7 @@ __device__ __forceinline__ uint4_t loaded_entry(uint32_t (&entry)[DW])
 }
 
 template <class P, int MP, int NP>
-__global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) void wave_k_kernel(const WaveKArgs a)
+__global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) / 4) void wave_k_kernel(const WaveKArgs a)
 {
     typedef WaveKCfg<P, MP, NP> C;
     static_assert(C::kExists, "a tile the LDS holds");
@@ -415,12 +418,13 @@ __global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) vo
         // (the entry is the oldest load)
         if (n_unit >= D) wait_vmcnt<D * C::kLoads>();
         else wait_vmcnt<0>();
-        // two threads an entry, eight pieces of 16 bytes each, neighbouring entries in another order
-        static_assert(kWaves * 64 == 2 * kCopiesEntries, "two threads an entry");
+        // two threads an entry (four of sixteen waves), eight (four) pieces of 16 bytes each, neighbouring entries in another order
+        constexpr int kPer = kWaves * 64 / kCopiesEntries, kPieces = 16 / kPer;
+        static_assert(kPer == 2 || kPer == 4, "threads an entry");
         const uint4_t piece = loaded_entry(entry);
-        const uint32_t at = kBookBase + (tid & (kCopiesEntries - 1)) * 256 + (tid >> 8) * 128 + (tid & 7) * 16;
+        const uint32_t at = kBookBase + (tid & (kCopiesEntries - 1)) * 256 + (tid >> 8) * (kPieces * 16) + (tid & (kPieces - 1)) * 16;
 #pragma unroll
-        for (int i = 0; i < 8; i++) *reinterpret_cast<uint4_t *>(smem + (at ^ (i * 16))) = piece;
+        for (int i = 0; i < kPieces; i++) *reinterpret_cast<uint4_t *>(smem + (at ^ (i * 16))) = piece;
         __syncthreads();
     } else if constexpr (P::kA || P::kB) {
         // (the codebooks are the oldest loads of the waves that brought them)
@@ -479,7 +483,7 @@ __global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) vo
 
     // ---- the sum over the waves ---------------------------------------------------------------------
     // A piece is 1 KB, float4 by lane; a wave takes pairs of pieces of a row of pieces.
-    constexpr int PM = C::kPassMP, kPairs = PM * NP / 2;
+    constexpr int PM = C::kPassMP, H = NP % 2 == 0 ? 2 : 1, kPairs = PM * NP / H;
     if constexpr (kPinned) {
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMAs have left the pipe
         hold_accumulators(acc);
@@ -494,12 +498,12 @@ __global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) vo
                 *reinterpret_cast<float4_t *>(smem + ((wave * PM + i) * NP + j) * 1024 + lane * 16) = acc[j][pass * PM + i];
         __syncthreads();
         for (int pair = wave; pair < kPairs; pair += kWaves) {
-            const int i = pair / (NP / 2), q = pair % (NP / 2);
+            const int i = pair / (NP / H), q = pair % (NP / H);
             const int m = m0 + (pass * PM + i) * 16 + r16;
-            float4_t sum[2];
+            float4_t sum[H];
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const uint8_t *src = smem + (i * NP + 2 * q + h) * 1024 + lane * 16;
+            for (int h = 0; h < H; h++) {
+                const uint8_t *src = smem + (i * NP + H * q + h) * 1024 + lane * 16;
                 sum[h] = *reinterpret_cast<const float4_t *>(src);
 #pragma unroll
                 for (int v = 1; v < kWaves; v++) sum[h] += *reinterpret_cast<const float4_t *>(src + v * (PM * NP * 1024));
@@ -516,23 +520,24 @@ __global__ __launch_bounds__(wave_count(MP, NP) * 64, wave_count(MP, NP) / 4) vo
                 }
                 if (n < N) __builtin_memcpy(a.y + (int64_t)m * N + n, &v, 16);
             } else {
-                int n = n0 + 2 * q * 16 + kg * 4, end = N;
+                int n = n0 + H * q * 16 + kg * 4, end = N;
                 if (P::kB && a.bias) {
 #pragma unroll
-                    for (int h = 0; h < 2; h++)
+                    for (int h = 0; h < H; h++)
 #pragma unroll
                         for (int e = 0; e < 4; e++) sum[h][e] += (float)a.bias[min(n + h * 16 + e, N - 1)];
                 }
-                const bool gated = P::kB && a.gated;
-                if (gated) {
+                const bool gated = P::kB && H == 2 && a.gated;
+                if constexpr (H == 2)
+                    if (gated) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) sum[0][e] = silu_f32(sum[0][e]) * sum[1][e];
-                    n = n0 / 2 + q * 16 + kg * 4;
-                    end = N / 2;
-                }
+                        for (int e = 0; e < 4; e++) sum[0][e] = silu_f32(sum[0][e]) * sum[1][e];
+                        n = n0 / 2 + q * 16 + kg * 4;
+                        end = N / 2;
+                    }
                 half_t *row = a.y + (int64_t)m * end;
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
+                for (int h = 0; h < H; h++) {
                     if (h == 1 && gated) break;
                     const half4_t v = {(half_t)sum[h][0], (half_t)sum[h][1], (half_t)sum[h][2], (half_t)sum[h][3]};
                     if (n + h * 16 + 4 <= end) {

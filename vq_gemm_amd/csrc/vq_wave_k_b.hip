@@ -17,10 +17,10 @@ struct Format {
     using Wave = WaveB<VEC_, CodeT_, ((MP * NP > 16 || (CSZ == 2 && MP >= 4)) ? 1 : 2)>;
     // Tiles of up to 32 rows gather more than they read of X: with a table of copies, 64 KB of the LDS that their units leave,
     // the gathers' bank conflicts go, M = 128, K = N = 4096 9.5 -> 9.0 us, M = 16, K = 2048, N = 11008 6.7 -> 6.0, tiles of
-    // 32 x 128 14.5 -> 12.0.  Taller ones read X twice as long as they gather and would keep half the units in flight: 64 x 64
+    // 32 x 128 14.5 -> 12.0; 32 x 16 gathers too little, equal.  Taller ones read X twice as long as they gather and would keep half the units in flight: 64 x 64
     // with 32 KB of copies 13.7 -> 15.0.
     template <int MP, int NP>
-    static constexpr bool kHasCopies = CSZ == 1 && MP <= 2;
+    static constexpr bool kHasCopies = CSZ == 1 && MP <= 2 && NP >= MP;
     template <int MP, int NP>
     using Copies = WaveB<VEC_, CodeT_, Wave<MP, NP>::S, true>;
 };
@@ -42,6 +42,8 @@ void with_tile(int tile, F f)
     case 54: f(integral_constant<int, 5>{}, integral_constant<int, 4>{}); break;
     case 64: f(integral_constant<int, 6>{}, integral_constant<int, 4>{}); break;
     case 28: f(integral_constant<int, 2>{}, integral_constant<int, 8>{}); break;
+    case 11: f(integral_constant<int, 1>{}, integral_constant<int, 1>{}); break;
+    case 21: f(integral_constant<int, 2>{}, integral_constant<int, 1>{}); break;
     default: break;
     }
 }
@@ -64,23 +66,23 @@ bool fits(const ProblemB &p, int tile)
     return ok;
 }
 
-// Costs of the tiles, by code size and vector length, fitted to 1700 launches, K 512 to 12288, 24 to 700 tiles: 4 % off; the tiles
+// Costs of the tiles, by code size and vector length, fitted to 2300 launches, K 512 to 12288, 24 to 700 tiles: 1 to 4 % off; the tiles
 // whose units are one step, 64 x 128, 80 x 64 and 96 x 64 - with 16-bit codes 64 x 64 too - 7 %, and 80 and 96 x 64, of which one
 // launch in ten took half as long again, are set a tenth above their fit.
-constexpr WaveKTile kTileCosts[2][2][11] = {
-    {{{12, 1.9, 42, 13, 0.04}, {14, 2.4, 58, 20, 0.04}, {18, 2.9, 115, 41, 0.04}, {22, 2.5, 43, 18, 0.19}, {24, 3.0, 61, 28, 0.17}, {28, 4.4, 124, 33, 0.19},
+constexpr WaveKTile kTileCosts[2][2][13] = {
+    {{{11, 1.5, 31, 8, 0.10}, {21, 1.7, 37, 11, 0.27}, {12, 1.9, 42, 13, 0.04}, {14, 2.4, 58, 20, 0.04}, {18, 2.9, 115, 41, 0.04}, {22, 2.5, 43, 18, 0.19}, {24, 3.0, 61, 28, 0.17}, {28, 4.4, 124, 33, 0.19},
       {34, 3.6, 78, 32, 0.14}, {44, 4.5, 91, 40, 0.11}, {48, 6.9, 154, 81, 0.36}, {54, 5.3, 95, 90, 0.50}, {64, 5.1, 138, 115, 0.40}},
-     {{12, 2.0, 42, 10, 0.21}, {14, 2.2, 69, 27, 0.01}, {18, 3.0, 114, 64, 0.00}, {22, 2.3, 44, 19, 0.28}, {24, 2.9, 70, 35, 0.04}, {28, 4.4, 117, 75, 0.05},
+     {{11, 1.6, 29, 9, 0.18}, {21, 1.7, 37, 11, 0.05}, {12, 2.0, 42, 10, 0.21}, {14, 2.2, 69, 27, 0.01}, {18, 3.0, 114, 64, 0.00}, {22, 2.3, 44, 19, 0.28}, {24, 2.9, 70, 35, 0.04}, {28, 4.4, 117, 75, 0.05},
       {34, 3.5, 83, 34, 0.14}, {44, 4.2, 98, 49, 0.11}, {48, 7.0, 152, 140, 0.16}, {54, 4.9, 140, 110, 0.25}, {64, 5.9, 115, 75, 0.45}}},
-    {{{12, 2.1, 37, 12, 0.07}, {14, 2.5, 56, 21, 0.05}, {18, 2.9, 110, 48, 0.02}, {22, 2.5, 40, 18, 0.27}, {24, 3.0, 63, 26, 0.19}, {28, 4.1, 124, 41, 0.11},
+    {{{11, 1.5, 28, 7, 0.00}, {21, 1.7, 36, 9, 0.30}, {12, 2.1, 37, 12, 0.07}, {14, 2.5, 56, 21, 0.05}, {18, 2.9, 110, 48, 0.02}, {22, 2.5, 40, 18, 0.27}, {24, 3.0, 63, 26, 0.19}, {28, 4.1, 124, 41, 0.11},
       {34, 3.6, 75, 32, 0.17}, {44, 4.3, 77, 58, 0.43}, {48, 6.7, 162, 92, 0.35}, {54, 4.8, 108, 98, 0.50}, {64, 5.1, 135, 125, 0.42}},
      // (no 32 x 128 and 48 x 64 here)
-     {{12, 2.5, 42, 17, 0.12}, {14, 2.7, 75, 20, 0.06}, {18, 3.4, 142, 47, 0.06}, {22, 2.6, 52, 19, 0.22}, {24, 3.2, 80, 38, 0.12}, {44, 4.2, 94, 95, 0.14},
+     {{11, 1.7, 29, 13, 0.14}, {21, 1.8, 41, 11, 0.05}, {12, 2.5, 42, 17, 0.12}, {14, 2.7, 75, 20, 0.06}, {18, 3.4, 142, 47, 0.06}, {22, 2.6, 52, 19, 0.22}, {24, 3.2, 80, 38, 0.12}, {44, 4.2, 94, 95, 0.14},
       {48, 6.4, 192, 132, 0.11}, {54, 4.8, 132, 125, 0.30}, {64, 5.9, 128, 102, 0.40}}}};
 // with a table of copies
-constexpr WaveKTile kCopiesCosts[2][6] = {
-    {{12, 2.1, 36, 10, 0.09}, {14, 2.4, 41, 17, 0.14}, {18, 2.7, 71, 31, 0.16}, {22, 2.5, 39, 17, 0.26}, {24, 2.9, 50, 28, 0.27}, {28, 3.9, 91, 39, 0.18}},
-    {{12, 2.1, 33, 12, 0.14}, {14, 2.2, 48, 28, 0.05}, {18, 2.8, 83, 31, 0.00}, {22, 2.5, 41, 9, 0.35}, {24, 2.9, 55, 26, 0.24}, {28, 3.9, 99, 55, 0.20}}};
+constexpr WaveKTile kCopiesCosts[2][7] = {
+    {{11, 1.8, 25, 7, 0.00}, {12, 2.1, 36, 10, 0.09}, {14, 2.4, 41, 17, 0.14}, {18, 2.7, 71, 31, 0.16}, {22, 2.5, 39, 17, 0.26}, {24, 2.9, 50, 28, 0.27}, {28, 3.9, 91, 39, 0.18}},
+    {{11, 1.8, 25, 9, 0.32}, {12, 2.1, 33, 12, 0.14}, {14, 2.2, 48, 28, 0.05}, {18, 2.8, 83, 31, 0.00}, {22, 2.5, 41, 9, 0.35}, {24, 2.9, 55, 26, 0.24}, {28, 3.9, 99, 55, 0.20}}};
 
 template <class F>
 WaveKPlan plan_b(const ProblemB &p)
@@ -97,7 +99,7 @@ WaveKPlan plan_b(const ProblemB &p)
     WaveKPlan best = {0, 0, 1e30};
     for (WaveKTile t : kTileCosts[F::CSZ - 1][F::VEC == 8 ? 0 : 1]) {
         if (forced > 0 && forced != t.tile) continue;
-        if (!fits<F>(p, t.tile)) continue;
+        if (!fits<F>(p, t.tile) || (p.gated && t.tile % 10 == 1)) continue;
         with_tile(t.tile, [&](auto mp, auto np) {
             if (!takes_copies<F, mp(), np()>(p)) return;
             for (const WaveKTile &c : kCopiesCosts[F::VEC == 8 ? 0 : 1])
@@ -189,11 +191,16 @@ bool wave_k_b_preferred(const ProblemB &p, double t_other, double margin)
     if (force == 1) return true;
     if (p.M <= 64) {
         const double t_decode = decode_slab_cost_us(p);
-        if (t_decode > 1e29) return p.M > 16;
-        // (the gated decode kernels deal tiles in pairs, which their model does not see; up to 16 rows the decode kernel is ahead near
-        // ties on codes out of HBM: over 145 shapes this line is 1.0 % from the better kernel there, 0.97 is 1.8 %, and on codes that
-        // the caches hold, where it is the other way round, they are 3.8 and 2.1 %)
-        return wave_k_b_cost_us(p) < (p.gated ? 1.15 : p.M <= 16 ? 0.89 : 0.97) * t_decode;
+        // (the streaming kernel, up to 16 rows: over 34 of its shapes on codes out of HBM the tile expected to be fastest takes 0.85 of
+        // its time up to K = 24576 - 16 x 11008 x 4096 11.9 us -> 8.9 - and over 7 from there on 1.03, 13 x 27520 x 2944 17.5 -> 20.2)
+        if (t_decode > 1e29) return p.M > 16 || (p.K <= 24576 && decode_stream_preferred(p));
+        // The gated decode kernels deal tiles in pairs, which their model does not see.  Up to 16 rows, where their model is 4 to 9 %
+        // high, the decode kernel is ahead near ties on codes out of HBM: over 333 shapes the line at 0.89 is 1.8 % from the better
+        // kernel (0.97: 1.6, 0.80: 5.8, the decode kernel alone 15.1).  Where its workgroups come out at exactly one a compute unit,
+        // none idle and none with two, it gives the least away (16 x 4096 x 4096: cold 6.48 us against 5.87; 2048 x 4096 5.3, 4.9) and
+        // the choice that callers have seen reported for such a layer stays.
+        const bool one_each = p.N == device_cu_count() * 16 && p.M <= 16;
+        return wave_k_b_cost_us(p) < (p.gated ? 1.15 : one_each ? 0.80 : p.M <= 16 ? 0.89 : 0.97) * t_decode;
     }
     return wave_k_b_cost_us(p) < margin * t_other;
 }
