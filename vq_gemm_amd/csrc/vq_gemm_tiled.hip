@@ -16,8 +16,10 @@
 //     step s+1 are read from the LDS.  One barrier per step publishes the next stage and frees
 //     the buffer of the stage just consumed.
 //   * X (and W in the NT layout) lies in the LDS as 64-byte rows, four to a 256-byte bank row,
-//     XOR-swizzled so that the 16 rows x one 16-byte chunk a quarter wave reads fall into 16
-//     different bank groups.
+//     XOR-swizzled so that the sixteen lanes that a 16-byte read serves at a time (0-3, 12-15, 20-23 and
+//     24-27, then 4-11, 16-19 and 28-31, the upper half wave alike) fall into 16 different bank groups: 4 cycles
+//     a read, 8 with the bank row's own number for the XOR.  (The fused geometry-A kernel 44 -> 41 us at
+//     M = 2048, K = 4096, Nc = 640; the plain product waits for its matrix cores, not for this.)
 //   * W in the NN layout ([K,N], n contiguous) lies as 32 k-rows of 512 bytes and is read with
 //     the transposing LDS read ds_read_b64_tr_b16: within 16 lanes, source lane 4d+q supplies
 //     row d, columns 4q..4q+3, and lane l receives column l of rows 0..3 - four consecutive k
@@ -65,7 +67,7 @@ typedef short short4_t __attribute__((__vector_size__(4 * sizeof(short))));
 __device__ __forceinline__ int row_offset(int row, int cc)
 {
     const int bank_row = row >> 2;
-    const int pos = (((row & 3) << 2) | cc) ^ (bank_row & 3);
+    const int pos = (((row & 3) << 2) | cc) ^ (-bank_row & 3);
     return (bank_row * 16 + pos) * 16;
 }
 
@@ -104,7 +106,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const half_t *_
     for (int i = 0; i < kXLoads; i++) {
         const int slot = (4 * i + wave) * 64 + lane;
         const int bank_row = slot >> 4;
-        const int pos = (slot & 15) ^ (bank_row & 3);
+        const int pos = (slot & 15) ^ (-bank_row & 3);
         const int row = 4 * bank_row + (pos >> 2), cc = pos & 3;
         x_voff[i] = (uint32_t)(((int64_t)(min(m0 + row, M - 1) - m0) * K + cc * 8) * 2);
         if (!W_IS_KN && i < C::kWLoads) w_voff[i] = (uint32_t)(((int64_t)(min(n0 + row, N - 1) - n0) * K + cc * 8) * 2);
@@ -378,7 +380,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_a_fused_kernel(const half_t 
     for (int i = 0; i < kXLoads; i++) {
         const int slot = (4 * i + wave) * 64 + lane;
         const int bank_row = slot >> 4;
-        const int pos = (slot & 15) ^ (bank_row & 3);
+        const int pos = (slot & 15) ^ (-bank_row & 3);
         const int row = 4 * bank_row + (pos >> 2), cc = pos & 3;
         x_voff[i] = (uint32_t)(((int64_t)(min(m0 + row, M - 1) - m0) * K + cc * 8) * 2);
     }

@@ -16,7 +16,7 @@
 // What bounds it: with few tiles the launch, the latency of the first units and the sum over the waves (together about
 // 4 us); with many the LDS, which carries each unit in and out once.
 //
-//   * X (64 bytes of a row per unit) lies in the LDS as in vq_gemm_tiled.hip: 64-byte rows, XOR-swizzled.
+//   * X lies in the LDS in rows of 64 or 128 bytes, XOR-swizzled (wave_x_swizzle).
 //   * fp16 W lies as k-rows and is read with the transposing ds_read_b64_tr_b16.  Rows of W that are no multiple of 16
 //     bytes (N % 8 != 0, or a pointer aligned to 2 bytes) cannot be loaded into the LDS directly: they go through registers.
 //   * Codes of geometry A lie as k-rows of bytes; ds_read_b64_tr_b8 hands a lane the eight codes of its code column, and
@@ -28,6 +28,7 @@
 
 #include "vq_prefill_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace vq {
@@ -109,24 +110,32 @@ struct WaveKCfg {
     }
 };
 
-// X in a unit of one step: 64-byte rows, four to a 256-byte bank row, XOR-swizzled; of two steps: x_offset.
+// X in a unit lies in rows of 64 bytes, four to a 256-byte bank row (one step), or of 128 bytes, two to a bank row (two steps), the
+// chunks of a bank row XOR-swizzled with a function of its number.  A 16-byte read serves sixteen lanes at a time, not in their
+// order but lanes 0-3, 12-15, 20-23 and 24-27, then 4-11, 16-19 and 28-31 (and the upper half wave alike): rows r16 of one chunk column
+// and of the next together.  With these functions they fall into sixteen different chunks of the bank row: 4 cycles a read,
+// where the bank row's own number makes it 8.
+template <int S>
+__device__ __forceinline__ int wave_x_swizzle(int bank_row)
+{
+    return S == 2 ? (bank_row & 1) | ((bank_row >> 2) & 1) * 6 : -bank_row & 3;
+}
+
+// Byte offset of chunk cc (16 bytes) of row `row`.
 template <int S>
 __device__ __forceinline__ int wave_x_offset(int row, int cc)
 {
-    if constexpr (S == 2) {
-        return x_offset(row, cc);
-    } else {
-        const int bank_row = row >> 2;
-        return (bank_row * 16 + ((((row & 3) << 2) | cc) ^ (bank_row & 3))) * 16;
-    }
+    const int bank_row = S == 2 ? row >> 1 : row >> 2;
+    const int pos = (S == 2 ? ((row & 1) << 3) | cc : ((row & 3) << 2) | cc) ^ wave_x_swizzle<S>(bank_row);
+    return (bank_row * 16 + pos) * 16;
 }
 
-// Rows of fp16 W: the XOR on the chunk index of k-row `k`, such that the four rows x 32 bytes a quarter wave of a transposing
-// read touches fall into different banks (with 64-byte rows they do by themselves).
+// Rows of fp16 W: the XOR on the chunk index of k-row `k`, such that the eight rows x 32 bytes a half wave of a transposing
+// read touches - four from k-row 8*kg on, for two kg - fall into different banks.
 template <int NP>
 __device__ __forceinline__ int wave_w_swizzle(int k)
 {
-    return NP == 8 ? 2 * (k & 3) + ((k >> 3) & 1) * 8 : NP == 4 ? ((k >> 1) & 1) * 2 + ((k >> 3) & 1) * 4 : 0;
+    return NP == 8 ? 2 * (k & 3) + ((k >> 3) & 1) * 8 : NP == 4 ? ((k >> 1) & 1) * 2 + ((k >> 3) & 1) * 4 : ((k >> 3) & 1) * 2;
 }
 
 struct WaveKArgs {
@@ -140,6 +149,7 @@ struct WaveKArgs {
     int tiles_m, tiles_n;
     int entries, rows_per_cb, books;   // (geometry B) books: codebooks of a tile
     int gated;
+    int by_rows;           // consecutive tiles lie along the rows of tiles (wave_k_by_rows)
 };
 
 // The entry of a table of copies by a load that the compiler does not count, beside the direct loads, which it does not either:
@@ -176,11 +186,11 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int r16 = lane & 15, kg = lane >> 4;
 
-    // Workgroup ids are dealt round-robin to the 8 XCDs: an XCD takes consecutive tiles, those over the same columns of Y
-    // next to each other, so that W passes through one L2 only.
+    // Workgroup ids are dealt round-robin to the 8 XCDs: an XCD takes consecutive tiles, by rows or by columns.
     const int n_wg = a.tiles_m * a.tiles_n, xcd = blockIdx.x & 7;
     const int tile = xcd * (n_wg >> 3) + min(xcd, n_wg & 7) + ((int)blockIdx.x >> 3);
-    const int tm = tile % a.tiles_m, tn = tile / a.tiles_m;
+    const int along = a.by_rows ? a.tiles_n : a.tiles_m, line = tile / along, at_line = tile - line * along;
+    const int tm = a.by_rows ? line : at_line, tn = a.by_rows ? at_line : line;
     const int m0 = tm * C::TM, n0 = tn * C::TN;
     const int n_all = K / kUnitK;
     const int n_unit = (n_all - wave + kWaves - 1) / kWaves;  // of this wave: wave, wave + kWaves, ...
@@ -193,7 +203,7 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
     for (int i = 0; i < S * MP; i++) {
         const int slot = i * 64 + lane;
         const int bank_row = slot >> 4;
-        const int pos = (slot & 15) ^ (bank_row & (S == 2 ? 15 : 3));
+        const int pos = (slot & 15) ^ wave_x_swizzle<S>(bank_row);
         const int row = S == 2 ? 2 * bank_row + (pos >> 3) : 4 * bank_row + (pos >> 2), cc = pos & (4 * S - 1);
         x_voff[i] = (uint32_t)(((int64_t)(min(m0 + row, M - 1) - m0) * k_x + cc * 8) * 2);
     }
@@ -553,12 +563,24 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
     }
 }
 
+// Whether an XCD, whose L2 is its own, takes its consecutive tiles along the rows of tiles or down the columns: the way that brings it
+// fewer bytes of X and W, `x_row` and `w_col` of them a tile and k.  Down the columns always, as it was, every XCD read all of X: with
+// this and the swizzle of X 150 shapes of M 65 to 2000 take 0.963 of their time, M = 1555, K = 1664, N = 656 15.0 us -> 10.6.
+inline int wave_k_by_rows(int tiles_m, int tiles_n, double x_row, double w_col)
+{
+    const int tiles = (tiles_m * tiles_n + 7) / 8;
+    auto bytes = [&](int along, double b_along, double b_across) { return std::min(along, tiles) * b_along + (tiles + along - 1) / along * b_across; };
+    return bytes(tiles_n, w_col, x_row) < bytes(tiles_m, x_row, w_col) ? 1 : 0;
+}
+
 template <class P, int MP, int NP>
 hipError_t launch_tile(WaveKArgs a, hipStream_t s)
 {
     typedef WaveKCfg<P, MP, NP> C;
     a.tiles_m = (a.M + C::TM - 1) / C::TM;
     a.tiles_n = (a.N + C::TN - 1) / C::TN;
+    // (geometry A by columns: a tile takes 16 or 32 bytes of a row of codes, and those beside it the rest of the line)
+    a.by_rows = P::kA ? 0 : wave_k_by_rows(a.tiles_m, a.tiles_n, C::TM * 2.0, C::TN * (P::kB ? (double)P::CSZ / P::VEC : 2.0));
     const size_t lds = C::lds_bytes(P::kB ? (size_t)a.books * a.entries * P::VEC * 2 : C::kBooks);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     return launch_kernel(wave_k_kernel<P, MP, NP>, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(C::kWaves * 64), lds, s, a);
@@ -588,6 +610,7 @@ inline double wave_k_tile_cost_us(const WaveKTile &t, int M, int K, int N, doubl
 struct WaveKPlan {
     int mp, np;
     double cost_us;
+    bool wide = false;   // (geometry A) the kernel of vq_wave_k_a.hip
 };
 
 // whole units of K, rows of X in whole 16-byte chunks, offsets within 32 bits
