@@ -2286,6 +2286,18 @@ def test_k_dealt_out_to_waves_geometry_a(M, K, Nc):
         _check_gemm(y, x, w, cb, geometry=GEOM_A, what=f"tile {tile}")
 
 
+@pytest.mark.parametrize("M,K,Nc", [(1, 64, 16), (130, 192, 48), (97, 320, 80), (65, 1088, 112), (129, 2112, 64), (257, 576, 96)])
+def test_k_dealt_out_to_waves_geometry_a_table_of_copies(M, K, Nc):
+    """The tiles of vq_wave_k_a.hip: waves with no step, one and an odd number of them, edges on both sides."""
+    spec = ProblemSpec("A", GEOM_A, M, K, 2 * Nc, 2, 256, Nc // 4, 8, codebook_std=0.05)
+    x, w, cb = make_problem(spec, seed=96, device=DEV)
+    for tile in (144, 164, 166, 184, 186):
+        _say("wave_k geometry A", M, K, Nc, "tile", tile)
+        y = _with_wave_tile(tile, lambda: cabi.e2e_gemm_a(x, w, cb, variant=cabi.VARIANT_PREFILL))
+        torch.cuda.synchronize()
+        _check_gemm(y, x, w, cb, geometry=GEOM_A, what=f"tile {tile}")
+
+
 @pytest.mark.parametrize("what", ["weights", "entries", "entry 0 is NaN", "both", "equal vectors and entries", "all zero"])
 @pytest.mark.parametrize("N,K,v,E,G", [(64, 256, 8, 256, 2), (48, 520, 8, 100, 1), (40, 128, 4, 4096, 1), (50, 64, 2, 77, 1), (24, 64, 8, 5000, 1), (24, 64, 8, 3430, 1)])
 def test_encoder_keeps_the_rule_where_nothing_is_finite_or_everything_is_equal(N, K, v, E, G, what):

@@ -32,7 +32,7 @@ HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 KERNEL_SOURCES = ["vq_api.hip", "vq_dequant.hip", "vq_encode.hip", "vq_lloyd.hip", "vq_generic.hip", "vq_decode.hip", "vq_decode_gemv.hip", "vq_decode_stream.hip", "vq_decode_general.hip", "vq_prefill.hip",
-                  "vq_prefill_small.hip", "vq_prefill_mid.hip", "vq_gemm_plain.hip", "vq_gemm_tiled.hip", "vq_wave_k.hip", "vq_wave_k_b.hip", "vq_epilogue.hip", "vq_check.hip", "vq_noalloc.hip"]
+                  "vq_prefill_small.hip", "vq_prefill_mid.hip", "vq_gemm_plain.hip", "vq_gemm_tiled.hip", "vq_wave_k.hip", "vq_wave_k_a.hip", "vq_wave_k_b.hip", "vq_epilogue.hip", "vq_check.hip", "vq_noalloc.hip"]
 
 # sources with no kernel of their own (argument validation and dispatch)
 HOST_ONLY_SOURCES = {"vq_api.hip", "vq_noalloc.hip"}

@@ -198,6 +198,7 @@ hipError_t launch_gemm_wave_k(const half_t *x, const half_t *w, half_t *y, int M
 bool wave_k_a_supports(const ProblemA &p);
 double wave_k_a_cost_us(const ProblemA &p);
 hipError_t launch_wave_k_a(const ProblemA &p, hipStream_t s);
+hipError_t launch_wave_k_a_wide(const ProblemA &p, int tile, hipStream_t s);
 bool wave_k_b_supports(const ProblemB &p);
 double wave_k_b_cost_us(const ProblemB &p);
 // whether the automatic choice takes this kernel (`t_other`: what the best of the others is expected to take, by their cost models)

@@ -717,12 +717,15 @@ static bool fused_a_tall(const ProblemA &p)
     return (double)((n_tall + cus - 1) / cus) <= 0.8 * (double)((n_short + cus - 1) / cus);
 }
 
+// fitted to 430 launches, M 20 to 4096, K 512 to 8192, N 512 to 8192: 8 % off
 double fused_a_cost_us(const ProblemA &p)
 {
     const int cus = device_cu_count();
     const bool tall = fused_a_tall(p);
     const int64_t tiles = (int64_t)((p.M + (tall ? 255 : 127)) / (tall ? 256 : 128)) * ((2 * p.Nc + kABN - 1) / kABN);
-    return (double)((tiles + cus - 1) / cus) * (4.0 + p.K * (tall ? 0.0132 : 0.0102));
+    const int64_t rounds = (tiles + cus - 1) / cus;
+    const double busy = (double)tiles / (double)(rounds * cus);
+    return (double)rounds * (5.6 + p.K * (tall ? 0.0117 + 0.0060 * busy : 0.0095 + 0.0016 * busy)) - 1.1;
 }
 
 hipError_t launch_fused_a(const ProblemA &p, hipStream_t s)

@@ -10,15 +10,20 @@ enum WaveKind { kDense, kDenseAnyN, kGeometryA };
 WaveKPlan wave_k_plan(int kind, int M, int K, int N)
 {
     const int forced = (int)tuning().wave_k_force_tile;
-    constexpr WaveKTile kTilesA[] = {{12, 1.4, 86, 30}, {22, 1.5, 96, 56}, {24, 2.1, 139, 56}, {42, 1.7, 96, 104}, {44, 2.7, 144, 106}, {84, 4.4, 168, 236}, {86, 5.0, 407, 95}};
+    // Geometry A: over 450 shapes, M 20 to 4096, K 512 to 8192, N 512 to 8192, the tile chosen is 0.7 % from the fastest.  Numbered from
+    // 100 on: the kernel of vq_wave_k_a.hip (3 to 6 % off; the others, which wait for memory more, 8 to 15 %).
+    constexpr WaveKTile kTilesA[] = {{12, 1.6, 86, 27}, {22, 1.5, 96, 59}, {24, 2.4, 132, 47}, {42, 1.7, 102, 93}, {44, 2.6, 139, 96},
+                                     {144, 3.4, 159, 47}, {164, 3.8, 188, 88}, {166, 5.3, 254, 94}, {184, 4.1, 205, 165}, {186, 7.0, 275, 133}};
     // (fp16 rows that straddle the memory's 128-byte lines cost a third more)
     constexpr WaveKTile kTilesDense[] = {{12, 1.6, 106, 13}, {22, 1.5, 137, 17}, {24, 1.5, 175, 10}, {42, 1.2, 167, 63}, {44, 1.8, 214, 45}};
     WaveKPlan best = {0, 0, 1e30};
     auto consider = [&](WaveKTile t) {
-        if (forced > 0 && forced != t.tile) return;
+        const bool wide = t.tile > 100;
+        if (forced > 0 && forced != t.tile && forced != t.tile % 100) return;
+        t.tile %= 100;
         if (kind != kGeometryA && N % 64 != 0) t.idle_clk *= 1.38;
         const double us = wave_k_tile_cost_us(t, M, K, N, (double)K * N * (kind == kGeometryA ? 0.5 : 2.0) + 2.0 * (double)M * (K + N));
-        if (us < best.cost_us) best = {t.tile / 10, t.tile % 10, us};
+        if (us < best.cost_us) best = {t.tile / 10, t.tile % 10, us, wide};
     };
     if (kind == kGeometryA)
         for (const WaveKTile &t : kTilesA) consider(t);
@@ -36,12 +41,7 @@ hipError_t launch_wave_k(const WaveKArgs &a, const WaveKPlan &plan, hipStream_t 
     case 24: return launch_tile<P, 2, 4>(a, s);
     case 42: return launch_tile<P, 4, 2>(a, s);
     case 44: return launch_tile<P, 4, 4>(a, s);
-    default:
-        if constexpr (P::kA) {
-            if (plan.mp == 8 && plan.np == 4) return launch_tile<P, 8, 4>(a, s);
-            if (plan.mp == 8 && plan.np == 6) return launch_tile<P, 8, 6>(a, s);
-        }
-        return hipErrorInvalidValue;
+    default: return hipErrorInvalidValue;
     }
 }
 
@@ -75,8 +75,10 @@ double wave_k_a_cost_us(const ProblemA &p) { return wave_k_plan(kGeometryA, p.M,
 hipError_t launch_wave_k_a(const ProblemA &p, hipStream_t s)
 {
     if (!wave_k_a_supports(p)) return hipErrorInvalidValue;
+    const WaveKPlan plan = wave_k_plan(kGeometryA, p.M, p.K, 2 * p.Nc);
+    if (plan.wide) return launch_wave_k_a_wide(p, plan.mp * 10 + plan.np, s);
     const WaveKArgs a = {p.x, p.w, p.cb, p.y, nullptr, p.M, p.K, 2 * p.Nc, p.K, 0, 0, 0, 1, 0, 0};
-    return launch_wave_k<WaveA>(a, wave_k_plan(kGeometryA, p.M, p.K, 2 * p.Nc), s);
+    return launch_wave_k<WaveA>(a, plan, s);
 }
 
 }  // namespace vq
