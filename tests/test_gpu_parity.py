@@ -2222,15 +2222,15 @@ def test_k_dealt_out_to_waves_tall_and_wide_tiles(row):
 
 @pytest.mark.parametrize("row", WAVE_K_B + [(16, 128, 17, 8, 256, 8, 1), (15, 1152, 48, 4, 256, 8, 1), (9, 4224, 50, 8, 37, 8, 1), (32, 2048, 15, 8, 512, 16, 1)],
                          ids=lambda r: "x".join(map(str, r)))
-def test_k_dealt_out_to_waves_one_piece_wide(row):
-    """16 and 32 x 16: sixteen waves and the table of copies where one codebook serves, eight waves elsewhere, more waves than units.
+def test_k_dealt_out_to_waves_an_odd_number_of_pieces_wide(row):
+    """16 and 32 x 16 and x 48: sixteen waves and the table of copies where one codebook serves, eight waves elsewhere, more waves than units.
     A gated product needs pairs of pieces and refuses them."""
     M, K, N, v, E, bits, G = row
     spec = ProblemSpec("wave_k", GEOM_B, M, K, N, v, E, G, bits, codebook_3d=(G > 1), codebook_std=0.05)
     x, codes, cb = make_problem(spec, seed=95, device=DEV)
     bias = torch.randn(N, generator=torch.Generator().manual_seed(8)).half().to(DEV)
     want = _np(x).astype(np.float64) @ vo.dequant_b(_np(codes), _np(cb)).astype(np.float64).T
-    for tile in (11, 21):
+    for tile in (11, 13, 21, 23):
         _say("wave_k", row, "tile", tile)
         for b in (None, bias):
             y = _with_wave_tile(tile, lambda: cabi.e2e_gemm_b(x, codes, cb, variant=cabi.VARIANT_WAVE_K, bias=b))

@@ -44,6 +44,8 @@ void with_tile(int tile, F f)
     case 28: f(integral_constant<int, 2>{}, integral_constant<int, 8>{}); break;
     case 11: f(integral_constant<int, 1>{}, integral_constant<int, 1>{}); break;
     case 21: f(integral_constant<int, 2>{}, integral_constant<int, 1>{}); break;
+    case 13: f(integral_constant<int, 1>{}, integral_constant<int, 3>{}); break;
+    case 23: f(integral_constant<int, 2>{}, integral_constant<int, 3>{}); break;
     default: break;
     }
 }
@@ -66,23 +68,28 @@ bool fits(const ProblemB &p, int tile)
     return ok;
 }
 
-// Costs of the tiles, by code size and vector length, fitted to 2300 launches, K 512 to 12288, 24 to 700 tiles: 1 to 4 % off; the tiles
-// whose units are one step, 64 x 128, 80 x 64 and 96 x 64 - with 16-bit codes 64 x 64 too - 7 %, and 80 and 96 x 64, of which one
+// Costs of the tiles, by code size and vector length, fitted to 3200 launches, K 512 to 12288, 24 to 700 tiles: 1 to 6 % off; the tiles
+// whose units are one step, 64 x 128, 80 x 64 and 96 x 64 - with 16-bit codes 64 x 64 too - 7 to 12 %, and 80 and 96 x 64, of which one
 // launch in ten took half as long again, are set a tenth above their fit.
-constexpr WaveKTile kTileCosts[2][2][13] = {
-    {{{11, 1.5, 31, 8, 0.10}, {21, 1.7, 37, 11, 0.27}, {12, 1.9, 42, 13, 0.04}, {14, 2.4, 58, 20, 0.04}, {18, 2.9, 115, 41, 0.04}, {22, 2.5, 43, 18, 0.19}, {24, 3.0, 61, 28, 0.17}, {28, 4.4, 124, 33, 0.19},
-      {34, 3.6, 78, 32, 0.14}, {44, 4.5, 91, 40, 0.11}, {48, 6.9, 154, 81, 0.36}, {54, 5.3, 95, 90, 0.50}, {64, 5.1, 138, 115, 0.40}},
-     {{11, 1.6, 29, 9, 0.18}, {21, 1.7, 37, 11, 0.05}, {12, 2.0, 42, 10, 0.21}, {14, 2.2, 69, 27, 0.01}, {18, 3.0, 114, 64, 0.00}, {22, 2.3, 44, 19, 0.28}, {24, 2.9, 70, 35, 0.04}, {28, 4.4, 117, 75, 0.05},
-      {34, 3.5, 83, 34, 0.14}, {44, 4.2, 98, 49, 0.11}, {48, 7.0, 152, 140, 0.16}, {54, 4.9, 140, 110, 0.25}, {64, 5.9, 115, 75, 0.45}}},
-    {{{11, 1.5, 28, 7, 0.00}, {21, 1.7, 36, 9, 0.30}, {12, 2.1, 37, 12, 0.07}, {14, 2.5, 56, 21, 0.05}, {18, 2.9, 110, 48, 0.02}, {22, 2.5, 40, 18, 0.27}, {24, 3.0, 63, 26, 0.19}, {28, 4.1, 124, 41, 0.11},
-      {34, 3.6, 75, 32, 0.17}, {44, 4.3, 77, 58, 0.43}, {48, 6.7, 162, 92, 0.35}, {54, 4.8, 108, 98, 0.50}, {64, 5.1, 135, 125, 0.42}},
+constexpr WaveKTile kTileCosts[2][2][15] = {
+    {{{11, 1.5, 31, 10, 0.00}, {12, 2.2, 36, 12, 0.00}, {13, 1.8, 48, 11, 0.00}, {14, 2.4, 58, 17, 0.00}, {18, 3.3, 112, 19, 0.00}, {21, 1.6, 37, 11, 0.00}, {22, 2.4, 42, 16, 0.00},
+      {23, 2.2, 49, 24, 0.00}, {24, 3.0, 62, 24, 0.00}, {28, 4.6, 107, 43, 0.02}, {34, 3.3, 75, 31, 0.05}, {44, 3.8, 90, 44, 0.06}, {48, 6.0, 132, 127, 0.27}, {54, 5.1, 108, 54, 0.06},
+      {64, 4.8, 122, 67, 0.35}},
+     {{11, 1.5, 29, 10, 0.00}, {12, 2.1, 40, 9, 0.00}, {13, 1.8, 51, 13, 0.04}, {14, 2.3, 62, 26, 0.00}, {18, 3.0, 120, 30, 0.00}, {21, 1.5, 37, 13, 0.01}, {22, 2.4, 41, 17, 0.24},
+      {23, 2.2, 49, 27, 0.01}, {24, 2.9, 67, 32, 0.02}, {28, 4.3, 121, 60, 0.08}, {34, 3.3, 76, 33, 0.01}, {44, 3.6, 98, 42, 0.13}, {48, 6.8, 140, 102, 0.50}, {54, 5.4, 113, 47, 0.50},
+      {64, 6.1, 117, 51, 0.50}}},
+    {{{11, 1.5, 25, 9, 0.00}, {12, 2.1, 32, 13, 0.00}, {13, 1.8, 45, 12, 0.00}, {14, 2.4, 59, 17, 0.00}, {18, 3.2, 102, 41, 0.00}, {21, 1.6, 36, 11, 0.03}, {22, 2.4, 40, 16, 0.00},
+      {23, 2.2, 48, 25, 0.08}, {24, 3.0, 60, 28, 0.01}, {28, 4.2, 110, 47, 0.08}, {34, 3.3, 72, 36, 0.07}, {44, 3.6, 80, 72, 0.11}, {48, 5.6, 149, 120, 0.26}, {54, 4.6, 110, 81, 0.50},
+      {64, 4.8, 135, 64, 0.50}},
      // (no 32 x 128 and 48 x 64 here)
-     {{11, 1.7, 29, 13, 0.14}, {21, 1.8, 41, 11, 0.05}, {12, 2.5, 42, 17, 0.12}, {14, 2.7, 75, 20, 0.06}, {18, 3.4, 142, 47, 0.06}, {22, 2.6, 52, 19, 0.22}, {24, 3.2, 80, 38, 0.12}, {44, 4.2, 94, 95, 0.14},
-      {48, 6.4, 192, 132, 0.11}, {54, 4.8, 132, 125, 0.30}, {64, 5.9, 128, 102, 0.40}}}};
+     {{11, 1.8, 29, 11, 0.00}, {12, 2.4, 42, 13, 0.00}, {13, 2.2, 50, 26, 0.00}, {14, 2.7, 69, 33, 0.18}, {18, 3.5, 136, 60, 0.00}, {21, 1.8, 41, 15, 0.03}, {22, 2.6, 51, 17, 0.19},
+      {23, 2.2, 59, 39, 0.12}, {24, 3.0, 85, 38, 0.32}, {44, 3.4, 114, 51, 0.50}, {48, 5.6, 160, 178, 0.46}, {54, 5.1, 121, 52, 0.50}, {64, 5.8, 127, 90, 0.50}}}};
 // with a table of copies
-constexpr WaveKTile kCopiesCosts[2][7] = {
-    {{11, 1.8, 25, 7, 0.00}, {12, 2.1, 36, 10, 0.09}, {14, 2.4, 41, 17, 0.14}, {18, 2.7, 71, 31, 0.16}, {22, 2.5, 39, 17, 0.26}, {24, 2.9, 50, 28, 0.27}, {28, 3.9, 91, 39, 0.18}},
-    {{11, 1.8, 25, 9, 0.32}, {12, 2.1, 33, 12, 0.14}, {14, 2.2, 48, 28, 0.05}, {18, 2.8, 83, 31, 0.00}, {22, 2.5, 41, 9, 0.35}, {24, 2.9, 55, 26, 0.24}, {28, 3.9, 99, 55, 0.20}}};
+constexpr WaveKTile kCopiesCosts[2][9] = {
+    {{11, 1.9, 25, 7, 0.00}, {12, 2.1, 33, 10, 0.00}, {13, 1.8, 36, 13, 0.00}, {14, 2.4, 42, 17, 0.00}, {18, 2.9, 65, 38, 0.03}, {22, 2.4, 42, 16, 0.00}, {23, 2.1, 43, 23, 0.00},
+     {24, 2.8, 55, 22, 0.23}, {28, 3.8, 86, 60, 0.05}},
+    {{11, 1.9, 24, 9, 0.01}, {12, 2.2, 30, 13, 0.00}, {13, 1.9, 38, 14, 0.00}, {14, 2.4, 48, 20, 0.00}, {18, 3.0, 78, 39, 0.00}, {22, 2.4, 38, 18, 0.00}, {23, 2.2, 45, 25, 0.02},
+     {24, 2.9, 56, 30, 0.12}, {28, 3.8, 101, 47, 0.00}}};
 
 template <class F>
 WaveKPlan plan_b(const ProblemB &p)
@@ -99,7 +106,7 @@ WaveKPlan plan_b(const ProblemB &p)
     WaveKPlan best = {0, 0, 1e30};
     for (WaveKTile t : kTileCosts[F::CSZ - 1][F::VEC == 8 ? 0 : 1]) {
         if (forced > 0 && forced != t.tile) continue;
-        if (!fits<F>(p, t.tile) || (p.gated && t.tile % 10 == 1)) continue;
+        if (!fits<F>(p, t.tile) || (p.gated && t.tile % 2 == 1)) continue;
         with_tile(t.tile, [&](auto mp, auto np) {
             if (!takes_copies<F, mp(), np()>(p)) return;
             for (const WaveKTile &c : kCopiesCosts[F::VEC == 8 ? 0 : 1])
