@@ -77,6 +77,35 @@ def test_dequant_b_bit_exact(row):
     assert np.array_equal(want.view(np.uint16), c_oracle.dequant_b(_np(codes), _np(cb)).view(np.uint16))
 
 
+@pytest.mark.parametrize("N,K,v,E,G,bits", [(70, 1000, 8, 8, 1, 8), (66, 2052, 4, 16, 2, 16), (129, 2050, 2, 31, 3, 8), (2000, 1032, 4, 250, 4, 8), (4100, 4096, 8, 256, 1, 8)])
+def test_dequant_b_through_a_table_bit_exact(N, K, v, E, G, bits):
+    """Enough weights for a codebook in the LDS: runs that are no multiple of a store or a pass, a result and codes off 16 bytes, codes
+    past the last entry (which read that entry)."""
+    g = torch.Generator().manual_seed(17)
+    J = K // v
+    wide = torch.randint(0, E + 3, (N * J + 1,), generator=g, dtype=torch.int32)
+    codes = (wide.to(torch.uint8) if bits == 8 else wide.to(torch.int16).view(torch.uint16)).to(DEV)[1:].view(N, J)
+    cb = torch.randn(G, E, v, generator=g).half().to(DEV)
+    out = torch.full((N * K + 2 * v,), 7.0, dtype=torch.float16, device=DEV)
+    _say("dequant_b table", N, K, v, E, G, bits)
+    w = cabi.dequant_b(codes, cb, out=out[v:v + N * K].view(N, K))
+    torch.cuda.synchronize()
+    want = vo.dequant_b(np.minimum(_np(codes), E - 1), _np(cb))
+    assert np.array_equal(_np(w).view(np.uint16), want.view(np.uint16))
+    assert (out[:v] == 7.0).all() and (out[v + N * K:] == 7.0).all()
+
+
+@pytest.mark.parametrize("K,Nc", [(1030, 1028), (4200, 256), (300, 4000)])
+def test_dequant_a_through_a_table_bit_exact(K, Nc):
+    g = torch.Generator().manual_seed(18)
+    w = torch.randint(0, 256, (K, Nc), generator=g, dtype=torch.int32).to(torch.uint8).to(DEV)
+    cb = torch.randn(Nc // 4, 256, 2, generator=g).half().to(DEV)
+    _say("dequant_a table", K, Nc)
+    got = cabi.dequant_a(w, cb)
+    torch.cuda.synchronize()
+    assert np.array_equal(_np(got).view(np.uint16), vo.dequant_a(_np(w), _np(cb)).view(np.uint16))
+
+
 @pytest.mark.parametrize("row", SMALL_B, ids=[r[0] for r in SMALL_B])
 def test_e2e_gemm_b_all_variants(row):
     spec = _spec(row)
