@@ -17,8 +17,8 @@ __device__ __forceinline__ void lds_add(double *p, double v)
 }
 
 // The assignment step of a Lloyd iteration: codes, and one row of partial results per workgroup, lloyd_assign_rows(p) of them
-// per codebook.  Codebooks whose sums do not fit the LDS beside the table are not supported.
+// per codebook; `sums` false: the errors only.  Codebooks whose sums do not fit the LDS beside the table are not supported.
 int lloyd_assign_rows(const ProblemB &p);
-hipError_t launch_lloyd_assign(const half_t *w, const ProblemB &p, void *codes_out, float *partials, hipStream_t s);
+hipError_t launch_lloyd_assign(const half_t *w, const ProblemB &p, void *codes_out, float *partials, bool sums, hipStream_t s);
 
 }  // namespace vq

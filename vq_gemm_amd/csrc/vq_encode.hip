@@ -19,6 +19,8 @@
 //     fp32; all lanes read the same entry at a time (a broadcast), each thread scores four vectors against it.
 #include "vq_encode.h"
 
+#include <type_traits>
+
 namespace vq {
 
 namespace {
@@ -156,13 +158,16 @@ __device__ __forceinline__ HalfWaves swap_half_waves(uint32_t a, uint32_t b)
 }
 
 // LDS: entries padded to whole tiles of 32: halves with flipped signs, then |c|^2 / 2 (infinity behind the last entry),
-// then with ACCUMULATE the sums of the vectors assigned to each entry and their number, [entry][VEC + 1], then n_buckets words.
+// then with SUMS the sums of the vectors assigned to each entry and their number, [entry][VEC + 1], then n_buckets words.
 //
-// ACCUMULATE (a Lloyd iteration): every vector is added to its entry's sums, its distance to the workgroup's error, and
+// SUMS (a Lloyd iteration): every vector is added to its entry's sums, its distance to the workgroup's error, and
 // both leave as the workgroup's row of `partials`: entries * (VEC + 1) sums and counts, then the error.  The sums are kept in
 // double: an LDS addition of doubles takes a fifth of the time of one of floats on this device (2.1 M vectors of 8 elements:
-// 19 against 99 us), and is exact for weights of any usual range.
-template <int VEC, typename CodeT, int GROUP, bool ACCUMULATE, int kScanBatches>
+// 19 against 99 us), and is exact for weights of any usual range.  kErrorOnly: the last assignment, whose sums nothing reads (44.2 -> 38.7 us;
+// as a flag of the one kernel it cost every assignment half a microsecond).
+enum ScanKeeps { kCodesOnly, kErrorOnly, kSums };
+
+template <int VEC, typename CodeT, int GROUP, ScanKeeps KEEPS, int kScanBatches>
 __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t *__restrict__ w, const half_t *__restrict__ cb,
                                                                    CodeT *__restrict__ codes, int64_t vectors_per_cb, int entries,
                                                                    int wgs_per_cb, float *__restrict__ partials, int bucket_off,
@@ -170,6 +175,7 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
 {
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ float reduce[kScanThreads / 64];
+    constexpr bool ACCUMULATE = KEEPS != kCodesOnly, SUMS = KEEPS == kSums;
     constexpr int DW = VEC / 2;                       // dwords of a vector
     constexpr int kScanVectors = 32 * kScanBatches;   // of a wave
     // An entry's place in the table: one is left out after every 256 bytes of them, or the entries of all best groups, which
@@ -232,7 +238,7 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
             largest = n2 < __builtin_inff() ? fmaxf(largest, n2) : __builtin_inff();
             if (n_buckets && e < entries) atomicMin(&bucket[bucket_of(c)], (uint32_t)e);
         }
-        if constexpr (ACCUMULATE)
+        if constexpr (SUMS)
             for (int i = tid; i < entries * (VEC + 1); i += kScanThreads) sums[i] = 0.0;
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) largest = fmaxf(largest, __shfl_xor(largest, d));
@@ -404,14 +410,16 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
                     uint32_t c[DW];
                     read_entry<DW>(table, at(e_best), c);
                     error += rule_distance<DW>(full, c);
-                    double *sum = sums + e_best * (VEC + 1);
+                    if constexpr (SUMS) {
+                        double *sum = sums + e_best * (VEC + 1);
 #pragma unroll
-                    for (int i = 0; i < DW; i++) {
-                        const half2_t v = __builtin_bit_cast(half2_t, full[i]);
-                        lds_add(sum + 2 * i, (double)(float)v[0]);
-                        lds_add(sum + 2 * i + 1, (double)(float)v[1]);
+                        for (int i = 0; i < DW; i++) {
+                            const half2_t v = __builtin_bit_cast(half2_t, full[i]);
+                            lds_add(sum + 2 * i, (double)(float)v[0]);
+                            lds_add(sum + 2 * i + 1, (double)(float)v[1]);
+                        }
+                        lds_add(sum + VEC, 1.0);
                     }
-                    lds_add(sum + VEC, 1.0);
                 }
             }
         }
@@ -423,7 +431,8 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
         if (lane == 0) reduce[wave] = error;
         __syncthreads();
         float *row = partials + (int64_t)blockIdx.x * lloyd_row(entries, VEC);
-        for (int i = tid; i < entries * (VEC + 1); i += kScanThreads) row[i] = (float)sums[i];
+        if constexpr (SUMS)
+            for (int i = tid; i < entries * (VEC + 1); i += kScanThreads) row[i] = (float)sums[i];
         if (tid == 0) {
             float e = 0.f;
             for (int i = 0; i < kScanThreads / 64; i++) e += reduce[i];
@@ -470,17 +479,18 @@ bool scan_supports(const half_t *w, const ProblemB &p, bool accumulate)
     return ((uintptr_t)w & (align - 1)) == 0 && ((uintptr_t)p.cb & 3) == 0 && scan_lds_bytes(p, accumulate) <= kScanLds;
 }
 
-template <int VEC, typename CodeT, bool ACCUMULATE>
+template <int VEC, typename CodeT, ScanKeeps KEEPS>
 hipError_t launch_scan(const half_t *w, const ProblemB &p, void *codes_out, float *partials, hipStream_t s)
 {
     const int64_t vectors_per_cb = (int64_t)p.rows_per_cb * (p.K / VEC);
     if (vectors_per_cb == 0) return hipSuccess;
-    const ScanPlan plan = scan_plan(p, ACCUMULATE);
-    const size_t smem = scan_lds_bytes(p, ACCUMULATE);
-    const int buckets = scan_buckets(p, ACCUMULATE);
+    constexpr bool accumulate = KEEPS != kCodesOnly;   // (the last assignment in the same workgroups as the others)
+    const ScanPlan plan = scan_plan(p, accumulate);
+    const size_t smem = scan_lds_bytes(p, accumulate);
+    const int buckets = scan_buckets(p, accumulate);
     const bool narrow = p.entries < kScanWideGroupEntries;
-    auto kern = plan.batches == 4 ? (narrow ? encode_scan_kernel<VEC, CodeT, 8, ACCUMULATE, 4> : encode_scan_kernel<VEC, CodeT, 16, ACCUMULATE, 4>)
-                                  : (narrow ? encode_scan_kernel<VEC, CodeT, 8, ACCUMULATE, 2> : encode_scan_kernel<VEC, CodeT, 16, ACCUMULATE, 2>);
+    auto kern = plan.batches == 4 ? (narrow ? encode_scan_kernel<VEC, CodeT, 8, KEEPS, 4> : encode_scan_kernel<VEC, CodeT, 16, KEEPS, 4>)
+                                  : (narrow ? encode_scan_kernel<VEC, CodeT, 8, KEEPS, 2> : encode_scan_kernel<VEC, CodeT, 16, KEEPS, 2>);
     return launch_kernel(kern, dim3((unsigned)(plan.wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem + 4 * (size_t)buckets, s, w, p.cb,
                        static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, plan.wgs_per_cb, partials, (int)smem, buckets);
 }
@@ -488,7 +498,7 @@ hipError_t launch_scan(const half_t *w, const ProblemB &p, void *codes_out, floa
 template <int VEC, typename CodeT>
 hipError_t encode_b_typed(const half_t *w, const ProblemB &p, void *codes_out, hipStream_t s)
 {
-    if (scan_supports(w, p, false)) return launch_scan<VEC, CodeT, false>(w, p, codes_out, nullptr, s);
+    if (scan_supports(w, p, false)) return launch_scan<VEC, CodeT, kCodesOnly>(w, p, codes_out, nullptr, s);
     const int64_t vectors_per_cb = (int64_t)p.rows_per_cb * (p.K / VEC);
     if (vectors_per_cb == 0) return hipSuccess;
     // enough workgroups per codebook to fill the device a few times over, none without work
@@ -518,14 +528,19 @@ bool lloyd_supports(const ProblemB &p) { return encode_supports(p) && scan_lds_b
 
 int lloyd_assign_rows(const ProblemB &p) { return scan_plan(p, true).wgs_per_cb; }
 
-hipError_t launch_lloyd_assign(const half_t *w, const ProblemB &p, void *codes_out, float *partials, hipStream_t s)
+hipError_t launch_lloyd_assign(const half_t *w, const ProblemB &p, void *codes_out, float *partials, bool sums, hipStream_t s)
 {
     if (!lloyd_supports(p) || !scan_supports(w, p, true)) return hipErrorInvalidValue;
-    const bool u8 = p.code_bits == 8;
+    auto launch = [&](auto vec, auto code) {
+        typedef decltype(code) CodeT;
+        return sums ? launch_scan<vec(), CodeT, kSums>(w, p, codes_out, partials, s) : launch_scan<vec(), CodeT, kErrorOnly>(w, p, codes_out, partials, s);
+    };
+    auto with_code = [&](auto vec) { return p.code_bits == 8 ? launch(vec, uint8_t{}) : launch(vec, uint16_t{}); };
+    using std::integral_constant;
     switch (p.vec) {
-    case 8: return u8 ? launch_scan<8, uint8_t, true>(w, p, codes_out, partials, s) : launch_scan<8, uint16_t, true>(w, p, codes_out, partials, s);
-    case 4: return u8 ? launch_scan<4, uint8_t, true>(w, p, codes_out, partials, s) : launch_scan<4, uint16_t, true>(w, p, codes_out, partials, s);
-    default: return u8 ? launch_scan<2, uint8_t, true>(w, p, codes_out, partials, s) : launch_scan<2, uint16_t, true>(w, p, codes_out, partials, s);
+    case 8: return with_code(integral_constant<int, 8>{});
+    case 4: return with_code(integral_constant<int, 4>{});
+    default: return with_code(integral_constant<int, 2>{});
     }
 }
 
