@@ -261,6 +261,14 @@ __device__ __forceinline__ float wave_sum_to_uniform(float v)
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// Where the piece of x that code c of lane l's dword meets lies in its run: the pieces of a code together, so that the lanes of a
+// wave read 64 neighbouring ones.  ROTATED: by four a code, so that the sixteen lanes that a 16-byte write serves at a time (four
+// of them one code apart each) meet in no bank, 9 cycles a write and not 36 - for a long row of X or two rows (K = 11008, N = 4096
+// 5.66 -> 5.60 us, K = 28672, N = 8192 12.4 -> 12.0, two rows at K = 14336 8.5 -> 8.25); one of up to 8192 halves has too few
+// writes to pay for the rotation (K = N = 4096 3.78 -> 3.83).
+template <bool ROTATED>
+__device__ __forceinline__ int wide_x_slot(int c, int l) { return c * 64 + (ROTATED ? (l + 4 * c) & 63 : l & 63); }
+
 // floor(x / d) for 0 <= x < 2^23 or so through a float reciprocal and one correction step; rcp = 1.0f / d.
 __device__ __forceinline__ int small_quotient(int x, int d, float rcp)
 {
@@ -457,13 +465,13 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
         }
     } else {
         // x: piece i = q*256 + 4*l + c (the 8 halves that code c of lane l's dword in run q meets) is kept at
-        // q*256 + c*64 + l, so that the lanes of a wave read 64 neighbouring pieces.
+        // q*256 + wide_x_slot(c, l).
 #pragma unroll
         for (int i = 0; i < kXPerThread; i++) {
             const int xi = xt + i * kDutyThreads;
             // (the long form: zeros behind the end of x, up to whole pieces of rows)
             if (LONG && xi - (XM > 1 && xi >= kXChunks ? kXChunks : 0) >= J) xpiece[i] = uint4_t{0u, 0u, 0u, 0u};
-            if (xi < XM * kXChunks) xs[(xi & ~255) + (xi & 3) * 64 + ((xi >> 2) & 63)] = xpiece[i];
+            if (xi < XM * kXChunks) xs[(xi & ~255) + wide_x_slot<LONG || XM == 2>(xi & 3, xi >> 2)] = xpiece[i];
         }
     }
     __syncthreads();
@@ -475,7 +483,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
 #pragma unroll
             for (int q = 0; q < RUNS; q++)
 #pragma unroll
-                for (int c = 0; c < 4; c++) xr[m][q][c] = xs[m * kXChunks + (piece * RUNS + q) * kRunCodes + c * 64 + lane];
+                for (int c = 0; c < 4; c++) xr[m][q][c] = xs[m * kXChunks + (piece * RUNS + q) * kRunCodes + wide_x_slot<LONG || XM == 2>(c, lane)];
     };
     load_x_piece(0);
 
@@ -663,7 +671,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
                 for (int j = lane; j < J; j += 64) {
                     const uint4_t wv = *reinterpret_cast<const uint4_t *>(tbl + row[j] * (uint32_t)(kWideCopies * 16) + copy_base);
                     const int xi = m * kXChunks + j;
-                    const uint4_t xv = xs[(xi & ~255) + (xi & 3) * 64 + ((xi >> 2) & 63)];
+                    const uint4_t xv = xs[(xi & ~255) + wide_x_slot<LONG || XM == 2>(xi & 3, xi >> 2)];
 #pragma unroll
                     for (int d = 0; d < 4; d++) {
                         const uint32_t wd = wv[d], xd = xv[d];
