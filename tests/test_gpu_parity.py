@@ -77,7 +77,7 @@ def test_dequant_b_bit_exact(row):
     assert np.array_equal(want.view(np.uint16), c_oracle.dequant_b(_np(codes), _np(cb)).view(np.uint16))
 
 
-@pytest.mark.parametrize("N,K,v,E,G,bits", [(70, 1000, 8, 8, 1, 8), (66, 2052, 4, 16, 2, 16), (129, 2050, 2, 31, 3, 8), (2000, 1032, 4, 250, 4, 8), (4100, 4096, 8, 256, 1, 8)])
+@pytest.mark.parametrize("N,K,v,E,G,bits", [(1030, 3080, 8, 8, 1, 8), (1026, 3100, 4, 16, 2, 16), (1551, 2050, 2, 31, 3, 8), (2000, 2056, 4, 250, 4, 8), (4100, 4096, 8, 256, 1, 8)])
 def test_dequant_b_through_a_table_bit_exact(N, K, v, E, G, bits):
     """Enough weights for a codebook in the LDS: runs that are no multiple of a store or a pass, a result and codes off 16 bytes, codes
     past the last entry (which read that entry)."""

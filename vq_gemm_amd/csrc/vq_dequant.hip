@@ -100,13 +100,13 @@ static hipError_t dequant_b_typed(const ProblemB &p, half_t *w_out, hipStream_t 
     dim3 grid((unsigned)blocks), block(256);
     // Vector copies need codeword-aligned source and destination; otherwise copy scalars.
     const bool aligned = (((uintptr_t)w_out | (uintptr_t)p.cb) % (uintptr_t)(p.vec * 2)) == 0;
-    // a table for every workgroup, where a compute unit, and a codebook's rows, come to four times as much or more (at half of that, 1024 x 1024,
-    // 3.0 and 3.3 us)
+    // a table for every workgroup, where a compute unit, and a codebook's rows, come to four times as much or more and there are
+    // workgroups for three units in eight (4-vectors: 1024 x 3072, 96 of them, 4.4 us -> 4.0; 2320 x 576, 42, 3.3 -> 3.7)
     const size_t table = (size_t)p.entries * p.vec * 2;
-    const int64_t per_cb = (int64_t)p.rows_per_cb * J;
-    if (aligned && table <= kDequantTable && total * p.vec * 2 >= 4 * (int64_t)table * device_cu_count() && per_cb >= 4 * p.entries) {
-        const int64_t step = (int64_t)kDequantThreads * kDequantUnroll * 8 / p.vec;
-        const int64_t want = (2 * device_cu_count() + p.n_codebooks - 1) / p.n_codebooks, have = (per_cb + step - 1) / step;
+    const int64_t per_cb = (int64_t)p.rows_per_cb * J, step = (int64_t)kDequantThreads * kDequantUnroll * 8 / p.vec, have = (per_cb + step - 1) / step;
+    if (aligned && table <= kDequantTable && total * p.vec * 2 >= 4 * (int64_t)table * device_cu_count() && per_cb >= 4 * p.entries &&
+        have * p.n_codebooks * 8 >= 3 * device_cu_count()) {
+        const int64_t want = (2 * device_cu_count() + p.n_codebooks - 1) / p.n_codebooks;
         const int wgs = (int)(want < have ? want : have);
         auto launch = [&](auto kern) { return launch_kernel(kern, dim3((unsigned)(wgs * p.n_codebooks)), dim3(kDequantThreads), table, s, codes, p.cb, w_out, per_cb, p.entries, wgs); };
         switch (p.vec) {
