@@ -579,8 +579,9 @@ hipError_t launch_tile(WaveKArgs a, hipStream_t s)
     typedef WaveKCfg<P, MP, NP> C;
     a.tiles_m = (a.M + C::TM - 1) / C::TM;
     a.tiles_n = (a.N + C::TN - 1) / C::TN;
-    // (geometry A by columns: a tile takes 16 or 32 bytes of a row of codes, and those beside it the rest of the line)
-    a.by_rows = P::kA ? 0 : wave_k_by_rows(a.tiles_m, a.tiles_n, C::TM * 2.0, C::TN * (P::kB ? (double)P::CSZ / P::VEC : 2.0));
+    // (geometry A by columns: a tile takes 16 or 32 bytes of a row of codes, and those beside it the rest of the line; so fp16 W, whose
+    // tiles bring as much of it as of X: M = 1306, K = 3712, N = 1280 34.5 us, by rows 36.5)
+    a.by_rows = P::kB ? wave_k_by_rows(a.tiles_m, a.tiles_n, C::TM * 2.0, C::TN * (double)P::CSZ / (P::kB ? P::VEC : 1)) : 0;
     const size_t lds = C::lds_bytes(P::kB ? (size_t)a.books * a.entries * P::VEC * 2 : C::kBooks);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     return launch_kernel(wave_k_kernel<P, MP, NP>, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(C::kWaves * 64), lds, s, a);
