@@ -230,6 +230,33 @@ static_assert(every_tile<Format<4, uint8_t>>() && every_tile<Format<4, uint16_t>
     assert res.returncode == 0, res.stdout + res.stderr
 
 
+def test_nothing_touches_the_registers_of_a_load_that_the_compiler_does_not_count(tmp_path):
+    """The codebook entries of the wave-K kernel's table of copies come by inline assembly into registers that the compiler takes for
+    written at once: no branch, at whose ends it may copy them, and no use may lie ahead of the wait.  On the assembly of
+    two of its kernels, as the build looks at it for all of them."""
+    import subprocess
+    from vq_gemm_amd import build
+    src, asm = tmp_path / "copies.hip", tmp_path / "copies.s"
+    src.write_text("""
+#include "vq_wave_k.h"
+namespace vq {
+namespace {
+template __global__ void wave_k_kernel<WaveB<8, uint8_t, 2, true>, 1, 2>(const WaveKArgs);
+template __global__ void wave_k_kernel<WaveB<4, uint8_t, 2, true>, 1, 1>(const WaveKArgs);
+}
+}
+""")
+    flags = [f for f in build.HIP_FLAGS if f not in ("-Wall", "-Wno-unused-function")]
+    res = subprocess.run([build.HIPCC] + flags + ["-x", "hip", "--offload-device-only", "-S", f"-I{build.CSRC}", str(src), "-o", str(asm)], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout + res.stderr
+    assert build.check_loads_in_flight(asm.read_text()) == 4   # (with as many units as are loaded ahead, and with fewer)
+    load, wait = ";;#ASMSTART\nglobal_load_dwordx4 v[2:5], v[0:1], off\n;;#ASMEND\n", "s_waitcnt vmcnt(3)\n"
+    assert build.check_loads_in_flight(load + "v_add_u32_e32 v6, 1, v7\n" + wait + "v_mov_b32_e32 v6, v2\n") == 1
+    for between in ("v_mov_b32_e32 v6, v2\n", "ds_write_b128 v8, v[4:7]\n", "s_cbranch_scc1 .L1\n", ".L1:\n"):
+        with pytest.raises(RuntimeError, match="being loaded"):
+            build.check_loads_in_flight(load + between + wait)
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="made-up addresses: only where no kernel can be launched")
 def test_stages_need_no_more_scratch_than_they_ask_for_wherever_the_operands_begin():
     lib = cabi.lib()

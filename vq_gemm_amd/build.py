@@ -15,6 +15,7 @@ compiler and linked against libvqgemm.so; no source passes through hipify.
 from __future__ import annotations
 
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -113,6 +114,36 @@ def _check_no_spills(asm_path: str) -> None:
     if bad:
         raise RuntimeError("register spills / scratch in a kernel that must have none:\n" + "\n".join(bad))
 
+# The wave-K kernel's one load by inline assembly into registers (a codebook entry per thread): between it and its wait the
+# compiler must not touch them, and no branch lies there.  (The batched decode kernel's go round its loop, held by the
+# bit-exact tests.)
+REGISTER_LOAD_SOURCES = {"vq_wave_k_b.hip"}
+
+
+def check_loads_in_flight(asm: str) -> int:
+    """Raises if, in the assembly `asm`, anything but a straight line without their registers lies between the register loads of
+    inline assembly and the next wait for loads.  Returns how many such loads there are."""
+    seen, in_asm, flying = 0, False, None
+    for line in asm.splitlines():
+        if "#ASMSTART" in line or "#ASMEND" in line:
+            in_asm = "#ASMSTART" in line
+            continue
+        text = line.split(";")[0].strip()
+        if not text or (text.startswith(".") and not text.endswith(":")):
+            continue
+        if flying:
+            regs = {r for a, b in re.findall(r"\bv\[(\d+):(\d+)\]", text) for r in range(int(a), int(b) + 1)} | {int(r) for r in re.findall(r"\bv(\d+)\b", text)}
+            if re.match(r"s_waitcnt\b.*vmcnt", text):
+                flying = None
+            elif regs & flying or text.endswith(":") or text.startswith(("s_cbranch", "s_branch", "s_endpgm", "s_setpc", "s_swappc")):
+                raise RuntimeError(f"a register that is being loaded: {text}")
+        elif in_asm:
+            m = re.match(r"global_load_dword\w* v\[(\d+):(\d+)\]", text)
+            if m:
+                flying = set(range(int(m[1]), int(m[2]) + 1))
+                seen += 1
+    return seen
+
 
 def _headers():
     hs = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".h")]
@@ -135,7 +166,12 @@ def build_lib(force: bool = True, jobs: int = 6) -> str:
             extra = KERNARG_PRELOAD_FLAGS if src in KERNARG_PRELOAD_SOURCES else []
             _run([HIPCC] + HIP_FLAGS + extra + ["--save-temps=obj", "-c", s, "-o", o])
             if src not in HOST_ONLY_SOURCES:
-                _check_no_spills(o.replace(".o", f"-hip-amdgcn-amd-amdhsa-{ARCH}.s"))
+                asm_path = o.replace(".o", f"-hip-amdgcn-amd-amdhsa-{ARCH}.s")
+                _check_no_spills(asm_path)
+                if src in REGISTER_LOAD_SOURCES:
+                    with open(asm_path) as f:
+                        if check_loads_in_flight(f.read()) == 0:
+                            raise RuntimeError(f"{asm_path}: no register load found, the check of those in flight did not run")
         return o
 
     with ThreadPoolExecutor(max_workers=jobs) as ex:

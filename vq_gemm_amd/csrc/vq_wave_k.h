@@ -152,28 +152,6 @@ struct WaveKArgs {
     int by_rows;           // consecutive tiles lie along the rows of tiles (wave_k_by_rows)
 };
 
-// The entry of a table of copies by a load that the compiler does not count, beside the direct loads, which it does not either:
-// it would wait for all of them.  The registers are not to be read ahead of loaded_entry, behind the wait.
-template <int DW>
-__device__ __forceinline__ void load_entry(uint32_t (&entry)[DW], const half_t *src)
-{
-    typedef uint32_t entry_t __attribute__((ext_vector_type(DW)));
-    entry_t v;
-    if constexpr (DW == 4) asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(v) : "v"(src) : "memory");
-    else asm volatile("global_load_dwordx2 %0, %1, off" : "=&v"(v) : "v"(src) : "memory");
-#pragma unroll
-    for (int i = 0; i < DW; i++) entry[i] = v[i];
-}
-
-// sixteen bytes of a row of copies: the entry, or two side by side
-template <int DW>
-__device__ __forceinline__ uint4_t loaded_entry(uint32_t (&entry)[DW])
-{
-#pragma unroll
-    for (int i = 0; i < DW; i++) asm volatile("" : "+v"(entry[i]));
-    return uint4_t{entry[0], entry[1], entry[DW == 4 ? 2 : 0], entry[DW == 4 ? 3 : 1]};
-}
-
 template <class P, int MP, int NP>
 __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) / 4) void wave_k_kernel(const WaveKArgs a)
 {
@@ -243,9 +221,11 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
     };
     const int64_t w_unit = P::kB ? C::kCodeBytes : kUnitK * w_row;     // bytes from unit to unit
     const half_t *x_tile = a.x + (int64_t)m0 * k_x;
-    int x_at = wave * kUnitK;
-    if constexpr (P::kB)
+    int x_at = wave * kUnitK, x_step = kWaves * kUnitK;   // (an X that repeats along K: modulo its columns)
+    if constexpr (P::kB) {
         while (x_at >= k_x) x_at -= k_x;
+        while (x_step >= k_x) x_step -= k_x;
+    }
     const uint8_t *w_ahead = static_cast<const uint8_t *>(a.w) + (P::kB ? (int64_t)n0 * w_row : w_col - w_skew) + wave * w_unit;
     auto issue = [&](int buf, int u) {
         const uint32_t at = ring + buf * C::kUnitBytes;
@@ -255,9 +235,8 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
 #pragma unroll
         for (int i = 0; i < S * MP; i++) load_to_lds_16(at + i * 1024, x_voff[i], x_tile + x_at);
         w_ahead += kWaves * w_unit;
-        x_at += kWaves * kUnitK;
-        if constexpr (P::kB)
-            while (x_at >= k_x) x_at -= k_x;
+        x_at += x_step;
+        if constexpr (P::kB) x_at = (int)min((uint32_t)x_at, (uint32_t)(x_at - k_x));
     };
 
     // ---- operands -------------------------------------------------------------------------------
@@ -406,12 +385,7 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
     };
 
     // ---- codebooks, first units -------------------------------------------------------------------
-    uint32_t entry[P::VEC == 4 ? 2 : 4];   // (copies) the thread's, on its way until the wait below
-    if constexpr (P::kCopies) {
-        static_assert(P::VEC == 8 || P::VEC == 4, "entries of 16 or 8 bytes");
-        const half_t *src = a.cb + ((int64_t)(n0 / a.rows_per_cb) * a.entries + min(tid & (kCopiesEntries - 1), a.entries - 1)) * P::VEC;
-        load_entry(entry, src);
-    } else if constexpr (P::kA || P::kB) {
+    if constexpr (!P::kCopies && (P::kA || P::kB)) {
         const int book_bytes = P::kA ? 1024 : a.entries * (P::VEC * 2);
         const int g_first = P::kA ? n0 / 8 : n0 / a.rows_per_cb;
         const int n16 = (P::kA ? C::TN / 8 : a.books) * book_bytes / 16;
@@ -421,22 +395,49 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
         for (int i0 = wave * 64; i0 < n16; i0 += kWaves * 64)
             load_to_lds_16(kBookBase + i0 * 16, (uint32_t)min(i0 + lane, last16) * 16u, src);
     }
-#pragma unroll
-    for (int d = 0; d < D; d++)
-        if (d < n_unit) issue(d, d);
     if constexpr (P::kCopies) {
-        // (the entry is the oldest load)
-        if (n_unit >= D) wait_vmcnt<D * C::kLoads>();
-        else wait_vmcnt<0>();
+        // The thread's entry comes by a load into registers, beside the others the first to be back.  The compiler does not count it: nothing
+        // but the units' loads, no branch, lies between it and the wait (the build looks at that), and where there are
+        // fewer units it goes last.
+        static_assert(P::VEC == 8 || P::VEC == 4, "entries of 16 or 8 bytes");
+        typedef uint32_t entry_t __attribute__((ext_vector_type(P::VEC / 2)));
+        const half_t *src = a.cb + ((int64_t)(n0 / a.rows_per_cb) * a.entries + min(tid & (kCopiesEntries - 1), a.entries - 1)) * P::VEC;
+        entry_t entry;
+        auto load_entry = [&]() {
+            if constexpr (P::VEC == 8) asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(entry) : "v"(src) : "memory");
+            else asm volatile("global_load_dwordx2 %0, %1, off" : "=&v"(entry) : "v"(src) : "memory");
+        };
         // two threads an entry (four of sixteen waves), eight (four) pieces of 16 bytes each, neighbouring entries in another order
-        constexpr int kPer = kWaves * 64 / kCopiesEntries, kPieces = 16 / kPer;
-        static_assert(kPer == 2 || kPer == 4, "threads an entry");
-        const uint4_t piece = loaded_entry(entry);
-        const uint32_t at = kBookBase + (tid & (kCopiesEntries - 1)) * 256 + (tid >> 8) * (kPieces * 16) + (tid & (kPieces - 1)) * 16;
+        auto write_copies = [&]() {
+            asm volatile("" : "+v"(entry));
+            constexpr int kPer = kWaves * 64 / kCopiesEntries, kPieces = 16 / kPer;
+            static_assert(kPer == 2 || kPer == 4, "threads an entry");
+            const uint4_t piece = {entry[0], entry[1], entry[P::VEC == 8 ? 2 : 0], entry[P::VEC == 8 ? 3 : 1]};
+            const uint32_t at = kBookBase + (tid & (kCopiesEntries - 1)) * 256 + (tid >> 8) * (kPieces * 16) + (tid & (kPieces - 1)) * 16;
 #pragma unroll
-        for (int i = 0; i < kPieces; i++) *reinterpret_cast<uint4_t *>(smem + (at ^ (i * 16))) = piece;
+            for (int i = 0; i < kPieces; i++) *reinterpret_cast<uint4_t *>(smem + (at ^ (i * 16))) = piece;
+        };
+        if (n_unit >= D) {
+            load_entry();
+#pragma unroll
+            for (int d = 0; d < D; d++) issue(d, d);
+            wait_vmcnt<D * C::kLoads>();
+            write_copies();
+        } else {
+#pragma unroll
+            for (int d = 0; d < D; d++)
+                if (d < n_unit) issue(d, d);
+            load_entry();
+            wait_vmcnt<0>();
+            write_copies();
+        }
         __syncthreads();
-    } else if constexpr (P::kA || P::kB) {
+    } else {
+#pragma unroll
+        for (int d = 0; d < D; d++)
+            if (d < n_unit) issue(d, d);
+    }
+    if constexpr (!P::kCopies && (P::kA || P::kB)) {
         // (the codebooks are the oldest loads of the waves that brought them)
         if (n_unit >= D) wait_vmcnt<D * C::kLoads>();
         else wait_vmcnt<0>();
