@@ -115,7 +115,7 @@ int vqgemm_e2e_gemm_b_bias(const void *x, const void *codes, const void *codeboo
  * one launch and the columns of W that are left over as a second one, in 128x128 tiles with K split there; either
  * only when `workspace_bytes` suffices (a workspace that is too small, or NULL, is no error for AUTO: it does without).  vqgemm_workspace_bytes_b says
  * how many bytes the given variant (AUTO, PREFILL_SPLITK, TWOPASS) wants for a shape: 0 when it uses none, a
- * negative error for an invalid shape (AUTO names split K's bytes too where the wave-K kernel, which needs none, is not far ahead of it).  `workspace` must be 256-byte aligned device memory; its contents before the
+ * negative error for an invalid shape.  `workspace` must be 256-byte aligned device memory; its contents before the
  * call do not matter and are undefined after it; two calls that overlap in time need a workspace each.  An explicit
  * variant with too small a workspace returns VQGEMM_E_SCRATCH.  The partial sums of a tile are added in the order
  * of the slices of K whichever workgroup finishes last: results are the same from run to run.  No counterpart in

@@ -1864,11 +1864,12 @@ def test_split_k_gives_the_same_bits_whatever_the_workspace_held():
 
 
 def test_split_k_is_what_the_automatic_choice_takes_for_medium_m_on_few_columns_and_only_with_a_workspace():
-    M, K, N = 512, 4096, 4096
-    spec = ProblemSpec("auto_split", GEOM_B, M, K, N, 8, 256, 32, 8, codebook_3d=True, codebook_std=0.05)
+    M, K, N = 954, 14080, 1920
+    spec = ProblemSpec("auto_split", GEOM_B, M, K, N, 8, 256, 15, 8, codebook_3d=True, codebook_std=0.05)
     x, codes, cb = make_problem(spec, seed=63, device=DEV)
-    need = cabi.workspace_bytes_b(M, K, N, 8, 256, 32, 8)
-    assert need > 0
+    dims = (M, K, N, 8, 256, 15, 8)
+    need = cabi.workspace_bytes_b(*dims)
+    assert need > 0 and cabi.auto_variant_name_b(*dims, need) == "prefill_splitk" != cabi.auto_variant_name_b(*dims)
     want = vo.vq_gemm_b(_np(x), _np(codes), _np(cb), acc=np.float64)
     y_plain = cabi.e2e_gemm_b(x, codes, cb)                      # no workspace: the unsplit choice
     y_split = cabi.e2e_gemm_b_ws(x, codes, cb)                   # allocates what workspace_bytes_b says
@@ -1876,8 +1877,11 @@ def test_split_k_is_what_the_automatic_choice_takes_for_medium_m_on_few_columns_
     # where a split cannot pay the automatic choice wants no workspace: one row of X, a full device of large tiles
     assert cabi.workspace_bytes_b(1, 4096, 4096, 8, 256, 1, 8) == 0 and cabi.workspace_bytes_b(14, 512, 768, 8, 256, 3, 8) == 0
     assert cabi.workspace_bytes_b(4096, 4096, 4096, 8, 256, 32, 8) == 0
+    # the kernels that were named are the ones that ran: the bits of the variants asked for
+    ws = torch.empty(max(need, cabi.workspace_bytes_b(*dims, cabi.VARIANT_PREFILL_SPLITK)), dtype=torch.uint8, device=DEV)
+    assert torch.equal(y_split, cabi.e2e_gemm_b_ws(x, codes, cb, variant=cabi.VARIANT_PREFILL_SPLITK, workspace=ws))
+    assert torch.equal(y_plain, cabi.e2e_gemm_b(x, codes, cb, variant=cabi.VARIANT_WAVE_K))
     # captured into a graph and replayed (the counters are cleared by a kernel, not a memset node)
-    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
     out = torch.empty(M, N, dtype=torch.float16, device=DEV)
     st = torch.cuda.Stream()
     with torch.cuda.stream(st):

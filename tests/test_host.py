@@ -313,12 +313,28 @@ def test_native_calls_let_other_threads_run():
 
 
 def test_split_k_is_asked_for_where_it_was_measured_faster():
-    """The workspace the automatic choice asks for: none where the wave-K kernel was measured at 0.75 to 0.85 of split K's time, slices
-    of K where it was the other way round (short K with a middling M here, few columns of a long K there)."""
-    for M, K, N, v, e, bits in ((203, 2816, 7040, 8, 256, 8), (489, 3072, 3328, 8, 256, 8), (72, 2304, 8832, 4, 4096, 16), (438, 2944, 3072, 4, 4096, 16)):
+    """The workspace the automatic choice asks for: none where the wave-K kernel was measured at 0.75 to 0.85 of split K's time (657 x
+    13376 x 1040: 28.1 us, split 34.3), slices of K where it was the other way round (3028 x 11264 x 640: 51.5 us, the wave-K kernel
+    61.3; 954 x 14080 x 1920 59.9, 70.1; 118 x 11008 x 14080 55.0, 65.1)."""
+    for M, K, N, v, e, bits in ((657, 13376, 1040, 8, 256, 8), (203, 2816, 7040, 8, 256, 8), (489, 3072, 3328, 8, 256, 8), (72, 2304, 8832, 4, 4096, 16), (438, 2944, 3072, 4, 4096, 16)):
         assert cabi.workspace_bytes_b(M, K, N, v, e, 1, bits) == 0, (M, K, N)
-    for M, K, N, v, e, bits in ((3028, 11264, 640, 8, 256, 8), (954, 14080, 1920, 8, 256, 8), (657, 13376, 1040, 8, 256, 8), (118, 11008, 14080, 4, 4096, 16)):
+    for M, K, N, v, e, bits in ((3028, 11264, 640, 8, 256, 8), (954, 14080, 1920, 8, 256, 8), (118, 11008, 14080, 4, 4096, 16)):
         assert cabi.workspace_bytes_b(M, K, N, v, e, 1, bits) > 0, (M, K, N)
+
+
+def test_a_workspace_is_asked_for_only_where_it_is_used():
+    """Over random shapes: a call with the workspace that is asked for launches a plan that needs one."""
+    import random
+    rng = random.Random(5)
+    asked = 0
+    for _ in range(600):
+        v, e, bits = rng.choice(((8, 256, 8), (4, 256, 8), (4, 4096, 16), (8, 512, 16)))
+        dims = (int(17 * 170 ** rng.random()), 64 * int(8 * 28 ** rng.random()), 16 * int(32 * 50 ** rng.random()), v, e, 1, bits)
+        need = cabi.workspace_bytes_b(*dims)
+        assert need == 0 or cabi.auto_variant_name_b(*dims, need) in ("prefill_splitk", "prefill_tail_split"), (dims, need)
+        asked += need > 0
+    assert asked >= 20
+    assert cabi.workspace_bytes_b(512, 4096, 4096, 8, 256, 32, 8) == 0 and cabi.auto_variant_name_b(512, 4096, 4096, 8, 256, 32, 8) == "wave_k"
 
 
 def test_the_report_of_the_automatic_choice_names_what_it_launches():

@@ -291,7 +291,7 @@ int splitk_auto(const ProblemB &p, double *t_best, int *plain_variant)
 // of large tiles with the left-over columns in 128x128 tiles and K split there (tail) - whichever the cost models
 // expect to be fastest by a margin.
 struct WorkspaceChoice {
-    bool wave;      // the wave-K kernel, which needs none (`bytes`: asked for all the same)
+    bool wave;      // the wave-K kernel, which needs none
     int sp;
     TailSplitPlan tail;
     size_t bytes;
@@ -300,9 +300,6 @@ struct WorkspaceChoice {
 // off.  Over 150 shapes of M 65 to 2000 the choice takes 0.91 of the time that it took before the tiles with a compute unit to
 // themselves, the wave-K kernel's last tile shapes and its faster reads of X (512 x 4096 x 4096: 27 us, split K 32).
 constexpr double kWaveMargin = 0.95;
-// Where split K was the plan until then, its workspace is still asked for, unless the wave-K kernel is far ahead: what a caller has
-// set aside by an earlier answer stays the answer.
-constexpr double kStillAsked = 0.75;
 
 WorkspaceChoice workspace_auto(const ProblemB &p)
 {
@@ -325,7 +322,7 @@ WorkspaceChoice workspace_auto(const ProblemB &p)
     const bool asked = tuning().splitk_force_splits >= 2.0 || tuning().tail_split_margin >= 1e3;
     const double t_other = c.tail.ok ? c.tail.cost_us : c.sp >= 2 ? t_best : prefill_cost_us(p);
     if (!(asked && c.bytes > 0) && (plain == VQGEMM_VARIANT_DECODE || plain == VQGEMM_VARIANT_PREFILL) && wave_k_b_preferred(p, t_other, kWaveMargin))
-        c = {true, 0, {false, 0, 0, 0, 1e30, 0}, c.sp >= 2 && wave_k_b_cost_us(p) > kStillAsked * t_other ? c.bytes : 0};
+        c = {true, 0, {false, 0, 0, 0, 1e30, 0}, 0};
     return c;
 }
 
