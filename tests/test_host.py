@@ -337,10 +337,19 @@ def test_a_workspace_is_asked_for_only_where_it_is_used():
     assert cabi.workspace_bytes_b(512, 4096, 4096, 8, 256, 32, 8) == 0 and cabi.auto_variant_name_b(512, 4096, 4096, 8, 256, 32, 8) == "wave_k"
 
 
+def test_no_width_is_an_exception_in_the_choice_between_decode_and_wave_k():
+    """One tile of the decode kernel to each of 256 compute units, and a tile less and more: 16 x 4096 x 4096 is 5.65 us by the wave-K
+    kernel and 6.50 by the decode kernel, as it is 5.66 and 6.49 on 4080 columns."""
+    name = cabi.auto_variant_name_b
+    for M, K, v, e, bits in ((16, 4096, 8, 256, 8), (16, 2048, 8, 256, 8), (8, 8192, 8, 256, 8), (16, 4096, 4, 256, 8), (5, 8192, 4, 256, 8), (8, 8192, 8, 512, 16)):
+        assert {name(M, K, N, v, e, 1, bits) for N in (4080, 4096, 4112)} == {"wave_k"}, (M, K, v, bits)
+    assert {name(3, 1024, N, 8, 256, 1, 8) for N in (4080, 4096)} == {"decode"}
+
+
 def test_the_report_of_the_automatic_choice_names_what_it_launches():
     """Host only; that the kernels named are the ones launched is held bit for bit on the GPU."""
     name = cabi.auto_variant_name_b
-    assert name(1, 4096, 4096, 8, 256, 1, 8) == "decode_gemv" and name(16, 4096, 4096, 8, 256, 1, 8) == "decode"
+    assert name(1, 4096, 4096, 8, 256, 1, 8) == "decode_gemv" and name(3, 4096, 4096, 8, 256, 1, 8) == "decode"
     assert name(64, 8192, 14336, 4, 4096, 1, 16) == "wave_k" and cabi.select_variant_b(64, 8192, 14336, 4, 4096, 1, 16) == cabi.VARIANT_DECODE
     assert name(4096, 4096, 4096, 8, 256, 32, 8) == "prefill" and name(4, 60, 20, 4, 256, 1, 8) == "generic"
     for dims, plan in (((954, 14080, 1920, 8, 256, 1, 8), "prefill_splitk"), ((1536, 4096, 11008, 8, 256, 43, 8), "prefill_tail_split")):

@@ -201,14 +201,10 @@ bool wave_k_b_preferred(const ProblemB &p, double t_other, double margin)
         // (the streaming kernel, up to 16 rows: over 34 of its shapes on codes out of HBM the tile expected to be fastest takes 0.85 of
         // its time up to K = 24576 - 16 x 11008 x 4096 11.9 us -> 8.9 - and over 7 from there on 1.03, 13 x 27520 x 2944 17.5 -> 20.2)
         if (t_decode > 1e29) return p.M > 16 || (p.K <= 24576 && decode_stream_preferred(p));
-        // The gated decode kernels deal tiles in pairs, which their model does not see.  Up to 16 rows: over 246 shapes on codes out of HBM
-        // and 146 on codes in the caches this line is 0.9 and 0.6 % from the better kernel (0.97: 0.8 and 0.3, 0.89: 1.6 and 1.0; 4 x 4096 x 8192,
-        // which is asked for in the packed layout, lies between; one and two rows of X, which the models know least,
-        // 2 x 1024 x 576 3.0 us and 3.4, by more).  Where the decode kernel's workgroups
-        // come out at exactly one a compute unit, none idle and none with two, it gives the least away (16 x 4096 x 4096: cold 6.48 us
-        // against 5.87; 2048 x 4096 5.3, 4.9) and the choice that callers have seen reported for such a layer stays.
-        const bool one_each = p.N == device_cu_count() * 16 && p.M <= 16;
-        return wave_k_b_cost_us(p) < (p.gated ? 1.15 : one_each ? 0.80 : p.M <= 2 ? 0.85 : p.M <= 16 ? 0.94 : 0.97) * t_decode;
+        // The gated decode kernels deal tiles in pairs, which their model does not see.  3 to 16 rows: over 425 shapes this line is 1.4 %
+        // from the better kernel on codes out of HBM and 0.9 % on codes in the caches (0.92: 1.3 and 1.2, 0.97: 1.8 and 0.8, 0.80: 3.6
+        // and 7.2); one and two rows of X, which the models know least (2 x 1024 x 576 3.0 us and 3.4), by more.
+        return wave_k_b_cost_us(p) < (p.gated ? 1.15 : p.M <= 2 ? 0.85 : p.M <= 16 ? 0.94 : 0.97) * t_decode;
     }
     return wave_k_b_cost_us(p) < margin * t_other;
 }
