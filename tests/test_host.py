@@ -346,6 +346,16 @@ def test_no_width_is_an_exception_in_the_choice_between_decode_and_wave_k():
     assert {name(3, 1024, N, 8, 256, 1, 8) for N in (4080, 4096)} == {"decode"}
 
 
+def test_many_codes_go_where_they_stream_faster():
+    """Codes out of HBM, us by the wave-K and by the decode kernel: 60.5 and 45.8, 45.0 and 35.1, 30.2 and 24.0, 39.7 and 35.0; where every
+    unit has a tile the other way round, 12.8 and 16.9, 15.8 and 21.2, 19.7 and 28.8."""
+    name = cabi.auto_variant_name_b
+    for dims, want in (((5, 11648, 27328, 4, 4096, 1, 16), "decode"), ((4, 8448, 26048, 4, 4096, 1, 16), "decode"), ((12, 5120, 24832, 4, 4096, 1, 16), "decode"),
+                       ((8, 12288, 27968, 8, 512, 1, 16), "decode"), ((8, 8192, 8192, 4, 4096, 1, 16), "wave_k"), ((3, 12288, 8192, 4, 4096, 64, 16), "wave_k"),
+                       ((3, 13440, 14848, 8, 512, 1, 16), "wave_k")):
+        assert name(*dims) == want, dims
+
+
 def test_the_report_of_the_automatic_choice_names_what_it_launches():
     """Host only; that the kernels named are the ones launched is held bit for bit on the GPU."""
     name = cabi.auto_variant_name_b

@@ -186,6 +186,21 @@ int wave_k_b_tile(const ProblemB &p)
     return tile;
 }
 
+// What the codes take to come out of HBM, at most 64 rows of X: the more of a row a unit of K brings (8, 16 or 32 bytes), the more are on
+// their way - 2.0, 3.3 or 3.8 TB/s when every compute unit works, its share of that when some have no tile -, where the decode
+// kernel, whose workgroups go on from tile to tile, draws up to 3.5 on any width.  (Without this 5 x 11648 x 27328, 159 MB of codes, 213
+// units of 256 at work, was taken at 60.5 us where the decode kernel takes 45.8, 4 x 8448 x 26048 at 45.0, 35.1, and a gated
+// 15 x 10112 x 20992 at 59.0, 43.1.  Over 236 shapes with 20 MB and more of codes the choice is 1.8 % from the better kernel, without 3.6;
+// with the codes in the last-level cache, where the wave-K kernel stands better, 1.8 and 1.2.)
+static double stream_us(const ProblemB &p, int tile)
+{
+    const int cus = device_cu_count(), tm = tile / 10 * 16, tn = tile % 10 * 16;
+    const int64_t tiles = (int64_t)((p.M + tm - 1) / tm) * ((p.N + tn - 1) / tn), rounds = (tiles + cus - 1) / cus;
+    const double bytes = (double)p.K * p.N / p.vec * (p.code_bits / 8) + 2.0 * (double)p.M * (p.K + p.N);
+    const int brings = 64 / p.vec * (p.code_bits / 8);
+    return 2.0 + bytes / (brings <= 8 ? 2.0e6 : brings <= 16 ? 3.3e6 : 3.8e6) * (double)(rounds * cus) / (double)tiles;
+}
+
 // The rule: whichever is expected to be faster.  Up to 64 rows of X the other is the decode path, whose model is as close as this
 // one's (with these margins the choice is 1 to 3 % from the better one over 540 measured shapes); where that
 // path would take its streaming or its general kernel it keeps up to 16 rows.  Above, the tiled kernels, by more than the models' error.
@@ -201,10 +216,9 @@ bool wave_k_b_preferred(const ProblemB &p, double t_other, double margin)
         // (the streaming kernel, up to 16 rows: over 34 of its shapes on codes out of HBM the tile expected to be fastest takes 0.85 of
         // its time up to K = 24576 - 16 x 11008 x 4096 11.9 us -> 8.9 - and over 7 from there on 1.03, 13 x 27520 x 2944 17.5 -> 20.2)
         if (t_decode > 1e29) return p.M > 16 || (p.K <= 24576 && decode_stream_preferred(p));
-        // The gated decode kernels deal tiles in pairs, which their model does not see.  3 to 16 rows: over 425 shapes this line is 1.4 %
-        // from the better kernel on codes out of HBM and 0.9 % on codes in the caches (0.92: 1.3 and 1.2, 0.97: 1.8 and 0.8, 0.80: 3.6
-        // and 7.2); one and two rows of X, which the models know least (2 x 1024 x 576 3.0 us and 3.4), by more.
-        return wave_k_b_cost_us(p) < (p.gated ? 1.15 : p.M <= 2 ? 0.85 : p.M <= 16 ? 0.94 : 0.97) * t_decode;
+        // The gated decode kernels deal tiles in pairs, which their model does not see.  3 to 16 rows: over 425 shapes this line is 1.2 %
+        // from the better kernel on codes out of HBM and 1.0 % on codes in the caches (0.92: 1.0 and 1.4, 0.97: 1.5 and 1.0); one and two rows of X, which the models know least (2 x 1024 x 576 3.0 us and 3.4), by more.
+        return std::fmax(wave_k_b_cost_us(p), stream_us(p, wave_k_b_tile(p))) < (p.gated ? 1.15 : p.M <= 2 ? 0.85 : p.M <= 16 ? 0.94 : 0.97) * t_decode;
     }
     return wave_k_b_cost_us(p) < margin * t_other;
 }
