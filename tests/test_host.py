@@ -356,6 +356,22 @@ def test_many_codes_go_where_they_stream_faster():
         assert name(*dims) == want, dims
 
 
+def test_geometry_a_takes_the_one_kernel_that_was_weighed_against_two_passes():
+    """Beyond one round of tiles the fused kernels take two passes' place for the wave-K kernel's sake only: not where the tuning table
+    rules that kernel out, and everywhere when the table asks for it."""
+    before = cabi.tuning()
+    wins, loses = (3262, 7488, 1376), (4096, 4096, 2048)
+    pick = lambda: [cabi.select_variant_a(*dims, has_workspace=True) for dims in (wins, loses)]
+    try:
+        assert pick() == [cabi.VARIANT_PREFILL, cabi.VARIANT_TWOPASS]
+        cabi.set_tuning(wave_k_force=2)
+        assert pick() == [cabi.VARIANT_TWOPASS, cabi.VARIANT_TWOPASS]
+        cabi.set_tuning(wave_k_force=1)
+        assert pick() == [cabi.VARIANT_PREFILL, cabi.VARIANT_PREFILL]
+    finally:
+        cabi.set_tuning(wave_k_force=before["wave_k_force"])
+
+
 def test_the_report_of_the_automatic_choice_names_what_it_launches():
     """Host only; that the kernels named are the ones launched is held bit for bit on the GPU."""
     name = cabi.auto_variant_name_b

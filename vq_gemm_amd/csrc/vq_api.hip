@@ -213,7 +213,8 @@ bool fused_a_preferred(const ProblemA &p, bool has_workspace)
     // ... unless the wave-K kernel, which multiplies more than it gathers, is expected to be ahead of it: M = 3262, K = 7488, Nc = 1376
     // 198.7 -> 155.7 us.  (The first pass: 2 us and 1 us a million codes; 5 % off with the second, over 18 such shapes, and the choice
     // 0.3 % from the better one.)
-    return wave_k_a_supports(p) && wave_k_a_cost_us(p) < 2.0 + 1.0e-6 * p.K * p.Nc + gemm_tiled_cost_us(p.M, p.K, 2 * p.Nc);
+    return wave_k_a_preferred(p) &&
+           ((int)tuning().wave_k_force == 1 || wave_k_a_cost_us(p) < 2.0 + 1.0e-6 * p.K * p.Nc + gemm_tiled_cost_us(p.M, p.K, 2 * p.Nc));
 }
 
 int check_b(int64_t M, int64_t K, int64_t N, int32_t vec, int32_t entries, int32_t n_codebooks, int32_t code_bits)
