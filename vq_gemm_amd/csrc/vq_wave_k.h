@@ -1,5 +1,5 @@
 // Products whose tiles of the large kernels are fewer than the compute units: a workgroup takes a small tile of Y
-// (16 to 128 rows by 32 to 128 columns) and its waves, eight in nearly all tiles, deal K out among themselves.
+// (16 to 96 rows by 16 to 128 columns) and its waves, eight in nearly all tiles, deal K out among themselves.
 //
 //   NN:        y[M,N] = x[M,K] . w[K,N], fp16 w
 //   geometry A: out[M, 2*Nc] = x[M,K] . W_dec, W_dec[k, 2n + r] = codebook[n/4][w[k,n]][r] (reference
@@ -10,8 +10,8 @@
 // LDS only it reads, so nothing in the loop waits for another wave - no barrier, only the wave's own loads - and an operand
 // of a wave serves the whole height (width) of the tile, where waves that share out a tile of this size would read every
 // operand once per wave.  Units in flight: 100 to 150 KB per compute unit, what it takes to keep the memory busy from few
-// workgroups.  At the end the eight partial tiles are added up through the LDS, in the order of the waves, in fp32, and
-// rounded once.
+// workgroups.  At the end the waves' partial tiles are added up through the LDS, in the order of the waves, in fp32, and
+// rounded once.  Geometry A's tiles of 64 x 64 and more are vq_wave_k_a.hip's.
 //
 // What bounds it: with few tiles the launch, the latency of the first units and the sum over the waves (together about
 // 4 us); with many the LDS, which carries each unit in and out once.
@@ -64,11 +64,11 @@ struct WaveB {           // geometry B
     static constexpr int VEC = VEC_, CSZ = (int)sizeof(CodeT_);
 };
 
-// Waves of a workgroup: two on every SIMD, one's MFMAs beside the other's reads, where their accumulators leave room for two; four for
+// Waves of a workgroup: two on every SIMD, one's MFMAs beside the other's reads; four on every SIMD for
 // the smallest tile on a table of copies, whose waves wait for one another's reads least (M = 16, K = 11008, N = 4096 9.2 -> 8.5 us; twice
 // as wide a tile gains nothing from it, 9.7, and loses at K = 4096, 6.0 -> 6.7).
 template <class P>
-constexpr int wave_count(int mp, int np) { return mp * np > 32 ? 4 : P::kB && P::kCopies && mp * np == 1 ? 16 : 8; }
+constexpr int wave_count(int mp, int np) { return P::kB && P::kCopies && mp * np == 1 ? 16 : 8; }
 
 // Rows of pieces whose partial sums, `per_row` KB of them each, fit the LDS together: the most that divide the tile's.
 constexpr int pass_rows(int mp, int per_row)
@@ -135,7 +135,8 @@ __device__ __forceinline__ int wave_x_offset(int row, int cc)
 template <int NP>
 __device__ __forceinline__ int wave_w_swizzle(int k)
 {
-    return NP == 8 ? 2 * (k & 3) + ((k >> 3) & 1) * 8 : NP == 4 ? ((k >> 1) & 1) * 2 + ((k >> 3) & 1) * 4 : ((k >> 3) & 1) * 2;
+    static_assert(NP == 2 || NP == 4, "32 or 64 columns");
+    return NP == 4 ? ((k >> 1) & 1) * 2 + ((k >> 3) & 1) * 4 : ((k >> 3) & 1) * 2;
 }
 
 struct WaveKArgs {
@@ -370,23 +371,11 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
     for (int j = 0; j < NP; j++)
 #pragma unroll
         for (int i = 0; i < MP; i++) acc[j][i] = float4_t{0.f, 0.f, 0.f, 0.f};
-    // The accumulators of the largest tiles are pinned to the AGPRs (mfma_in_place): the compiler does not see those MFMAs, so
-    // what it computed into their operands is kept two wait states ahead of them.
-    constexpr bool kPinned = MP * NP > 32;
     auto multiply = [&](int set) {
-        if constexpr (kPinned) {
-            __builtin_amdgcn_sched_barrier(0);
-            asm volatile("s_nop 1" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-        }
 #pragma unroll
         for (int j = 0; j < NP; j++)
 #pragma unroll
-            for (int i = 0; i < MP; i++) {
-                if constexpr (kPinned) mfma_in_place(acc[j][i], ws[set][j], xs[set][i]);
-                else acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ws[set][j], xs[set][i], acc[j][i], 0, 0, 0);
-            }
-        if constexpr (kPinned) __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < MP; i++) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ws[set][j], xs[set][i], acc[j][i], 0, 0, 0);
     };
 
     // ---- codebooks, first units -------------------------------------------------------------------
@@ -500,10 +489,6 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
     // ---- the sum over the waves ---------------------------------------------------------------------
     // A piece is 1 KB, float4 by lane; a wave takes pairs of pieces of a row of pieces.
     constexpr int PM = C::kPassMP, H = NP % 2 == 0 ? 2 : 1, kPairs = PM * NP / H;
-    if constexpr (kPinned) {
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMAs have left the pipe
-        hold_accumulators(acc);
-    }
 #pragma unroll
     for (int pass = 0; pass < MP / PM; pass++) {
         __syncthreads();

@@ -37,10 +37,10 @@ struct WaveACfg {
     static constexpr int kSumBytes = kWaves * kPassMP * NP * 1024;
     static constexpr int kUse = kCodeBase + kWaves * DC * kCodeBytes;
     static constexpr int kLdsBytes = kUse > kSumBytes ? kUse : kSumBytes;
-    static_assert(NP >= 4 && NP <= 8 && NP % 2 == 0 && MP * NP <= 64 && kLdsBytes <= 160 * 1024, "pairs of pieces, accumulators in the AGPRs");
+    static_assert((NP == 4 || NP == 6) && MP * NP <= 64 && kLdsBytes <= 160 * 1024, "pairs of pieces, accumulators in the AGPRs");
     // the table: the words of pair q in a row, from word first(q) on, two copies of each of the pair's four codebooks for every
     // lane of a quarter wave that gathers from it, or one
-    static constexpr int words(int q) { return NP == 4 || (NP == 6 && q == 0) ? 32 : 16; }
+    static constexpr int words(int q) { return NP == 4 || q == 0 ? 32 : 16; }
     static constexpr int first(int q) { return q == 0 ? 0 : first(q - 1) + words(q - 1); }
 };
 
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(256, 1) void wave_k_a_kernel(const half_t *__restri
     // (a wave writes four rows at a time, lane by lane sixteen bytes: four words of one codebook)
     uint32_t words[16];
     {
-        const int chunk = r16, q = NP == 4 ? chunk >> 3 : NP == 8 ? chunk >> 2 : chunk < 8 ? 0 : (chunk >> 2) - 1;
+        const int chunk = r16, q = NP == 4 ? chunk >> 3 : chunk < 8 ? 0 : (chunk >> 2) - 1;
         const int book = min(n0 / 8 + q * 4 + (chunk & 3), N / 8 - 1);   // (columns past the last: that one's codebook again)
         const uint32_t *src = reinterpret_cast<const uint32_t *>(cb) + (int64_t)book * 256 + wave * 64 + kg;
 #pragma unroll
