@@ -214,12 +214,20 @@ template <class C> constexpr bool holds_every_table()
 template <class F, int MP, int NP> constexpr bool holds()
 {
     typedef WaveKCfg<typename F::template Wave<MP, NP>, MP, NP> C;
-    if constexpr (C::kExists) return holds_every_table<C>();
-    else return true;
+    bool ok = true;
+    if constexpr (C::kExists) ok = holds_every_table<C>();
+    if constexpr (F::template kHasCopies<MP, NP>) {   // (one size of table: a row of the 64 banks for each of 256 entries)
+        typedef WaveKCfg<typename F::template Copies<MP, NP>, MP, NP> D;
+        static_assert(D::kExists);
+        ok = ok && D::lds_bytes(16) >= D::kRing + 256 * 256 && D::lds_bytes(4096) <= 160 * 1024;
+    }
+    return ok;
 }
 template <class F> constexpr bool every_tile()
 {
-    return holds<F, 1, 2>() && holds<F, 1, 4>() && holds<F, 1, 8>() && holds<F, 2, 2>() && holds<F, 2, 4>() && holds<F, 4, 4>() && holds<F, 4, 8>();
+    bool ok = holds<F, 1, 1>() && holds<F, 1, 2>() && holds<F, 1, 3>() && holds<F, 1, 4>() && holds<F, 1, 8>() && holds<F, 2, 1>() && holds<F, 2, 2>() && holds<F, 2, 3>();
+    ok = ok && holds<F, 2, 4>() && holds<F, 2, 8>() && holds<F, 3, 4>() && holds<F, 4, 4>() && holds<F, 4, 8>() && holds<F, 5, 4>() && holds<F, 6, 4>();
+    return ok;
 }
 static_assert(every_tile<Format<8, uint8_t>>() && every_tile<Format<8, uint16_t>>(), "8-vectors");
 static_assert(every_tile<Format<4, uint8_t>>() && every_tile<Format<4, uint16_t>>(), "4-vectors");
