@@ -1040,10 +1040,13 @@ def test_geometry_a(M, K, Nc):
         idx = torch.randint(0, K, (M,), generator=torch.Generator().manual_seed(9)).to(DEV)
         xo = torch.zeros(M, K, dtype=torch.float16, device=DEV)
         xo[torch.arange(M, device=DEV), idx] = 1
-        _say("geometry A fused one-hot", M, K, Nc)
-        y = cabi.e2e_gemm_a(xo, w, cb, variant=cabi.VARIANT_PREFILL)
-        torch.cuda.synchronize()
-        assert torch.equal(y, dec[idx])
+        for kernel in ("fused", "wave_k"):
+            _say("geometry A fused one-hot", M, K, Nc, kernel)
+            call = lambda a: _with_geometry_a_kernel(kernel, lambda: cabi.e2e_gemm_a(a, w, cb, variant=cabi.VARIANT_PREFILL))
+            y = call(xo)
+            torch.cuda.synchronize()
+            assert torch.equal(y, dec[idx]), kernel
+            _check_gemm(call(x), x, w, cb, geometry=GEOM_A, what=f"A/{kernel}")
 
 
 # ------------------------------------------------------------------ plain GEMM control and the hipBLASLt baseline
@@ -1466,28 +1469,40 @@ def test_modules_serve_reference_native_shapes_on_every_route(M, K, Nc, route):
     assert torch.equal(ops.load_module("s2_128").e2e_gemm(x, w, cb), cabi.e2e_gemm_a(x, w, cb, workspace=ws))
 
 
+def _with_geometry_a_kernel(kernel, call):
+    """`call` with geometry A's fused product by the one kernel or the other, whichever the cost models would take."""
+    before = cabi.tuning()["wave_k_force"]
+    try:
+        cabi.set_tuning(wave_k_force={"wave_k": 1, "fused": 2}[kernel])
+        return call()
+    finally:
+        cabi.set_tuning(wave_k_force=before)
+
+
+@pytest.mark.parametrize("kernel", ["fused", "wave_k"])
 @pytest.mark.parametrize("M,K,Nc", [(2048, 4096, 640), (512, 4096, 640), (2048, 2048, 2048)])
-def test_fused_reference_layout_kernel_gives_the_same_bits_on_every_launch(M, K, Nc):
-    # The fused kernel waits for its hand-issued loads by count, and a count that does not match the order of the
+def test_fused_reference_layout_kernel_gives_the_same_bits_on_every_launch(M, K, Nc, kernel):
+    # Both kernels wait for its hand-issued loads by count, and a count that does not match the order of the
     # loads shows as a rare wrong element on a fast launch, not as a steady error.  The reference's own shape
-    # (128x128 tiles, 160 of them), a shorter X on it and a shape of 256x128 tiles: 50 launches each on fixed
+    # (128x128 tiles of the fused kernel, 160 of them), a shorter X on it and a shape of its 256x128 tiles: 50 launches each on fixed
     # operands, every result equal to the first bit for bit, the first within the bar of the oracle on sampled rows.
     spec = ProblemSpec("A", GEOM_A, M, K, 2 * Nc, 2, 256, Nc // 4, 8, codebook_std=1.0)
     x, w, cb = make_problem(spec, seed=71, device=DEV)
-    _say("fused geometry A, 50 launches", M, K, Nc)
-    first = cabi.e2e_gemm_a(x, w, cb, variant=cabi.VARIANT_PREFILL).clone()
+    _say("fused geometry A, 50 launches", M, K, Nc, kernel)
+    launch = lambda: _with_geometry_a_kernel(kernel, lambda: cabi.e2e_gemm_a(x, w, cb, variant=cabi.VARIANT_PREFILL))
+    first = launch().clone()
     torch.cuda.synchronize()
     rows = np.unique(np.concatenate([np.arange(0, M, max(1, M // 32)), [M - 1]]))
     e1, e2 = vo.rel_err(_np(first)[rows], vo.vq_gemm_a(_np(x)[rows], _np(w), _np(cb), acc=np.float64))
     _say(f"  rel_err(floor)={e1:.3e} max/max={e2:.3e}")
     assert e1 <= TOL, (e1, e2)
     # back to back (the next launch's prologue runs beside the previous one's tail), then one at a time
-    outs = [cabi.e2e_gemm_a(x, w, cb, variant=cabi.VARIANT_PREFILL) for _ in range(25)]
+    outs = [launch() for _ in range(25)]
     torch.cuda.synchronize()
     for i, y in enumerate(outs):
         assert torch.equal(y, first), f"launch {i} differs"
     for i in range(25):
-        y = cabi.e2e_gemm_a(x, w, cb, variant=cabi.VARIANT_PREFILL)
+        y = launch()
         torch.cuda.synchronize()
         assert torch.equal(y, first), f"synchronised launch {i} differs"
 
