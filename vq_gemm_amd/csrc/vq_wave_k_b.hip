@@ -190,8 +190,9 @@ int wave_k_b_tile(const ProblemB &p)
 // their way - 2.0, 3.3 or 3.8 TB/s when every compute unit works, its share of that when some have no tile -, where the decode
 // kernel, whose workgroups go on from tile to tile, draws up to 3.5 on any width.  (Without this 5 x 11648 x 27328, 159 MB of codes, 213
 // units of 256 at work, was taken at 60.5 us where the decode kernel takes 45.8, 4 x 8448 x 26048 at 45.0, 35.1, and a gated
-// 15 x 10112 x 20992 at 59.0, 43.1.  Over 236 shapes with 20 MB and more of codes the choice is 1.8 % from the better kernel, without 3.6;
-// with the codes in the last-level cache, where the wave-K kernel stands better, 1.8 and 1.2.)
+// 15 x 10112 x 20992 at 59.0, 43.1.  Over 236 shapes with 20 MB and more of codes the choice is 1.9 % from the better kernel, without 3.6;
+// with the codes in the last-level cache, where the wave-K kernel stands better, 1.3 and 1.2.  There it would lose by more if this had to
+// beat the decode kernel by the margin below too: 1.7 and 1.6.)
 static double stream_us(const ProblemB &p, int tile)
 {
     const int cus = device_cu_count(), tm = tile / 10 * 16, tn = tile % 10 * 16;
@@ -218,7 +219,8 @@ bool wave_k_b_preferred(const ProblemB &p, double t_other, double margin)
         if (t_decode > 1e29) return p.M > 16 || (p.K <= 24576 && decode_stream_preferred(p));
         // The gated decode kernels deal tiles in pairs, which their model does not see.  3 to 16 rows: over 425 shapes this line is 1.2 %
         // from the better kernel on codes out of HBM and 1.0 % on codes in the caches (0.92: 1.0 and 1.4, 0.97: 1.5 and 1.0); one and two rows of X, which the models know least (2 x 1024 x 576 3.0 us and 3.4), by more.
-        return std::fmax(wave_k_b_cost_us(p), stream_us(p, wave_k_b_tile(p))) < (p.gated ? 1.15 : p.M <= 2 ? 0.85 : p.M <= 16 ? 0.94 : 0.97) * t_decode;
+        return wave_k_b_cost_us(p) < (p.gated ? 1.15 : p.M <= 2 ? 0.85 : p.M <= 16 ? 0.94 : 0.97) * t_decode &&
+               stream_us(p, wave_k_b_tile(p)) < (p.gated ? 1.15 : 1.0) * t_decode;
     }
     return wave_k_b_cost_us(p) < margin * t_other;
 }
