@@ -48,14 +48,14 @@ PROFILED_C2_TRAFFIC_SOURCE = "profiles/decode_gemv_wide_kernel_c2_decode_gemv.md
 # The same for the other configurations (name in `other_configs` -> bytes per launch, summary file): what the
 # per-configuration `roofline` objects carry as `traffic`.  None where no counter run exists.
 PROFILED_TRAFFIC = {
-    "C3": (24_371_000, "profiles/decode_batched_kernel_c3_m16_mlp_up.md"),
+    "C3": (24_283_000, "profiles/wave_k_kernel_c3_and_m16_k14336_n4096.md"),
     "decode_m1_k4096_n28672": (14_921_700, "profiles/decode_gemv_wide_kernel_m1_n28672.md"),
     "decode_m1_k8192_n28672": (29_657_000, "profiles/decode_gemv_wide_kernel_m1_n28672.md"),
     "decode_qkv_m1_k4096_n12288": (6_578_000, "profiles/decode_gemv_wide_kernel_m1_n28672.md"),
     "decode_m2_k4096_n28672": (15_187_968, "profiles/decode_gemv_wide_kernel_m2_two_rows_of_x.md"),
     "decode_down_m1_k14336_n4096": (7_692_288, "profiles/decode_gemv_wide_kernel_long_k_down_projection.md"),
     "decode_down_m1_k28672_n8192": (29_952_000, "profiles/decode_gemv_wide_kernel_long_k_down_projection.md"),
-    "decode_down_m16_k14336_n4096": (11_270_000, "profiles/decode_stream_kernel_m16_k14336_n4096.md"),
+    "decode_down_m16_k14336_n4096": (11_225_000, "profiles/wave_k_kernel_c3_and_m16_k14336_n4096.md"),
     "C4": (85_373_000, "profiles/prefill_kernel_c4_prefill_gemm.md"),
     "C5": (489_400_000, "profiles/prefill_kernel_c5_m2048_k8192_n28672.md"),
 }
@@ -486,7 +486,7 @@ def main():
         others["decode_down_m1_k28672_n8192"], _ = bench_config(
             ProblemSpec("decode_down_m1_k28672_n8192", GEOM_B, 1, 28672, 8192, 8, 256, 1, 8),
             max(200, args.steps // 5), max(20, args.warmup // 5), cold_pool=True)
-        # the same down-projection at a batch of sixteen: the streaming kernel of the K-sliced path
+        # the same down-projection at a batch of sixteen: K dealt out to the waves of 256 workgroups
         others["decode_down_m16_k14336_n4096"], _ = bench_config(
             ProblemSpec("decode_down_m16_k14336_n4096", GEOM_B, 16, 14336, 4096, 8, 256, 1, 8),
             max(200, args.steps // 5), max(20, args.warmup // 5), cold_pool=True)
