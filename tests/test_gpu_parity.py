@@ -2382,6 +2382,45 @@ def test_encoder_on_both_sides_of_the_line_between_its_wave_sizes(N, K, v):
     assert np.array_equal(_np(codes), c_oracle.encode_b(w.numpy(), cb.numpy(), 8))
 
 
+@pytest.mark.parametrize("scale", [2e-7, 2e-5, 0.02, 40.0, 2e4, 65504.0])   # subnormal halves to norms that take more than one part
+@pytest.mark.parametrize("N,K,v,E", [(96, 128, 4, 33), (96, 256, 4, 767), (64, 256, 4, 768), (40, 128, 4, 4096), (64, 256, 8, 513)])
+def test_encoder_at_the_ends_of_the_range_of_halves(N, K, v, E, scale):
+    """The half norms of 4-vectors as sums of halves: groups of eight and of sixteen, tiles left empty, entries of very different sizes."""
+    g = torch.Generator(device="cpu").manual_seed(23)
+    cb, w = torch.randn(1, E, v, generator=g), torch.randn(N, K, generator=g)
+    cb[:, ::7] *= 2.0 ** -12
+    w.view(N, K // v, v)[:, ::5] *= 2.0 ** -13
+    cb, w = ((t * scale).clamp(-65504, 65504).half() for t in (cb, w))
+    w.view(N, K // v, v)[:, ::3] = cb[0, torch.randint(0, E, (N, (K // v + 2) // 3), generator=g)]
+    bits = 8 if E <= 256 else 16
+    _say("encode", N, K, v, E, scale)
+    codes = cabi.encode_b(w.to(DEV), cb.to(DEV), bits)
+    torch.cuda.synchronize()
+    assert np.array_equal(_np(codes), c_oracle.encode_b(w.numpy(), cb.numpy(), bits))
+
+
+@pytest.mark.parametrize("scale", [2e-6, 0.02, 2e4])
+def test_lloyd_assignments_of_eight_vectors_with_the_norms_as_parts_of_k(scale):
+    """The first assignment of one iteration, whose kernel is another than the encoder's: the sums make the same codebook as the encoder's codes."""
+    from vq_gemm_amd.torch_ops import native
+    N, K, v, E = 1032, 1032, 8, 100
+    g = torch.Generator(device="cpu").manual_seed(24)
+    w = (torch.randn(N, K, generator=g) * scale).clamp(-65504, 65504).half().to(DEV)
+    pick = torch.randperm(N * K // v, generator=g)[:E].to(torch.int32).view(1, E)
+    _say("lloyd", N, K, v, E, scale)
+    _, cb, errors = native.kmeans(w, pick, v, E, 1, 8, 1)
+    vectors = w.view(-1, v)
+    first = vectors[pick.view(-1).long().to(DEV)].contiguous()
+    codes = cabi.encode_b(w, first).view(-1).long()
+    d = vectors.double() - first.double()[codes]
+    assert abs(float(errors[0]) - float((d * d).sum())) <= 1e-4 * float((d * d).sum())   # fp32 sums of a wave's, 131 K of them
+    sums = torch.zeros(E, v, dtype=torch.float64, device=DEV).index_add_(0, codes, vectors.double())
+    mean = sums / torch.bincount(codes, minlength=E)[:, None].clamp(min=1)
+    # a vector assigned to another entry moves a mean of a thousand vectors by a thousandth of them; the sums are fp32, the entries halves
+    step = torch.maximum(mean.abs() * 2.0 ** -11, torch.full_like(mean, 2.0 ** -25))
+    assert bool(((cb[0].double() - mean).abs() <= 1.01 * step + 1e-5 * scale).all())
+
+
 @pytest.mark.parametrize("M,K,N", [(257, 192, 263), (130, 448, 129), (40, 256, 300)])
 def test_rows_of_y_that_begin_anywhere(M, K, N):
     spec = ProblemSpec("odd_rows", GEOM_B, M, K, N, 8, 256, 1, 8, codebook_std=0.05)

@@ -92,14 +92,29 @@ __global__ __launch_bounds__(kEncThreads) void encode_b_kernel(const half_t *__r
 // ---- matrix-core scan -------------------------------------------------------------------------
 // What bounds it: the vector unit.  The rule costs 2 * vec + 2 vector instructions per vector and entry; a score costs
 // the matrix pipe 1/32 of a cycle (v_mfma_f32_32x32x8_f16: 32 entries by 32 vectors, vec <= 8 of its k in use) and the
-// vector unit one instruction: of a group of eight scores four to fold them to their minimum and four to keep the best
-// two groups (0.75 in groups of sixteen).  4096 x 4096, 8-vectors, 256 entries: 230 -> 32 us.
+// vector unit 13 instructions per 16: of each group of eight scores four to fold them to their minimum and one to put the group's number
+// into its low bits, then three that keep the best group and the second best of the two (11 per 16 in groups of sixteen).  All of them
+// take 4.2 cycles here; an MFMA adds 8 to the 54 of the fold of its results while other waves fold, of its own 32.  What a 4096 x
+// 4096 weight takes in 8-vectors with 256 entries: 29.5 us (with a comparison and a selection for the group's number, 16 instructions per
+// 16 scores, 36; by the rule 230), of which a tile of 32 entries is 1.9, the pass per vector behind the scan 9, table and launch 4.
 //
 // A wave takes 128 vectors as four batches of 32 (64 as two, where there are too few for a workgroup on every other unit), so that an entry tile read from the LDS (its halves and its
 // half norms) meets four MFMAs.  A lane of the result holds 16 scores of one vector - two groups of eight entries, or one -, and
 // the lane 32 further on the other 16.
+//
+// The half norms: as the MFMA's accumulators, 16 numbers a lane out of the LDS per tile, or (NORMS_IN_K) as products too, in the half of K
+// that a vector leaves unused (8-vectors: of the MFMA with 16 of K): as a sum of halves times powers of two, which are the same for
+// every vector.  What an LDS read writes into registers is not free to the vector unit: 16 cycles of a 4-vectors' tile and batch.
 // Scores per group: a larger one costs the scan less and the rule more; they meet at about this many entries.
 constexpr int kScanWideGroupEntries = 768;
+
+// The low bits of a score that hold a number: which of a run of groups it is the minimum of, which entry of a group it is of.
+constexpr uint32_t kRunMask = 15;
+constexpr float kHidden = 0x1.3p-16f, kHiddenManyParts = 0x1.9p-16f;  // derived in the kernel
+constexpr float kNumbered = 0x1p-18f;   // by which the number can move a score, and as much again for the rounding of what is made of it
+// Instead of the half norm of an entry that is never chosen, and the score that nothing has yet: far from any real one, and
+// finite with a number in its low bits.
+constexpr float kFar = 0x1p127f;
 
 // bytes of the scan's table: whole tiles of 32 entries, an entry left out after every 256 bytes, in whole 16-byte steps
 __host__ __device__ inline int scan_table_bytes(int entries, int vec)
@@ -130,6 +145,20 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c)
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, a), __builtin_bit_cast(half2_t, b), c, false);
 }
 
+__device__ __forceinline__ float min3(float a, float b, float c)
+{
+    // (as an instruction: the compiler would quiet operands that integer operations made)
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// `score` with a number in the low bits
+__device__ __forceinline__ float numbered(float score, uint32_t number)
+{
+    return __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, score) & ~kRunMask) | number);
+}
+
 // two halves with both zeros as one (-0 + 0 is 0)
 __device__ __forceinline__ uint32_t one_zero(uint32_t v) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) + half2_t{}); }
 
@@ -157,8 +186,8 @@ __device__ __forceinline__ HalfWaves swap_half_waves(uint32_t a, uint32_t b)
     return HalfWaves{r[0], r[1]};
 }
 
-// LDS: entries padded to whole tiles of 32: halves with flipped signs, then |c|^2 / 2 (infinity behind the last entry),
-// then with SUMS the sums of the vectors assigned to each entry and their number, [entry][VEC + 1], then n_buckets words.
+// LDS: entries padded to whole tiles of 32: halves with flipped signs, then with NORMS_IN_K the parts of |c|^2 / 2 likewise, then |c|^2 / 2
+// (kFar behind the last entry; not beside parts in groups of sixteen, which are scored again by the parts), then with SUMS the sums of the vectors assigned to each entry and their number, [entry][VEC + 1], then n_buckets words.
 //
 // SUMS (a Lloyd iteration): every vector is added to its entry's sums, its distance to the workgroup's error, and
 // both leave as the workgroup's row of `partials`: entries * (VEC + 1) sums and counts, then the error.  The sums are kept in
@@ -167,8 +196,8 @@ __device__ __forceinline__ HalfWaves swap_half_waves(uint32_t a, uint32_t b)
 // as a flag of the one kernel it cost every assignment half a microsecond).
 enum ScanKeeps { kCodesOnly, kErrorOnly, kSums };
 
-template <int VEC, typename CodeT, int GROUP, ScanKeeps KEEPS, int kScanBatches>
-__global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t *__restrict__ w, const half_t *__restrict__ cb,
+template <int VEC, typename CodeT, int GROUP, ScanKeeps KEEPS, int kScanBatches, bool NORMS_IN_K>
+__global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half_t *__restrict__ w, const half_t *__restrict__ cb,
                                                                    CodeT *__restrict__ codes, int64_t vectors_per_cb, int entries,
                                                                    int wgs_per_cb, float *__restrict__ partials, int bucket_off,
                                                                    int n_buckets)
@@ -183,22 +212,42 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
     constexpr int kRow = 128 / VEC;
     auto at = [](int e) { return e + e / kRow; };
     constexpr int kGroups = 16 / GROUP, kQuads = GROUP / 4;  // groups of a lane's scores; runs of four entries in a group
+    constexpr int kRunTiles = (kRunMask + 1) / kGroups;      // tiles of a run of groups
+    constexpr bool kWideK = NORMS_IN_K && VEC == 8;          // sixteen of K per MFMA: the vector and the norm's parts
+    constexpr bool kNormTable = !NORMS_IN_K || GROUP == 8;   // the half norms lie in the LDS as floats
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, h = lane >> 5;         // vector of a batch, and which half of K (and of the rows) the lane holds
     const int n_tiles = (entries + 31) / 32;
     uint32_t *table = reinterpret_cast<uint32_t *>(smem);                         // [n_tiles * 32][DW]
-    float *norms = reinterpret_cast<float *>(smem + scan_table_bytes(entries, VEC));
-    double *sums = reinterpret_cast<double *>(norms + n_tiles * 32);
+    uint32_t *parts = table + scan_table_bytes(entries, VEC) / 4;                 // with NORMS_IN_K, as the table
+    float *norms = reinterpret_cast<float *>(parts + (NORMS_IN_K ? scan_table_bytes(entries, VEC) / 4 : 0));
+    double *sums = reinterpret_cast<double *>(norms + (kNormTable ? n_tiles * 32 : 0));
     uint32_t *bucket = reinterpret_cast<uint32_t *>(smem + bucket_off);
     const int g = blockIdx.x / wgs_per_cb, part = blockIdx.x % wgs_per_cb;
     const half_t *wg_w = w + (int64_t)g * vectors_per_cb * VEC;
     CodeT *wg_codes = codes + (int64_t)g * vectors_per_cb;
 
+    const int64_t step = (int64_t)wgs_per_cb * (kScanThreads / 64) * kScanVectors;
+    // a vector per lane, two batches of them at a time
+    typedef uint32_t dwords_of_vector_t __attribute__((ext_vector_type(DW)));
+    typedef dwords_of_vector_t vector_t __attribute__((aligned(DW < 2 ? 4 : 8)));
+    auto load_vectors = [&](int64_t base, vector_t (&v)[kScanBatches / 2]) {
+        const vector_t *from = reinterpret_cast<const vector_t *>(wg_w + base * VEC);
+        const uint32_t last = (uint32_t)min(vectors_per_cb - 1 - base, (int64_t)kScanVectors);
+#pragma unroll
+        for (int u = 0; u < kScanBatches / 2; u++) v[u] = from[min((uint32_t)(u * 64 + lane), last)];
+    };
+    vector_t coming[kScanBatches / 2];
+    int64_t base = ((int64_t)part * (kScanThreads / 64) + wave) * kScanVectors;
+    if (base < vectors_per_cb) load_vectors(base, coming);
+
     // table, half norms, whether all of them are finite (else every vector of the codebook is decided by the rule)
     bool book_finite;
+    float slack = 0.f, hides = kHidden;   // by which the parts of a half norm can miss it; what rounding can hide, as a share
+    half8_t scales{};                  // what the parts are multiplied by
     {
         // An entry that equals an earlier one is never chosen, but beside it no vector would be clear below, and a vector by the rule
-        // takes as long as twenty others: it gets an infinite norm.  The entries' hashes deal them out to buckets, and an entry looks
+        // takes as long as twenty others: its norm becomes kFar.  The entries' hashes deal them out to buckets, and an entry looks
         // at the first one in its bucket.  (What meets another entry there, and so stays, costs time, not the result.)  A codebook
         // half of whose entries equal the other half, 4096 x 4096 8-vectors: 749 -> 125 us, two equal ones and half of the weights
         // that value 435 -> 40; none equal 41.3 and 41.2.
@@ -234,7 +283,7 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
                 n2 = __builtin_fmaf((float)f[1], (float)f[1], n2);
                 table[at(e) * DW + i] = c[i] = own[i];
             }
-            norms[e] = e < entries ? 0.5f * n2 : __builtin_inff();
+            if constexpr (kNormTable) norms[e] = e < entries ? 0.5f * n2 : kFar;
             largest = n2 < __builtin_inff() ? fmaxf(largest, n2) : __builtin_inff();
             if (n_buckets && e < entries) atomicMin(&bucket[bucket_of(c)], (uint32_t)e);
         }
@@ -247,6 +296,57 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
 #pragma unroll
         for (int i = 0; i < kScanThreads / 64; i++) largest = fmaxf(largest, reduce[i]);
         book_finite = largest < __builtin_inff();
+        if constexpr (NORMS_IN_K) {
+            // |c|^2 / 2 as a sum of halves times powers of two: kTop parts at the scale that the largest needs (all but the first only for
+            // codebooks of norms beyond 2^31), then two for what halves leave out, 11 bits further down each.
+            constexpr int kParts = VEC == 8 ? 8 : 4, kTop = kParts - 2;
+            const int shift = min(max((int)(__builtin_bit_cast(uint32_t, largest) >> 23) - 127 - 15, -2), 15);
+            const float scale = __builtin_bit_cast(float, (uint32_t)(shift + 127) << 23), unscale = __builtin_bit_cast(float, (uint32_t)(127 - shift) << 23);
+            book_finite = book_finite && 0.5f * largest <= kTop * 65504.f * scale;
+            slack = 0x1p-44f * scale;
+            if (VEC == 8 && 0.5f * largest > 65504.f * scale) hides = kHiddenManyParts;
+#pragma unroll
+            for (int i = 0; i < kParts; i++) scales[i] = (half_t)(i < kTop ? scale : i == kTop ? scale * 0x1p-11f : scale * 0x1p-22f);
+            for (int e = tid; e < n_tiles * 32; e += kScanThreads) {
+                uint32_t c[DW];
+                read_entry<DW>(table, at(e), c);
+                float left = 0.f;
+#pragma unroll
+                for (int i = 0; i < DW; i++) {
+                    const half2_t f = __builtin_bit_cast(half2_t, c[i]);
+                    left = __builtin_fmaf((float)f[0], (float)f[0], left);
+                    left = __builtin_fmaf((float)f[1], (float)f[1], left);
+                }
+                bool never = e >= entries;
+                if (n_buckets && !never) {
+                    const int first = (int)bucket[bucket_of(c)];
+                    uint32_t other[DW];
+                    read_entry<DW>(table, at(first), other);
+                    uint32_t differ = first < e ? 0u : 1u;
+#pragma unroll
+                    for (int i = 0; i < DW; i++) differ |= one_zero(c[i]) ^ one_zero(other[i]);
+                    never = !differ;
+                }
+                if constexpr (kNormTable)
+                    if (never) norms[e] = kFar;
+                left = never ? kFar : 0.5f * left;
+                half_t part[kParts];
+                bool full = true;
+#pragma unroll
+                for (int i = 0; i < kTop; i++) {
+                    const float q = full ? left * unscale : 0.f;
+                    full = q > 65504.f;
+                    part[i] = (half_t)fminf(q, 65504.f);
+                    left = __builtin_fmaf(-(float)part[i], scale, left);
+                }
+                part[kTop] = never ? (half_t)0.f : (half_t)(left * unscale * 0x1p11f);
+                left = __builtin_fmaf(-(float)part[kTop], scale * 0x1p-11f, left);
+                part[kTop + 1] = never ? (half_t)0.f : (half_t)(left * unscale * 0x1p22f);
+#pragma unroll
+                for (int i = 0; i < DW; i++) parts[at(e) * DW + i] = __builtin_bit_cast(uint32_t, half2_t{part[2 * i], part[2 * i + 1]});
+            }
+            __syncthreads();
+        } else
         if (n_buckets) {
             for (int e = tid; e < entries; e += kScanThreads) {
                 uint32_t c[DW], other[DW];
@@ -256,7 +356,7 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
                 uint32_t differ = first < e ? 0u : 1u;
 #pragma unroll
                 for (int i = 0; i < DW; i++) differ |= one_zero(c[i]) ^ one_zero(other[i]);
-                if (!differ) norms[e] = __builtin_inff();
+                if (!differ) norms[e] = kFar;
             }
             __syncthreads();
         }
@@ -267,80 +367,145 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
     float above = __builtin_inff(), below = -__builtin_inff();
     asm volatile("" : "+v"(above), "+v"(below));
     float error = 0.f;
-    const int64_t step = (int64_t)wgs_per_cb * (kScanThreads / 64) * kScanVectors;
-    for (int64_t base = ((int64_t)part * (kScanThreads / 64) + wave) * kScanVectors; base < vectors_per_cb; base += step) {
-        // the vectors: lane (col, h) holds elements 4h .. 4h+3 of its vector in each batch (nothing where vec ends before)
-        half4_t b[kScanBatches];
-        float m1[kScanBatches], m2[kScanBatches];
-        int best[kScanBatches];
+    // a tile's entries as the matrix cores take them: the lower half wave the first half of K, the upper one the other
+    typedef std::conditional_t<kWideK, half8_t, half4_t> operand_t;
+    const uint32_t *a_from = (NORMS_IN_K && h ? parts : table) + at(col) * DW + (!NORMS_IN_K && VEC == 8 ? 2 * h : 0);
+    auto load_tile = [&](int t) {
+        if constexpr (VEC == 2) {
+            operand_t a = {};
+            const half2_t v = __builtin_bit_cast(half2_t, table[at(t * 32 + col)]);
+            if (h == 0) a = half4_t{v[0], v[1], (half_t)0.f, (half_t)0.f};
+            return a;
+        } else {
+            const operand_t a = *reinterpret_cast<const operand_t *>(a_from + t * (32 + 32 / kRow) * DW);
+            return NORMS_IN_K || VEC == 8 || h == 0 ? a : operand_t{};
+        }
+    };
+    auto load_norms = [&](int t, float16_t &c) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4_t v = *reinterpret_cast<const float4_t *>(norms + t * 32 + 8 * q + 4 * h);
+#pragma unroll
+            for (int i = 0; i < 4; i++) c[4 * q + i] = v[i];
+        }
+    };
+    auto multiply = [&](operand_t a, operand_t b, const float16_t &c) {
+        if constexpr (kWideK)
+            return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+        else
+            return __builtin_amdgcn_mfma_f32_32x32x8f16(a, b, c, 0, 0, 0);
+    };
+    const int quarter = (int)((vectors_per_cb + 4 * step - 1) / (4 * step));
+    for (int turn = 0; base < vectors_per_cb; base += step, turn++) {
+        // A SIMD issues for its oldest wave first, which would leave the youngest alone at the end, nobody covering its waits: a
+        // wave's priority falls by one with every quarter of its vectors (8-vectors 33.1 -> 30.5 us, 4-vectors 52 -> 47).
+        if (turn == 0)
+            __builtin_amdgcn_s_setprio(3);
+        else if (turn == quarter)
+            __builtin_amdgcn_s_setprio(2);
+        else if (turn == 2 * quarter)
+            __builtin_amdgcn_s_setprio(1);
+        else if (turn == 3 * quarter)
+            __builtin_amdgcn_s_setprio(0);
+        vector_t own[kScanBatches / 2];
+        operand_t b[kScanBatches];
+        float m1[kScanBatches], m2[kScanBatches];      // of this run of groups, with the group's number in the low bits
+        float all1[kScanBatches], all2[kScanBatches];  // of all runs
+        int best[kScanBatches];                        // the run that all1 is of
+#pragma unroll
+        for (int u = 0; u < kScanBatches; u += 2) {
+            own[u / 2] = coming[u / 2];
+            // One swap of half waves: .lo the lower lanes' dwords followed by what the upper half wave holds, .hi the upper lanes' likewise
+            if constexpr (NORMS_IN_K) {
+                typedef uint32_t dwords_t __attribute__((ext_vector_type(sizeof(operand_t) / 4)));
+                dwords_t lo, hi;
+#pragma unroll
+                for (int i = 0; i < DW; i++) {
+                    const HalfWaves r = swap_half_waves(own[u / 2][i], __builtin_bit_cast(uint32_t, half2_t{scales[2 * i], scales[2 * i + 1]}));
+                    lo[i] = r.lo;
+                    hi[i] = r.hi;
+                }
+                b[u] = __builtin_bit_cast(operand_t, lo);
+                b[u + 1] = __builtin_bit_cast(operand_t, hi);
+            } else {
+                // lanes (col, h): elements 4h .. 4h+3 of the vector (nothing where vec ends before)
+                uint2_t lo = {}, hi = {};
+#pragma unroll
+                for (int i = 0; i < (VEC == 2 ? 1 : 2); i++) {
+                    const HalfWaves r = swap_half_waves(own[u / 2][i], VEC == 8 ? own[u / 2][(i + 2) % DW] : 0u);
+                    lo[i] = r.lo;
+                    hi[i] = r.hi;
+                }
+                b[u] = __builtin_bit_cast(operand_t, lo);
+                b[u + 1] = __builtin_bit_cast(operand_t, hi);
+            }
+        }
 #pragma unroll
         for (int u = 0; u < kScanBatches; u++) {
-            const int64_t idx = min(base + u * 32 + col, vectors_per_cb - 1);
-            const half_t *src = wg_w + idx * VEC + (VEC == 8 ? 4 * h : 0);
-            b[u] = half4_t{};
-            if (VEC == 8 || h == 0) {
-                if constexpr (VEC == 2) {
-                    const half2_t v = *reinterpret_cast<const half2_t *>(src);
-                    b[u] = half4_t{v[0], v[1], (half_t)0.f, (half_t)0.f};
-                } else {
-                    b[u] = *reinterpret_cast<const half4_t *>(src);
-                }
-            }
-            m1[u] = m2[u] = __builtin_inff();
+            m1[u] = m2[u] = all1[u] = all2[u] = kFar;
             best[u] = 0;
         }
-        for (int t = 0; t < n_tiles; t++) {
-            half4_t a = {};
-            {
-                const uint32_t *src = table + at(t * 32 + col) * DW + (VEC == 8 ? 2 * h : 0);
-                if (VEC == 8 || h == 0) {
-                    if constexpr (VEC == 2) {
-                        const half2_t v = __builtin_bit_cast(half2_t, src[0]);
-                        a = half4_t{v[0], v[1], (half_t)0.f, (half_t)0.f};
+        load_vectors(base + step < vectors_per_cb ? base + step : base, coming);
+        operand_t ahead{};
+        if constexpr (NORMS_IN_K) ahead = load_tile(0);
+        for (int t0 = 0, run = 0; t0 < n_tiles; t0 += kRunTiles, run++) {
+            const int t1 = min(t0 + kRunTiles, n_tiles);
+            for (int t = t0; t < t1; t++) {
+                uint32_t number[2] = {(uint32_t)((t - t0) * kGroups), (uint32_t)((t - t0) * kGroups + 1)};
+                asm("" : "+s"(number[0]), "+s"(number[1]));
+                operand_t a;
+                float16_t c = {};
+                if constexpr (NORMS_IN_K) {
+                    a = ahead;
+                    ahead = load_tile(min(t + 1, n_tiles - 1));
+                } else {
+                    a = load_tile(t);
+                    load_norms(t, c);
+                }
+#pragma unroll
+                for (int u = 0; u < kScanBatches; u++) {
+                    const float16_t s = multiply(a, b[u], c);
+                    float x[kGroups];
+#pragma unroll
+                    for (int gr = 0; gr < kGroups; gr++) {
+                        float f = above;
+#pragma unroll
+                        for (int i = 0; i < GROUP; i++) f = fminf(f, s[gr * GROUP + i]);
+                        x[gr] = numbered(f, number[gr]);
+                    }
+                    if constexpr (kGroups == 2) {
+                        const float second = __builtin_amdgcn_fmed3f(m1[u], x[0], x[1]);
+                        m1[u] = min3(m1[u], x[0], x[1]);
+                        m2[u] = __builtin_amdgcn_fmed3f(m2[u], second, below);
                     } else {
-                        a = *reinterpret_cast<const half4_t *>(src);
+                        m2[u] = __builtin_amdgcn_fmed3f(m1[u], m2[u], x[0]);
+                        m1[u] = __builtin_amdgcn_fmed3f(m1[u], x[0], below);
                     }
                 }
             }
-            float16_t c;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float4_t v = *reinterpret_cast<const float4_t *>(norms + t * 32 + 8 * q + 4 * h);
-#pragma unroll
-                for (int i = 0; i < 4; i++) c[4 * q + i] = v[i];
-            }
+            if (t1 == n_tiles && run == 0) break;   // all there is
 #pragma unroll
             for (int u = 0; u < kScanBatches; u++) {
-                const float16_t s = __builtin_amdgcn_mfma_f32_32x32x8f16(a, b[u], c, 0, 0, 0);
+                best[u] = m1[u] < all1[u] ? run : best[u];
+                all2[u] = min3(all2[u], m2[u], __builtin_amdgcn_fmed3f(m1[u], all1[u], above));
+                all1[u] = __builtin_amdgcn_fmed3f(m1[u], all1[u], below);
+                m1[u] = m2[u] = kFar;
+            }
+        }
+        if (n_tiles > kRunTiles) {
 #pragma unroll
-                for (int gr = 0; gr < kGroups; gr++) {
-                    float x = above;
-#pragma unroll
-                    for (int i = 0; i < GROUP; i++) x = fminf(x, s[gr * GROUP + i]);
-                    best[u] = x < m1[u] ? kGroups * t + gr : best[u];
-                    m2[u] = __builtin_amdgcn_fmed3f(m1[u], m2[u], x);
-                    m1[u] = __builtin_amdgcn_fmed3f(m1[u], x, below);
-                }
+            for (int u = 0; u < kScanBatches; u++) {
+                m1[u] = all1[u];
+                m2[u] = all2[u];
             }
         }
         // Two batches at a time, a vector per lane: lane l takes vector l of the pair.  One swap of half waves brings a lane
-        // what its vector's two lanes hold: .lo of the rows (and elements) of half 0, .hi of half 1.
+        // what its vector's two lanes hold: .lo of the rows of half 0, .hi of half 1.
 #pragma unroll
         for (int u = 0; u < kScanBatches; u += 2) {
-            uint32_t full[DW];  // the vector, in element order
-            {
-                const uint2_t v0 = __builtin_bit_cast(uint2_t, b[u]), v1 = __builtin_bit_cast(uint2_t, b[u + 1]);
-                const HalfWaves p0 = swap_half_waves(v0[0], v1[0]);
-                full[0] = p0.lo;
-                if constexpr (VEC >= 4) {
-                    const HalfWaves p1 = swap_half_waves(v0[1], v1[1]);
-                    full[1] = p1.lo;
-                    if constexpr (VEC == 8) {
-                        full[2] = p0.hi;
-                        full[3] = p1.hi;
-                    }
-                }
-            }
+            uint32_t full[DW];  // the vector
+#pragma unroll
+            for (int i = 0; i < DW; i++) full[i] = own[u / 2][i];
             float w2 = 0.f;
 #pragma unroll
             for (int i = 0; i < DW; i++) w2 = dot2(full[i], full[i], w2);
@@ -349,59 +514,85 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
             const HalfWaves sb = swap_half_waves((uint32_t)best[u], (uint32_t)best[u + 1]);
             const float lo1 = __builtin_bit_cast(float, s1.lo), hi1 = __builtin_bit_cast(float, s1.hi);
             const bool lower = !(hi1 < lo1);  // the best group is among the rows of half 0
-            const int group = lower ? (int)sb.lo : (int)sb.hi;
-            const float next = fminf(fmaxf(lo1, hi1), fminf(__builtin_bit_cast(float, s2.lo), __builtin_bit_cast(float, s2.hi)));
-            // the scores of the group's entries once more, now one by one
-            const int e0 = (group / kGroups) * 32 + (group % kGroups) * 16 + (lower ? 0 : 4);
-            float first = above, second = above;
-            int e_best = 0;
+            const uint32_t group = (lower ? sb.lo : sb.hi) * (kRunMask + 1) + ((lower ? s1.lo : s1.hi) & kRunMask);
+            const float next = min3(__builtin_amdgcn_fmed3f(lo1, hi1, above), __builtin_bit_cast(float, s2.lo), __builtin_bit_cast(float, s2.hi));
+            // the scores of the group's entries once more, now one by one, with the entry's number in the group in the low bits
+            const uint32_t e0 = group * (32 / kGroups) + (lower ? 0u : 4u);
+            const uint32_t *entry = table + at(e0) * DW, *entry_parts = parts + at(e0) * DW;
+            float first = kFar, second = kFar;
 #pragma unroll
             for (int q = 0; q < kQuads; q++) {
-                const float4_t norm = *reinterpret_cast<const float4_t *>(norms + e0 + 8 * q);
+                constexpr int kPerQ = 8;
+                const int at_q = kPerQ * q + kPerQ * q / kRow;
+                float x[4];
+                if constexpr (kNormTable) {
+                    const float4_t norm = *reinterpret_cast<const float4_t *>(norms + e0 + kPerQ * q);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) x[i] = norm[i];
+                }
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    uint32_t c[DW];
-                    read_entry<DW>(table, at(e0 + 8 * q) + i, c);
-                    float x = norm[i];
+                    uint32_t e[DW];
+                    if constexpr (!kNormTable) {
+                        read_entry<DW>(entry_parts, at_q + i, e);
+                        x[i] = 0.f;
 #pragma unroll
-                    for (int k = 0; k < DW; k++) x = dot2(c[k], full[k], x);
-                    e_best = x < first ? e0 + 8 * q + i : e_best;
-                    second = __builtin_amdgcn_fmed3f(first, second, x);
-                    first = __builtin_amdgcn_fmed3f(first, x, below);
+                        for (int k = 0; k < DW; k++) x[i] = dot2(e[k], __builtin_bit_cast(uint32_t, half2_t{scales[2 * k], scales[2 * k + 1]}), x[i]);
+                    }
+                    read_entry<DW>(entry, at_q + i, e);
+#pragma unroll
+                    for (int k = 0; k < DW; k++) x[i] = dot2(e[k], full[k], x[i]);
+                    x[i] = numbered(x[i], 4 * q + i);
                 }
+                const float s01 = __builtin_amdgcn_fmed3f(first, x[0], x[1]);
+                first = min3(first, x[0], x[1]);
+                const float s23 = __builtin_amdgcn_fmed3f(first, x[2], x[3]);
+                first = min3(first, x[2], x[3]);
+                second = min3(second, s01, s23);
             }
-            // What rounding can hide.  With u = 2^-24: a score (nine exact terms, summed) is off by at most 24 u (|w||c| + |c|^2 / 2)
-            // <= 24 u (|w|^2 / 2 + |c|^2), the rule's distance by 10 u of itself.  Whatever entry the rule would choose is no
-            // further from w than the first one here, so that entry and the first both have |c| <= |w| + sqrt(D) with
+            const uint32_t in_group = __builtin_bit_cast(uint32_t, first) & kRunMask;
+            int e_best = (int)(e0 + in_group + (in_group & ~3u));
+            // What rounding can hide.  With u = 2^-24: a score is off by at most E u (|w||c| + |c|^2 / 2) <= E u (|w|^2 / 2 + |c|^2), the
+            // rule's distance by 10 u of itself.  (E = 28: 8 for the norm and 2 for each addition of up to eleven exact terms; 38 where
+            // the largest norm takes more than one part of the first scale, up to sixteen terms.)  Whatever entry the rule would choose
+            // is no further from w than the first one here, so that entry and the first both have |c| <= |w| + sqrt(D) with
             // D = |w|^2 + 2 first, |c|^2 <= 4 (|w|^2 + first).  Two scores and two halved distances: at most
-            // u (228 |w|^2 + 216 first) < 2^-16 (|w|^2 + first).  (Not clear either where anything is not finite.)
-            const float hidden = 1.52587890625e-5f * (w2 + first);
-            const bool clear = book_finite && fminf(next, second) - first > hidden;
+            // u ((9 E + 12) |w|^2 + (8 E + 24) first).  The number in the low bits of the first score moves it by 15 * 2^-23 of itself,
+            // at most 30 u (|w|^2 + first) (as first >= -|w|^2 / 2), so 294 u < kHidden (or 384 u < kHiddenManyParts) of |w|^2 + first; the
+            // number in those of the others moves them by 2^-19 of themselves.  (Not clear either where anything is not finite.)
+            const float other = __builtin_amdgcn_fmed3f(next, second, below);
+            const float hidden = __builtin_fmaf(hides, w2 + first, slack);
+            const bool clear = book_finite && __builtin_fmaf(-kNumbered, __builtin_fabsf(other), other) - first > hidden;
             // vectors that this does not decide: the rule on every entry, all lanes on one vector
+            // (Distances compare as their bits do: none is negative, and a NaN is above all.)
             for (uint64_t todo = __ballot(!clear); todo; todo &= todo - 1) {
                 const int v = __builtin_ctzll(todo);
                 uint32_t one[DW], c[DW];
 #pragma unroll
                 for (int i = 0; i < DW; i++) one[i] = __builtin_amdgcn_readlane(full[i], v);
-                read_entry<DW>(table, 0, c);
-                float d0 = rule_distance<DW>(one, c);  // entry 0 is taken as it is
-                int e_min = 0;
-                for (int e = lane; e < entries; e += 64) {
+                int e_min = min(lane, entries - 1);
+                read_entry<DW>(table, at(e_min), c);
+                uint32_t d_min = __builtin_bit_cast(uint32_t, rule_distance<DW>(one, c));
+                const bool entry_0_is_nan = (__builtin_amdgcn_readfirstlane(d_min) & 0x7fffffffu) > 0x7f800000u;  // and taken as it is
+                for (int e = lane + 64; e < entries; e += 64) {
                     read_entry<DW>(table, at(e), c);
-                    const float d = rule_distance<DW>(one, c);
-                    const bool take = d < d0;
-                    d0 = take ? d : d0;
-                    e_min = take ? e : e_min;
+                    const uint32_t d = __builtin_bit_cast(uint32_t, rule_distance<DW>(one, c));
+                    e_min = d < d_min ? e : e_min;
+                    d_min = min(d, d_min);
                 }
-#pragma unroll
-                for (int s = 32; s >= 1; s >>= 1) {
-                    const float od = __shfl_xor(d0, s);
-                    const int oe = __shfl_xor(e_min, s);
-                    const bool other = od < d0 || (od == d0 && oe < e_min);
-                    d0 = other ? od : d0;
-                    e_min = other ? oe : e_min;
-                }
-                e_best = lane == v ? e_min : e_best;
+                uint32_t least = d_min;
+#define VQ_LEAST(control) least = min(least, (uint32_t)__builtin_amdgcn_update_dpp((int)least, (int)least, control, 0xf, 0xf, false))
+                VQ_LEAST(0x128);  // rows of sixteen lanes, rotated by 8, 4, 2 and 1
+                VQ_LEAST(0x124);
+                VQ_LEAST(0x122);
+                VQ_LEAST(0x121);
+#undef VQ_LEAST
+                least = min(min((uint32_t)__builtin_amdgcn_readlane(least, 0), (uint32_t)__builtin_amdgcn_readlane(least, 16)),
+                            min((uint32_t)__builtin_amdgcn_readlane(least, 32), (uint32_t)__builtin_amdgcn_readlane(least, 48)));
+                int e_first = entries;
+                for (uint64_t at_least = __ballot(d_min == least); at_least; at_least &= at_least - 1)
+                    e_first = min(e_first, (int)__builtin_amdgcn_readlane(e_min, __builtin_ctzll(at_least)));
+                e_best = lane == v ? (entry_0_is_nan ? 0 : e_first) : e_best;
             }
             const int64_t idx = base + u * 32 + lane;
             if (idx < vectors_per_cb) {
@@ -441,25 +632,18 @@ __global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(const half_t 
     }
 }
 
-size_t scan_lds_bytes(const ProblemB &p, bool accumulate)
+size_t scan_lds_bytes(const ProblemB &p, bool accumulate, bool norms_in_k = false)
 {
-    const size_t padded = ((size_t)p.entries + 31) / 32 * 32;
-    return scan_table_bytes(p.entries, p.vec) + padded * 4 + (accumulate ? (size_t)p.entries * (p.vec + 1) * 8 : 0);
+    const size_t padded = ((size_t)p.entries + 31) / 32 * 32, table = scan_table_bytes(p.entries, p.vec);
+    const size_t norms = norms_in_k && p.entries >= kScanWideGroupEntries ? 0 : padded * 4;
+    return table + (norms_in_k ? table : 0) + norms + (accumulate ? (size_t)p.entries * (p.vec + 1) * 8 : 0);
 }
 
-constexpr size_t kScanLdsTwoPerUnit = 72 * 1024, kScanLds = 128 * 1024;
+// (two workgroups and their few static bytes in 160 KB)
+constexpr size_t kScanLdsTwoPerUnit = 79 * 1024, kScanLds = 128 * 1024;
 
-// Buckets for finding equal entries: four per entry where the LDS has room that neither keeps a second workgroup off the unit nor the
-// codebook off this kernel; none where not even one per two entries fits.
-int scan_buckets(const ProblemB &p, bool accumulate)
-{
-    const size_t bytes = scan_lds_bytes(p, accumulate), room = ((bytes <= kScanLdsTwoPerUnit ? kScanLdsTwoPerUnit : kScanLds) - bytes) / 4;
-    const size_t want = 4 * (size_t)p.entries;
-    return room >= want ? (int)want : 2 * room >= (size_t)p.entries ? (int)room : 0;
-}
-
-// Batches of a wave and workgroups per codebook: as many as are resident together (two of eight waves per unit while the LDS
-// allows), none without work.
+// Batches of a wave, workgroups per codebook: as many as are resident together (two of eight waves per unit while the LDS
+// allows), none without work.  The same for every assignment of a Lloyd iteration.
 struct ScanPlan {
     int batches, wgs_per_cb;
 };
@@ -471,6 +655,23 @@ ScanPlan scan_plan(const ProblemB &p, bool accumulate)
     auto have = [&](int batches) { return (vectors + kScanThreads / 2 * batches - 1) / (kScanThreads / 2 * batches); };
     const int batches = have(4) * p.n_codebooks * 2 <= device_cu_count() ? 2 : 4;
     return {batches, (int)(want < have(batches) ? want : have(batches))};
+}
+
+// Half norms as parts of K: of 4-vectors wherever two workgroups still share a unit (no MFMA more, and a quarter of the LDS reads: 4096 x
+// 4096 with 256 entries 57 -> 48 us, with 4096 entries 523 -> 447), of 8-vectors, whose MFMA is the longer one then, only beside the
+// LDS additions of a Lloyd iteration (35.5 -> 34.0; codes alone 29.5 -> 30.5) and not for waves of two batches, whose launches are
+// mostly prologue (512 x 512: 6.7 -> 6.9).
+bool scan_norms_in_k(const ProblemB &p, bool accumulate, bool sums, int batches)
+{
+    return (p.vec == 4 || (p.vec == 8 && sums && batches == 4)) && scan_lds_bytes(p, accumulate, true) <= kScanLdsTwoPerUnit;
+}
+
+// Buckets for finding equal entries: four per entry where the LDS has room that neither keeps a second workgroup off the unit nor the
+// codebook off this kernel; none where not even one per two entries fits.
+int scan_buckets(size_t bytes, int entries)
+{
+    const size_t room = ((bytes <= kScanLdsTwoPerUnit ? kScanLdsTwoPerUnit : kScanLds) - bytes) / 4, want = 4 * (size_t)entries;
+    return room >= want ? (int)want : 2 * room >= (size_t)entries ? (int)room : 0;
 }
 
 bool scan_supports(const half_t *w, const ProblemB &p, bool accumulate)
@@ -486,13 +687,23 @@ hipError_t launch_scan(const half_t *w, const ProblemB &p, void *codes_out, floa
     if (vectors_per_cb == 0) return hipSuccess;
     constexpr bool accumulate = KEEPS != kCodesOnly;   // (the last assignment in the same workgroups as the others)
     const ScanPlan plan = scan_plan(p, accumulate);
-    const size_t smem = scan_lds_bytes(p, accumulate);
-    const int buckets = scan_buckets(p, accumulate);
-    const bool narrow = p.entries < kScanWideGroupEntries;
-    auto kern = plan.batches == 4 ? (narrow ? encode_scan_kernel<VEC, CodeT, 8, KEEPS, 4> : encode_scan_kernel<VEC, CodeT, 16, KEEPS, 4>)
-                                  : (narrow ? encode_scan_kernel<VEC, CodeT, 8, KEEPS, 2> : encode_scan_kernel<VEC, CodeT, 16, KEEPS, 2>);
-    return launch_kernel(kern, dim3((unsigned)(plan.wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem + 4 * (size_t)buckets, s, w, p.cb,
-                       static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, plan.wgs_per_cb, partials, (int)smem, buckets);
+    const bool in_k = scan_norms_in_k(p, accumulate, KEEPS == kSums, plan.batches), narrow = p.entries < kScanWideGroupEntries;
+    const size_t smem = scan_lds_bytes(p, accumulate, in_k);
+    const int buckets = scan_buckets(smem, p.entries);
+    auto launch = [&](auto batches, auto norms_in_k) {
+        const auto kern = narrow ? encode_scan_kernel<VEC, CodeT, 8, KEEPS, batches(), norms_in_k()>
+                                 : encode_scan_kernel<VEC, CodeT, 16, KEEPS, batches(), norms_in_k()>;
+        return launch_kernel(kern, dim3((unsigned)(plan.wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem + 4 * (size_t)buckets, s, w, p.cb,
+                             static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, plan.wgs_per_cb, partials, (int)smem, buckets);
+    };
+    using std::integral_constant;
+    using four = integral_constant<int, 4>;
+    using two = integral_constant<int, 2>;
+    if constexpr (VEC == 4)
+        if (in_k) return plan.batches == 4 ? launch(four{}, std::true_type{}) : launch(two{}, std::true_type{});
+    if constexpr (VEC == 8 && KEEPS == kSums)
+        if (in_k) return launch(four{}, std::true_type{});
+    return plan.batches == 4 ? launch(four{}, std::false_type{}) : launch(two{}, std::false_type{});
 }
 
 template <int VEC, typename CodeT>
