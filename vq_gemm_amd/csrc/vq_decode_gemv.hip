@@ -6,7 +6,7 @@
 //   * A wave owns whole rows of W (four of them), so nothing is summed across waves: no partial
 //     sums in the LDS, no barrier behind the multiply.  A row's sum is folded inside the wave with
 //     DPP adds and four lane reads.
-//   * No matrix core: with one row of X fifteen of an MFMA's sixteen columns would be padding, and
+//   * No matrix core (the wide form further on has a use for it): with one row of X fifteen of an MFMA's sixteen columns would be padding, and
 //     feeding it means laying X out in operand order through the LDS first.  Here a lane keeps
 //     its share of x (the 8-vectors its codes meet) in registers, loaded straight from global
 //     memory while the codes are on their way, and multiplies with v_dot2_f32_f16: four per code.
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void decode_gemv_kernel(const half
 //     pending store would make it drain every load).  The loads are unconditional (past the end the
 //     last group is requested again) and only the multiply is skipped, for the same reason: a load
 //     inside a branch would make the counts at the join imprecise.
-//   * A row's sum is folded with six DPP additions (the last two broadcast row totals onward, so that
+//   * A row's sum is folded with six or seven DPP additions (the last two broadcast row totals onward, so that
 //     lane 63 holds the sum in a fixed order) and one lane read.
 constexpr int kWideWaves = 16;
 constexpr int kWideCopies = 16;
@@ -259,6 +259,25 @@ __device__ __forceinline__ float wave_sum_to_uniform(float v)
     v = dpp_add_row_bcast15(v);
     v = dpp_add_row_bcast31(v);
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+}
+
+template <int CONTROL>
+__device__ __forceinline__ float dpp_add(float moved, float v)
+{
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, moved), CONTROL, 0xf, 0xf, true));
+}
+
+// Sum over the 64 lanes of lane l's v[l % 4], valid in lane 63 (returned from there as a wave-uniform value).
+__device__ __forceinline__ float diagonal_sum_to_uniform(float4_t v)
+{
+    float s = dpp_add<0x00>(v[0], v[3]);   // the last lane of every four: its v[3], the first lane's v[0], ...
+    s = dpp_add<0x55>(v[1], s);
+    s = dpp_add<0xaa>(v[2], s);
+    s = dpp_add<0x114>(s, s);              // the last lane of a row of sixteen: the row (shifts by 4 and 8)
+    s = dpp_add<0x118>(s, s);
+    s = dpp_add_row_bcast15(s);
+    s = dpp_add_row_bcast31(s);
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 63));
 }
 
 // Where the piece of x that code c of lane l's dword meets lies in its run: the pieces of a code together, so that the lanes of a
@@ -298,6 +317,11 @@ __device__ __forceinline__ int small_quotient(int x, int d, float rcp)
 // K-sliced matrix-core kernel -> this: N = 11008 7.2 -> 5.3 us, N = 28672 10.5 -> 8.7).  K beyond 4096 is the long
 // form in pieces of two runs, both rows of x in the LDS (K = 14336, N = 4096: 10.9 -> 8.5 us).
 //
+// GATED: the epilogue of a gate/up pair, once for all of a wave's outputs behind its rows (an output at a time, and asked for at run
+// time in the kernel of every launch, K = 4096: N = 22016 5.9 -> 5.6 us gated; launches without it 0 to 3 % longer).
+//
+// ALL (the long form): all of a wave's NBUF pairs of row and piece are requested ahead of the barrier.
+//
 // XRUNS: runs of 2048 k of x that the LDS holds.  XRUNS == RUNS is the form described so far (K = RUNS * 2048, all of a
 // lane's x in registers).  XRUNS > RUNS is the form for a longer K, or one that is no multiple of 2048 (the
 // down-projection of an MLP: K = 11008, 14336, 28672): a row is cut into pieces of RUNS runs, a wave goes through
@@ -305,12 +329,12 @@ __device__ __forceinline__ int small_quotient(int x, int d, float rcp)
 // and a row's sum so far travels in its lane of `res`: the accumulator of lane 0 starts from it.  x is padded with
 // zeros up to whole pieces, and a load that would reach past the end of a row reads the row's last dword instead: what
 // it gathers meets zeros.  One codebook, or several without a workgroup whose rows reach into two; not gated.
-template <int RUNS, int G, int NBUF, int BOOKS, int COPIES, int XRUNS = RUNS, int XM = 1>
+template <int RUNS, int G, int NBUF, int BOOKS, int COPIES, int XRUNS, int XM, bool GATED, bool ALL>
 __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const half_t *__restrict__ x,
                                                                            const uint8_t *__restrict__ codes,
                                                                            const half_t *__restrict__ cb, int entries,
                                                                            int rows_q, int rows_r, int n_total,
-                                                                           int gated_row_bytes, int rows_per_cb,
+                                                                           int row_bytes, int rows_per_cb,
                                                                            float rcp_rows_per_cb, int n_books,
                                                                            const half_t *__restrict__ bias,
                                                                            half_t *__restrict__ y, int rotate_priority)
@@ -319,18 +343,26 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     // dwords of a kernel's arguments into scalar registers at wave launch, -amdgpu-kernarg-preload-count, and what the
     // first loads need - x, the codes, the codebook and the numbers the wave's rows follow from - lies inside them, so
     // that no wave waits for an argument fetch ahead of its first load.)
-    // gated: the epilogue of a gate/up pair.  The rows of W are gate and up rows interleaved in groups of 16; what
+    // GATED: the epilogue of a gate/up pair.  The rows of W are gate and up rows interleaved in groups of 16; what
     // is dealt out to the waves (rows_q, rows_r, n_total) are then the N/2 outputs, a wave's code rows are the gate
     // and the up row of each of its outputs in turn; a group of two rows is one output (G = 2), or the gate row and the
     // up row are two groups in turn (G = 1).
-    // gated_row_bytes: bit 31 = gated, below it the bytes of a row of codes (K / 8; read by the long form only) - one
-    // argument, so that everything the prologue needs stays inside the preloaded fourteen dwords.
+    // row_bytes: of codes, K / 8 (read by the long form only).
     constexpr bool TWO = BOOKS == 2;
+    // Products on the matrix cores (v_mfma_f32_4x4x4_16b_f16) instead of v_dot2_f32_f16: of sixteen 4x4 products by 4 of K, one to four lanes,
+    // the diagonal is lane l's four halves of W times its four of x - gathers and registers stay as they are, three quarters of the result
+    // are what nobody looks at, and the vector unit issues for 4 cycles where two v_dot2 take 8.5.  What a row costs it falls from 250
+    // cycles to 165 beside 128 of the matrix pipe; its sum, over the lanes' diagonals, takes one addition more.  Cold, K = 4096: N = 8192
+    // 3.75 -> 3.54 us, 16384 4.57 -> 4.40, 28672 5.8 -> 5.53, gated (with the one epilogue at the end) N = 22016 6.13 -> 5.48; K = N = 8192
+    // 4.68 -> 4.42.  Not for the chain of a single row, which is as long as its latencies (2.94 -> 2.97; K = 2048, a row at a time, 2.90 ->
+    // 2.93), not with two rows of X (no registers for eight sums more), and not for rows of five pieces (K = 28672, N = 8192 11.2 ->
+    // 11.6; of three, K = 22016, N = 4096, 7.07 -> 6.55).
+    constexpr bool kDiagonal = XM == 1 && NBUF > 1 && RUNS * G > 1 && !(RUNS == 3 && XRUNS == 16);
     constexpr bool LONG = XRUNS != RUNS;
-    static_assert(!LONG || (BOOKS < 2 && COPIES == kWideCopies && NBUF == 2), "the long form: one table, replicated");
+    static_assert(!LONG || (BOOKS < 2 && COPIES == kWideCopies && (NBUF == 2 || ALL)), "the long form: one table, replicated");
     static_assert(NBUF > 1 || G == 1, "a single group per wave: of one row");
     static_assert(XM == 1 || (XM == 2 && RUNS <= 2), "two rows of X: both in the lane's registers, 4096 k of each at a time");
-    const int gated = LONG ? 0 : (gated_row_bytes < 0 ? 1 : 0);
+    static_assert(!GATED || (!LONG && NBUF > 1 && BOOKS != 1), "a gate/up pair: two rows of W at least");
     constexpr int kXChunks = XRUNS * kRunCodes;  // 16-byte pieces of x
     // table of the first codebook (at LDS address 0: a gather address is used as it comes out of the byte
     // permute) | table of the second one (TWO) | x
@@ -340,7 +372,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     uint4_t *table = lds, *xs = lds + kTableSlots;
     const int tid = threadIdx.x;
     // codes (bytes) per row, and the pieces a row is worked through in
-    const int J = LONG ? (gated_row_bytes & 0xffffff) : RUNS * kRunCodes;
+    const int J = LONG ? row_bytes : RUNS * kRunCodes;
     constexpr int kPieceBytes = RUNS * kRunCodes;
     const int n_pieces = LONG ? (J + kPieceBytes - 1) / kPieceBytes : 1;
 
@@ -356,8 +388,8 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
         // the workgroup's first and last share (rows, or outputs when gated) and the rows of W they reach
         const int wg_first = min((int)blockIdx.x * kWideWaves * rows_q + min((int)blockIdx.x * kWideWaves, rows_r), n_total - 1);
         const int wg_last = min(((int)blockIdx.x + 1) * kWideWaves * rows_q + min(((int)blockIdx.x + 1) * kWideWaves, rows_r), n_total) - 1;
-        const int wg_row0 = gated ? gate_row(wg_first) : wg_first;
-        const int wg_row_last = gated ? gate_row(max(wg_last, wg_first)) + 16 : wg_last;
+        const int wg_row0 = GATED ? gate_row(wg_first) : wg_first;
+        const int wg_row_last = GATED ? gate_row(max(wg_last, wg_first)) + 16 : wg_last;
         book0 = small_quotient(wg_row0, rows_per_cb, rcp_rows_per_cb);
         if (TWO) second_book_row = (book0 + 1) * rows_per_cb;
         // (only the workgroups whose rows cross into the next codebook fetch and fill the second table)
@@ -391,17 +423,17 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     const int gw = blockIdx.x * kWideWaves + wave;
     const int row0 = min(gw * rows_q + min(gw, rows_r), n_total - 1);  // (a wave without a share reads the last row)
     const int n_share = rows_q + (gw < rows_r ? 1 : 0);
-    const int n_rows = gated ? 2 * n_share : n_share;
+    const int n_rows = GATED ? 2 * n_share : n_share;
     const int n_groups = (n_rows + G - 1) / G;
     // code row t of the wave (clamped: loads past the end read the last row again)
     auto code_row = [&](int t) {
         t = min(t, max(n_rows, 1) - 1);
-        return gated ? gate_row(row0 + (t >> 1)) + 16 * (t & 1) : row0 + t;
+        return GATED ? gate_row(row0 + (t >> 1)) + 16 * (t & 1) : row0 + t;
     };
     // gated with a bias: lane i keeps the bias of its i-th output's gate and up row (loaded ahead of the codes, so
     // that the loop stays free of loads other than the codes)
     float bias_gate = 0.f, bias_up = 0.f;
-    if (gated && bias) {
+    if (GATED && bias) {
         const int o = row0 + min((int)lane, max(n_share, 1) - 1);
         bias_gate = (float)bias[gate_row(o)];
         bias_up = (float)bias[gate_row(o) + 16];
@@ -439,12 +471,10 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
         if (++req_group >= n_groups) req_group = 0, ++req_piece;
     };
 #pragma unroll
-    for (int u = 0; u < NBUF - 1; u++) {
+    for (int u = 0; u < (ALL || NBUF == 1 ? NBUF : NBUF - 1); u++) {
         if constexpr (LONG) request_next(cw[u]);
         else load_group(0, min(u, max(n_groups, 1) - 1), cw[u]);
     }
-    // (NBUF == 1: no wave has more than one group - its codes are all the loads there are, and there is no loop)
-    if constexpr (NBUF == 1) load_group(0, 0, cw[0]);
 
     if (table_duty) {
         // Table: thread (e, h) writes copies 8h .. 8h+7 of entry e, in an order that sends the sixteen lanes
@@ -492,23 +522,26 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     const uint32_t copy_base = (lane & (kWideCopies - 1)) * 16u;
     const uint8_t *tbl = reinterpret_cast<const uint8_t *>(table);
     float res[XM];       // lane i: the sum of the wave's row i (for each row of X)
-    float gate_sum[XM];  // gated, G = 1: the gate row's sum (wave-uniform) until the up row's group has run
+    float gate_sum[XM];  // gated: lane i's is the gate row's sum of output i, `res` the up row's
 #pragma unroll
     for (int m = 0; m < XM; m++) res[m] = gate_sum[m] = 0.f;
     // rows [g*G, g*G + R) of the wave, R <= G (a compile-time count: the last group may be short)
     auto multiply_rows = [&](int g, const uint32_t (&cur)[G][RUNS], auto r_const) {
         constexpr int R = decltype(r_const)::value;
-        float acc[XM][R];
+        std::conditional_t<kDiagonal, float4_t, float> acc[XM][R];
         uint32_t base[R];
 #pragma unroll
         for (int r = 0; r < R; r++) {
 #pragma unroll
-            for (int m = 0; m < XM; m++) acc[m][r] = 0.f;
+            for (int m = 0; m < XM; m++) acc[m][r] = {};
             // (the long form: the row's sum over the pieces before this one, zero at the first)
             if constexpr (LONG) {
 #pragma unroll
-                for (int m = 0; m < XM; m++)
-                    acc[m][r] = lane == 0 ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, res[m]), g * G + r)) : 0.f;
+                for (int m = 0; m < XM; m++) {
+                    const float so_far = lane == 0 ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, res[m]), g * G + r)) : 0.f;
+                    if constexpr (kDiagonal) acc[m][r][0] = so_far;
+                    else acc[m][r] = so_far;
+                }
             }
             if constexpr (COPIES == 1) base[r] = TWO && code_row(g * G + r) >= second_book_row ? 4096u : 0u;
             else base[r] = TWO ? copy_base | (code_row(g * G + r) >= second_book_row ? 0x10000u : 0u) : copy_base;
@@ -532,48 +565,44 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
 #pragma unroll
                 for (int r = 0; r < R; r++)
 #pragma unroll
-                    for (int d = 0; d < 4; d++)
+                    for (int d = 0; d < 4; d += 2)
 #pragma unroll
                         for (int m = 0; m < XM; m++) {
-                            const uint32_t wd = w[r][c][d], xd = xr[m][q][c][d];
-                            acc[m][r] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, wd), __builtin_bit_cast(half2_t, xd), acc[m][r], false);
+                            const uint2_t wd = {w[r][c][d], w[r][c][d + 1]}, xd = {xr[m][q][c][d], xr[m][q][c][d + 1]};
+                            if constexpr (kDiagonal) {
+                                acc[m][r] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, wd), __builtin_bit_cast(half4_t, xd), acc[m][r], 0, 0, 0);
+                            } else {
+                                const uint32_t w0 = wd[0], w1 = wd[1], x0 = xd[0], x1 = xd[1];
+                                acc[m][r] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, w0), __builtin_bit_cast(half2_t, x0), acc[m][r], false);
+                                acc[m][r] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, w1), __builtin_bit_cast(half2_t, x1), acc[m][r], false);
+                            }
                         }
         }
-        if (G == 2 && R == 2 && gated) {
-            // one output: gate and up sums, the bias of the output's lane, silu(gate) * up
+        auto total = [](auto v) {
+            if constexpr (kDiagonal) return diagonal_sum_to_uniform(v);
+            else return wave_sum_to_uniform(v);
+        };
+        auto keep = [&](float &where, float s, int i) {
+            // (the sum goes from the scalar register straight into lane i: one v_writelane instead of a move, a compare and a select;
+            // on this target the instruction takes one scalar register: the lane number goes through m0)
+            asm("s_mov_b32 m0, %2\n\tv_writelane_b32 %0, %1, m0" : "+v"(where) : "s"(s), "s"(i) : "m0");
+        };
+        if constexpr (GATED) {
+            // rows are the gate and the up row of an output in turn
 #pragma unroll
-            for (int m = 0; m < XM; m++) {
-                const float sg = wave_sum_to_uniform(acc[m][0]) + __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bias_gate), g));
-                const float su = wave_sum_to_uniform(acc[m][R - 1]) + __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bias_up), g));
-                res[m] = (int)lane == g ? silu_f32(sg) * su : res[m];
-            }
-            return;
-        }
-        if (G == 1 && gated) {
-            // even groups are gate rows, odd groups the up rows of the same output
-            const int o = g >> 1;
+            for (int r = 0; r < R; r++)
 #pragma unroll
-            for (int m = 0; m < XM; m++) {
-                const float s = wave_sum_to_uniform(acc[m][0]);
-                if ((g & 1) == 0) {
-                    gate_sum[m] = s + __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bias_gate), o));
-                } else {
-                    const float su = s + __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bias_up), o));
-                    res[m] = (int)lane == o ? silu_f32(gate_sum[m]) * su : res[m];
+                for (int m = 0; m < XM; m++) {
+                    const float s = total(acc[m][r]);
+                    if (((g * G + r) & 1) == 0) keep(gate_sum[m], s, (g * G + r) >> 1);
+                    else keep(res[m], s, (g * G + r) >> 1);
                 }
-            }
-            return;
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int m = 0; m < XM; m++) keep(res[m], total(acc[m][r]), g * G + r);
         }
-#pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int m = 0; m < XM; m++) {
-                // (the row's sum goes from the scalar register straight into lane g*G + r: one v_writelane instead of a
-                // move, a compare and a select)
-                const float s = wave_sum_to_uniform(acc[m][r]);
-                // (on this target the instruction takes one scalar register: the lane number goes through m0)
-                asm("s_mov_b32 m0, %2\n\tv_writelane_b32 %0, %1, m0" : "+v"(res[m]) : "s"(s), "s"(g * G + r) : "m0");
-            }
     };
     auto multiply_group = [&](int g, const uint32_t (&cur)[G][RUNS]) {
         const int left = n_rows - g * G;  // wave-uniform
@@ -601,6 +630,18 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     };
     if constexpr (NBUF == 1) {
         multiply_group(0, cw[0]);
+    } else if constexpr (ALL) {
+        // every pair is on its way: nothing to request
+        int piece = 0, g = 0;
+#pragma unroll
+        for (int u = 0; u < NBUF; u++) {
+            if (rotate_priority) set_priority(age - u);
+            if (piece < n_pieces) {
+                if (g == 0 && piece > 0) load_x_piece(piece);
+                multiply_group(g, cw[u]);
+                if (++g >= n_groups) g = 0, ++piece;
+            }
+        }
     } else if constexpr (LONG) {
         int piece = 0, g = 0, turn = 0;
         while (piece < n_pieces) {
@@ -651,7 +692,11 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
         }
     }
     if ((int)lane < n_share) {
-        const float b = bias && !gated ? (float)bias[row0 + lane] : 0.f;
+        const float b = bias && !GATED ? (float)bias[row0 + lane] : 0.f;
+        if constexpr (GATED) {
+#pragma unroll
+            for (int m = 0; m < XM; m++) res[m] = silu_f32(gate_sum[m] + bias_gate) * (res[m] + bias_up);
+        }
 #pragma unroll
         for (int m = 0; m < XM; m++) y[(int64_t)m * n_total + row0 + lane] = (half_t)(res[m] + b);   // (a row of y: what was dealt out)
     }
@@ -807,87 +852,93 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
     const int rotate_priority = tuning().gemv_wide_rotate_priority >= 1.0 && (n_dealt + waves - 1) / waves >= 2 ? 1 : 0;
     auto launch = [&](auto kern) {
         return launch_kernel(kern, grid, block, 0, s, p.x, codes, p.cb, p.entries, n_dealt / waves, n_dealt % waves, n_dealt,
-                           (int)((p.gated ? 0x80000000u : 0u) | (uint32_t)(p.K / 8)), p.rows_per_cb,
+                           (int)(p.K / 8), p.rows_per_cb,
                            1.0f / (float)p.rows_per_cb, p.n_codebooks, p.bias, p.y, rotate_priority);
     };
     using std::integral_constant;
-    const int g = wide_rows_per_group(p);
-    if (const LongK f = long_k_form(p); p.M == 2 && f.is_long) {
-        auto pick_long2 = [&](auto g_c, auto x_c) {
-            constexpr int GG = decltype(g_c)::value, XR = decltype(x_c)::value;
-            return books == 0 ? launch(decode_gemv_wide_kernel<2, GG, 2, 0, kWideCopies, XR, 2>)
-                              : launch(decode_gemv_wide_kernel<2, GG, 2, 1, kWideCopies, XR, 2>);
+    using std::true_type;
+    using std::false_type;
+    using one = integral_constant<int, 1>;
+    using two = integral_constant<int, 2>;
+    using three = integral_constant<int, 3>;
+    using four = integral_constant<int, 4>;
+    using eight = integral_constant<int, 8>;
+    using sixteen = integral_constant<int, 16>;
+    const int g = wide_rows_per_group(p), rows_per_wave = (n_dealt + waves - 1) / waves;
+    // the plain or the replicated table, and how many of them
+    auto launch_form = [&](auto runs, auto group, auto nbuf, auto copies, auto x_runs, auto x_rows, auto gated, auto all) {
+        if constexpr (!gated() && x_runs() != runs())
+            return books == 0 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), false, all()>)
+                              : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 1, copies(), x_runs(), x_rows(), false, all()>);
+        else if constexpr (gated())   // (a codebook boundary may lie anywhere)
+            return books == 0 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), true, all()>)
+                              : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 2, copies(), x_runs(), x_rows(), true, all()>);
+        else
+            return books == 0   ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), false, all()>)
+                   : books == 1 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 1, copies(), x_runs(), x_rows(), false, all()>)
+                                : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 2, copies(), x_runs(), x_rows(), false, all()>);
+    };
+    using replicated = integral_constant<int, kWideCopies>;
+    if (const LongK f = long_k_form(p); f.is_long) {
+        // (the replicated table, one table per workgroup)
+        if (p.M == 2) {
+            auto go = [&](auto group, auto x_runs) { return launch_form(two{}, group, two{}, replicated{}, x_runs, two{}, false_type{}, false_type{}); };
+            if (f.x_runs == 4) return g == 2 ? go(two{}, four{}) : go(one{}, four{});
+            return g == 2 ? go(two{}, eight{}) : go(one{}, eight{});
+        }
+        // Two pairs of a row and a piece (one row in two pieces, one of them a wave's only row): both requested ahead of the barrier (K =
+        // 11008, N = 4096 4.74 -> 4.64 us, K = 14336 5.39 -> 5.20).  More of them two in flight: three were measured and are slower,
+        // K = 11008 to 28672, N = 4096 to 16384: +3 to +6 %, one shape -3 %.
+        auto go = [&](auto runs, auto x_runs) {
+            const int pieces = (int)((p.K / 8 + runs() * kRunCodes - 1) / (runs() * kRunCodes));
+            if (g == 2) return launch_form(runs, two{}, two{}, replicated{}, x_runs, one{}, false_type{}, false_type{});
+            return rows_per_wave * pieces <= 2 ? launch_form(runs, one{}, two{}, replicated{}, x_runs, one{}, false_type{}, true_type{})
+                                               : launch_form(runs, one{}, two{}, replicated{}, x_runs, one{}, false_type{}, false_type{});
         };
-        auto pick_x2 = [&](auto g_c) {
-            return f.x_runs == 4 ? pick_long2(g_c, integral_constant<int, 4>{}) : pick_long2(g_c, integral_constant<int, 8>{});
-        };
-        return g == 2 ? pick_x2(integral_constant<int, 2>{}) : pick_x2(integral_constant<int, 1>{});
+        if (f.x_runs == 8) return f.runs == 3 ? go(three{}, eight{}) : go(four{}, eight{});
+        return f.runs == 3 ? go(three{}, sixteen{}) : go(four{}, sixteen{});
     }
+    // (a launch in which no wave has more than one row: no second group to request)
+    const bool single = !p.gated && rows_per_wave <= 1;
     if (p.M == 2) {
         // two rows of X against every gathered codeword: the replicated table, one or two groups
-        auto pick2 = [&](auto runs_c, auto g_c, auto nbuf_c) {
-            constexpr int R = decltype(runs_c)::value, GG = decltype(g_c)::value, NB = decltype(nbuf_c)::value;
-            return books == 0 ? launch(decode_gemv_wide_kernel<R, GG, NB, 0, kWideCopies, R, 2>)
-                 : books == 1 ? launch(decode_gemv_wide_kernel<R, GG, NB, 1, kWideCopies, R, 2>)
-                              : launch(decode_gemv_wide_kernel<R, GG, NB, 2, kWideCopies, R, 2>);
+        auto go = [&](auto runs, auto group, auto nbuf, auto gated) { return launch_form(runs, group, nbuf, replicated{}, runs, two{}, gated, false_type{}); };
+        auto with_runs = [&](auto group, auto nbuf, auto gated) {
+            return p.K / kRunK == 1 ? go(one{}, group, nbuf, gated) : go(two{}, group, nbuf, gated);
         };
-        auto pick2_runs = [&](auto g_c, auto nbuf_c) {
-            return p.K / kRunK == 1 ? pick2(integral_constant<int, 1>{}, g_c, nbuf_c) : pick2(integral_constant<int, 2>{}, g_c, nbuf_c);
-        };
-        if (!p.gated && (n_dealt + waves - 1) / waves <= 1) return pick2_runs(integral_constant<int, 1>{}, integral_constant<int, 1>{});
-        return g == 2 ? pick2_runs(integral_constant<int, 2>{}, integral_constant<int, 2>{})
-                      : pick2_runs(integral_constant<int, 1>{}, integral_constant<int, 2>{});
-    }
-    if (const LongK f = long_k_form(p); f.is_long) {
-        // (the replicated table, one table per workgroup, two groups in flight: three were measured and are slower,
-        // K = 11008 to 28672, N = 4096 to 16384: +3 to +6 %, one shape -3 %)
-        auto pick_long = [&](auto runs_c, auto g_c, auto x_c) {
-            constexpr int R = decltype(runs_c)::value, GG = decltype(g_c)::value, XR = decltype(x_c)::value;
-            return books == 0 ? launch(decode_gemv_wide_kernel<R, GG, 2, 0, kWideCopies, XR>)
-                              : launch(decode_gemv_wide_kernel<R, GG, 2, 1, kWideCopies, XR>);
-        };
-        auto pick_x = [&](auto runs_c, auto g_c) {
-            return f.x_runs == 8 ? pick_long(runs_c, g_c, integral_constant<int, 8>{}) : pick_long(runs_c, g_c, integral_constant<int, 16>{});
-        };
-        auto pick_g = [&](auto runs_c) {
-            return g == 2 ? pick_x(runs_c, integral_constant<int, 2>{}) : pick_x(runs_c, integral_constant<int, 1>{});
-        };
-        return f.runs == 3 ? pick_g(integral_constant<int, 3>{}) : pick_g(integral_constant<int, 4>{});
+        if (single) return with_runs(one{}, one{}, false_type{});
+        if (p.gated) return g == 2 ? with_runs(two{}, two{}, true_type{}) : with_runs(one{}, two{}, true_type{});
+        return g == 2 ? with_runs(two{}, two{}, false_type{}) : with_runs(one{}, two{}, false_type{});
     }
     // The plain table while a wave gathers for at most Tuning::gemv_wide_plain_table_max_runs runs of 2048 k (8 gathers per
     // lane and run): measured cold, plain -> replicated, K = 4096: one row per wave 3.29 -> 3.43 us, two rows
     // 4.07 -> 3.89; K = 2048, one row 2.93 -> 3.12; K = 8192, one row 4.26 -> 4.02.
     const int code_rows_per_wave = (int)((p.N + waves - 1) / waves);
     const bool plain_table = (double)code_rows_per_wave * (double)(p.K / kRunK) <= tuning().gemv_wide_plain_table_max_runs;
-    auto pick = [&](auto runs_c, auto g_c, auto nbuf_c) {
-        constexpr int R = decltype(runs_c)::value, GG = decltype(g_c)::value, NB = decltype(nbuf_c)::value;
-        if (plain_table)
-            return books == 0 ? launch(decode_gemv_wide_kernel<R, GG, NB, 0, 1>)
-                 : books == 1 ? launch(decode_gemv_wide_kernel<R, GG, NB, 1, 1>) : launch(decode_gemv_wide_kernel<R, GG, NB, 2, 1>);
-        return books == 0 ? launch(decode_gemv_wide_kernel<R, GG, NB, 0, kWideCopies>)
-             : books == 1 ? launch(decode_gemv_wide_kernel<R, GG, NB, 1, kWideCopies>) : launch(decode_gemv_wide_kernel<R, GG, NB, 2, kWideCopies>);
+    auto go = [&](auto runs, auto group, auto nbuf, auto gated) {
+        return plain_table ? launch_form(runs, group, nbuf, one{}, runs, one{}, gated, false_type{})
+                           : launch_form(runs, group, nbuf, replicated{}, runs, one{}, gated, false_type{});
     };
-    auto pick_runs = [&](auto g_c, auto nbuf_c) {
+    auto with_runs = [&](auto group, auto nbuf, auto gated) {
         switch (p.K / kRunK) {
-        case 1: return pick(integral_constant<int, 1>{}, g_c, nbuf_c);
-        case 2: return pick(integral_constant<int, 2>{}, g_c, nbuf_c);
+        case 1: return go(one{}, group, nbuf, gated);
+        case 2: return go(two{}, group, nbuf, gated);
         default: break;
         }
         // (two rows per group with three groups in flight do not fit the registers beyond K = 4096: not built)
-        if constexpr (decltype(g_c)::value * decltype(nbuf_c)::value <= 4) {
-            if (p.K / kRunK == 3) return pick(integral_constant<int, 3>{}, g_c, nbuf_c);
-            return pick(integral_constant<int, 4>{}, g_c, nbuf_c);
+        if constexpr (group() * nbuf() <= 4) {
+            if (p.K / kRunK == 3) return go(three{}, group, nbuf, gated);
+            return go(four{}, group, nbuf, gated);
         }
         return hipErrorInvalidValue;
     };
-    // (a launch in which no wave has more than one row: no second group to request)
-    const bool single = !p.gated && tuning().gemv_wide_single_rows_max >= 1.0 && (n_dealt + waves - 1) / waves <= 1;
-    if (single) return pick_runs(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    if (single && tuning().gemv_wide_single_rows_max >= 1.0) return with_runs(one{}, one{}, false_type{});
     const int nbuf = (g == 2 && p.K / kRunK > 2) ? 2 : wide_groups_in_flight(p);
-    if (g == 2) return nbuf == 3 ? pick_runs(integral_constant<int, 2>{}, integral_constant<int, 3>{})
-                                 : pick_runs(integral_constant<int, 2>{}, integral_constant<int, 2>{});
-    return nbuf == 3 ? pick_runs(integral_constant<int, 1>{}, integral_constant<int, 3>{})
-                     : pick_runs(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+    auto with_groups = [&](auto gated) {
+        if (g == 2) return nbuf == 3 ? with_runs(two{}, three{}, gated) : with_runs(two{}, two{}, gated);
+        return nbuf == 3 ? with_runs(one{}, three{}, gated) : with_runs(one{}, two{}, gated);
+    };
+    return p.gated ? with_groups(true_type{}) : with_groups(false_type{});
 }
 
 bool decode_gemv_wide_preferred(const ProblemB &p);
