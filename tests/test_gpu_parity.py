@@ -2034,6 +2034,27 @@ def test_infinite_codewords_reach_their_own_rows_only_and_as_infinities(M, K, N,
     assert cabi.VARIANT_GENERIC in ran and (M > 64 or cabi.VARIANT_DECODE in ran)
 
 
+@pytest.mark.parametrize("K,N,v,E,G,gated", [(8192, 48, 4, 256, 1, False), (8192, 64, 4, 200, 2, True), (4096, 48, 4, 4096, 3, False), (6144, 32, 8, 300, 1, False),
+                                             (8192, 32, 4, 1000, 1, True), (6144, 32, 4, 256, 1, False), (2048, 16, 8, 300, 1, False)])
+def test_gemv_kernel_products_of_the_diagonal(K, N, v, E, G, gated):
+    bits = 8 if E <= 256 else 16
+    spec = ProblemSpec("diag4", GEOM_B, 1, K, N, v, E, G, bits, codebook_3d=(G > 1), codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=99, device=DEV)
+    _say("gemv diagonal", K, N, v, E, G, gated)
+    if gated:
+        e1, e2 = vo.rel_err(_np(cabi.e2e_gemm_b_gated(x, codes, cb, variant=cabi.VARIANT_DECODE_GEMV)), vo.gated_gemm_b(_np(x), _np(codes), _np(cb)).astype(np.float64))
+        assert e2 <= TOL and e1 <= 2 * TOL   # (a product of two sums, as in test_gated_epilogue_against_the_oracle)
+        return
+    w = vo.dequant_b(_np(codes), _np(cb))
+    y = cabi.e2e_gemm_b(x, codes, cb, variant=cabi.VARIANT_DECODE_GEMV)
+    assert vo.rel_err(_np(y), _np(x).astype(np.float64) @ w.astype(np.float64).T)[0] <= TOL
+    for c in (0, K // 2 + 3, K - 1):
+        eye = torch.zeros(1, K, dtype=torch.float16, device=DEV)
+        eye[0, c] = 1.0
+        yw = cabi.e2e_gemm_b(eye, codes, cb, variant=cabi.VARIANT_DECODE_GEMV)
+        assert np.array_equal(_np(yw).view(np.uint16), w[:, [c]].T.copy().view(np.uint16)), c
+
+
 # K, N, codebooks, gated: products on the matrix cores or not, by rows per wave (4096 of them), pieces of a row and codebook boundaries
 @pytest.mark.parametrize("K,N,G,gated", [(2048, 8200, 1, False), (2048, 12289, 1, False), (4096, 4097, 1, False), (4096, 16383, 3, False), (8192, 8193, 1, False),
                                          (4096, 96, 1, True), (2048, 16416, 1, True), (4096, 24608, 1, True), (8192, 8224, 257, True), (6144, 8192, 8, True),

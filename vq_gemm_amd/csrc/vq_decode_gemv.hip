@@ -72,6 +72,40 @@ __device__ __forceinline__ float wave_sum(float v)
     return (r0 + r1) + (r2 + r3);
 }
 
+// (One instruction each: the rows the mask leaves out keep their value, which the compiler does not
+// express through the builtin.  The s_nop covers the two wait states a DPP read needs behind a VALU write.)
+__device__ __forceinline__ float dpp_add_row_bcast15(float v)
+{
+    // lane 15 of rows 0 and 2 is added to every lane of rows 1 and 3
+    asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ float dpp_add_row_bcast31(float v)
+{
+    // lane 31 is added to every lane of rows 2 and 3
+    asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf" : "+v"(v));
+    return v;
+}
+
+template <int CONTROL>
+__device__ __forceinline__ float dpp_add(float moved, float v)
+{
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, moved), CONTROL, 0xf, 0xf, true));
+}
+
+// Sum over the 64 lanes of lane l's v[l % 4], valid in lane 63 (returned from there as a wave-uniform value).
+__device__ __forceinline__ float diagonal_sum_to_uniform(float4_t v)
+{
+    float s = dpp_add<0x00>(v[0], v[3]);   // the last lane of every four: its v[3], the first lane's v[0], ...
+    s = dpp_add<0x55>(v[1], s);
+    s = dpp_add<0xaa>(v[2], s);
+    s = dpp_add<0x114>(s, s);              // the last lane of a row of sixteen: the row (shifts by 4 and 8)
+    s = dpp_add<0x118>(s, s);
+    s = dpp_add_row_bcast15(s);
+    s = dpp_add_row_bcast31(s);
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 63));
+}
+
 // Format of the codes: a lane takes the 32 / VEC codes that meet 32 consecutive halves of x in every
 // run of 2048 k, as one load of 4, 8 or 16 bytes.
 template <int VEC, typename CodeT>
@@ -149,11 +183,16 @@ __global__ __launch_bounds__(kGemvWaves * 64) void decode_gemv_kernel(const half
     for (int i = threadIdx.x + kGemvWaves * 64; i < chunks; i += kGemvWaves * 64) table[i] = tsrc[i];
     __syncthreads();
 
-    float acc[MX][kGemvRows];
+    // Products on the matrix cores' diagonals (see the wide form's kDiagonal) for one row of X and K = 8192 - 4-vectors with 8-bit codes N =
+    // 8192 9.1 -> 6.3 us, N = 4096 5.4 -> 4.9, with 16-bit codes N = 8192 13.2 -> 11.1 - or 16-bit codes from K = 4096 on (N = 4096 5.3 ->
+    // 5.15, N = 2048 4.5 -> 4.35).  Elsewhere the longer chain costs more than the vector unit gains (4-vectors with 8-bit codes, K = N =
+    // 4096 3.45 -> 3.53, K = 6144 4.33 -> 4.5; 512 8-vectors, K = 2048 2.71 -> 2.74).
+    constexpr bool kDiagonal = VEC >= 4 && MX == 1 && (RUNS == 4 || (sizeof(CodeT) == 2 && RUNS > 1));
+    std::conditional_t<kDiagonal, float4_t, float> acc[MX][kGemvRows];
 #pragma unroll
     for (int m = 0; m < MX; m++)
 #pragma unroll
-        for (int r = 0; r < kGemvRows; r++) acc[m][r] = 0.f;
+        for (int r = 0; r < kGemvRows; r++) acc[m][r] = {};
     const uint8_t *tbl = reinterpret_cast<const uint8_t *>(table);
 #pragma unroll
     for (int q = 0; q < RUNS; q++)
@@ -179,6 +218,13 @@ __global__ __launch_bounds__(kGemvWaves * 64) void decode_gemv_kernel(const half
                 }
 #pragma unroll
                 for (int m = 0; m < MX; m++)
+                    if constexpr (kDiagonal) {
+#pragma unroll
+                        for (int d = 0; d < VEC / 2; d += 2) {
+                            const uint2_t wd = {w[d], w[d + 1]}, xd = {xr[m][q][c * (VEC / 2) + d], xr[m][q][c * (VEC / 2) + d + 1]};
+                            acc[m][r] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, wd), __builtin_bit_cast(half4_t, xd), acc[m][r], 0, 0, 0);
+                        }
+                    } else
 #pragma unroll
                     for (int d = 0; d < VEC / 2; d++) {
                         // (through scalars: a bit cast applied to a vector element reads element 0)
@@ -192,7 +238,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void decode_gemv_kernel(const half
         float sum[kGemvRows];
 #pragma unroll
         for (int r = 0; r < kGemvRows; r++) {
-            sum[r] = wave_sum(acc[m][r]);
+            if constexpr (kDiagonal) sum[r] = diagonal_sum_to_uniform(acc[m][r]);
+            else sum[r] = wave_sum(acc[m][r]);
             if (bias) sum[r] += (float)bias[code_row(r)];
         }
         if constexpr (GATED) {
@@ -234,21 +281,6 @@ constexpr int kWideWaves = 16;
 constexpr int kWideCopies = 16;
 constexpr int kWideTableBytes = 256 * kWideCopies * 16;  // 64 KB
 
-// (One instruction each: the rows the mask leaves out keep their value, which the compiler does not
-// express through the builtin.  The s_nop covers the two wait states a DPP read needs behind a VALU write.)
-__device__ __forceinline__ float dpp_add_row_bcast15(float v)
-{
-    // lane 15 of rows 0 and 2 is added to every lane of rows 1 and 3
-    asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf" : "+v"(v));
-    return v;
-}
-__device__ __forceinline__ float dpp_add_row_bcast31(float v)
-{
-    // lane 31 is added to every lane of rows 2 and 3
-    asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf" : "+v"(v));
-    return v;
-}
-
 // Sum of v over the 64 lanes, valid in lane 63 (returned from there as a wave-uniform value).
 __device__ __forceinline__ float wave_sum_to_uniform(float v)
 {
@@ -259,25 +291,6 @@ __device__ __forceinline__ float wave_sum_to_uniform(float v)
     v = dpp_add_row_bcast15(v);
     v = dpp_add_row_bcast31(v);
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
-
-template <int CONTROL>
-__device__ __forceinline__ float dpp_add(float moved, float v)
-{
-    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, moved), CONTROL, 0xf, 0xf, true));
-}
-
-// Sum over the 64 lanes of lane l's v[l % 4], valid in lane 63 (returned from there as a wave-uniform value).
-__device__ __forceinline__ float diagonal_sum_to_uniform(float4_t v)
-{
-    float s = dpp_add<0x00>(v[0], v[3]);   // the last lane of every four: its v[3], the first lane's v[0], ...
-    s = dpp_add<0x55>(v[1], s);
-    s = dpp_add<0xaa>(v[2], s);
-    s = dpp_add<0x114>(s, s);              // the last lane of a row of sixteen: the row (shifts by 4 and 8)
-    s = dpp_add<0x118>(s, s);
-    s = dpp_add_row_bcast15(s);
-    s = dpp_add_row_bcast31(s);
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 63));
 }
 
 // Where the piece of x that code c of lane l's dword meets lies in its run: the pieces of a code together, so that the lanes of a
