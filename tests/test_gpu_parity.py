@@ -2450,19 +2450,35 @@ def test_encoder_at_the_ends_of_the_range_of_halves(N, K, v, E, scale):
     assert np.array_equal(_np(codes), c_oracle.encode_b(w.numpy(), cb.numpy(), bits))
 
 
-@pytest.mark.parametrize("scale", [2e-6, 0.02, 2e4])
-def test_lloyd_assignments_of_eight_vectors_with_the_norms_as_parts_of_k(scale):
-    """The first assignment of one iteration, whose kernel is another than the encoder's: the sums make the same codebook as the encoder's codes."""
+@pytest.mark.parametrize("N,K", [(4096, 1024), (4096, 1032)])
+def test_encoder_in_workgroups_of_sixteen_waves(N, K):
+    """Codebooks that leave no room for a second workgroup on the unit, every unit at work: rows picked from all over against the oracle."""
+    v, E = 8, 5000
+    g = torch.Generator(device="cpu").manual_seed(25)
+    cb, w = torch.randn(1, E, v, generator=g).half(), torch.randn(N, K, generator=g).half()
+    _say("encode", N, K, v, E)
+    codes = cabi.encode_b(w.to(DEV), cb.to(DEV), 16)
+    torch.cuda.synchronize()
+    rows = list(range(0, N, 97)) + [N - 1]
+    assert np.array_equal(_np(codes)[rows], c_oracle.encode_b(w[rows].contiguous().numpy(), cb.numpy(), 16))
+
+
+@pytest.mark.parametrize("N,K,v,E,scale", [(1032, 1032, 8, 100, 2e-6), (1032, 1032, 8, 100, 0.02), (1032, 1032, 8, 100, 2e4),
+                                           (4096, 1032, 8, 128, 0.02), (4104, 1024, 8, 900, 0.02), (2056, 1024, 4, 129, 2e-5), (4096, 1032, 8, 127, 0.02)])
+def test_lloyd_assignments_make_the_codebook_of_the_encoders_codes(N, K, v, E, scale):
+    """The first assignment of one iteration, whose kernel is another than the encoder's: half norms as parts of K, workgroups of sixteen
+    waves (from 2**19 vectors and 128 entries on)."""
     from vq_gemm_amd.torch_ops import native
-    N, K, v, E = 1032, 1032, 8, 100
     g = torch.Generator(device="cpu").manual_seed(24)
     w = (torch.randn(N, K, generator=g) * scale).clamp(-65504, 65504).half().to(DEV)
     pick = torch.randperm(N * K // v, generator=g)[:E].to(torch.int32).view(1, E)
     _say("lloyd", N, K, v, E, scale)
-    _, cb, errors = native.kmeans(w, pick, v, E, 1, 8, 1)
+    bits = 8 if E <= 256 else 16
+    _, cb, errors = native.kmeans(w, pick, v, E, 1, bits, 1)
     vectors = w.view(-1, v)
     first = vectors[pick.view(-1).long().to(DEV)].contiguous()
-    codes = cabi.encode_b(w, first).view(-1).long()
+    codes = cabi.encode_b(w, first, bits).view(-1)
+    codes = (codes if bits == 8 else codes.view(torch.int16)).long()
     d = vectors.double() - first.double()[codes]
     assert abs(float(errors[0]) - float((d * d).sum())) <= 1e-4 * float((d * d).sum())   # fp32 sums of a wave's, 131 K of them
     sums = torch.zeros(E, v, dtype=torch.float64, device=DEV).index_add_(0, codes, vectors.double())

@@ -5,7 +5,8 @@
 
 namespace vq {
 
-constexpr int kScanThreads = 512;  // eight waves per workgroup of the matrix-core scan (more per unit than two such, in smaller workgroups, gained nothing)
+// eight waves per workgroup of the matrix-core scan (more per unit than two such, in smaller workgroups, gained nothing), or sixteen
+constexpr int kScanThreads = 512, kScanWideThreads = 1024;
 
 // floats of one workgroup's partial result of a Lloyd iteration: per entry `vec` sums and a count, then the error
 __host__ __device__ inline int64_t lloyd_row(int entries, int vec) { return (int64_t)entries * (vec + 1) + 1; }

@@ -92,11 +92,12 @@ __global__ __launch_bounds__(kEncThreads) void encode_b_kernel(const half_t *__r
 // ---- matrix-core scan -------------------------------------------------------------------------
 // What bounds it: the vector unit.  The rule costs 2 * vec + 2 vector instructions per vector and entry; a score costs
 // the matrix pipe 1/32 of a cycle (v_mfma_f32_32x32x8_f16: 32 entries by 32 vectors, vec <= 8 of its k in use) and the
-// vector unit 13 instructions per 16: of each group of eight scores four to fold them to their minimum and one to put the group's number
-// into its low bits, then three that keep the best group and the second best of the two (11 per 16 in groups of sixteen).  All of them
-// take 4.2 cycles here; an MFMA adds 8 to the 54 of the fold of its results while other waves fold, of its own 32.  What a 4096 x
-// 4096 weight takes in 8-vectors with 256 entries: 29.5 us (with a comparison and a selection for the group's number, 16 instructions per
-// 16 scores, 36; by the rule 230), of which a tile of 32 entries is 1.9, the pass per vector behind the scan 9, table and launch 4.
+// vector unit 12.5 instructions per 16: of each group of eight scores four to fold them to their minimum and one to put the group's number
+// into its low bits, then five per two tiles that keep the best group and the second best (10.5 per 16 in groups of sixteen).  All of them
+// take 4.2 cycles here; an MFMA adds 8 to the 52 of the fold of its results while other waves fold, of its own 32.  What a 4096 x
+// 4096 weight takes in 8-vectors with 256 entries: 28.9 us (the second best kept after every tile, 13 per 16, 29.5; with a comparison and
+// a selection for the group's number, 16 per 16 scores, 36; by the rule 230), of which a tile of 32 entries is 1.8, the pass per vector
+// behind the scan 9, table and launch 4.
 //
 // A wave takes 128 vectors as four batches of 32 (64 as two, where there are too few for a workgroup on every other unit), so that an entry tile read from the LDS (its halves and its
 // half norms) meets four MFMAs.  A lane of the result holds 16 scores of one vector - two groups of eight entries, or one -, and
@@ -196,14 +197,14 @@ __device__ __forceinline__ HalfWaves swap_half_waves(uint32_t a, uint32_t b)
 // as a flag of the one kernel it cost every assignment half a microsecond).
 enum ScanKeeps { kCodesOnly, kErrorOnly, kSums };
 
-template <int VEC, typename CodeT, int GROUP, ScanKeeps KEEPS, int kScanBatches, bool NORMS_IN_K>
-__global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half_t *__restrict__ w, const half_t *__restrict__ cb,
+template <int VEC, typename CodeT, int GROUP, ScanKeeps KEEPS, int kScanBatches, bool NORMS_IN_K, int THREADS>
+__global__ __launch_bounds__(THREADS, 4) void encode_scan_kernel(const half_t *__restrict__ w, const half_t *__restrict__ cb,
                                                                    CodeT *__restrict__ codes, int64_t vectors_per_cb, int entries,
                                                                    int wgs_per_cb, float *__restrict__ partials, int bucket_off,
                                                                    int n_buckets)
 {
     extern __shared__ __align__(16) uint8_t smem[];
-    __shared__ float reduce[kScanThreads / 64];
+    __shared__ float reduce[THREADS / 64];
     constexpr bool ACCUMULATE = KEEPS != kCodesOnly, SUMS = KEEPS == kSums;
     constexpr int DW = VEC / 2;                       // dwords of a vector
     constexpr int kScanVectors = 32 * kScanBatches;   // of a wave
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half
     const half_t *wg_w = w + (int64_t)g * vectors_per_cb * VEC;
     CodeT *wg_codes = codes + (int64_t)g * vectors_per_cb;
 
-    const int64_t step = (int64_t)wgs_per_cb * (kScanThreads / 64) * kScanVectors;
+    const int64_t step = (int64_t)wgs_per_cb * (THREADS / 64) * kScanVectors;
     // a vector per lane, two batches of them at a time
     typedef uint32_t dwords_of_vector_t __attribute__((ext_vector_type(DW)));
     typedef dwords_of_vector_t vector_t __attribute__((aligned(DW < 2 ? 4 : 8)));
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half
         for (int u = 0; u < kScanBatches / 2; u++) v[u] = from[min((uint32_t)(u * 64 + lane), last)];
     };
     vector_t coming[kScanBatches / 2];
-    int64_t base = ((int64_t)part * (kScanThreads / 64) + wave) * kScanVectors;
+    int64_t base = ((int64_t)part * (THREADS / 64) + wave) * kScanVectors;
     if (base < vectors_per_cb) load_vectors(base, coming);
 
     // table, half norms, whether all of them are finite (else every vector of the codebook is decided by the rule)
@@ -270,9 +271,9 @@ __global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half
             for (int i = 0; i < DW; i++) own[i] = (e < entries ? own[i] : 0u) ^ 0x80008000u;
         };
         load(tid);
-        for (int i = tid; i < n_buckets; i += kScanThreads) bucket[i] = ~0u;
+        for (int i = tid; i < n_buckets; i += THREADS) bucket[i] = ~0u;
         if (n_buckets) __syncthreads();
-        for (int e = tid; e < n_tiles * 32; e += kScanThreads) {
+        for (int e = tid; e < n_tiles * 32; e += THREADS) {
             if (e != tid) load(e);
             float n2 = 0.f;
             uint32_t c[DW];
@@ -288,13 +289,13 @@ __global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half
             if (n_buckets && e < entries) atomicMin(&bucket[bucket_of(c)], (uint32_t)e);
         }
         if constexpr (SUMS)
-            for (int i = tid; i < entries * (VEC + 1); i += kScanThreads) sums[i] = 0.0;
+            for (int i = tid; i < entries * (VEC + 1); i += THREADS) sums[i] = 0.0;
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) largest = fmaxf(largest, __shfl_xor(largest, d));
         if (lane == 0) reduce[wave] = largest;
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < kScanThreads / 64; i++) largest = fmaxf(largest, reduce[i]);
+        for (int i = 0; i < THREADS / 64; i++) largest = fmaxf(largest, reduce[i]);
         book_finite = largest < __builtin_inff();
         if constexpr (NORMS_IN_K) {
             // |c|^2 / 2 as a sum of halves times powers of two: kTop parts at the scale that the largest needs (all but the first only for
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half
             if (VEC == 8 && 0.5f * largest > 65504.f * scale) hides = kHiddenManyParts;
 #pragma unroll
             for (int i = 0; i < kParts; i++) scales[i] = (half_t)(i < kTop ? scale : i == kTop ? scale * 0x1p-11f : scale * 0x1p-22f);
-            for (int e = tid; e < n_tiles * 32; e += kScanThreads) {
+            for (int e = tid; e < n_tiles * 32; e += THREADS) {
                 uint32_t c[DW];
                 read_entry<DW>(table, at(e), c);
                 float left = 0.f;
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half
             __syncthreads();
         } else
         if (n_buckets) {
-            for (int e = tid; e < entries; e += kScanThreads) {
+            for (int e = tid; e < entries; e += THREADS) {
                 uint32_t c[DW], other[DW];
                 read_entry<DW>(table, at(e), c);
                 const int first = (int)bucket[bucket_of(c)];
@@ -450,7 +451,8 @@ __global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half
         if constexpr (NORMS_IN_K) ahead = load_tile(0);
         for (int t0 = 0, run = 0; t0 < n_tiles; t0 += kRunTiles, run++) {
             const int t1 = min(t0 + kRunTiles, n_tiles);
-            for (int t = t0; t < t1; t++) {
+            // one tile: the best and the second best of its groups and of m1's, the one kept in m1, the other returned
+            auto scan_tile = [&](int t, float (&second)[kScanBatches]) {
                 uint32_t number[2] = {(uint32_t)((t - t0) * kGroups), (uint32_t)((t - t0) * kGroups + 1)};
                 asm("" : "+s"(number[0]), "+s"(number[1]));
                 operand_t a;
@@ -474,14 +476,26 @@ __global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half
                         x[gr] = numbered(f, number[gr]);
                     }
                     if constexpr (kGroups == 2) {
-                        const float second = __builtin_amdgcn_fmed3f(m1[u], x[0], x[1]);
+                        second[u] = __builtin_amdgcn_fmed3f(m1[u], x[0], x[1]);
                         m1[u] = min3(m1[u], x[0], x[1]);
-                        m2[u] = __builtin_amdgcn_fmed3f(m2[u], second, below);
                     } else {
-                        m2[u] = __builtin_amdgcn_fmed3f(m1[u], m2[u], x[0]);
+                        second[u] = __builtin_amdgcn_fmed3f(m1[u], x[0], above);
                         m1[u] = __builtin_amdgcn_fmed3f(m1[u], x[0], below);
                     }
                 }
+            };
+            int t = t0;
+            float second0[kScanBatches], second1[kScanBatches];
+            for (; t + 1 < t1; t += 2) {
+                scan_tile(t, second0);
+                scan_tile(t + 1, second1);
+#pragma unroll
+                for (int u = 0; u < kScanBatches; u++) m2[u] = min3(m2[u], second0[u], second1[u]);
+            }
+            if (t < t1) {
+                scan_tile(t, second0);
+#pragma unroll
+                for (int u = 0; u < kScanBatches; u++) m2[u] = __builtin_amdgcn_fmed3f(m2[u], second0[u], below);
             }
             if (t1 == n_tiles && run == 0) break;   // all there is
 #pragma unroll
@@ -623,10 +637,10 @@ __global__ __launch_bounds__(kScanThreads, 4) void encode_scan_kernel(const half
         __syncthreads();
         float *row = partials + (int64_t)blockIdx.x * lloyd_row(entries, VEC);
         if constexpr (SUMS)
-            for (int i = tid; i < entries * (VEC + 1); i += kScanThreads) row[i] = (float)sums[i];
+            for (int i = tid; i < entries * (VEC + 1); i += THREADS) row[i] = (float)sums[i];
         if (tid == 0) {
             float e = 0.f;
-            for (int i = 0; i < kScanThreads / 64; i++) e += reduce[i];
+            for (int i = 0; i < THREADS / 64; i++) e += reduce[i];
             row[entries * (VEC + 1)] = e;
         }
     }
@@ -642,19 +656,23 @@ size_t scan_lds_bytes(const ProblemB &p, bool accumulate, bool norms_in_k = fals
 // (two workgroups and their few static bytes in 160 KB)
 constexpr size_t kScanLdsTwoPerUnit = 79 * 1024, kScanLds = 128 * 1024;
 
-// Batches of a wave, workgroups per codebook: as many as are resident together (two of eight waves per unit while the LDS
-// allows), none without work.  The same for every assignment of a Lloyd iteration.
+// Threads of a workgroup, batches of a wave, workgroups per codebook: as many as are resident together - two of eight waves per
+// unit, or one of sixteen where every unit has work for it and two do not fit (4096 x 4096 in 8-vectors: 5000 entries 376 -> 338 us; a
+// Lloyd iteration's sums of 1000 entries 101.6 -> 85) or leave sums behind, which the update has to read (256 entries 33.8 -> 32.7; 32
+// entries, whose additions meet, 28.9 -> 29.6) -, none without work.  The same for every assignment of a Lloyd iteration.
 struct ScanPlan {
-    int batches, wgs_per_cb;
+    int threads, batches, wgs_per_cb;
 };
 ScanPlan scan_plan(const ProblemB &p, bool accumulate)
 {
-    const int64_t vectors = (int64_t)p.rows_per_cb * (p.K / p.vec);
-    const int per_cu = scan_lds_bytes(p, accumulate) <= kScanLdsTwoPerUnit ? 2 : 1;
-    const int64_t want = ((int64_t)device_cu_count() * per_cu + p.n_codebooks - 1) / p.n_codebooks;
-    auto have = [&](int batches) { return (vectors + kScanThreads / 2 * batches - 1) / (kScanThreads / 2 * batches); };
-    const int batches = have(4) * p.n_codebooks * 2 <= device_cu_count() ? 2 : 4;
-    return {batches, (int)(want < have(batches) ? want : have(batches))};
+    const int64_t vectors = (int64_t)p.rows_per_cb * (p.K / p.vec), cus = device_cu_count();
+    const bool two = scan_lds_bytes(p, accumulate) <= kScanLdsTwoPerUnit;
+    const bool wide = (!two || (accumulate && p.entries >= 128)) && vectors * p.n_codebooks >= cus * (kScanWideThreads / 64) * 128;
+    const int threads = wide ? kScanWideThreads : kScanThreads, per_cu = wide || !two ? 1 : 2;
+    const int64_t want = (cus * per_cu + p.n_codebooks - 1) / p.n_codebooks;
+    auto have = [&](int batches) { return (vectors + threads / 2 * batches - 1) / (threads / 2 * batches); };
+    const int batches = have(4) * p.n_codebooks * 2 <= cus ? 2 : 4;
+    return {threads, batches, (int)(want < have(batches) ? want : have(batches))};
 }
 
 // Half norms as parts of K: of 4-vectors wherever two workgroups still share a unit (no MFMA more, and a quarter of the LDS reads: 4096 x
@@ -690,20 +708,30 @@ hipError_t launch_scan(const half_t *w, const ProblemB &p, void *codes_out, floa
     const bool in_k = scan_norms_in_k(p, accumulate, KEEPS == kSums, plan.batches), narrow = p.entries < kScanWideGroupEntries;
     const size_t smem = scan_lds_bytes(p, accumulate, in_k);
     const int buckets = scan_buckets(smem, p.entries);
-    auto launch = [&](auto batches, auto norms_in_k) {
-        const auto kern = narrow ? encode_scan_kernel<VEC, CodeT, 8, KEEPS, batches(), norms_in_k()>
-                                 : encode_scan_kernel<VEC, CodeT, 16, KEEPS, batches(), norms_in_k()>;
-        return launch_kernel(kern, dim3((unsigned)(plan.wgs_per_cb * p.n_codebooks)), dim3(kScanThreads), smem + 4 * (size_t)buckets, s, w, p.cb,
-                             static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, plan.wgs_per_cb, partials, (int)smem, buckets);
+    auto launch = [&](auto threads, auto batches, auto norms_in_k) {
+        auto go = [&](auto kern) {
+            return launch_kernel(kern, dim3((unsigned)(plan.wgs_per_cb * p.n_codebooks)), dim3(threads()), smem + 4 * (size_t)buckets, s, w, p.cb,
+                                 static_cast<CodeT *>(codes_out), vectors_per_cb, p.entries, plan.wgs_per_cb, partials, (int)smem, buckets);
+        };
+        if (narrow) return go(encode_scan_kernel<VEC, CodeT, 8, KEEPS, batches(), norms_in_k(), threads()>);
+        return go(encode_scan_kernel<VEC, CodeT, 16, KEEPS, batches(), norms_in_k(), threads()>);
     };
     using std::integral_constant;
     using four = integral_constant<int, 4>;
     using two = integral_constant<int, 2>;
-    if constexpr (VEC == 4)
-        if (in_k) return plan.batches == 4 ? launch(four{}, std::true_type{}) : launch(two{}, std::true_type{});
-    if constexpr (VEC == 8 && KEEPS == kSums)
-        if (in_k) return launch(four{}, std::true_type{});
-    return plan.batches == 4 ? launch(four{}, std::false_type{}) : launch(two{}, std::false_type{});
+    using wide = integral_constant<int, kScanWideThreads>;
+    using usual = integral_constant<int, kScanThreads>;
+    const bool wide_wg = plan.threads == kScanWideThreads;
+    if constexpr (VEC == 4 || (VEC == 8 && KEEPS == kSums))
+        if (in_k) {
+            if constexpr (accumulate)
+                if (wide_wg) return launch(wide{}, four{}, std::true_type{});
+            if constexpr (VEC == 4)
+                if (plan.batches == 2) return launch(usual{}, two{}, std::true_type{});
+            return launch(usual{}, four{}, std::true_type{});
+        }
+    if (wide_wg) return launch(wide{}, four{}, std::false_type{});
+    return plan.batches == 4 ? launch(usual{}, four{}, std::false_type{}) : launch(usual{}, two{}, std::false_type{});
 }
 
 template <int VEC, typename CodeT>
