@@ -2059,7 +2059,8 @@ def test_gemv_kernel_products_of_the_diagonal(K, N, v, E, G, gated):
 @pytest.mark.parametrize("K,N,G,gated", [(2048, 8200, 1, False), (2048, 12289, 1, False), (4096, 4097, 1, False), (4096, 16383, 3, False), (8192, 8193, 1, False),
                                          (4096, 96, 1, True), (2048, 16416, 1, True), (4096, 24608, 1, True), (8192, 8224, 257, True), (6144, 8192, 8, True),
                                          (8224, 4096, 1, False), (12288, 4097, 1, False), (16384, 4096, 1, False), (24576, 130, 1, False),
-                                         (26624, 130, 1, False), (11008, 8192, 2, False)])
+                                         (26624, 130, 1, False), (11008, 8192, 2, False), (14336, 300, 1, False), (11008, 5003, 1, False), (8192, 10241, 1, False),
+                                         (4096, 1001, 1, False), (6144, 33, 1, False), (8192, 9248, 1, True)])
 def test_gemv_wide_form_products_of_the_diagonal(K, N, G, gated):
     spec = ProblemSpec("diag", GEOM_B, 1, K, N, 8, 256, G, 8, codebook_3d=(G > 1), codebook_std=0.05)
     x, codes, cb = make_problem(spec, seed=98, device=DEV)

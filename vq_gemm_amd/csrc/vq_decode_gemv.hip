@@ -262,7 +262,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void decode_gemv_kernel(const half
 // each entry in one 256-byte bank row, lane l reading copy l % 16, so the gathers never collide):
 // four waves per SIMD cover the latency of each other's gathers.  One or two rows of X, 8-vectors, 8-bit codes.
 //   * The rows of W are dealt out to the waves of the whole grid in contiguous runs of equal length
-//     (one more for the first N % waves), so no unit idles while another finishes a longer share.
+//     (one more for the first N % waves, or for the first waves of every workgroup: wide_deals_by_units).
 //     A workgroup's rows may reach into a second codebook: it then holds two tables (128 KB) and a
 //     row picks its table through the third byte of the gather address.
 //   * x goes through the LDS once per workgroup (4 to 16 KB, laid out so that a wave reads its 16-byte
@@ -310,6 +310,12 @@ __device__ __forceinline__ int small_quotient(int x, int d, float rcp)
     q -= rem < 0 ? 1 : 0;
     return q;
 }
+
+// Whether every workgroup gets the same share.  Where the rows are long a unit with more of them than others is what a launch ends with
+// (K = 11008, N = 5120 6.1 -> 5.7 us, K = N = 8192 gated 9.6 -> 9.1, K = 14336, N = 1024 4.63 -> 4.0), and fewer than one a wave come
+// from more units (K = 4096, N = 1024 2.57 -> 2.42); launches of a few shorter ones take longer when no unit is done ahead of
+// the others (K = 4096, N = 14336 4.22 -> 4.34, K = 2048, N = 1024 2.13 -> 2.27).
+constexpr bool wide_deals_by_units(int runs, int nbuf, int x_runs) { return x_runs != runs || runs > 2 || (runs == 2 && nbuf == 1); }
 
 // BOOKS: 0 = one codebook; 1 = several, no workgroup's rows reach into a second one; 2 = some workgroup's rows
 // do, and every workgroup then fills two tables.  (A compile-time flag, like the unconditional loads below: a
@@ -397,10 +403,16 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     // row of W behind a gated output: its gate row (the up row lies 16 further on)
     auto gate_row = [](int o) { return 32 * (o >> 4) + (o & 15); };
     bool second_table = false;
+    // The first row (or output) of a wave: evenly to all waves, one more for the first rows_r of them, or (kByUnits) for the first rows_r
+    // of every workgroup.  (kByUnits and one codebook: the launch says which, and a workgroup's share, in arguments that nothing
+    // else reads then.)
+    constexpr bool kByUnits = wide_deals_by_units(RUNS, NBUF, XRUNS);
+    const int waves_counted = !kByUnits ? kWideWaves : BOOKS == 0 ? n_books : 0;
+    const int wg_share = kByUnits && BOOKS == 0 ? rows_per_cb : kWideWaves * rows_q + (kByUnits ? rows_r : 0);
+    auto dealt_from = [&](int wg, int wave) { return wg * wg_share + wave * rows_q + min(wg * waves_counted + wave, rows_r); };
     if constexpr (BOOKS > 0) {
         // the workgroup's first and last share (rows, or outputs when gated) and the rows of W they reach
-        const int wg_first = min((int)blockIdx.x * kWideWaves * rows_q + min((int)blockIdx.x * kWideWaves, rows_r), n_total - 1);
-        const int wg_last = min(((int)blockIdx.x + 1) * kWideWaves * rows_q + min(((int)blockIdx.x + 1) * kWideWaves, rows_r), n_total) - 1;
+        const int wg_first = min(dealt_from(blockIdx.x, 0), n_total - 1), wg_last = min(dealt_from(blockIdx.x + 1, 0), n_total) - 1;
         const int wg_row0 = GATED ? gate_row(wg_first) : wg_first;
         const int wg_row_last = GATED ? gate_row(max(wg_last, wg_first)) + 16 : wg_last;
         book0 = small_quotient(wg_row0, rows_per_cb, rcp_rows_per_cb);
@@ -433,9 +445,8 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     // result per lane
     const uint32_t lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int gw = blockIdx.x * kWideWaves + wave;
-    const int row0 = min(gw * rows_q + min(gw, rows_r), n_total - 1);  // (a wave without a share reads the last row)
-    const int n_share = rows_q + (gw < rows_r ? 1 : 0);
+    const int from = dealt_from(blockIdx.x, wave), row0 = min(from, n_total - 1);  // (a wave without a share reads the last row)
+    const int most = rows_q + ((int)blockIdx.x * waves_counted + wave < rows_r ? 1 : 0), n_share = kByUnits ? min(most, n_total - from) : most;
     const int n_rows = GATED ? 2 * n_share : n_share;
     const int n_groups = (n_rows + G - 1) / G;
     // code row t of the wave (clamped: loads past the end read the last row again)
@@ -863,10 +874,15 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
     // the waves of a SIMD take turns at the issue priority (see the kernel) once they have two rows or more each: a
     // single row per wave is over before a turn would come
     const int rotate_priority = tuning().gemv_wide_rotate_priority >= 1.0 && (n_dealt + waves - 1) / waves >= 2 ? 1 : 0;
-    auto launch = [&](auto kern) {
-        return launch_kernel(kern, grid, block, 0, s, p.x, codes, p.cb, p.entries, n_dealt / waves, n_dealt % waves, n_dealt,
-                           (int)(p.K / 8), p.rows_per_cb,
-                           1.0f / (float)p.rows_per_cb, p.n_codebooks, p.bias, p.y, rotate_priority);
+    auto launch_dealt = [&](auto kern, bool can_by_units) {
+        // (With hardly a row more than whole ones for every wave the first workgroups take them, which begin a little before the others:
+        // K = 12288, N = 4097 5.0 us, and 5.45 with a row more in every workgroup.)
+        const bool by_units = can_by_units && (books > 0 || n_dealt < waves || n_dealt % waves >= waves / 16);
+        const int share = by_units ? (n_dealt + cus - 1) / cus : n_dealt, of = by_units ? kWideWaves : waves;
+        const int wg_share = by_units ? share : kWideWaves * (share / of), waves_counted = by_units ? 0 : kWideWaves;
+        return launch_kernel(kern, grid, block, 0, s, p.x, codes, p.cb, p.entries, share / of, share % of, n_dealt,
+                           (int)(p.K / 8), can_by_units && books == 0 ? wg_share : p.rows_per_cb,
+                           1.0f / (float)p.rows_per_cb, can_by_units && books == 0 ? waves_counted : p.n_codebooks, p.bias, p.y, rotate_priority);
     };
     using std::integral_constant;
     using std::true_type;
@@ -880,6 +896,7 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
     const int g = wide_rows_per_group(p), rows_per_wave = (n_dealt + waves - 1) / waves;
     // the plain or the replicated table, and how many of them
     auto launch_form = [&](auto runs, auto group, auto nbuf, auto copies, auto x_runs, auto x_rows, auto gated, auto all) {
+        auto launch = [&](auto kern) { return launch_dealt(kern, wide_deals_by_units(runs(), nbuf(), x_runs())); };
         if constexpr (!gated() && x_runs() != runs())
             return books == 0 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), false, all()>)
                               : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 1, copies(), x_runs(), x_rows(), false, all()>);
