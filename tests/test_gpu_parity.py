@@ -2361,6 +2361,24 @@ def test_copies_of_the_codebook_change_no_bit(vec, M, K, N, E):
             assert torch.equal(one.view(torch.int16), two.view(torch.int16)), tile
 
 
+@pytest.mark.parametrize("vec", [4, 8])
+@pytest.mark.parametrize("M,K,N,E", [(1, 128, 6, 512), (16, 192, 258, 300), (33, 1088, 130, 512), (40, 4160, 34, 8), (5, 2048, 642, 512)])
+def test_copies_of_a_codebook_with_16_bit_codes_change_no_bit(vec, M, K, N, E):
+    """As above, up to 512 entries in rows of half the banks; 513 entries and more have no such table."""
+    spec = ProblemSpec("wave_k", GEOM_B, M, K, N, vec, E, 1, 16, codebook_std=0.05)
+    x, codes, cb = make_problem(spec, seed=95, device=DEV)
+    cb[E - 1, 0], cb[E // 2, vec - 1] = float("inf"), float("nan")
+    twice = torch.stack([cb, cb]).contiguous()
+    more = torch.cat([cb, torch.ones(520 - E if E < 512 else 8, vec, dtype=torch.float16, device=DEV)]).contiguous()
+    for tile in (12, 13, 14, 18, 23, 24, 28):
+        if vec == 4 and tile == 28:
+            continue
+        _say("copies", vec, M, K, N, E, "tile", tile)
+        one, two, plain = (_with_wave_tile(tile, lambda: cabi.e2e_gemm_b(x, codes, book, variant=cabi.VARIANT_WAVE_K)) for book in (cb, twice, more))
+        torch.cuda.synchronize()
+        assert torch.equal(one.view(torch.int16), two.view(torch.int16)) and torch.equal(one.view(torch.int16), plain.view(torch.int16)), tile
+
+
 @pytest.mark.parametrize("M,K,N", [(1, 64, 8), (17, 96, 40), (33, 320, 65), (65, 1056, 2047), (130, 2048, 129), (16, 512, 64)])
 @pytest.mark.parametrize("shift", [0, 1])   # elements by which w is off a 16-byte boundary
 def test_k_dealt_out_to_waves_plain_gemm(M, K, N, shift):

@@ -36,7 +36,7 @@ namespace vq {
 namespace {
 
 constexpr int kStepK = 32;                // k of one MFMA step
-constexpr int kCopiesEntries = 256, kCopiesBytes = kCopiesEntries * 256;   // a table of copies: a row of banks per entry
+constexpr int kCopiesBytes = 64 * 1024;   // a table of copies: a row of banks for each of 256 entries, or half of one for each of 512
 
 // What W is and how a unit of it is laid out.  S: MFMA steps of a unit.
 struct WaveDense {       // fp16 [K,N], rows of whole 16-byte chunks
@@ -55,10 +55,12 @@ struct WaveA {           // geometry A
     static constexpr int VEC = 2, CSZ = 1;
 };
 // COPIES: the table holds one codebook of at most 256 entries, each as often as fills a row of the 64 banks (16 copies of
-// an 8-vector, 32 of a 4-vector), and a lane gathers its own copy: no two lanes of a gather meet in a bank.
+// an 8-vector, 32 of a 4-vector), and a lane gathers its own copy: no two lanes of a gather meet in a bank.  16-bit codes: of at
+// most 512 entries, each half as often; two lanes meet where their entries lie in the same half of a row.
 template <int VEC_, typename CodeT_, int S_, bool COPIES_ = false>
 struct WaveB {           // geometry B
     static constexpr bool kCopies = COPIES_;
+    static constexpr int kCopyRow = sizeof(CodeT_) == 1 ? 256 : 128, kCopyEntries = kCopiesBytes / kCopyRow;
     static constexpr int S = S_;
     static constexpr bool kDense = false, kAnyN = false, kA = false, kB = true;
     static constexpr int VEC = VEC_, CSZ = (int)sizeof(CodeT_);
@@ -276,7 +278,8 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
         const int g_first = n0 / a.rows_per_cb;
 #pragma unroll
         for (int j = 0; j < NP; j++)
-            w_rd[j] = P::kCopies ? kBookBase + (uint32_t)(lane * (P::VEC * 2) & 255) : kBookBase + (uint32_t)((min(n0 + j * 16 + r16, N - 1) / a.rows_per_cb - g_first) * a.entries * (P::VEC * 2));
+            if constexpr (P::kCopies) w_rd[j] = kBookBase + (uint32_t)(lane * (P::VEC * 2) & (P::kCopyRow - 1));
+            else w_rd[j] = kBookBase + (uint32_t)((min(n0 + j * 16 + r16, N - 1) / a.rows_per_cb - g_first) * a.entries * (P::VEC * 2));
     }
     const uint32_t code_rd = ring + C::kXBytes + (C::kCodeBytes == 32 ? (kg >> 1) * (C::kRows * 16) + (kg & 1) * 8 : kg * (C::kCodeBytes / 4)) + r16 * 16;
     typedef short short4_t __attribute__((__vector_size__(4 * sizeof(short))));
@@ -336,7 +339,10 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
                 ws[set][2 * q + 1] = __builtin_bit_cast(half8_t, odd);
             }
         } else if constexpr (P::kB) {
-            constexpr int kEntry = P::kCopies ? 256 : P::VEC * 2;   // bytes from entry to entry
+            constexpr int kEntry = []() constexpr {   // bytes from entry to entry
+                if constexpr (P::kCopies) return P::kCopyRow;
+                else return P::VEC * 2;
+            }();
 #pragma unroll
             for (int j = 0; j < NP; j++) {
                 if constexpr (P::VEC == 8) {
@@ -395,19 +401,20 @@ __global__ __launch_bounds__(wave_count<P>(MP, NP) * 64, wave_count<P>(MP, NP) /
         // fewer units it goes last.
         static_assert(P::VEC == 8 || P::VEC == 4, "entries of 16 or 8 bytes");
         typedef uint32_t entry_t __attribute__((ext_vector_type(P::VEC / 2)));
-        const half_t *src = a.cb + ((int64_t)(n0 / a.rows_per_cb) * a.entries + min(tid & (kCopiesEntries - 1), a.entries - 1)) * P::VEC;
+        const half_t *src = a.cb + ((int64_t)(n0 / a.rows_per_cb) * a.entries + min(tid & (P::kCopyEntries - 1), a.entries - 1)) * P::VEC;
         entry_t entry;
         auto load_entry = [&]() {
             if constexpr (P::VEC == 8) asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(entry) : "v"(src) : "memory");
             else asm volatile("global_load_dwordx2 %0, %1, off" : "=&v"(entry) : "v"(src) : "memory");
         };
-        // two threads an entry (four of sixteen waves), eight (four) pieces of 16 bytes each, neighbouring entries in another order
+        // two threads an entry (four of sixteen waves; half of that for 512 entries), four or eight pieces of 16 bytes each, neighbouring entries
+        // in another order
         auto write_copies = [&]() {
             asm volatile("" : "+v"(entry));
-            constexpr int kPer = kWaves * 64 / kCopiesEntries, kPieces = 16 / kPer;
-            static_assert(kPer == 2 || kPer == 4, "threads an entry");
+            constexpr int kPer = kWaves * 64 / P::kCopyEntries, kPieces = P::kCopyRow / 16 / kPer;
+            static_assert(kPer >= 1 && kPer <= 4 && (kPieces == 4 || kPieces == 8), "threads an entry");
             const uint4_t piece = {entry[0], entry[1], entry[P::VEC == 8 ? 2 : 0], entry[P::VEC == 8 ? 3 : 1]};
-            const uint32_t at = kBookBase + (tid & (kCopiesEntries - 1)) * 256 + (tid >> 8) * (kPieces * 16) + (tid & (kPieces - 1)) * 16;
+            const uint32_t at = kBookBase + (tid & (P::kCopyEntries - 1)) * P::kCopyRow + tid / P::kCopyEntries * (kPieces * 16) + (tid & (kPieces - 1)) * 16;
 #pragma unroll
             for (int i = 0; i < kPieces; i++) *reinterpret_cast<uint4_t *>(smem + (at ^ (i * 16))) = piece;
         };

@@ -18,9 +18,11 @@ struct Format {
     // Tiles of up to 32 rows gather more than they read of X: with a table of copies, 64 KB of the LDS that their units leave,
     // the gathers' bank conflicts go, M = 128, K = N = 4096 9.5 -> 9.0 us, M = 16, K = 2048, N = 11008 6.7 -> 6.0, tiles of
     // 32 x 128 14.5 -> 12.0; 32 x 16 gathers too little, equal.  Taller ones read X twice as long as they gather and would keep half the units in flight: 64 x 64
-    // with 32 KB of copies 13.7 -> 15.0.
+    // with 32 KB of copies 13.7 -> 15.0.  16-bit codes of up to 512 entries (two stages of 256) in tiles wider than tall, with half as many
+    // copies: M = 16, K = 4096, N = 11008 7.5 -> 6.8, M = 32, K = 4096, N = 11008 8.5 -> 8.35, tiles of 16 x 64 8.6 -> 7.4, 4-vectors
+    // 2 to 7 %; 16 x 16 and 32 x 32 gather too little (M = 5, K = 8192, N = 4096 7.0 -> 7.5).
     template <int MP, int NP>
-    static constexpr bool kHasCopies = CSZ == 1 && MP <= 2 && NP >= MP;
+    static constexpr bool kHasCopies = MP <= 2 && (CSZ == 1 ? NP >= MP : NP > MP) && WaveKCfg<WaveB<VEC_, CodeT_, Wave<MP, NP>::S, true>, MP, NP>::kExists;
     template <int MP, int NP>
     using Copies = WaveB<VEC_, CodeT_, Wave<MP, NP>::S, true>;
 };
@@ -50,11 +52,15 @@ void with_tile(int tile, F f)
     }
 }
 
-// Whether the tile's kernel with a table of copies serves the problem: 8-bit codes, tiles that meet one codebook.
+// Whether the tile's kernel with a table of copies serves the problem: at most as many entries, tiles that meet one codebook.
 template <class F, int MP, int NP>
 bool takes_copies(const ProblemB &p)
 {
-    return F::template kHasCopies<MP, NP> && codebooks_per_tile(p, NP * 16) == 1;
+    // (16-bit codes, 16 rows: a longer K wants the units that the copies take the room of: M = 16, N = 11008, K = 8192 9.73 -> 9.15, 9216
+    // 10.32 -> 10.27, 10240 12.4 -> 12.9, 16384 16.8 -> 17.4.)
+    if constexpr (F::template kHasCopies<MP, NP>)
+        return codebooks_per_tile(p, NP * 16) == 1 && p.entries <= F::template Copies<MP, NP>::kCopyEntries && (F::CSZ == 1 || MP > 1 || p.K <= 8192);
+    return false;
 }
 
 template <class F>
@@ -108,7 +114,7 @@ WaveKPlan plan_b(const ProblemB &p)
         if (forced > 0 && forced != t.tile) continue;
         if (!fits<F>(p, t.tile) || (p.gated && t.tile % 2 == 1)) continue;
         with_tile(t.tile, [&](auto mp, auto np) {
-            if (!takes_copies<F, mp(), np()>(p)) return;
+            if (F::CSZ == 2 || !takes_copies<F, mp(), np()>(p)) return;   // (16-bit codes: the tile as without copies, a little above its time)
             for (const WaveKTile &c : kCopiesCosts[F::VEC == 8 ? 0 : 1])
                 if (c.tile == t.tile) t = c;
         });
