@@ -2055,23 +2055,24 @@ def test_gemv_kernel_products_of_the_diagonal(K, N, v, E, G, gated):
         assert np.array_equal(_np(yw).view(np.uint16), w[:, [c]].T.copy().view(np.uint16)), c
 
 
-# K, N, codebooks, gated: products on the matrix cores or not, by rows per wave (4096 of them), pieces of a row and codebook boundaries
-@pytest.mark.parametrize("K,N,G,gated", [(2048, 8200, 1, False), (2048, 12289, 1, False), (4096, 4097, 1, False), (4096, 16383, 3, False), (8192, 8193, 1, False),
-                                         (4096, 96, 1, True), (2048, 16416, 1, True), (4096, 24608, 1, True), (8192, 8224, 257, True), (6144, 8192, 8, True),
-                                         (8224, 4096, 1, False), (12288, 4097, 1, False), (16384, 4096, 1, False), (24576, 130, 1, False),
-                                         (26624, 130, 1, False), (11008, 8192, 2, False), (14336, 300, 1, False), (11008, 5003, 1, False), (8192, 10241, 1, False),
-                                         (4096, 1001, 1, False), (6144, 33, 1, False), (8192, 9248, 1, True)])
-def test_gemv_wide_form_products_of_the_diagonal(K, N, G, gated):
-    spec = ProblemSpec("diag", GEOM_B, 1, K, N, 8, 256, G, 8, codebook_3d=(G > 1), codebook_std=0.05)
+# rows of X, K, N, codebooks, gated: products on the matrix cores or not, by rows per wave (4096 of them), pieces of a row and codebook boundaries
+@pytest.mark.parametrize("M,K,N,G,gated", [(1, 2048, 8200, 1, False), (1, 2048, 12289, 1, False), (1, 4096, 4097, 1, False), (1, 4096, 16383, 3, False), (1, 8192, 8193, 1, False),
+                                         (1, 4096, 96, 1, True), (1, 2048, 16416, 1, True), (1, 4096, 24608, 1, True), (1, 8192, 8224, 257, True), (1, 6144, 8192, 8, True),
+                                         (1, 8224, 4096, 1, False), (1, 12288, 4097, 1, False), (1, 16384, 4096, 1, False), (1, 24576, 130, 1, False),
+                                         (1, 26624, 130, 1, False), (1, 11008, 8192, 2, False), (1, 14336, 300, 1, False), (1, 11008, 5003, 1, False), (1, 8192, 10241, 1, False),
+                                         (1, 4096, 1001, 1, False), (1, 6144, 33, 1, False), (1, 8192, 9248, 1, True), (2, 4096, 8193, 1, False), (2, 4096, 24608, 1, True), (2, 2048, 8224, 1, True),
+                                           (2, 11008, 4100, 1, False), (2, 16384, 300, 1, False), (2, 4096, 8192, 2, False), (2, 4096, 28672, 1, False)])
+def test_gemv_wide_form_products_of_the_diagonal(M, K, N, G, gated):
+    spec = ProblemSpec("diag", GEOM_B, M, K, N, 8, 256, G, 8, codebook_3d=(G > 1), codebook_std=0.05)
     x, codes, cb = make_problem(spec, seed=98, device=DEV)
-    _say("gemv diagonal", K, N, G, gated)
+    _say("gemv diagonal", M, K, N, G, gated)
     bias = torch.linspace(-1, 1, N, device=DEV).half()
     if gated:
         y = cabi.e2e_gemm_b_gated(x, codes, cb, bias=bias)
         e1, e2 = vo.rel_err(_np(y), vo.gated_gemm_b(_np(x), _np(codes), _np(cb), _np(bias)).astype(np.float64))
         assert e2 <= TOL and e1 <= 2 * TOL   # (a product of two sums, as in test_gated_epilogue_against_the_oracle)
         return
-    assert cabi.select_variant_b(1, K, N, 8, 256, G, 8) == cabi.VARIANT_DECODE_GEMV
+    assert cabi.select_variant_b(M, K, N, 8, 256, G, 8) == cabi.VARIANT_DECODE_GEMV
     y = cabi.e2e_gemm_b(x, codes, cb, bias=bias)
     w = vo.dequant_b(_np(codes), _np(cb))
     want = _np(x).astype(np.float64) @ w.astype(np.float64).T + _np(bias).astype(np.float64)
@@ -2081,9 +2082,10 @@ def test_gemv_wide_form_products_of_the_diagonal(K, N, G, gated):
     cb[..., 3, :], cb[..., 5, :] = 6e-8, 3e-5
     w = vo.dequant_b(_np(codes), _np(cb))
     for c in (0, 5, K // 2 + 3, K - 1):
-        eye = torch.zeros(1, K, dtype=torch.float16, device=DEV)
-        eye[0, c] = 1.0
-        assert np.array_equal(_np(cabi.e2e_gemm_b(eye, codes, cb)).view(np.uint16), w[:, [c]].T.copy().view(np.uint16)), c
+        eye = torch.zeros(M, K, dtype=torch.float16, device=DEV)
+        cols = [c, (c + 9) % K][:M]
+        eye[torch.arange(M), torch.tensor(cols)] = 1.0
+        assert np.array_equal(_np(cabi.e2e_gemm_b(eye, codes, cb)).view(np.uint16), w[:, cols].T.copy().view(np.uint16)), c
 
 
 @pytest.mark.parametrize("M,K,N,G", [(1, 2080, 48, 1), (2, 2080, 33, 1), (1, 8224, 64, 1), (2, 6176, 4096, 1), (1, 14336, 40, 1), (2, 14336, 2048, 1), (1, 4096, 32, 1)])

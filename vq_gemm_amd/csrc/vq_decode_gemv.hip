@@ -374,9 +374,9 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     // cycles to 165 beside 128 of the matrix pipe; its sum, over the lanes' diagonals, takes one addition more.  Cold, K = 4096: N = 8192
     // 3.75 -> 3.54 us, 16384 4.57 -> 4.40, 28672 5.8 -> 5.53, gated (with the one epilogue at the end) N = 22016 6.13 -> 5.48; K = N = 8192
     // 4.68 -> 4.42.  Not for the chain of a single row, which is as long as its latencies (2.94 -> 2.97; K = 2048, a row at a time, 2.90 ->
-    // 2.93), not with two rows of X (no registers for eight sums more), and not for rows of five pieces (K = 28672, N = 8192 11.2 ->
+    // 2.93), with two rows of X only a row of W at a time (registers), and not for rows of five pieces (K = 28672, N = 8192 11.2 ->
     // 11.6; of three, K = 22016, N = 4096, 7.07 -> 6.55).
-    constexpr bool kDiagonal = XM == 1 && NBUF > 1 && RUNS * G > 1 && !(RUNS == 3 && XRUNS == 16);
+    constexpr bool kDiagonal = NBUF > 1 && (XM == 1 ? RUNS * G > 1 && !(RUNS == 3 && XRUNS == 16) : G == 1);
     constexpr bool LONG = XRUNS != RUNS;
     static_assert(!LONG || (BOOKS < 2 && COPIES == kWideCopies && (NBUF == 2 || ALL)), "the long form: one table, replicated");
     static_assert(NBUF > 1 || G == 1, "a single group per wave: of one row");
@@ -912,9 +912,10 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
     if (const LongK f = long_k_form(p); f.is_long) {
         // (the replicated table, one table per workgroup)
         if (p.M == 2) {
-            auto go = [&](auto group, auto x_runs) { return launch_form(two{}, group, two{}, replicated{}, x_runs, two{}, false_type{}, false_type{}); };
-            if (f.x_runs == 4) return g == 2 ? go(two{}, four{}) : go(one{}, four{});
-            return g == 2 ? go(two{}, eight{}) : go(one{}, eight{});
+            // (a row at a time, the products on the diagonals: two a group, which leave no registers for that, were 1 to 5 % behind, K = 6144 to
+            // 16384, N = 4096 to 11008)
+            auto go = [&](auto x_runs) { return launch_form(two{}, one{}, two{}, replicated{}, x_runs, two{}, false_type{}, false_type{}); };
+            return f.x_runs == 4 ? go(four{}) : go(eight{});
         }
         // Two pairs of a row and a piece (one row in two pieces, one of them a wave's only row): both requested ahead of the barrier (K =
         // 11008, N = 4096 4.74 -> 4.64 us, K = 14336 5.39 -> 5.20).  More of them two in flight: three were measured and are slower,
@@ -937,8 +938,11 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
             return p.K / kRunK == 1 ? go(one{}, group, nbuf, gated) : go(two{}, group, nbuf, gated);
         };
         if (single) return with_runs(one{}, one{}, false_type{});
-        if (p.gated) return g == 2 ? with_runs(two{}, two{}, true_type{}) : with_runs(one{}, two{}, true_type{});
-        return g == 2 ? with_runs(two{}, two{}, false_type{}) : with_runs(one{}, two{}, false_type{});
+        // A row at a time leaves registers for the diagonals of both sums: cold, K = 4096, N = 12288 5.3 -> 5.05 us, 16384 6.0 -> 5.8, K = 2048
+        // gated N = 22016 5.5 -> 5.4; from there on two rows of W a group are ahead (K = 4096, N = 28672 7.8 and 8.1, gated 22016 7.3 and 7.45).
+        const bool singly = g == 1 || (int64_t)(p.gated ? 2 : 1) * rows_per_wave * (p.K / kRunK) <= 8;
+        if (p.gated) return singly ? with_runs(one{}, two{}, true_type{}) : with_runs(two{}, two{}, true_type{});
+        return singly ? with_runs(one{}, two{}, false_type{}) : with_runs(two{}, two{}, false_type{});
     }
     // The plain table while a wave gathers for at most Tuning::gemv_wide_plain_table_max_runs runs of 2048 k (8 gathers per
     // lane and run): measured cold, plain -> replicated, K = 4096: one row per wave 3.29 -> 3.43 us, two rows
