@@ -183,8 +183,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void decode_gemv_kernel(const half
     for (int i = threadIdx.x + kGemvWaves * 64; i < chunks; i += kGemvWaves * 64) table[i] = tsrc[i];
     __syncthreads();
 
-    // Products on the matrix cores' diagonals (see the wide form's kDiagonal) for one row of X and K = 8192 - 4-vectors with 8-bit codes N =
-    // 8192 9.1 -> 6.3 us, N = 4096 5.4 -> 4.9, with 16-bit codes N = 8192 13.2 -> 11.1 - or 16-bit codes from K = 4096 on (N = 4096 5.3 ->
+    // Products on the matrix cores' diagonals (see the wide form's DIAGONAL) for one row of X and K = 8192 - codes out of HBM, 4-vectors
+    // with 8-bit codes N = 16384 18.4 -> 11.2 us, 8192 9.95 -> 7.14, 4096 5.6 -> 5.1, with 16-bit codes N = 8192 15.1 -> 12.75 - or 16-bit codes from K = 4096 on (N = 4096 5.3 ->
     // 5.15, N = 2048 4.5 -> 4.35).  Elsewhere the longer chain costs more than the vector unit gains (4-vectors with 8-bit codes, K = N =
     // 4096 3.45 -> 3.53, K = 6144 4.33 -> 4.5; 512 8-vectors, K = 2048 2.71 -> 2.74).
     constexpr bool kDiagonal = VEC >= 4 && MX == 1 && (RUNS == 4 || (sizeof(CodeT) == 2 && RUNS > 1));
@@ -317,6 +317,14 @@ __device__ __forceinline__ int small_quotient(int x, int d, float rcp)
 // the others (K = 4096, N = 14336 4.22 -> 4.34, K = 2048, N = 1024 2.13 -> 2.27).
 constexpr bool wide_deals_by_units(int runs, int nbuf, int x_runs) { return x_runs != runs || runs > 2 || (runs == 2 && nbuf == 1); }
 
+// The forms that have an instance with the products on the diagonals.  Not the chain of a single row, which is as long as its latencies
+// (K = N = 4096 2.94 -> 2.97 us, K = 2048 a row at a time 2.90 -> 2.93), two rows of X only a row of W at a time (registers), and not rows of
+// five pieces (K = 28672, N = 8192 11.2 -> 11.6; of three, K = 22016, N = 4096, 7.07 -> 6.55).
+constexpr bool wide_has_diagonal(int runs, int group, int nbuf, int x_runs, int x_rows)
+{
+    return nbuf > 1 && (x_rows == 1 ? runs * group > 1 && !(runs == 3 && x_runs == 16) : group == 1);
+}
+
 // BOOKS: 0 = one codebook; 1 = several, no workgroup's rows reach into a second one; 2 = some workgroup's rows
 // do, and every workgroup then fills two tables.  (A compile-time flag, like the unconditional loads below: a
 // load inside a branch makes the compiler's wait counts at the join imprecise, and the table would then
@@ -337,7 +345,12 @@ constexpr bool wide_deals_by_units(int runs, int nbuf, int x_runs) { return x_ru
 // form in pieces of two runs, both rows of x in the LDS (K = 14336, N = 4096: 10.9 -> 8.5 us).
 //
 // GATED: the epilogue of a gate/up pair, once for all of a wave's outputs behind its rows (an output at a time, and asked for at run
-// time in the kernel of every launch, K = 4096: N = 22016 5.9 -> 5.6 us gated; launches without it 0 to 3 % longer).
+// time in the kernel of every launch, K = 4096: N = 22016 5.9 -> 5.6 us gated; launches without it 0 to 3 % longer; codes out of HBM 5.96 -> 5.51 with the diagonals, 28672 7.13 -> 6.49).
+//
+// DIAGONAL: products on the matrix cores (v_mfma_f32_4x4x4_16b_f16) instead of v_dot2_f32_f16: of sixteen 4x4 products by 4 of K, one to four
+// lanes, the diagonal is lane l's four halves of W times its four of x - gathers and registers stay as they are, three quarters of the
+// result are what nobody looks at, and the vector unit issues for 4 cycles where two v_dot2 take 8.5.  What a row of 4096 costs it falls
+// from 250 cycles to 165 beside 128 of the matrix pipe; its sum, over the lanes' diagonals, takes one addition more.
 //
 // ALL (the long form): all of a wave's NBUF pairs of row and piece are requested ahead of the barrier.
 //
@@ -348,7 +361,7 @@ constexpr bool wide_deals_by_units(int runs, int nbuf, int x_runs) { return x_ru
 // and a row's sum so far travels in its lane of `res`: the accumulator of lane 0 starts from it.  x is padded with
 // zeros up to whole pieces, and a load that would reach past the end of a row reads the row's last dword instead: what
 // it gathers meets zeros.  One codebook, or several without a workgroup whose rows reach into two; not gated.
-template <int RUNS, int G, int NBUF, int BOOKS, int COPIES, int XRUNS, int XM, bool GATED, bool ALL>
+template <int RUNS, int G, int NBUF, int BOOKS, int COPIES, int XRUNS, int XM, bool GATED, bool ALL, bool DIAGONAL>
 __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const half_t *__restrict__ x,
                                                                            const uint8_t *__restrict__ codes,
                                                                            const half_t *__restrict__ cb, int entries,
@@ -368,15 +381,6 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     // up row are two groups in turn (G = 1).
     // row_bytes: of codes, K / 8 (read by the long form only).
     constexpr bool TWO = BOOKS == 2;
-    // Products on the matrix cores (v_mfma_f32_4x4x4_16b_f16) instead of v_dot2_f32_f16: of sixteen 4x4 products by 4 of K, one to four lanes,
-    // the diagonal is lane l's four halves of W times its four of x - gathers and registers stay as they are, three quarters of the result
-    // are what nobody looks at, and the vector unit issues for 4 cycles where two v_dot2 take 8.5.  What a row costs it falls from 250
-    // cycles to 165 beside 128 of the matrix pipe; its sum, over the lanes' diagonals, takes one addition more.  Cold, K = 4096: N = 8192
-    // 3.75 -> 3.54 us, 16384 4.57 -> 4.40, 28672 5.8 -> 5.53, gated (with the one epilogue at the end) N = 22016 6.13 -> 5.48; K = N = 8192
-    // 4.68 -> 4.42.  Not for the chain of a single row, which is as long as its latencies (2.94 -> 2.97; K = 2048, a row at a time, 2.90 ->
-    // 2.93), with two rows of X only a row of W at a time (registers), and not for rows of five pieces (K = 28672, N = 8192 11.2 ->
-    // 11.6; of three, K = 22016, N = 4096, 7.07 -> 6.55).
-    constexpr bool kDiagonal = NBUF > 1 && (XM == 1 ? RUNS * G > 1 && !(RUNS == 3 && XRUNS == 16) : G == 1);
     constexpr bool LONG = XRUNS != RUNS;
     static_assert(!LONG || (BOOKS < 2 && COPIES == kWideCopies && (NBUF == 2 || ALL)), "the long form: one table, replicated");
     static_assert(NBUF > 1 || G == 1, "a single group per wave: of one row");
@@ -552,7 +556,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
     // rows [g*G, g*G + R) of the wave, R <= G (a compile-time count: the last group may be short)
     auto multiply_rows = [&](int g, const uint32_t (&cur)[G][RUNS], auto r_const) {
         constexpr int R = decltype(r_const)::value;
-        std::conditional_t<kDiagonal, float4_t, float> acc[XM][R];
+        std::conditional_t<DIAGONAL, float4_t, float> acc[XM][R];
         uint32_t base[R];
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -563,7 +567,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
 #pragma unroll
                 for (int m = 0; m < XM; m++) {
                     const float so_far = lane == 0 ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, res[m]), g * G + r)) : 0.f;
-                    if constexpr (kDiagonal) acc[m][r][0] = so_far;
+                    if constexpr (DIAGONAL) acc[m][r][0] = so_far;
                     else acc[m][r] = so_far;
                 }
             }
@@ -593,7 +597,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
 #pragma unroll
                         for (int m = 0; m < XM; m++) {
                             const uint2_t wd = {w[r][c][d], w[r][c][d + 1]}, xd = {xr[m][q][c][d], xr[m][q][c][d + 1]};
-                            if constexpr (kDiagonal) {
+                            if constexpr (DIAGONAL) {
                                 acc[m][r] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, wd), __builtin_bit_cast(half4_t, xd), acc[m][r], 0, 0, 0);
                             } else {
                                 const uint32_t w0 = wd[0], w1 = wd[1], x0 = xd[0], x1 = xd[1];
@@ -603,7 +607,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void decode_gemv_wide_kernel(const
                         }
         }
         auto total = [](auto v) {
-            if constexpr (kDiagonal) return diagonal_sum_to_uniform(v);
+            if constexpr (DIAGONAL) return diagonal_sum_to_uniform(v);
             else return wave_sum_to_uniform(v);
         };
         auto keep = [&](float &where, float s, int i) {
@@ -895,18 +899,33 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
     using sixteen = integral_constant<int, 16>;
     const int g = wide_rows_per_group(p), rows_per_wave = (n_dealt + waves - 1) / waves;
     // the plain or the replicated table, and how many of them
-    auto launch_form = [&](auto runs, auto group, auto nbuf, auto copies, auto x_runs, auto x_rows, auto gated, auto all) {
+    auto launch_with = [&](auto runs, auto group, auto nbuf, auto copies, auto x_runs, auto x_rows, auto gated, auto all, auto diagonal) {
         auto launch = [&](auto kern) { return launch_dealt(kern, wide_deals_by_units(runs(), nbuf(), x_runs())); };
         if constexpr (!gated() && x_runs() != runs())
-            return books == 0 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), false, all()>)
-                              : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 1, copies(), x_runs(), x_rows(), false, all()>);
+            return books == 0 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), false, all(), diagonal()>)
+                              : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 1, copies(), x_runs(), x_rows(), false, all(), diagonal()>);
         else if constexpr (gated())   // (a codebook boundary may lie anywhere)
-            return books == 0 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), true, all()>)
-                              : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 2, copies(), x_runs(), x_rows(), true, all()>);
+            return books == 0 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), true, all(), diagonal()>)
+                              : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 2, copies(), x_runs(), x_rows(), true, all(), diagonal()>);
         else
-            return books == 0   ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), false, all()>)
-                   : books == 1 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 1, copies(), x_runs(), x_rows(), false, all()>)
-                                : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 2, copies(), x_runs(), x_rows(), false, all()>);
+            return books == 0   ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 0, copies(), x_runs(), x_rows(), false, all(), diagonal()>)
+                   : books == 1 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 1, copies(), x_runs(), x_rows(), false, all(), diagonal()>)
+                                : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 2, copies(), x_runs(), x_rows(), false, all(), diagonal()>);
+    };
+    // The products on the diagonals up to eleven runs of 2048 k a wave (v_dot2 beyond): codes out of HBM, K = 4096, N = 8192 3.42 -> 3.34 us,
+    // 12288 in three codebooks 4.16 -> 3.90, 20480 (10 runs) 5.18 -> 5.08, K = N = 8192 4.54 -> 4.46; but K = 4096, N = 28672 (14) 6.24 ->
+    // 6.53, 65536 11.9 -> 12.3, K = 6144, N = 16384 (12) 5.85 -> 5.92, K = 8192, N = 12288 (12) 5.98 -> 6.74, K = 14336, N = 16384 (28) 12.0 ->
+    // 12.5, although out of the caches they gain there too (5.89 -> 5.70, 5.49 -> 5.35, 5.51 -> 5.46).
+    const bool diagonals = (double)p.N * (double)((p.K + kRunK - 1) / kRunK) <= 11.0 * (double)waves;
+    auto launch_form = [&](auto runs, auto group, auto nbuf, auto copies, auto x_runs, auto x_rows, auto gated, auto all) {
+        constexpr bool has = wide_has_diagonal(runs(), group(), nbuf(), x_runs(), x_rows());
+        // (forms that only launches of few runs take)
+        constexpr bool always = has && (copies() == 1 || all() || (x_rows() == 2 && x_runs() == runs()));
+        if constexpr (always) return launch_with(runs, group, nbuf, copies, x_runs, x_rows, gated, all, true_type{});
+        else if constexpr (has)
+            return diagonals ? launch_with(runs, group, nbuf, copies, x_runs, x_rows, gated, all, true_type{})
+                             : launch_with(runs, group, nbuf, copies, x_runs, x_rows, gated, all, false_type{});
+        else return launch_with(runs, group, nbuf, copies, x_runs, x_rows, gated, all, false_type{});
     };
     using replicated = integral_constant<int, kWideCopies>;
     if (const LongK f = long_k_form(p); f.is_long) {
@@ -938,7 +957,7 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
             return p.K / kRunK == 1 ? go(one{}, group, nbuf, gated) : go(two{}, group, nbuf, gated);
         };
         if (single) return with_runs(one{}, one{}, false_type{});
-        // A row at a time leaves registers for the diagonals of both sums: cold, K = 4096, N = 12288 5.3 -> 5.05 us, 16384 6.0 -> 5.8, K = 2048
+        // A row at a time leaves registers for the diagonals of both sums: codes out of the Infinity Cache, K = 4096, N = 12288 5.3 -> 5.05 us, 16384 6.0 -> 5.8, K = 2048
         // gated N = 22016 5.5 -> 5.4; from there on two rows of W a group are ahead (K = 4096, N = 28672 7.8 and 8.1, gated 22016 7.3 and 7.45).
         const bool singly = g == 1 || (int64_t)(p.gated ? 2 : 1) * rows_per_wave * (p.K / kRunK) <= 8;
         if (p.gated) return singly ? with_runs(one{}, two{}, true_type{}) : with_runs(two{}, two{}, true_type{});
