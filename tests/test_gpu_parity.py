@@ -2062,9 +2062,9 @@ def test_gemv_kernel_products_of_the_diagonal(K, N, v, E, G, gated):
                                          (1, 26624, 130, 1, False), (1, 11008, 8192, 2, False), (1, 14336, 300, 1, False), (1, 11008, 5003, 1, False), (1, 8192, 10241, 1, False),
                                          (1, 4096, 1001, 1, False), (1, 6144, 33, 1, False), (1, 8192, 9248, 1, True), (2, 4096, 8193, 1, False), (2, 4096, 24608, 1, True), (2, 2048, 8224, 1, True),
                                            (2, 11008, 4100, 1, False), (2, 16384, 300, 1, False), (2, 4096, 8192, 2, False), (2, 4096, 28672, 1, False),
-                                           # (eleven runs a wave and hardly more)
-                                           (1, 4096, 22528, 1, False), (1, 4096, 22529, 1, False), (1, 4096, 22560, 3, True), (1, 8192, 11272, 2, False),
-                                           (1, 6144, 15032, 1, False), (1, 11008, 7512, 1, False), (2, 8192, 11265, 1, False)])
+                                           # (ten runs a wave and hardly more; six with two rows of X)
+                                           (1, 4096, 20480, 1, False), (1, 4096, 20481, 1, False), (1, 4096, 20544, 3, True), (1, 8192, 10248, 2, False),
+                                           (1, 6144, 13672, 1, False), (1, 11008, 6840, 1, False), (2, 8192, 10241, 1, False), (2, 4096, 12289, 1, False)])
 def test_gemv_wide_form_products_of_the_diagonal(M, K, N, G, gated):
     spec = ProblemSpec("diag", GEOM_B, M, K, N, 8, 256, G, 8, codebook_3d=(G > 1), codebook_std=0.05)
     x, codes, cb = make_problem(spec, seed=98, device=DEV)

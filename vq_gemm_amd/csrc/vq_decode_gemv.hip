@@ -184,9 +184,9 @@ __global__ __launch_bounds__(kGemvWaves * 64) void decode_gemv_kernel(const half
     __syncthreads();
 
     // Products on the matrix cores' diagonals (see the wide form's DIAGONAL) for one row of X and K = 8192 - codes out of HBM, 4-vectors
-    // with 8-bit codes N = 16384 18.4 -> 11.2 us, 8192 9.95 -> 7.14, 4096 5.6 -> 5.1, with 16-bit codes N = 8192 15.1 -> 12.75 - or 16-bit codes from K = 4096 on (N = 4096 5.3 ->
-    // 5.15, N = 2048 4.5 -> 4.35).  Elsewhere the longer chain costs more than the vector unit gains (4-vectors with 8-bit codes, K = N =
-    // 4096 3.45 -> 3.53, K = 6144 4.33 -> 4.5; 512 8-vectors, K = 2048 2.71 -> 2.74).
+    // with 8-bit codes N = 16384 18.4 -> 11.2 us, 8192 9.95 -> 7.14, 4096 5.6 -> 5.1, with 16-bit codes N = 8192 15.1 -> 12.75 - or 16-bit
+    // codes from K = 4096 on (N = 4096 5.3 -> 5.15, N = 2048 4.5 -> 4.35).  Elsewhere the longer chain costs more than the vector unit
+    // gains (4-vectors with 8-bit codes, K = N = 4096 3.45 -> 3.53, K = 6144 4.33 -> 4.5; 512 8-vectors, K = 2048 2.71 -> 2.74).
     constexpr bool kDiagonal = VEC >= 4 && MX == 1 && (RUNS == 4 || (sizeof(CodeT) == 2 && RUNS > 1));
     std::conditional_t<kDiagonal, float4_t, float> acc[MX][kGemvRows];
 #pragma unroll
@@ -345,7 +345,8 @@ constexpr bool wide_has_diagonal(int runs, int group, int nbuf, int x_runs, int 
 // form in pieces of two runs, both rows of x in the LDS (K = 14336, N = 4096: 10.9 -> 8.5 us).
 //
 // GATED: the epilogue of a gate/up pair, once for all of a wave's outputs behind its rows (an output at a time, and asked for at run
-// time in the kernel of every launch, K = 4096: N = 22016 5.9 -> 5.6 us gated; launches without it 0 to 3 % longer; codes out of HBM 5.96 -> 5.51 with the diagonals, 28672 7.13 -> 6.49).
+// time in the kernel of every launch, K = 4096: N = 22016 5.9 -> 5.6 us gated; launches
+// without it 0 to 3 % longer; codes out of HBM 5.95 -> 5.57, 28672 7.13 -> 6.49).
 //
 // DIAGONAL: products on the matrix cores (v_mfma_f32_4x4x4_16b_f16) instead of v_dot2_f32_f16: of sixteen 4x4 products by 4 of K, one to four
 // lanes, the diagonal is lane l's four halves of W times its four of x - gathers and registers stay as they are, three quarters of the
@@ -912,11 +913,12 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
                    : books == 1 ? launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 1, copies(), x_runs(), x_rows(), false, all(), diagonal()>)
                                 : launch(decode_gemv_wide_kernel<runs(), group(), nbuf(), 2, copies(), x_runs(), x_rows(), false, all(), diagonal()>);
     };
-    // The products on the diagonals up to eleven runs of 2048 k a wave (v_dot2 beyond): codes out of HBM, K = 4096, N = 8192 3.42 -> 3.34 us,
+    // The products on the diagonals up to ten runs of 2048 k a wave (v_dot2 beyond): codes out of HBM, K = 4096, N = 8192 3.42 -> 3.34 us,
     // 12288 in three codebooks 4.16 -> 3.90, 20480 (10 runs) 5.18 -> 5.08, K = N = 8192 4.54 -> 4.46; but K = 4096, N = 28672 (14) 6.24 ->
     // 6.53, 65536 11.9 -> 12.3, K = 6144, N = 16384 (12) 5.85 -> 5.92, K = 8192, N = 12288 (12) 5.98 -> 6.74, K = 14336, N = 16384 (28) 12.0 ->
-    // 12.5, although out of the caches they gain there too (5.89 -> 5.70, 5.49 -> 5.35, 5.51 -> 5.46).
-    const bool diagonals = (double)p.N * (double)((p.K + kRunK - 1) / kRunK) <= 11.0 * (double)waves;
+    // 12.5, although out of the caches they gain there too (5.89 -> 5.70, 5.49 -> 5.35, 5.51 -> 5.46); between (gated K = 4096, N =
+    // 22016, 10.75) they are level, 5.57 and 5.55, or behind, by device.
+    const bool diagonals = (double)p.N * (double)((p.K + kRunK - 1) / kRunK) <= 10.0 * (double)waves;
     auto launch_form = [&](auto runs, auto group, auto nbuf, auto copies, auto x_runs, auto x_rows, auto gated, auto all) {
         constexpr bool has = wide_has_diagonal(runs(), group(), nbuf(), x_runs(), x_rows());
         // (forms that only launches of few runs take)
@@ -957,9 +959,9 @@ hipError_t launch_decode_gemv_wide(const ProblemB &p, hipStream_t s)
             return p.K / kRunK == 1 ? go(one{}, group, nbuf, gated) : go(two{}, group, nbuf, gated);
         };
         if (single) return with_runs(one{}, one{}, false_type{});
-        // A row at a time leaves registers for the diagonals of both sums: codes out of the Infinity Cache, K = 4096, N = 12288 5.3 -> 5.05 us, 16384 6.0 -> 5.8, K = 2048
-        // gated N = 22016 5.5 -> 5.4; from there on two rows of W a group are ahead (K = 4096, N = 28672 7.8 and 8.1, gated 22016 7.3 and 7.45).
-        const bool singly = g == 1 || (int64_t)(p.gated ? 2 : 1) * rows_per_wave * (p.K / kRunK) <= 8;
+        // A row at a time leaves registers for the diagonals of both sums: codes out of HBM, K = 4096, N = 12288 (6 runs a wave) 5.17 -> 4.97 us, 8192
+        // 4.18 -> 3.97.  From there on two rows of W a group, with v_dot2, are ahead (N = 16384 5.60 and 5.81, 28672 8.3 and 8.6).
+        const bool singly = g == 1 || (int64_t)(p.gated ? 2 : 1) * rows_per_wave * (p.K / kRunK) <= 6;
         if (p.gated) return singly ? with_runs(one{}, two{}, true_type{}) : with_runs(two{}, two{}, true_type{});
         return singly ? with_runs(one{}, two{}, false_type{}) : with_runs(two{}, two{}, false_type{});
     }
